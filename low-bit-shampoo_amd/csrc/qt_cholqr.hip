@@ -41,14 +41,9 @@ constexpr int kSolvePanel = 256;       // diagonal blocks of the factor are inve
 // `set_aside`, if not null: the columns taken out are reported there (bit k of set_aside[b * aside_stride]) instead of in info, and
 // their columns of `inv` are zero, so that Q inv has zero columns in their place for the caller to fill.
 //
-// Lane i of every wave stands for row i of the (full, symmetric) trailing matrix; wave w keeps the columns 16 w ..
-// 16 w + 15 of that row in registers, and the same columns of the right-hand side e_i of the forward substitution,
-// which ends as column i of L^-1 (L = U^T), so the inverse costs no second pass.  A right-looking factorisation in
-// four blocks of sixteen columns: the wave that owns a block factors it alone (1 / sqrt(pivot) from v_rsq_f32 plus one
-// Newton step; a[i][j] -= L[i][k] L[j][k], s[j] -= L[j][k] x[k] for its own columns j behind k), the waves behind it
-// apply the block's sixteen steps to their columns from the copy in LDS.  (With one wave per matrix and all 64 columns
-// in a lane's registers a step costs twice 64 - k multiply-adds per lane and the kernel 25-29 us; a barrier per step
-// between four waves costs as much in waiting.)
+// A right-looking factorisation L L^T (L = U^T) of blocks of sixteen columns, the matrix in LDS, with the inverse beside it
+// (factor64 below): the wave that owns a block of columns takes them into registers, lane i standing for row i, and
+// factors them alone; the blocks behind it and the inverse are products of 16 x 16 blocks on the fp32 matrix instruction.
 //
 // SCALED: `gram` is the Gram matrix S = P^T P of a panel whose columns are not of unit length yet.  The kernel factors
 // D^-1 S D^-1 (D = the column lengths, from the diagonal of S) and `inv` receives D^-1 U^-1, so that P inv is the
@@ -57,11 +52,179 @@ constexpr int kSolvePanel = 256;       // diagonal blocks of the factor are inve
 // unit column is rounding noise; a NaN counts) is set aside like a dropped one -- it takes no part in the
 // factorisation, its column of inv is zero, its bit of set_aside is set -- whatever aside_pivots says; aside_pivots
 // == 0 keeps the columns dropped for their pivot where they are (bit 1 of info) and reports only the short ones.
-constexpr int LDC = NB + 4;                      // LDS row stride: rows stay 16-byte aligned
+constexpr int LDC = NB + 4;                      // LDS row stride: 16-byte reads of one column by 64 rows meet no bank twice
 constexpr int kCholWaves = 4, kCholCols = NB / kCholWaves;
+typedef float qt_acc4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float lane_value(float x, int lane) {
     return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), lane));
+}
+
+// acc += sign A B for 16 x 16 blocks in LDS: A row by row (16-byte reads), B either the transpose of such a block
+// (B_TURNED: B[k][n] = b[n][k]) or as it lies.  v_mfma_f32_16x16x4f32: lane l supplies row (A) or column (B) l % 16 and
+// k = 4 (l / 16) + t in step t, and holds column l % 16 of rows 4 (l / 16) .. + 3 of the result.
+template <bool B_TURNED>
+__device__ __forceinline__ qt_acc4 block_product(const float *a, const float *b, float sign, qt_acc4 acc) {
+    const int lane = threadIdx.x & 63, at = lane & 15, g = (lane >> 4) * 4;
+    const float4 av = *reinterpret_cast<const float4 *>(a + at * LDC + g);
+    float bv[4];
+    if (B_TURNED) {
+        const float4 v = *reinterpret_cast<const float4 *>(b + at * LDC + g);
+        bv[0] = v.x; bv[1] = v.y; bv[2] = v.z; bv[3] = v.w;
+    } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) bv[t] = b[(g + t) * LDC + at];
+    }
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sign * av.x, bv[0], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sign * av.y, bv[1], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sign * av.z, bv[2], acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(sign * av.w, bv[3], acc, 0, 0, 0);
+}
+__device__ __forceinline__ qt_acc4 block_load(const float *c) {
+    const int lane = threadIdx.x & 63, at = lane & 15, g = (lane >> 4) * 4;
+    qt_acc4 acc;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = c[(g + r) * LDC + at];
+    return acc;
+}
+__device__ __forceinline__ void block_store(float *c, qt_acc4 acc) {
+    const int lane = threadIdx.x & 63, at = lane & 15, g = (lane >> 4) * 4;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c[(g + r) * LDC + at] = acc[r];
+}
+
+// What became of the pivots of a factorisation (the same in every thread).
+struct PivotOutcome {
+    unsigned long long dropped;          // columns taken out (pivot at or below the floor)
+    int failed;                          // a pivot that is not a number, or not positive with a floor of zero
+};
+struct PivotNotes {                      // (LDS) one slot per wave
+    unsigned long long dropped[kCholWaves];
+    int failed[kCholWaves];
+};
+
+// `a` (64 rows, LDC floats apart): the lower triangle of a symmetric matrix on entry, L on exit (above the diagonal
+// blocks: undefined).  `y`: L^-1 on exit, zeros above its diagonal.  All 256 threads of a workgroup; a barrier
+// before the call makes `a` visible, the last thing the call does is one as well.
+// What bounds it is the chain of the 64 pivots (about 250 cycles each: the pivot through v_readlane, v_rsq_f32 and one
+// Newton step, the column, the next pivot, with the multiply-adds of the step before in its shadow).  A launch takes
+// 13.2 us for one matrix and 14.6 for 99; with the trailing updates and the substitution for the inverse as vector
+// multiply-adds of the waves behind (300 cycles a step on top of 300 for the pivot) it took 18.9 and 21.7.
+__device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes &notes, float pivot_floor) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    {
+        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int i = threadIdx.x; i < NB * (NB / 4); i += NB * kCholWaves)
+            *reinterpret_cast<float4 *>(y + (i / (NB / 4)) * LDC + 4 * (i % (NB / 4))) = zero;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int p = 0; p < kCholWaves; ++p) {
+        const int c0 = p * kCholCols;
+        if (wave == p) {                         // (uniform over the wave)
+            float row[kCholCols], s[kCholCols];  // columns c0 .. c0 + 15 of row `lane`; the same columns of the right-hand side e_lane of L x = e
+#pragma unroll
+            for (int q = 0; q < kCholCols; q += 4) {
+                const float4 v = *reinterpret_cast<const float4 *>(a + lane * LDC + c0 + q);
+                row[q] = v.x; row[q + 1] = v.y; row[q + 2] = v.z; row[q + 3] = v.w;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[q + e] = lane == c0 + q + e ? 1.0f : 0.0f;
+            }
+            // Step kk works on the chain of its own pivot -- v_readlane, v_rsq_f32, one Newton step, the column of L -- and, in
+            // the shadow of those dependent instructions, subtracts the step before from the columns behind kk (column kk
+            // itself had that done at once).  The scheduling barriers keep the compiler from putting those updates off
+            // for good, which costs it the scalar registers.  A pivot that is not above the floor is replaced and its
+            // column of L cleared by selects (no branch on a value that comes out of a vector compare).
+            const float instead = pivot_floor > 0.0f ? pivot_floor : 1.0f, root = pivot_floor > 0.0f ? sqrtf(pivot_floor) : 1.0f;
+            float own = 0.0f, l_before = 0.0f, x_before = 0.0f;                // own: the pivot of column `lane`, before it is replaced
+#pragma unroll
+            for (int kk = 0; kk < kCholCols; ++kk) {
+                const bool here = lane == c0 + kk;
+                own = here ? row[kk] : own;
+                float d = lane_value(row[kk], c0 + kk), v[kCholCols];
+                const bool fine = d > pivot_floor;
+                d = fine ? d : instead;
+                float r = __builtin_amdgcn_rsqf(d);
+                const float alone = here ? root : 0.0f, half_d = -0.5f * d;
+#pragma unroll
+                for (int jj = kk + 1; jj < kCholCols; ++jj) v[jj] = kk > 0 ? lane_value(l_before, c0 + jj) : 0.0f;   // L[j][k - 1]
+                __builtin_amdgcn_sched_barrier(0);
+                r = r * __builtin_fmaf(half_d * r, r, 1.5f);
+                const float l = fine ? row[kk] * r : alone;                // L[lane][k] (lanes above k: unused values)
+                row[kk] = l;                                               // (replaced pivot: nothing below the diagonal)
+                s[kk] *= r;                                                // x[k] = s[k] / L[k][k]
+                if (kk > 0) {
+#pragma unroll
+                    for (int jj = kk + 1; jj < kCholCols; ++jj) {
+                        row[jj] = __builtin_fmaf(-l_before, v[jj], row[jj]);
+                        s[jj] = __builtin_fmaf(-v[jj], x_before, s[jj]);
+                    }
+                }
+                if (kk + 1 < kCholCols) {
+                    const float next = lane_value(l, c0 + kk + 1);
+                    row[kk + 1] = __builtin_fmaf(-l, next, row[kk + 1]);
+                    s[kk + 1] = __builtin_fmaf(-next, s[kk], s[kk + 1]);
+                }
+                l_before = l;
+                x_before = s[kk];
+#pragma unroll
+                for (int jj = kk + 1; jj < kCholCols; ++jj) asm volatile("" : "+v"(s[jj]));   // (now, not at the end)
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const bool mine = (lane >> 4) == p;
+            const unsigned long long replaced = __ballot(mine && !(own > pivot_floor)), not_a_number = __ballot(mine && own != own);
+#pragma unroll
+            for (int q = 0; q < kCholCols; q += 4)
+                *reinterpret_cast<float4 *>(a + lane * LDC + c0 + q) = make_float4(row[q], row[q + 1], row[q + 2], row[q + 3]);
+            if (mine) {
+#pragma unroll
+                for (int jj = 0; jj < kCholCols; ++jj) y[(c0 + jj) * LDC + lane] = s[jj];     // L_pp^-1 (zero above its diagonal)
+            }
+            if (lane == 0) {
+                notes.dropped[p] = pivot_floor > 0.0f ? replaced & ~not_a_number : 0ull;
+                notes.failed[p] = (pivot_floor > 0.0f ? not_a_number : replaced) != 0 ? 1 : 0;
+            }
+        }
+        __syncthreads();
+        // the blocks behind: A_ij -= L_ip L_jp^T for i >= j > p, dealt out over the waves
+        const int rest = kCholWaves - 1 - p, count = rest * (rest + 1) / 2;
+        for (int q = wave; q < count; q += kCholWaves) {
+            int i = p + 1, left = q;
+            while (left > i - p - 1) { left -= i - p; ++i; }
+            const int j = p + 1 + left;
+            float *c = a + 16 * i * LDC + 16 * j;
+            block_store(c, block_product<true>(a + 16 * i * LDC + c0, a + 16 * j * LDC + c0, -1.0f, block_load(c)));
+        }
+        __syncthreads();
+    }
+    // The inverse below its diagonal blocks, by halves: Y_10 = -Y_11 (L_10 Y_00) and Y_32 likewise, then the lower left
+    // 32 x 32 from the two 32 x 32 inverses.  The strict upper triangle of `a` holds the inner products.
+    const qt_acc4 none = {0.f, 0.f, 0.f, 0.f};
+    if (wave < 2) {
+        const int i = 2 * wave + 1, j = 2 * wave;
+        float *inner = a + 16 * j * LDC + 16 * i;
+        block_store(inner, block_product<false>(a + 16 * i * LDC + 16 * j, y + 16 * j * LDC + 16 * j, 1.0f, none));
+        wave_lds_sync();
+        block_store(y + 16 * i * LDC + 16 * j, block_product<false>(y + 16 * i * LDC + 16 * i, inner, -1.0f, none));
+    }
+    __syncthreads();
+    const int bi = 2 + (wave >> 1), bj = wave & 1;               // this wave's block of the lower left half
+    {
+        qt_acc4 m = none;                                        // M = L_BA Y_A
+        for (int k = bj; k < 2; ++k) m = block_product<false>(a + 16 * bi * LDC + 16 * k, y + 16 * k * LDC + 16 * bj, 1.0f, m);
+        block_store(a + 16 * bj * LDC + 16 * bi, m);
+    }
+    __syncthreads();
+    {
+        qt_acc4 m = none;                                        // Y_BA = -Y_B M
+        for (int k = 2; k <= bi; ++k) m = block_product<false>(y + 16 * bi * LDC + 16 * k, a + 16 * bj * LDC + 16 * k, -1.0f, m);
+        block_store(y + 16 * bi * LDC + 16 * bj, m);
+    }
+    PivotOutcome out = {0, 0};
+#pragma unroll
+    for (int w = 0; w < kCholWaves; ++w) { out.dropped |= notes.dropped[w]; out.failed |= notes.failed[w]; }
+    __syncthreads();
+    return out;
 }
 
 template <bool SCALED>
@@ -70,22 +233,25 @@ __global__ __launch_bounds__(NB * kCholWaves) void cholesky64_kernel(const float
                                                                      int ldi, float *panel_inv, int *info, float pivot_floor,
                                                                      unsigned long long *set_aside, int aside_stride,
                                                                      float too_short, int stand_in, int aside_pivots) {
-    __shared__ __attribute__((aligned(16))) float cols[NB][LDC];
-    __shared__ __attribute__((aligned(16))) float handed[NB][2][NB];      // [k][column k of L | x[k] of every row][row]
+    __shared__ __attribute__((aligned(16))) float a[NB * LDC], y[NB * LDC];
     __shared__ float lengths[NB];
-    __shared__ unsigned long long s_dropped[kCholWaves];
-    __shared__ int s_failed[kCholWaves];
+    __shared__ PivotNotes notes;
     const int b = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c0 = wave * kCholCols;
     const float *G = gram + (long long)b * g_stride;
-    for (int r = wave; r < NB; r += kCholWaves) cols[r][lane] = G[(long long)r * ldg + lane];
-    __syncthreads();
-    float row[kCholCols];                        // columns c0 .. c0 + 15 of row `lane` of the symmetric matrix; end as L[lane][c0 ..]
-    float s[kCholCols];                          // the same columns of the right-hand side e_lane; end as L^-1[c0 ..][lane]
+    float in[NB / kCholWaves];                   // rows wave, wave + 4, ... of column `lane` (all loads in flight at once)
+#pragma unroll
+    for (int i = 0; i < NB / kCholWaves; ++i) in[i] = G[(long long)(wave + kCholWaves * i) * ldg + lane];
     float own_scale = 1.0f;                      // SCALED: 1 / length of column `lane` (0 for a column set aside or of length 0)
     unsigned long long early = 0;                // SCALED: the columns set aside for their length (uniform over the workgroup)
     bool shrunk = false;                         // SCALED: a column kept although the projections left little of it
     if constexpr (SCALED) {
-        const float norm2 = cols[lane][lane];
+        if (lane % kCholWaves == wave) {
+#pragma unroll
+            for (int i = 0; i < NB / kCholWaves; ++i)
+                if (wave + kCholWaves * i == lane) lengths[lane] = in[i];
+        }
+        __syncthreads();
+        const float norm2 = lengths[lane];
         const bool aside = stand_in != 0 && !(norm2 >= too_short);
         own_scale = 0.0f;
         if (!aside) {
@@ -103,86 +269,29 @@ __global__ __launch_bounds__(NB * kCholWaves) void cholesky64_kernel(const float
         // (A column that depends on the ones before it gets here when an earlier pass could not tell: next to an
         // ill-conditioned panel that one Cholesky QR round had not made orthonormal yet.)
         shrunk = stand_in == 0 && __ballot(!(norm2 >= too_short)) != 0;
-        if (wave == 0) lengths[lane] = own_scale;
-        __syncthreads();
     }
+    // the upper triangle of the input turned into the lower one of `a`
 #pragma unroll
-    for (int jj = 0; jj < kCholCols; ++jj) {
-        const int j = c0 + jj;
-        row[jj] = j >= lane ? cols[lane][j] : cols[j][lane];
+    for (int i = 0; i < NB / kCholWaves; ++i) {
+        const int r = wave + kCholWaves * i;
+        float v = in[i];
         if constexpr (SCALED) {
-            const bool out = ((early >> j) & 1ull) || ((early >> lane) & 1ull);
-            row[jj] = out ? (j == lane ? 1.0f : 0.0f) : row[jj] * own_scale * lengths[j];
+            const bool out = ((early >> r) & 1ull) || ((early >> lane) & 1ull);
+            v = out ? (r == lane ? 1.0f : 0.0f) : v * lane_value(own_scale, r) * own_scale;
         }
-        s[jj] = j == lane ? 1.0f : 0.0f;
+        if (r <= lane) a[lane * LDC + r] = v;
     }
-    bool ok = true;
-    uint32_t taken_out = 0;                      // which of its sixteen columns this wave took out of the factorisation (uniform over the wave)
-    // Four phases.  In phase p wave p factors its sixteen columns on its own -- step k: pivot, column k of L, then its
-    // columns behind k at once, their L[j][k] through v_readlane -- and leaves every column of L, with the
-    // substitution's x[k] of every row, in LDS; behind the barrier the waves after it bring their columns up to date
-    // with those sixteen steps (the same multiply-adds in the same order as step by step), and the next one goes on.
+    PivotOutcome pivots = factor64(a, y, notes, pivot_floor);                      // (begins with a barrier)
+    unsigned long long dropped = pivots.dropped;
+    float s[kCholCols];                          // row `lane` of U^-1, columns c0 ..: U^-1[lane][c] = L^-1[c][lane]
 #pragma unroll
-    for (int p = 0; p < kCholWaves; ++p) {
-        if (wave == p) {                         // (uniform over the wave)
-#pragma unroll
-            for (int kk = 0; kk < kCholCols; ++kk) {
-                const int k = p * kCholCols + kk;
-                float d = lane_value(row[kk], k);
-                bool drop = false;
-                if (!(d > pivot_floor)) {
-                    if (pivot_floor > 0.0f && d == d) { drop = true; taken_out |= 1u << kk; d = pivot_floor; }
-                    else { ok = false; d = 1.0f; }
-                }
-                float r = __builtin_amdgcn_rsqf(d);
-                r = r * __builtin_fmaf(-0.5f * d * r, r, 1.5f);
-                float l = row[kk] * r;           // L[lane][k] (lanes above k: unused values)
-                if (drop) l = lane == k ? d * r : 0.0f;   // sqrt(floor) on the diagonal, nothing below it
-                row[kk] = l;
-                s[kk] *= r;                      // x[k] = s[k] / L[k][k]
-                const float xk = s[kk];
-                handed[k][0][lane] = l;
-                handed[k][1][lane] = xk;
-#pragma unroll
-                for (int jj = kk + 1; jj < kCholCols; ++jj) {
-                    const float v = lane_value(l, p * kCholCols + jj);     // L[j][k]
-                    row[jj] = __builtin_fmaf(-l, v, row[jj]);
-                    s[jj] = __builtin_fmaf(-v, xk, s[jj]);
-                }
-            }
-        }
-        if (p + 1 == kCholWaves) break;
-        __syncthreads();
-        if (wave > p) {
-#pragma unroll
-            for (int kk = 0; kk < kCholCols; ++kk) {
-                const int k = p * kCholCols + kk;
-                const float l = handed[k][0][lane], xk = handed[k][1][lane];
-#pragma unroll
-                for (int q = 0; q < kCholCols; q += 4) {
-                    const float4 v4 = *reinterpret_cast<const float4 *>(&handed[k][0][c0 + q]);     // L[j][k] for four columns j
-                    const float v[4] = {v4.x, v4.y, v4.z, v4.w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        row[q + e] = __builtin_fmaf(-l, v[e], row[q + e]);
-                        s[q + e] = __builtin_fmaf(-v[e], xk, s[q + e]);
-                    }
-                }
-            }
-        }
-    }
-    if (lane == 0) { s_dropped[wave] = (unsigned long long)taken_out << c0; s_failed[wave] = ok ? 0 : 1; }
-    __syncthreads();
-    unsigned long long dropped = 0;
-    int failed = 0;
-#pragma unroll
-    for (int w = 0; w < kCholWaves; ++w) { dropped |= s_dropped[w]; failed |= s_failed[w]; }
+    for (int jj = 0; jj < kCholCols; ++jj) s[jj] = y[(c0 + jj) * LDC + lane];
     float *I = inv + (long long)b * inv_stride + (long long)lane * ldi + c0;
     if constexpr (!SCALED) {
         float *U = u + (long long)b * u_stride;
 #pragma unroll
         for (int jj = 0; jj < kCholCols; ++jj)                                      // U[r][lane] = L[lane][r]
-            U[(long long)(c0 + jj) * ldu + lane] = c0 + jj <= lane ? row[jj] : 0.0f;
+            U[(long long)(c0 + jj) * ldu + lane] = c0 + jj <= lane ? a[lane * LDC + c0 + jj] : 0.0f;
     }
     if (set_aside != nullptr) {
         const unsigned long long out = SCALED ? early | (aside_pivots != 0 ? dropped : 0ull) : dropped;
@@ -197,7 +306,7 @@ __global__ __launch_bounds__(NB * kCholWaves) void cholesky64_kernel(const float
         for (int jj = 0; jj < kCholCols; ++jj) s[jj] *= own_scale;                 // row `lane` of D^-1 U^-1
     }
 #pragma unroll
-    for (int jj = 0; jj < kCholCols; jj += 4)    // U^-1[lane][c] = L^-1[c][lane] = s[c] of this lane (zero for c < lane)
+    for (int jj = 0; jj < kCholCols; jj += 4)
         *reinterpret_cast<float4 *>(I + jj) = make_float4(s[jj], s[jj + 1], s[jj + 2], s[jj + 3]);
     if (!SCALED && panel_inv != nullptr) {
         float *P = panel_inv + (long long)b * inv_stride + (long long)lane * ldi + c0;
@@ -209,7 +318,8 @@ __global__ __launch_bounds__(NB * kCholWaves) void cholesky64_kernel(const float
             *reinterpret_cast<float4 *>(P + jj) = make_float4(v[0], v[1], v[2], v[3]);
         }
     }
-    if ((failed != 0 || dropped != 0 || shrunk) && threadIdx.x == 0) info[b] |= (failed != 0 ? 1 : 0) | (dropped != 0 || shrunk ? 2 : 0);
+    if ((pivots.failed != 0 || dropped != 0 || shrunk) && threadIdx.x == 0)
+        info[b] |= (pivots.failed != 0 ? 1 : 0) | (dropped != 0 || shrunk ? 2 : 0);
 }
 
 // How far a stack of Gram matrices is from the identity: per matrix max |G - I| and ||G - I||_F^2, in
