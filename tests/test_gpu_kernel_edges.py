@@ -39,3 +39,50 @@ def test_64_column_factor_with_a_dependent_column_at_the_edges_of_its_blocks_of_
     # U U^-1 = I: forward error n * 2^-24 * condition of U (1 / sqrt(floor) = 70 at most)
     assert float((upper.double() @ inv[0].double().cpu() - torch.eye(64)).abs().max()) <= 64 * 2 ** -24 * 70
     assert float(torch.tril(inv[0], -1).abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("order,blocksize", [(1, 64), (3, 64), (27, 64), (66, 64), (100, 64), (129, 128), (255, 256), (260, 2048),
+                                             (1200, 64), (1201, 64), (1202, 512), (2049, 2048), (4099, 2048)])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_general_quantizer_over_ragged_segments_shared_bytes_and_odd_addresses(X, order, blocksize, bits):
+    import numpy as np
+    import qtensor.functional as F
+    from oracle import quant_np as Q
+    code = F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)
+    g = torch.Generator().manual_seed(order)
+    for diagonal, dtype, skew in ((True, torch.float32, 0), (False, torch.float32, 1), (True, torch.bfloat16, 1)):
+        A = torch.randn(order, order, generator=g).to(dtype)
+        A[order // 2] = 0.0                                                # zero segments, and one NaN segment
+        A[order - 1, order - 1 if order < 3 else 1] = float("nan")
+        dev = torch.empty(order * order + skew, dtype=dtype, device="cuda")[skew:].view(order, order).copy_(A)
+        n_bytes = -(-order * order * bits // 8)
+        room = torch.full((n_bytes + 8,), 0xA5, dtype=torch.uint8, device="cuda")
+        out = room[4 + skew:4 + skew + n_bytes]
+        o = Q.quantize_c(A.float().numpy(), code.numpy(), order, blocksize, bits, diagonal)
+        if diagonal:
+            got = F.quantize_blockwise_diagreal(dev, code.cuda(), order, blocksize=blocksize, bits=bits, out=out)
+            assert np.array_equal(got[2].cpu().numpy(), o[2], equal_nan=True)
+            back = F.dequantize_blockwise_diagreal(out, code.cuda(), order, got[1], got[2], blocksize=blocksize, bits=bits, outdtype=dtype)
+        else:
+            got = F.quantize_blockwise(dev, code.cuda(), order, blocksize=blocksize, bits=bits, out=out)
+            land = torch.empty(order * order + 1, device="cuda")[1:].view(order, order)
+            back = F.dequantize_blockwise(out, code.cuda(), order, got[1], blocksize=blocksize, bits=bits, out=land)
+        assert np.array_equal(out.cpu().numpy(), o[0])
+        assert np.array_equal(got[1].cpu().numpy(), o[1], equal_nan=True)
+        assert (room[:4 + skew] == 0xA5).all() and (room[4 + skew + n_bytes:] == 0xA5).all()
+        want = Q.dequantize_c(o[0], code.numpy(), order, o[1], blocksize, bits, diag=o[2] if diagonal else None,
+                              to_bf16=dtype == torch.bfloat16)
+        assert np.array_equal(back.float().cpu().numpy().reshape(-1), np.asarray(want).reshape(-1), equal_nan=True)
+
+
+@pytest.mark.parametrize("order", [27, 100, 257])
+def test_general_quantizer_over_a_stack_is_the_single_matrix_one(X, order):
+    import qtensor.functional as F
+    code = F.create_linear_map(True, 4, 2).cuda()
+    mats = torch.randn(5, order, order, device="cuda", generator=torch.Generator(device="cuda").manual_seed(order))
+    q = X.quantize_stack(mats, X.empty_quantized(5, order, 64, 4, code, True))
+    back = X.dequantize_stack(q)
+    for b in range(5):
+        codes, absmax, diag = F.quantize_blockwise_diagreal(mats[b], code, order, blocksize=64, bits=4)
+        assert torch.equal(q.codes[b], codes) and torch.equal(q.absmax[b], absmax) and torch.equal(q.diag[b], diag)
+        assert torch.equal(back[b], F.dequantize_blockwise_diagreal(codes, code, order, absmax, diag, blocksize=64, bits=4))
