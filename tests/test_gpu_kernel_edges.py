@@ -86,3 +86,37 @@ def test_general_quantizer_over_a_stack_is_the_single_matrix_one(X, order):
         codes, absmax, diag = F.quantize_blockwise_diagreal(mats[b], code, order, blocksize=64, bits=4)
         assert torch.equal(q.codes[b], codes) and torch.equal(q.absmax[b], absmax) and torch.equal(q.diag[b], diag)
         assert torch.equal(back[b], F.dequantize_blockwise_diagreal(codes, code, order, absmax, diag, blocksize=64, bits=4))
+
+
+@pytest.mark.parametrize("table", ["descending", "shuffled", "repeated", "neighbours", "tiny", "lopsided"])
+@pytest.mark.parametrize("order", [64, 1024])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_threshold_tables_of_unusual_code_tables(X, bits, order, table):
+    """Thresholds bracketed around the middle of a gap, the table taken as it stands where it ascends: codes, maxima and
+    the dequantized matrix are the oracle's, bit for bit (small matrices search, large ones use the bucket table)."""
+    import numpy as np
+    import qtensor.functional as F
+    from oracle import quant_np as Q
+    n = 1 << bits
+    g = torch.Generator().manual_seed(n)
+    code = F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)
+    if table == "descending":
+        code = code.flip(0).contiguous()
+    elif table == "shuffled":
+        code = code[torch.randperm(n, generator=g)].contiguous()
+    elif table == "repeated":
+        code = code.clone()
+        code[n // 4:n // 2] = code[n // 4]
+    elif table == "neighbours":                                            # gaps of one, two, ... values of fp32 around a half
+        code = (0.5 + torch.cumsum(torch.arange(n), 0).double() * 2.0 ** -24).float()
+    elif table == "tiny":                                                  # thresholds too near zero for the fast quotient
+        code = code * 2.0 ** -60
+    else:                                                                  # one gap over many binades on either side of zero
+        code = torch.cat([torch.tensor([-1.0, -2.0 ** -40, 0.0]), torch.linspace(2.0 ** -20, 1.0, n - 3)])
+    A = torch.randn(order, order, generator=g)
+    A.view(-1)[:n] = code.abs().max() * code                                  # values at the entries themselves
+    out, absmax = F.quantize_blockwise(A.cuda(), code.cuda(), order, blocksize=64, bits=bits)
+    back = F.dequantize_blockwise(out, code.cuda(), order, absmax, blocksize=64, bits=bits)
+    want, want_absmax = Q.quantize_c(A.numpy(), code.numpy(), order, 64, bits, False)
+    assert np.array_equal(out.cpu().numpy(), want) and np.array_equal(absmax.cpu().numpy(), want_absmax)
+    assert np.array_equal(back.cpu().numpy(), Q.dequantize_c(want, code.numpy(), order, want_absmax, bits=bits, blocksize=64))
