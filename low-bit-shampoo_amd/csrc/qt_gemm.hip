@@ -35,6 +35,9 @@
 #ifndef QT_STREAMK
 #define QT_STREAMK 1
 #endif
+#ifndef QT_GEMM_AHEAD
+#define QT_GEMM_AHEAD 4                // k tiles that the loads of a lone workgroup's tile run ahead
+#endif
 // Tuning knobs of the tile / k-cut choice (environment variables QT_GEMM_TILE, QT_GEMM_SPLIT, QT_GEMM_STREAM_WGS,
 // QT_GEMM_STREAM_MIN) exist only in builds made with -DQT_TUNING_KNOBS: they change the summation order of a
 // product, which a release build promises not to depend on anything but the operands' shapes.
@@ -621,7 +624,7 @@ template <int BM, int BN, int KA, int KB, int EPI, int PREC>
 constexpr int kWavesPerSimd = (PREC == kPipeSplit && BM == 128 && BN == 128 &&
                                (KA >= kQuant4 || KB >= kQuant4 || EPI == kRequant8)) ? 2 : 3;   // (the 256-entry tables of the 8-bit re-encoding leave LDS for two)
 
-template <int BM, int BN, int KA, int KB, int EPI, int PREC = kPipeF32>
+template <int BM, int BN, int KA, int KB, int EPI, int PREC = kPipeF32, bool DEEP = false>
 __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) void gemm_kernel(const GemmArgs args) {   // three waves per SIMD mean at most 168 registers, two 256
     constexpr int WM = BM / 2, WN = BN / 2, MI = WM / 32, NI = WN / 32;
     // Workgroups are dealt round-robin to the 8 accelerator dies, each with its own L2.  Renumber
@@ -808,12 +811,68 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     const int k_last = (args.triangular & 2) ? min(n0 + BN, args.K) : args.K;
     const int n_tiles = streamed ? seg_tiles : max((k_last - k_first + BK - 1) / BK, 1) / slices;
     const int k_begin = streamed ? seg_first * BK : k_first + slice * n_tiles * BK;
+    // DEEP (dense 64 x 64 tiles, one workgroup to a unit: launch_gemm).  A k tile is then 192 cycles of matrix
+    // instructions against a load latency of several times that with nothing else on the unit to hide it, so the loads
+    // are kept kAhead tiles ahead in as many sets of registers (eight words a set).  Loads and commits beyond the last
+    // tile repeat it instead of being left out: without a branch around a load every wait is for its own set alone.
+    static_assert(!DEEP || (kSplit && BM == 64 && BN == 64 && KA < kQuant4 && KB < kQuant4), "built for dense 64 x 64 tiles");
+    const int frag_row = lane & 31, half = lane >> 5;
+    constexpr int STEPS = BK / 2;
+    if constexpr (DEEP) {
+        constexpr int kAhead = QT_GEMM_AHEAD;
+        static_assert(kAhead % 2 == 0, "the LDS stage of a tile follows from its set");
+        using LA = SplitLayout<BM>;
+        using LB = SplitLayout<BN>;
+        constexpr int pa_of[6] = {0, 2, 1, 0, 1, 0}, pb_of[6] = {2, 0, 1, 1, 0, 0};       // smallest products first, as below
+        LoaderA ra[kAhead];
+        LoaderB rb[kAhead];
+        auto at_tile = [&](int t) { return (long long)(k_begin + max(min(t, n_tiles - 1), 0) * BK); };
+        auto fetch_a = [&](LoaderA &l, int t) { l.fetch_fast(A + (KA == kDense ? at_tile(t) : at_tile(t) * args.lda)); };
+        auto fetch_b = [&](LoaderB &l, int t) { l.fetch_fast(B + (KB == kDenseT ? at_tile(t) : at_tile(t) * args.ldb)); };
+        fetch(k_begin);
+#pragma unroll
+        for (int u = 1; u <= kAhead; ++u) {
+            ra[u % kAhead] = la;
+            rb[u % kAhead] = lb;
+            fetch_a(ra[u % kAhead], u);
+            fetch_b(rb[u % kAhead], u);
+        }
+        commit(0);
+        __syncthreads();
+        for (int t0 = 0; t0 < n_tiles; t0 += kAhead) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                if (t0 + u >= n_tiles) break;
+                const int cur = u & 1, set = (u + 1) % kAhead;
+                const unsigned char *sa = reinterpret_cast<const unsigned char *>(s_mem) + cur * SPLIT_STAGE + half * LA::kHalf + (wm + frag_row) * 16;
+                const unsigned char *sb = reinterpret_cast<const unsigned char *>(s_mem) + cur * SPLIT_STAGE + SPLIT_A + half * LB::kHalf + (wn + frag_row) * 16;
+                unsigned char *next = reinterpret_cast<unsigned char *>(s_mem) + (cur ^ 1) * SPLIT_STAGE;
+                qt_bf16x8 fa[3], fb[3];
+#pragma unroll
+                for (int p = 0; p < 3; ++p) {
+                    fa[p] = *reinterpret_cast<const qt_bf16x8 *>(sa + p * LA::kPlane);
+                    fb[p] = *reinterpret_cast<const qt_bf16x8 *>(sb + p * LB::kPlane);
+                }
+#pragma unroll
+                for (int q = 0; q < 6; ++q) {
+                    if (q == 2) {
+                        ra[set].commit_split(next);
+                        fetch_a(ra[set], t0 + u + 1 + kAhead);
+                    }
+                    if (q == 4) {
+                        rb[set].commit_split(next + SPLIT_A);
+                        fetch_b(rb[set], t0 + u + 1 + kAhead);
+                    }
+                    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa_of[q]], fb[pb_of[q]], acc[0][0], 0, 0, 0);
+                }
+                __syncthreads();
+            }
+        }
+    } else {
     fetch(k_begin);
     commit(0);
     if (n_tiles > 1) fetch(k_begin + BK);
     __syncthreads();
-    const int frag_row = lane & 31, half = lane >> 5;
-    constexpr int STEPS = BK / 2;
     if constexpr (kSplit) {
         using LA = SplitLayout<BM>;
         using LB = SplitLayout<BN>;
@@ -919,6 +978,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                 }
         }
         __syncthreads();
+    }
     }
 
     // Split pipe, diagonal tile of a symmetric product: a b and b a add the pieces of a product in different orders,
@@ -1329,7 +1389,18 @@ void launch_gemm(const GemmArgs &a, int batch, hipStream_t stream) {
         blocks = (runs + a.stream_per - 1) / a.stream_per;
     }
     if (blocks > 0x7fffffffLL) { set_error(kBadArgument, "gemm: too many tiles (%lld)", blocks); return; }
-    hipLaunchKernelGGL((gemm_kernel<BM, BN, KA, KB, EPI, PREC>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+    if constexpr (PREC == kPipeSplit && BM == 64 && BN == 64 && KA < kQuant4 && KB < kQuant4 && EPI <= kAxpbyDense) {
+        // Loads far ahead where no workgroup shares its unit (up to half as many workgroups as units, so that a launch on
+        // another stream does not either): a per-parameter optimizer step over convolution weights, chains of products of
+        // 2 to 38 tiles, 34.4 -> 31.4 ms.  With the line at one or two workgroups per unit it is the same to the noise,
+        // and for every launch the stacks lose (a step that takes statistics in 3.81 -> 3.92 ms): other workgroups hide
+        // the latency there and the registers cost occupancy.
+        if (blocks <= compute_units() / 2) {
+            hipLaunchKernelGGL((gemm_kernel<BM, BN, KA, KB, EPI, PREC, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+        } else
+            hipLaunchKernelGGL((gemm_kernel<BM, BN, KA, KB, EPI, PREC>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+    } else
+        hipLaunchKernelGGL((gemm_kernel<BM, BN, KA, KB, EPI, PREC>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
     if (EPI == kStore && a.stream_per > 0) {
         hipLaunchKernelGGL(reduce_pieces_kernel, dim3((unsigned)(tn * tm * batch), 4), dim3(256), 0, stream, a.workspace, a.C, a.ldc,
                            a.M, a.N, BM, BN, (int)tm, (int)tn, a.K / BK, a.stream_per, a.stream_lcm);

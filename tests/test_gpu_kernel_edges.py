@@ -120,3 +120,26 @@ def test_threshold_tables_of_unusual_code_tables(X, bits, order, table):
     want, want_absmax = Q.quantize_c(A.numpy(), code.numpy(), order, 64, bits, False)
     assert np.array_equal(out.cpu().numpy(), want) and np.array_equal(absmax.cpu().numpy(), want_absmax)
     assert np.array_equal(back.cpu().numpy(), Q.dequantize_c(want, code.numpy(), order, want_absmax, bits=bits, blocksize=64))
+
+
+@pytest.mark.parametrize("trans", ["", "a", "b"])
+@pytest.mark.parametrize("k", [32, 48, 64, 80, 96, 112, 144, 1216])
+@pytest.mark.parametrize("m,n", [(64, 64), (65, 128), (2, 3), (200, 70)])
+def test_products_of_a_few_tiles_equal_the_same_products_in_a_large_stack(X, m, n, k, trans):
+    """Loads several k tiles ahead (k ranges around the number of register sets, ragged tiles): the bits of the large stack's
+    kernels, and fp32 accuracy against float64; beta E + alpha A B over it as well."""
+    g = torch.Generator().manual_seed(m + n + k)
+    A, B = torch.randn(m, k, generator=g), torch.randn(k, n, generator=g)
+    a = (A.T if trans == "a" else A).contiguous().cuda()
+    b = (B.T if trans == "b" else B).contiguous().cuda()
+    E = torch.randn(m, n, generator=g).cuda()
+    kw = dict(trans_a=trans == "a", trans_b=trans == "b")
+    few = X.gemm(a.unsqueeze(0), b.unsqueeze(0), addend=E.unsqueeze(0), alpha=-1.0, beta=1.0, **kw)[0]
+    many = X.gemm(a.repeat(400, 1, 1), b.repeat(400, 1, 1), addend=E.repeat(400, 1, 1), alpha=-1.0, beta=1.0, **kw)
+    assert torch.equal(few, many[0]) and torch.equal(few, many[399])
+    want = E.cpu().double() - A.double() @ B.double()
+    # dropped pieces 2^-24 |a b| each and k fp32 additions: (k + 2) 2^-24 sum |a b|, plus the last sum's rounding
+    bound = (k + 2) * 2 ** -24 * (A.abs().double() @ B.abs().double()) + 2 ** -23 * want.abs() + 1e-30
+    assert bool(((few.cpu().double() - want).abs() <= bound).all())
+    plain = X.gemm(a.unsqueeze(0), b.unsqueeze(0), **kw)[0].cpu().double()
+    assert bool(((plain - A.double() @ B.double()).abs() <= bound + 2 ** -23 * (A.double() @ B.double()).abs()).all())
