@@ -4,7 +4,7 @@
 // (torch.linalg.qr at qtensor/utils.py:157 of the reference).
 //
 // The only arithmetic done outside the matrix-core GEMM (qtensor_hip_gemm) is the 64 x 64 diagonal
-// block: four waves per matrix factor it in registers and also invert the factor.
+// block: four waves per matrix factor it in LDS, sixteen columns at a time, and also invert the factor.
 //   factor:  for each block row j:  U_jj = chol(G_jj);  U_j,> = U_jj^-T G_j,>;  G_>,> -= U_j,>^T U_j,>
 //            (the last step for the rows of the current 256-row panel at once, for the rest per panel)
 //   solve :  the inverted diagonal blocks are doubled up to 256 x 256 -- with blocks A, C already
@@ -43,7 +43,7 @@ constexpr int kSolvePanel = 256;       // diagonal blocks of the factor are inve
 //
 // A right-looking factorisation L L^T (L = U^T) of blocks of sixteen columns, the matrix in LDS, with the inverse beside it
 // (factor64 below): the wave that owns a block of columns takes them into registers, lane i standing for row i, and
-// factors them alone; the blocks behind it and the inverse are products of 16 x 16 blocks on the fp32 matrix instruction.
+// factors them alone; the blocks behind it in the matrix and in the inverse are updated on the fp32 matrix instruction.
 //
 // SCALED: `gram` is the Gram matrix S = P^T P of a panel whose columns are not of unit length yet.  The kernel factors
 // D^-1 S D^-1 (D = the column lengths, from the diagonal of S) and `inv` receives D^-1 U^-1, so that P inv is the
@@ -60,25 +60,21 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
     return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), lane));
 }
 
-// acc += sign A B for 16 x 16 blocks in LDS: A row by row (16-byte reads), B either the transpose of such a block
-// (B_TURNED: B[k][n] = b[n][k]) or as it lies.  v_mfma_f32_16x16x4f32: lane l supplies row (A) or column (B) l % 16 and
-// k = 4 (l / 16) + t in step t, and holds column l % 16 of rows 4 (l / 16) .. + 3 of the result.
-template <bool B_TURNED>
-__device__ __forceinline__ qt_acc4 block_product(const float *a, const float *b, float sign, qt_acc4 acc) {
-    const int lane = threadIdx.x & 63, at = lane & 15, g = (lane >> 4) * 4;
-    const float4 av = *reinterpret_cast<const float4 *>(a + at * LDC + g);
-    float bv[4];
-    if (B_TURNED) {
-        const float4 v = *reinterpret_cast<const float4 *>(b + at * LDC + g);
-        bv[0] = v.x; bv[1] = v.y; bv[2] = v.z; bv[3] = v.w;
-    } else {
+// acc -= A B for 16 x 16 blocks in LDS, one multiply-add per k in ascending order.  b_row, b_col: the strides of B, so that
+// its transpose can be taken as well.  v_mfma_f32_16x16x4f32: lane l supplies row (A) or column (B) l % 16 and k = l / 16 of
+// the four k of a step, which the instruction adds one after the other, each with one rounding; the lane holds column
+// l % 16 of rows 4 (l / 16) .. + 3 of the result.
+__device__ __forceinline__ qt_acc4 block_subtract(const float *a, const float *b, int b_row, int b_col, qt_acc4 acc) {
+    const int lane = threadIdx.x & 63, at = lane & 15, g = lane >> 4;
+    float av[4], bv[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) bv[t] = b[(g + t) * LDC + at];
+    for (int t = 0; t < 4; ++t) {
+        av[t] = a[at * LDC + 4 * t + g];
+        bv[t] = b[(4 * t + g) * b_row + at * b_col];
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sign * av.x, bv[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sign * av.y, bv[1], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sign * av.z, bv[2], acc, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(sign * av.w, bv[3], acc, 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(-av[t], bv[t], acc, 0, 0, 0);
+    return acc;
 }
 __device__ __forceinline__ qt_acc4 block_load(const float *c) {
     const int lane = threadIdx.x & 63, at = lane & 15, g = (lane >> 4) * 4;
@@ -104,38 +100,45 @@ struct PivotNotes {                      // (LDS) one slot per wave
 };
 
 // `a` (64 rows, LDC floats apart): the lower triangle of a symmetric matrix on entry, L on exit (above the diagonal
-// blocks: undefined).  `y`: L^-1 on exit, zeros above its diagonal.  All 256 threads of a workgroup; a barrier
-// before the call makes `a` visible, the last thing the call does is one as well.
+// blocks: undefined).  `y`: L^-1 on exit, zeros above its diagonal.  All 256 threads of a workgroup; the call begins and
+// ends with a barrier.
+// Step k subtracts L[i][k] L[j][k] from element (i, j) behind it and L[j][k] x[k] from every right-hand side of L X = I, one
+// multiply-add each, k ascending for every element: the inverse is the forward substitution and |L Y - I| stays within
+// 64 x 2^-24 |L| |Y| element by element.  (An inverse put together from the inverses of diagonal blocks, Y_10 = -Y_11 (L_10 Y_00),
+// does not: its residual on ill-conditioned panels was up to three times as large.)
 // What bounds it is the chain of the 64 pivots (about 250 cycles each: the pivot through v_readlane, v_rsq_f32 and one
-// Newton step, the column, the next pivot, with the multiply-adds of the step before in its shadow).  A launch takes
-// 13.2 us for one matrix and 14.6 for 99; with the trailing updates and the substitution for the inverse as vector
-// multiply-adds of the waves behind (300 cycles a step on top of 300 for the pivot) it took 18.9 and 21.7.
+// Newton step, the column, the next pivot, with the multiply-adds of the step before in its shadow).  Back to back a launch
+// takes 12.1 us for one matrix and 12.8 for 99; with the trailing updates and the substitution behind a block as vector
+// multiply-adds of the waves behind (300 cycles a step on top of 300 for the pivot) it took 15.4 and 16.3, with the
+// inverse from the inverses of diagonal blocks 12.0 and 12.7.
 __device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes &notes, float pivot_floor) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    {
-        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int i = threadIdx.x; i < NB * (NB / 4); i += NB * kCholWaves)
-            *reinterpret_cast<float4 *>(y + (i / (NB / 4)) * LDC + 4 * (i % (NB / 4))) = zero;
+    for (int i = threadIdx.x; i < NB * (NB / 4); i += NB * kCholWaves) {
+        const int r = i / (NB / 4), c = 4 * (i % (NB / 4));
+        *reinterpret_cast<float4 *>(y + r * LDC + c) =
+            make_float4(r == c ? 1.0f : 0.0f, r == c + 1 ? 1.0f : 0.0f, r == c + 2 ? 1.0f : 0.0f, r == c + 3 ? 1.0f : 0.0f);
     }
     __syncthreads();
 #pragma unroll 1
     for (int p = 0; p < kCholWaves; ++p) {
         const int c0 = p * kCholCols;
         if (wave == p) {                         // (uniform over the wave)
-            float row[kCholCols], s[kCholCols];  // columns c0 .. c0 + 15 of row `lane`; the same columns of the right-hand side e_lane of L x = e
+            float row[kCholCols], s[kCholCols];  // columns c0 .. c0 + 15 of row `lane`; the same rows of right-hand side `lane` of L X = I
 #pragma unroll
             for (int q = 0; q < kCholCols; q += 4) {
                 const float4 v = *reinterpret_cast<const float4 *>(a + lane * LDC + c0 + q);
                 row[q] = v.x; row[q + 1] = v.y; row[q + 2] = v.z; row[q + 3] = v.w;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) s[q + e] = lane == c0 + q + e ? 1.0f : 0.0f;
+                for (int e = 0; e < 4; ++e) s[q + e] = y[(c0 + q + e) * LDC + lane];
             }
             // Step kk works on the chain of its own pivot -- v_readlane, v_rsq_f32, one Newton step, the column of L -- and, in
             // the shadow of those dependent instructions, subtracts the step before from the columns behind kk (column kk
             // itself had that done at once).  The scheduling barriers keep the compiler from putting those updates off
             // for good, which costs it the scalar registers.  A pivot that is not above the floor is replaced and its
             // column of L cleared by selects (no branch on a value that comes out of a vector compare).
-            const float instead = pivot_floor > 0.0f ? pivot_floor : 1.0f, root = pivot_floor > 0.0f ? sqrtf(pivot_floor) : 1.0f;
+            const float instead = pivot_floor > 0.0f ? pivot_floor : 1.0f;
+            float root = __builtin_amdgcn_rsqf(instead);
+            root = instead * (root * __builtin_fmaf(-0.5f * instead * root, root, 1.5f));
             float own = 0.0f, l_before = 0.0f, x_before = 0.0f;                // own: the pivot of column `lane`, before it is replaced
 #pragma unroll
             for (int kk = 0; kk < kCholCols; ++kk) {
@@ -176,54 +179,34 @@ __device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes 
 #pragma unroll
             for (int q = 0; q < kCholCols; q += 4)
                 *reinterpret_cast<float4 *>(a + lane * LDC + c0 + q) = make_float4(row[q], row[q + 1], row[q + 2], row[q + 3]);
-            if (mine) {
 #pragma unroll
-                for (int jj = 0; jj < kCholCols; ++jj) y[(c0 + jj) * LDC + lane] = s[jj];     // L_pp^-1 (zero above its diagonal)
-            }
+            for (int jj = 0; jj < kCholCols; ++jj) y[(c0 + jj) * LDC + lane] = s[jj];
             if (lane == 0) {
                 notes.dropped[p] = pivot_floor > 0.0f ? replaced & ~not_a_number : 0ull;
                 notes.failed[p] = (pivot_floor > 0.0f ? not_a_number : replaced) != 0 ? 1 : 0;
             }
         }
         __syncthreads();
-        // the blocks behind: A_ij -= L_ip L_jp^T for i >= j > p, dealt out over the waves
-        const int rest = kCholWaves - 1 - p, count = rest * (rest + 1) / 2;
+        // the blocks behind, dealt out over the waves: A_ij -= L_ip L_jp^T for i >= j > p and Y_ij -= L_ip Y_pj for i > p >= j
+        const int rest = kCholWaves - 1 - p, own = rest * (rest + 1) / 2, count = own + rest * (p + 1);
         for (int q = wave; q < count; q += kCholWaves) {
-            int i = p + 1, left = q;
-            while (left > i - p - 1) { left -= i - p; ++i; }
-            const int j = p + 1 + left;
-            float *c = a + 16 * i * LDC + 16 * j;
-            block_store(c, block_product<true>(a + 16 * i * LDC + c0, a + 16 * j * LDC + c0, -1.0f, block_load(c)));
+            if (q < own) {
+                int i = p + 1, left = q;
+                while (left > i - p - 1) { left -= i - p; ++i; }
+                const int j = p + 1 + left;
+                float *c = a + 16 * i * LDC + 16 * j;
+                block_store(c, block_subtract(a + 16 * i * LDC + c0, a + 16 * j * LDC + c0, 1, LDC, block_load(c)));
+            } else {
+                const int i = p + 1 + (q - own) % rest, j = (q - own) / rest;
+                float *c = y + 16 * i * LDC + 16 * j;
+                block_store(c, block_subtract(a + 16 * i * LDC + c0, y + c0 * LDC + 16 * j, LDC, 1, block_load(c)));
+            }
         }
         __syncthreads();
-    }
-    // The inverse below its diagonal blocks, by halves: Y_10 = -Y_11 (L_10 Y_00) and Y_32 likewise, then the lower left
-    // 32 x 32 from the two 32 x 32 inverses.  The strict upper triangle of `a` holds the inner products.
-    const qt_acc4 none = {0.f, 0.f, 0.f, 0.f};
-    if (wave < 2) {
-        const int i = 2 * wave + 1, j = 2 * wave;
-        float *inner = a + 16 * j * LDC + 16 * i;
-        block_store(inner, block_product<false>(a + 16 * i * LDC + 16 * j, y + 16 * j * LDC + 16 * j, 1.0f, none));
-        wave_lds_sync();
-        block_store(y + 16 * i * LDC + 16 * j, block_product<false>(y + 16 * i * LDC + 16 * i, inner, -1.0f, none));
-    }
-    __syncthreads();
-    const int bi = 2 + (wave >> 1), bj = wave & 1;               // this wave's block of the lower left half
-    {
-        qt_acc4 m = none;                                        // M = L_BA Y_A
-        for (int k = bj; k < 2; ++k) m = block_product<false>(a + 16 * bi * LDC + 16 * k, y + 16 * k * LDC + 16 * bj, 1.0f, m);
-        block_store(a + 16 * bj * LDC + 16 * bi, m);
-    }
-    __syncthreads();
-    {
-        qt_acc4 m = none;                                        // Y_BA = -Y_B M
-        for (int k = 2; k <= bi; ++k) m = block_product<false>(y + 16 * bi * LDC + 16 * k, a + 16 * bj * LDC + 16 * k, -1.0f, m);
-        block_store(y + 16 * bi * LDC + 16 * bj, m);
     }
     PivotOutcome out = {0, 0};
 #pragma unroll
     for (int w = 0; w < kCholWaves; ++w) { out.dropped |= notes.dropped[w]; out.failed |= notes.failed[w]; }
-    __syncthreads();
     return out;
 }
 
@@ -277,7 +260,7 @@ __global__ __launch_bounds__(NB * kCholWaves) void cholesky64_kernel(const float
         float v = in[i];
         if constexpr (SCALED) {
             const bool out = ((early >> r) & 1ull) || ((early >> lane) & 1ull);
-            v = out ? (r == lane ? 1.0f : 0.0f) : v * lane_value(own_scale, r) * own_scale;
+            v = out ? (r == lane ? 1.0f : 0.0f) : v * own_scale * lane_value(own_scale, r);
         }
         if (r <= lane) a[lane * LDC + r] = v;
     }

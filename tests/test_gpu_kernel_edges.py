@@ -41,6 +41,56 @@ def test_64_column_factor_with_a_dependent_column_at_the_edges_of_its_blocks_of_
     assert float(torch.tril(inv[0], -1).abs().max()) == 0.0
 
 
+def fma32(a, b, c):
+    """a b + c of float32 arrays, rounded once: the float64 sum is made odd where it is inexact, so that its own rounding
+    decides no tie of the second one."""
+    import numpy as np
+    p, c = a.astype(np.float64) * b.astype(np.float64), c.astype(np.float64)               # (the product is exact)
+    s = p + c
+    t = s - p
+    low = (p - (s - t)) + (c - t)                                                          # what the sum lost, exactly
+    odd = np.where(low > 0, np.nextafter(s, np.inf), np.nextafter(s, -np.inf))
+    return np.where((low != 0) & (s.view(np.int64) % 2 == 0), odd, s).astype(np.float32)
+
+
+@pytest.mark.parametrize("condition", [1.0, 30.0, 1000.0])
+@pytest.mark.parametrize("dependent", [None, 1, 16, 31, 47, 63])
+def test_64_column_factor_and_inverse_are_the_column_by_column_recurrences(X, condition, dependent):
+    """U and U^-1 bit for bit: L[i][k] = a[i][k] r_k, a[i][j] -= L[i][k] L[j][k], x[k] = s[k] r_k, s[j] -= L[j][k] x[k], one
+    rounding each, k ascending (r_k = 1 / sqrt(pivot) is the diagonal of the inverse)."""
+    import numpy as np
+    floor = 2e-4
+    g = torch.Generator().manual_seed(int(condition) + (dependent or 0))
+    A = torch.linalg.qr(torch.randn(256, 64, generator=g, dtype=torch.float64))[0]
+    A = A * torch.logspace(0, -float(np.log10(condition)), 64, dtype=torch.float64)
+    A = A @ torch.linalg.qr(torch.randn(64, 64, generator=g, dtype=torch.float64))[0]
+    if dependent is not None:
+        A[:, dependent] = A[:, :dependent] @ torch.randn(dependent, generator=g, dtype=torch.float64)
+    A = A / A.norm(dim=0, keepdim=True)
+    gram = (A.T @ A).float()
+    U, inv = torch.zeros(1, 64, 64, device="cuda"), torch.zeros(1, 64, 64, device="cuda")
+    X.cholesky_upper(gram[None].cuda().contiguous(), U, inv, torch.zeros(1, dtype=torch.int32, device="cuda"), pivot_floor=floor)
+    U, inv = torch.triu(U[0]).cpu().numpy(), inv[0].cpu().numpy()
+    a, s = gram.numpy().T.copy(), np.eye(64, dtype=np.float32)               # (the upper triangle is what is read)
+    L = np.zeros((64, 64), np.float32)
+    for k in range(64):
+        d, r = a[k, k], inv[k, k]
+        dropped = not d > floor
+        d = np.float32(floor) if dropped else d
+        assert abs(float(r) ** 2 * float(d) - 1.0) <= 8 * 2.0 ** -24          # a reciprocal root off by two roundings at most, squared
+        L[k:, k] = a[k:, k] * r
+        if dropped:
+            L[k:, k] = 0.0
+            L[k, k] = d * r
+        s[k] *= r
+        for j in range(k + 1, 64):
+            v = np.full(64, L[j, k])
+            a[j:, j] = fma32(-L[j:, k], v[j:], a[j:, j])
+            s[j] = fma32(-v, s[k], s[j])
+    assert np.array_equal(U, L.T)
+    assert np.array_equal(inv, s.T)
+
+
 @pytest.mark.parametrize("order,blocksize", [(1, 64), (3, 64), (27, 64), (66, 64), (100, 64), (129, 128), (255, 256), (260, 2048),
                                              (1200, 64), (1201, 64), (1202, 512), (2049, 2048), (4099, 2048)])
 @pytest.mark.parametrize("bits", [4, 8])
