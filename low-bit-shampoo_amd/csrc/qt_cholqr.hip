@@ -108,7 +108,7 @@ struct PivotNotes {                      // (LDS) one slot per wave
 // does not: its residual on ill-conditioned panels was up to three times as large.)
 // What bounds it is the chain of the 64 pivots (about 250 cycles each: the pivot through v_readlane, v_rsq_f32 and one
 // Newton step, the column, the next pivot, with the multiply-adds of the step before in its shadow).  Back to back a launch
-// takes 12.1 us for one matrix and 12.8 for 99; with the trailing updates and the substitution behind a block as vector
+// takes 12.4 us for one matrix and 13.1 for 99; with the trailing updates and the substitution behind a block as vector
 // multiply-adds of the waves behind (300 cycles a step on top of 300 for the pivot) it took 15.4 and 16.3, with the
 // inverse from the inverses of diagonal blocks 12.0 and 12.7.
 __device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes &notes, float pivot_floor) {
@@ -134,9 +134,11 @@ __device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes 
             // Step kk works on the chain of its own pivot -- v_readlane, v_rsq_f32, one Newton step, the column of L -- and, in
             // the shadow of those dependent instructions, subtracts the step before from the columns behind kk (column kk
             // itself had that done at once).  The scheduling barriers keep the compiler from putting those updates off
-            // for good, which costs it the scalar registers.  A pivot that is not above the floor is replaced and its
-            // column of L cleared by selects (no branch on a value that comes out of a vector compare).
+            // for good, which costs it the scalar registers.  A pivot at or below a positive floor is replaced by it and its
+            // column of L cleared, by selects (no branch on a value that comes out of a vector compare); any other that
+            // is not above the floor is replaced by 1 and its column kept, so that what was not a number stays one.
             const float instead = pivot_floor > 0.0f ? pivot_floor : 1.0f;
+            const float drop_at = pivot_floor > 0.0f ? pivot_floor : __builtin_nanf("");         // (no comparison with a NaN holds)
             float root = __builtin_amdgcn_rsqf(instead);
             root = instead * (root * __builtin_fmaf(-0.5f * instead * root, root, 1.5f));
             float own = 0.0f, l_before = 0.0f, x_before = 0.0f;                // own: the pivot of column `lane`, before it is replaced
@@ -145,16 +147,17 @@ __device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes 
                 const bool here = lane == c0 + kk;
                 own = here ? row[kk] : own;
                 float d = lane_value(row[kk], c0 + kk), v[kCholCols];
-                const bool fine = d > pivot_floor;
-                d = fine ? d : instead;
+                const bool drop = d <= drop_at, fine = d > pivot_floor;
+                d = drop ? instead : d;
+                d = drop || fine ? d : 1.0f;
                 float r = __builtin_amdgcn_rsqf(d);
                 const float alone = here ? root : 0.0f, half_d = -0.5f * d;
 #pragma unroll
                 for (int jj = kk + 1; jj < kCholCols; ++jj) v[jj] = kk > 0 ? lane_value(l_before, c0 + jj) : 0.0f;   // L[j][k - 1]
                 __builtin_amdgcn_sched_barrier(0);
                 r = r * __builtin_fmaf(half_d * r, r, 1.5f);
-                const float l = fine ? row[kk] * r : alone;                // L[lane][k] (lanes above k: unused values)
-                row[kk] = l;                                               // (replaced pivot: nothing below the diagonal)
+                const float l = drop ? alone : row[kk] * r;                // L[lane][k] (lanes above k: unused values)
+                row[kk] = l;                                               // (dropped column: nothing below the diagonal)
                 s[kk] *= r;                                                // x[k] = s[k] / L[k][k]
                 if (kk > 0) {
 #pragma unroll

@@ -91,6 +91,23 @@ def test_64_column_factor_and_inverse_are_the_column_by_column_recurrences(X, co
     assert np.array_equal(inv, s.T)
 
 
+@pytest.mark.parametrize("column", [0, 15, 16, 40, 63])
+def test_64_column_factor_keeps_the_column_of_a_pivot_that_fails(X, column):
+    """A NaN shows in the factor (not only in info), and without a floor a pivot that is not positive counts as 1."""
+    gram = torch.eye(64).repeat(2, 1, 1) + 2.0 ** -8 * torch.triu(torch.ones(64, 64), 1)
+    gram[0, column, column] = float("nan")
+    gram[1, column, column] = -4.0
+    U, inv = torch.zeros(2, 64, 64, device="cuda"), torch.zeros(2, 64, 64, device="cuda")
+    for floor in (2e-4, 0.0):
+        info = torch.zeros(2, dtype=torch.int32, device="cuda")
+        X.cholesky_upper(gram.cuda(), U, inv, info, pivot_floor=floor)
+        assert info[0].item() & 1 and info[1].item() == (2 if floor else 1)
+        assert bool(torch.isnan(U[0, column, column])) and bool(torch.isfinite(U[0, :column]).all())
+    row = U[1].cpu()[column]                                                 # floor 0: L[i][column] = a[i][column] / 1
+    assert row[column] < -3.9
+    assert column == 63 or bool((row[column + 1:] > 0).all())
+
+
 @pytest.mark.parametrize("order,blocksize", [(1, 64), (3, 64), (27, 64), (66, 64), (100, 64), (129, 128), (255, 256), (260, 2048),
                                              (1200, 64), (1201, 64), (1202, 512), (2049, 2048), (4099, 2048)])
 @pytest.mark.parametrize("bits", [4, 8])
