@@ -148,11 +148,45 @@ __global__ __launch_bounds__(kFlatThreads) void dequantize_flat_kernel(
 }
 
 // General path: any order and alignment, a stack of matrices with a run of code bytes, maxima and diagonal entries each.
-// Bound by the store stream: a thread turns E consecutive elements of the flat matrix into 16-byte (bf16: 8-byte) stores,
+// Few elements (the line is drawn in dequantize_dispatch): bound by the latency of a thread's chain of loads and integer
+// divisions, not by memory, so a thread takes one code byte and the launch has as many threads as it can.
+template <typename T, int BITS, bool DIAG>
+__global__ __launch_bounds__(kThreads) void dequantize_bytes_kernel(
+    const uint8_t *__restrict__ q, const float *__restrict__ code, uint32_t order, uint32_t bs_shift, uint32_t nb, uint32_t total,
+    const float *__restrict__ absmax, const float *__restrict__ diag, T *__restrict__ out) {
+    constexpr int NCODE = 1 << BITS;
+    constexpr uint32_t EPB = 8 / BITS;
+    __shared__ float s_code[NCODE];
+    for (int i = threadIdx.x; i < NCODE; i += kThreads) s_code[i] = code[i];
+    __syncthreads();
+    const uint32_t n_bytes = (total + EPB - 1) / EPB;
+    // blockIdx.y = matrix of a stack
+    q += (size_t)blockIdx.y * n_bytes;
+    absmax += (size_t)blockIdx.y * order * nb;
+    if (DIAG) diag += (size_t)blockIdx.y * order;
+    out += (size_t)blockIdx.y * total;
+    for (uint32_t j = blockIdx.x * kThreads + threadIdx.x; j < n_bytes; j += gridDim.x * kThreads) {
+        const uint32_t byte = q[j];
+#pragma unroll
+        for (uint32_t e = 0; e < EPB; ++e) {
+            const uint32_t k = j * EPB + e;
+            if (k >= total) break;
+            const uint32_t id = BITS == 8 ? byte : (e == 0 ? byte >> 4 : byte & 15u);
+            const uint32_t r = k / order, c = k - r * order;
+            const float a = absmax[r * nb + (c >> bs_shift)];
+            float y = a == 0.0f ? 0.0f : s_code[id] * a;
+            if (DIAG && r == c) y = diag[r];
+            Vec4Store<T>::store1(out, k, y);
+        }
+    }
+}
+
+// More elements: bound by the store stream.  A thread turns E consecutive elements of the flat matrix into 16-byte (bf16: 8-byte) stores,
 // one division by the order and one or two maxima per E.  WHOLE: the order is a multiple of four, E = 4 elements lie in
 // one segment of one row and their codes are whole, aligned bytes.  Otherwise E = 8 (whole bytes again) and the thread
 // walks over the ends of segments and rows.
-// One 1200 x 1200 matrix: 4.3 us against 6.0 with a thread per code byte; the stacks of a convolution net 8.3 against 14.1.
+// One 1200 x 1200 matrix: 3.6 us against 4.8 with a thread per code byte; 1301 x 1301: 5.0 against 5.7; 30 x 576 x 576: 11.8
+// against 21.5 (4-bit codes, back to back).
 template <typename T> struct AnyAligned4;                  // four elements at any address of an element
 template <> struct AnyAligned4<float> {
     typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
@@ -300,10 +334,18 @@ void dequantize_dispatch(const uint8_t *q, const float *code, int order_i, const
         const uint32_t nb = (order + bs - 1) / bs;
         const uint32_t one = order * order;
         const bool whole = order % 4 == 0 && is_aligned(q, BITS == 4 ? 2 : 4);
-        const uint32_t n_units = whole ? one / 4 : (one + 7) / 8;
+        // A thread per code byte where that is the faster one, back to back: walking over eight elements costs it 3.3 us
+        // against 2.6 for 261 x 261, 3.7 against 2.6 for 100 x 27 x 27, 3.8 against 3.7 for 801 x 801, 4.1 against 4.2 for
+        // 1001 x 1001; four whole elements 2.6 against 2.5 for 260 x 260 in 8 bits, the same from 340 x 340, and never
+        // more in 4 bits.
+        const bool bytes = total < (whole ? (BITS == 8 ? 1u << 17 : 0u) : 1000000u);
+        const uint32_t n_units = bytes ? (one * BITS + 7) / 8 : whole ? one / 4 : (one + 7) / 8;
         const FastDiv quad_div = make_fastdiv(whole ? order / 4 : 1);
         const dim3 grid(capped_grid((n_units + kThreads - 1) / kThreads, 16), batch);
-        if (whole)
+        if (bytes)
+            hipLaunchKernelGGL((dequantize_bytes_kernel<T, BITS, DIAG>), grid, dim3(kThreads), 0, stream,
+                               q, code, order, (uint32_t)bs_shift, nb, one, absmax, diag, out);
+        else if (whole)
             hipLaunchKernelGGL((dequantize_general_kernel<T, BITS, DIAG, true>), grid, dim3(kThreads), 0, stream,
                                q, code, order, (uint32_t)bs_shift, nb, quad_div, one, absmax, diag, out);
         else

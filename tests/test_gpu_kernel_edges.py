@@ -155,6 +155,36 @@ def test_general_quantizer_over_a_stack_is_the_single_matrix_one(X, order):
         assert torch.equal(back[b], F.dequantize_blockwise_diagreal(codes, code, order, absmax, diag, blocksize=64, bits=4))
 
 
+@pytest.mark.parametrize("order,batch", [(5, 39999), (5, 40001), (27, 1371), (27, 1372), (101, 99), (999, 1), (1001, 1), (60, 36), (60, 37)])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_general_dequantizer_on_either_side_of_the_size_at_which_a_thread_takes_more_than_a_byte(X, order, batch, bits):
+    """(odd orders: a million elements in the stack; multiples of four: 2^17 in 8 bits).  The first, the middle and the last
+    matrix against the oracle, bit for bit, the others against the single-matrix entry point's arithmetic."""
+    import numpy as np
+    import qtensor.functional as F
+    from oracle import quant_np as Q
+    code = F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)
+    mats = torch.randn(batch, order, order, device="cuda", generator=torch.Generator(device="cuda").manual_seed(order))
+    mats[batch // 2, order // 2] = 0.0                                     # zero segments
+    for diagonal, dtype in ((True, torch.float32), (False, torch.bfloat16)):
+        q = X.quantize_stack(mats, X.empty_quantized(batch, order, 64, bits, code.cuda(), diagonal))
+        room = torch.full((2 + batch * order * order + 2,), -7.0, dtype=dtype, device="cuda")
+        back = X.dequantize_stack(q, out=room[2:-2].view(batch, order, order), outdtype=dtype)
+        assert bool((room[:2] == -7.0).all()) and bool((room[-2:] == -7.0).all())
+        for b in {0, batch // 2, batch - 1}:
+            want = Q.dequantize_c(q.codes[b].cpu().numpy(), code.numpy(), order, q.absmax[b].cpu().numpy(), 64, bits,
+                                  diag=q.diag[b].cpu().numpy() if diagonal else None, to_bf16=dtype == torch.bfloat16)
+            assert np.array_equal(back[b].float().cpu().numpy().reshape(-1), np.asarray(want).reshape(-1))
+        # every other element: code[id] * maximum in fp32, by torch
+        ids = q.codes.long() if bits == 8 else torch.stack([q.codes.long() >> 4, q.codes.long() & 15], 2).flatten(1)
+        ids = ids[:, :order * order].view(batch, order, order)
+        a = q.absmax.view(batch, order, -1).repeat_interleave(64, 2)[:, :, :order]
+        full = torch.where(a == 0, torch.zeros_like(a), code.cuda()[ids] * a)
+        if diagonal:
+            full.diagonal(dim1=1, dim2=2).copy_(q.diag)
+        assert torch.equal(back, full.to(dtype))
+
+
 @pytest.mark.parametrize("table", ["descending", "shuffled", "repeated", "neighbours", "tiny", "lopsided"])
 @pytest.mark.parametrize("order", [64, 1024])
 @pytest.mark.parametrize("bits", [4, 8])
