@@ -155,6 +155,26 @@ def test_general_quantizer_over_a_stack_is_the_single_matrix_one(X, order):
         assert torch.equal(back[b], F.dequantize_blockwise_diagreal(codes, code, order, absmax, diag, blocksize=64, bits=4))
 
 
+@pytest.mark.parametrize("order,blocksize", [(1, 2048), (27, 512), (32, 64), (33, 128), (64, 2048), (65, 2048), (100, 2048), (128, 256), (129, 512),
+                                             (256, 512), (300, 2048), (511, 1024), (513, 2048), (1025, 2048), (1090, 1024), (1600, 512)])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_general_quantizer_with_segments_longer_than_the_row(X, order, blocksize, bits):
+    """Stacks whose rows are one segment, shorter than the blocksize by less or more than a factor of two, and rows with a short
+    last segment: every matrix against the oracle, bit for bit."""
+    import numpy as np
+    from oracle import quant_np as Q
+    import qtensor.functional as F
+    code = F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)
+    for diagonal, dtype in ((True, torch.float32), (False, torch.bfloat16)):
+        mats = torch.randn(3, order, order, generator=torch.Generator().manual_seed(order)).to(dtype)
+        mats[1, order // 2] = 0.0
+        q = X.quantize_stack(mats.cuda(), X.empty_quantized(3, order, blocksize, bits, code.cuda(), diagonal))
+        for b in range(3):
+            want = Q.quantize_c(mats[b].float().numpy(), code.numpy(), order, blocksize, bits, diagonal)
+            assert np.array_equal(q.codes[b].cpu().numpy(), want[0]) and np.array_equal(q.absmax[b].cpu().numpy(), want[1])
+            assert not diagonal or np.array_equal(q.diag[b].cpu().numpy(), want[2])
+
+
 @pytest.mark.parametrize("order,batch", [(5, 39999), (5, 40001), (27, 1371), (27, 1372), (101, 99), (999, 1), (1001, 1), (60, 36), (60, 37)])
 @pytest.mark.parametrize("bits", [4, 8])
 def test_general_dequantizer_on_either_side_of_the_size_at_which_a_thread_takes_more_than_a_byte(X, order, batch, bits):
