@@ -811,10 +811,12 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     const int k_last = (args.triangular & 2) ? min(n0 + BN, args.K) : args.K;
     const int n_tiles = streamed ? seg_tiles : max((k_last - k_first + BK - 1) / BK, 1) / slices;
     const int k_begin = streamed ? seg_first * BK : k_first + slice * n_tiles * BK;
-    // DEEP (dense 64 x 64 tiles, one workgroup to a unit: launch_gemm).  A k tile is then 192 cycles of matrix
-    // instructions against a load latency of several times that with nothing else on the unit to hide it, so the loads
-    // are kept kAhead tiles ahead in as many sets of registers (eight words a set).  Loads and commits beyond the last
-    // tile repeat it instead of being left out: without a branch around a load every wait is for its own set alone.
+    // DEEP (dense 64 x 64 tiles, few workgroups and four k tiles or more: launch_gemm).  A k tile is then 192 cycles of
+    // matrix instructions against a load latency of several times that with next to nothing else on the unit to hide
+    // it, so the loads are kept kAhead tiles ahead in as many sets of registers (eight words a set).  Loads and commits
+    // beyond the last tile repeat it instead of being left out: a branch around a load would make the next wait one for
+    // all loads in flight.  (An operand with k contiguous and rows that are not 16-byte aligned still takes one, the
+    // loader's choice between one wide load and four of a word.)
     static_assert(!DEEP || (kSplit && BM == 64 && BN == 64 && KA < kQuant4 && KB < kQuant4), "built for dense 64 x 64 tiles");
     const int frag_row = lane & 31, half = lane >> 5;
     constexpr int STEPS = BK / 2;
@@ -1390,12 +1392,17 @@ void launch_gemm(const GemmArgs &a, int batch, hipStream_t stream) {
     }
     if (blocks > 0x7fffffffLL) { set_error(kBadArgument, "gemm: too many tiles (%lld)", blocks); return; }
     if constexpr (PREC == kPipeSplit && BM == 64 && BN == 64 && KA < kQuant4 && KB < kQuant4 && EPI <= kAxpbyDense) {
-        // Loads far ahead where no workgroup shares its unit (up to half as many workgroups as units, so that a launch on
-        // another stream does not either): a per-parameter optimizer step over convolution weights, chains of products of
-        // 2 to 38 tiles, 34.4 -> 31.4 ms.  With the line at one or two workgroups per unit it is the same to the noise,
-        // and for every launch the stacks lose (a step that takes statistics in 3.81 -> 3.92 ms): other workgroups hide
-        // the latency there and the registers cost occupancy.
-        if (blocks <= compute_units() / 2) {
+        // Loads far ahead where the launch's own workgroups have a unit each and half of the units stay free: a per-parameter
+        // optimizer step over convolution weights, chains of products of 2 to 38 tiles, 34.4 -> 31.4 ms.  Both lines are
+        // measured.  Workgroups: at one or two per unit the step is the same to the noise, and for every launch the
+        // stacks lose (a step that takes statistics in 3.81 -> 3.92 ms): other workgroups hide the latency there and the
+        // registers cost occupancy.  (A launch on another stream may share the units all the same.)  k tiles of a
+        // workgroup, on operands that another kernel has just written, us with and without: one 320 x 320 result, k = 1024
+        // 28.5 and 45.7, 128 6.4 and 8.1, 64 4.9 and 5.4, 48 4.6 and 4.6, 32 4.3 and 4.0; one 64 x 64 result, 1024 27.0 and
+        // 37.7, 128 6.1 and 6.9, 64 4.5 and 4.4, 32 3.8 and 3.3; the per-parameter step with the line at four tiles
+        // 31.7 ms, at five 32.0.  (With operands that the unit's own die still holds in its cache 64 takes 4.5 against
+        // 4.1, 128 6.0 against 5.6, and from 512 on it is the same.)
+        if (blocks <= compute_units() / 2 && (a.K + BK - 1) / BK / (EPI == kStore ? a.split_k : 1) >= 4) {
             hipLaunchKernelGGL((gemm_kernel<BM, BN, KA, KB, EPI, PREC, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
         } else
             hipLaunchKernelGGL((gemm_kernel<BM, BN, KA, KB, EPI, PREC>), dim3((unsigned)blocks), dim3(256), 0, stream, a);

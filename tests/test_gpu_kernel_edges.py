@@ -260,3 +260,56 @@ def test_products_of_a_few_tiles_equal_the_same_products_in_a_large_stack(X, m, 
     assert bool(((few.cpu().double() - want).abs() <= bound).all())
     plain = X.gemm(a.unsqueeze(0), b.unsqueeze(0), **kw)[0].cpu().double()
     assert bool(((plain - A.double() @ B.double()).abs() <= bound + 2 ** -23 * (A.double() @ B.double()).abs()).all())
+
+
+@pytest.mark.parametrize("form", ["plain", "addend", "symmetric", "symmetric addend", "upper a", "upper b", "skip", "word rows"])
+@pytest.mark.parametrize("k", [48, 64, 80, 96, 112, 128, 144, 208])
+@pytest.mark.parametrize("m", [64, 130, 208])
+def test_launches_on_either_side_of_the_lines_of_the_loads_far_ahead_have_the_same_bits(X, m, k, form):
+    """Dense products of at most half as many 64 x 64 tiles as units, on four k tiles or more, load several tiles ahead: a stack
+    at that line against one beyond it, entry by entry, in every form that reaches the variant.  (Below k = 256 no product is
+    cut along k, and up to as many tiles as units the tiles are 64 x 64 ones.)"""
+    if form.startswith("upper"):
+        m = k
+    tiles_1 = -(-m // 64)
+    tiles = tiles_1 * (tiles_1 + 1) // 2 if form.startswith("symmetric") else tiles_1 * tiles_1
+    half = torch.cuda.get_device_properties(0).multi_processor_count // 2
+    few, many = half // tiles, half // tiles + 1
+    assert few >= 1 and few * tiles <= half < many * tiles <= 2 * half
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    A = torch.randn(many, m, k, device="cuda", generator=g)
+    B = torch.randn(many, k, m, device="cuda", generator=g)
+    kw = {}
+    if form == "word rows":                                                # rows that are not 16-byte aligned: the other loads of the loaders
+        A = torch.randn(many, m, k + 1, device="cuda", generator=g)[:, :, 1:]
+        B = torch.randn(many, m, k + 3, device="cuda", generator=g)[:, :, 3:]
+        kw = dict(trans_b=True)
+    elif form.startswith("symmetric"):
+        B, kw = A, dict(trans_b=True, symmetric=True)
+    elif form == "upper a":
+        A, kw = A.triu(), dict(upper_a=True)
+    elif form == "upper b":
+        B, kw = B.triu(), dict(upper_b=True)
+    E = torch.randn(many, m, m, device="cuda", generator=g)
+    E = E + E.transpose(1, 2)
+    flags = (torch.arange(many, device="cuda") % 3 == 0).int()
+
+    def product(count):
+        more = dict(kw)
+        if form.endswith("addend"):
+            more.update(addend=E[:count], alpha=-1.0, beta=1.0)
+        if form == "skip":
+            more.update(skip=flags[:count].contiguous())
+        out = torch.full((count, m, m), -7.0, device="cuda")
+        return X.gemm(A[:count], B[:count], out=out, **more)
+
+    a, b = product(few), product(many)
+    assert torch.equal(a, b[:few])
+    want = A.double().cpu() @ (B.transpose(1, 2) if kw.get("trans_b") else B).double().cpu()
+    size = A.abs().double().cpu() @ (B.transpose(1, 2) if kw.get("trans_b") else B).abs().double().cpu()
+    if form.endswith("addend"):
+        want, size = E.double().cpu() - want, size + E.abs().double().cpu()
+    if form == "skip":
+        want[flags.bool().cpu()] = -7.0
+    # dropped pieces 2^-24 |a b| each and k fp32 additions, plus the last sum's rounding
+    assert bool(((b.cpu().double() - want).abs() <= (k + 4) * 2 ** -24 * size + 1e-30).all())
