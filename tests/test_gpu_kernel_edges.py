@@ -205,38 +205,87 @@ def test_general_dequantizer_on_either_side_of_the_size_at_which_a_thread_takes_
         assert torch.equal(back, full.to(dtype))
 
 
-@pytest.mark.parametrize("table", ["descending", "shuffled", "repeated", "neighbours", "tiny", "lopsided"])
-@pytest.mark.parametrize("order", [64, 1024])
+def table_of(kind, bits):
+    import qtensor.functional as F
+    n = 1 << bits
+    code = F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)
+    if kind == "descending":
+        return code.flip(0).contiguous()
+    if kind == "shuffled":
+        return code[torch.randperm(n, generator=torch.Generator().manual_seed(n))].contiguous()
+    if kind == "repeated":
+        code = code.clone()
+        code[n // 4:n // 2] = code[n // 4]
+    elif kind == "neighbours":                                             # gaps of one, two, ... values of fp32 around a half
+        code = (0.5 + torch.cumsum(torch.arange(n), 0).double() * 2.0 ** -24).float()
+    elif kind == "tiny":                                                   # thresholds too near zero for the fast quotient
+        code = code * 2.0 ** -60
+    elif kind == "lopsided":                                               # one gap over many binades on either side of zero
+        code = torch.cat([torch.tensor([-1.0, -2.0 ** -40, 0.0]), torch.linspace(2.0 ** -20, 1.0, n - 3)])
+    return code
+
+
+def around_the_thresholds(code):
+    """(values, below, above): every entry, and up to six values of fp32 on either side of every gap's middle and of the value at
+    which |v - lo| > |hi - v| (each difference rounded to fp32) turns true; below, above: the two values at that turn, per gap."""
+    import numpy as np
+
+    def key(x):
+        b = x.view(np.int32).astype(np.int64)
+        return np.where(b >= 0, b, -(b & 0x7fffffff))
+
+    def value(k):
+        return np.where(k >= 0, k, (-k) | 0x80000000).astype(np.uint32).view(np.float32)
+
+    c = np.unique(code.numpy() + np.float32(0.0))                          # (no -0)
+    lo, hi = c[:-1], c[1:]
+    low, high = key(lo), key(hi)
+    for _ in range(33):
+        mid = (low + high) // 2
+        upper = np.abs(value(mid) - lo) > np.abs(hi - value(mid))
+        inside = high - low > 1
+        low, high = np.where(inside & ~upper, mid, low), np.where(inside & upper, mid, high)
+    middle = key((np.float32(0.5) * lo + np.float32(0.5) * hi).astype(np.float32))
+    steps = np.arange(-6, 7)[:, None]
+    values = np.concatenate([c, value(middle + steps).ravel(), value(high + steps).ravel()])
+    return np.clip(values, -1.0, 1.0), value(high - 1), value(high)
+
+
+@pytest.mark.parametrize("table", ["as it ships", "descending", "shuffled", "repeated", "neighbours", "tiny", "lopsided"])
+@pytest.mark.parametrize("order", [64, 66, 1024])
 @pytest.mark.parametrize("bits", [4, 8])
 def test_threshold_tables_of_unusual_code_tables(X, bits, order, table):
     """Thresholds bracketed around the middle of a gap, the table taken as it stands where it ascends: codes, maxima and
-    the dequantized matrix are the oracle's, bit for bit (small matrices search, large ones use the bucket table)."""
+    the dequantized matrix are the oracle's, bit for bit, on either side of every threshold and of the bracket's ends (small
+    matrices search, ragged ones in chunks, large ones use the bucket table)."""
     import numpy as np
     import qtensor.functional as F
     from oracle import quant_np as Q
-    n = 1 << bits
-    g = torch.Generator().manual_seed(n)
-    code = F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)
-    if table == "descending":
-        code = code.flip(0).contiguous()
-    elif table == "shuffled":
-        code = code[torch.randperm(n, generator=g)].contiguous()
-    elif table == "repeated":
-        code = code.clone()
-        code[n // 4:n // 2] = code[n // 4]
-    elif table == "neighbours":                                            # gaps of one, two, ... values of fp32 around a half
-        code = (0.5 + torch.cumsum(torch.arange(n), 0).double() * 2.0 ** -24).float()
-    elif table == "tiny":                                                  # thresholds too near zero for the fast quotient
-        code = code * 2.0 ** -60
-    else:                                                                  # one gap over many binades on either side of zero
-        code = torch.cat([torch.tensor([-1.0, -2.0 ** -40, 0.0]), torch.linspace(2.0 ** -20, 1.0, n - 3)])
-    A = torch.randn(order, order, generator=g)
-    A.view(-1)[:n] = code.abs().max() * code                                  # values at the entries themselves
-    out, absmax = F.quantize_blockwise(A.cuda(), code.cuda(), order, blocksize=64, bits=bits)
-    back = F.dequantize_blockwise(out, code.cuda(), order, absmax, blocksize=64, bits=bits)
-    want, want_absmax = Q.quantize_c(A.numpy(), code.numpy(), order, 64, bits, False)
-    assert np.array_equal(out.cpu().numpy(), want) and np.array_equal(absmax.cpu().numpy(), want_absmax)
-    assert np.array_equal(back.cpu().numpy(), Q.dequantize_c(want, code.numpy(), order, want_absmax, bits=bits, blocksize=64))
+    code = table_of(table, bits)
+    values, below, above = around_the_thresholds(code)
+    # segments of 64 with a 1 in each, so that the quotients are the values themselves (a row of 66 has a short one as well)
+    g = torch.Generator().manual_seed(order)
+    per = order * (order - -(-order // 64))
+    count = -(-len(values) // per)
+    rows = torch.ones(count * order, order)
+    free = torch.arange(order) % 64 != 0
+    fill = torch.from_numpy(np.resize(values, count * per).copy())[torch.randperm(count * per, generator=g)]
+    rows[:, free] = fill.view(count * order, -1)
+    seen, want_code = [], []
+    for A in rows.view(count, order, order):
+        want, want_absmax = Q.quantize_c(A.numpy(), code.numpy(), order, 64, bits, False)
+        assert (want_absmax == 1.0).all()
+        out, absmax = F.quantize_blockwise(A.cuda(), code.cuda(), order, blocksize=64, bits=bits)
+        back = F.dequantize_blockwise(out, code.cuda(), order, absmax, blocksize=64, bits=bits)
+        assert np.array_equal(out.cpu().numpy(), want) and np.array_equal(absmax.cpu().numpy(), want_absmax)
+        assert np.array_equal(back.cpu().numpy(), Q.dequantize_c(want, code.numpy(), order, want_absmax, bits=bits, blocksize=64))
+        seen.append(A.numpy().ravel())
+        ids = want if bits == 8 else np.stack([want >> 4, want & 15], 1).ravel()
+        want_code.append(code.numpy()[ids[:order * order]])
+    # the matrices held both sides of every gap's threshold, and the oracle put them on different entries
+    seen, want_code = np.concatenate(seen), np.concatenate(want_code)
+    entry_of = dict(zip(seen.tolist(), want_code.tolist()))
+    assert all(entry_of[b] < entry_of[a] for b, a in zip(below.tolist(), above.tolist()))
 
 
 @pytest.mark.parametrize("trans", ["", "a", "b"])
