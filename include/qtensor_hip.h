@@ -95,8 +95,8 @@ void cdequantize_blockwise_diagreal_4bit_bf16_stream(unsigned char *A, float *co
  * diagonal entries, ceil(order * order * bits / 8) code bytes per matrix: the codes of an odd order are
  * padded to a whole byte per matrix).  batch*order*order < 2^31.  With blocksize dividing order and
  * 16-byte aligned A/out the whole stack is one stream of segments (the fast path); any other order goes
- * through the general path, one matrix per grid row, at most 65535 matrices per launch.  diag == NULL
- * selects the plain form. */
+ * through the general path, at most 65535 matrices per launch (a limit of the dequantizer's grid, kept the
+ * same for both directions).  diag == NULL selects the plain form. */
 void qtensor_hip_quantize_batched(const void *A, int a_is_bf16, const float *code, int bits, int order, int batch,
                                   float *absmax, float *diag, unsigned char *out, int blocksize, qtensor_stream_t stream);
 void qtensor_hip_dequantize_batched(const unsigned char *q, const float *code, int bits, int order, int batch,

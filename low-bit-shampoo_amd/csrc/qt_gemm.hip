@@ -1393,7 +1393,7 @@ void launch_gemm(const GemmArgs &a, int batch, hipStream_t stream) {
     if (blocks > 0x7fffffffLL) { set_error(kBadArgument, "gemm: too many tiles (%lld)", blocks); return; }
     if constexpr (PREC == kPipeSplit && BM == 64 && BN == 64 && KA < kQuant4 && KB < kQuant4 && EPI <= kAxpbyDense) {
         // Loads far ahead where the launch's own workgroups have a unit each and half of the units stay free: a per-parameter
-        // optimizer step over convolution weights, chains of products of 2 to 38 tiles, 34.4 -> 31.4 ms.  Both lines are
+        // optimizer step over convolution weights, chains of products of 2 to 38 tiles, 34.1 -> 32.3 ms.  Both lines are
         // measured.  Workgroups: at one or two per unit the step is the same to the noise, and for every launch the
         // stacks lose (a step that takes statistics in 3.81 -> 3.92 ms): other workgroups hide the latency there and the
         // registers cost occupancy.  (A launch on another stream may share the units all the same.)  k tiles of a
