@@ -96,8 +96,24 @@ struct PivotOutcome {
 };
 struct PivotNotes {                      // (LDS) one slot per wave
     unsigned long long dropped[kCholWaves];
-    int failed[kCholWaves];
+    int failed[kCholWaves];              // bit 0: as above; bit 1: a pivot that is not finite
 };
+
+// A right-hand side of the forward substitution is zero down to its one, and factor64 leaves out those blocks.  Zero times
+// a number that is not finite is a NaN all the same, and from then on so is everything below it: right-hand side c is NaN
+// from the first row j on whose L[j][k] is not finite for some k < c.  (Such a number always makes the pivot of row j one
+// that is not finite.)
+__device__ __forceinline__ void spread_not_finite(const float *a, float *y) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int first = NB;                          // of row `lane`
+    for (int k = NB - 1; k >= 0; --k)
+        if (k < lane && !(fabsf(a[lane * LDC + k]) < __builtin_inff())) first = k;
+    bool gone = false;                       // in right-hand side `lane`
+    for (int j = 0; j < NB; ++j) {
+        gone = gone || __builtin_amdgcn_readlane(first, j) < lane;
+        if (gone && j % kCholWaves == wave) y[j * LDC + lane] = __builtin_nanf("");
+    }
+}
 
 // `a` (64 rows, LDC floats apart): the lower triangle of a symmetric matrix on entry, L on exit (above the diagonal
 // blocks: undefined).  `y`: L^-1 on exit, zeros above its diagonal.  All 256 threads of a workgroup; the call begins and
@@ -178,7 +194,8 @@ __device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes 
                 __builtin_amdgcn_sched_barrier(0);
             }
             const bool mine = (lane >> 4) == p;
-            const unsigned long long replaced = __ballot(mine && !(own > pivot_floor)), not_a_number = __ballot(mine && own != own);
+            const unsigned long long replaced = __ballot(mine && !(own > pivot_floor)), not_a_number = __ballot(mine && own != own),
+                                     not_finite = __ballot(mine && !(fabsf(own) < __builtin_inff()));
 #pragma unroll
             for (int q = 0; q < kCholCols; q += 4)
                 *reinterpret_cast<float4 *>(a + lane * LDC + c0 + q) = make_float4(row[q], row[q + 1], row[q + 2], row[q + 3]);
@@ -186,7 +203,7 @@ __device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes 
             for (int jj = 0; jj < kCholCols; ++jj) y[(c0 + jj) * LDC + lane] = s[jj];
             if (lane == 0) {
                 notes.dropped[p] = pivot_floor > 0.0f ? replaced & ~not_a_number : 0ull;
-                notes.failed[p] = (pivot_floor > 0.0f ? not_a_number : replaced) != 0 ? 1 : 0;
+                notes.failed[p] = ((pivot_floor > 0.0f ? not_a_number : replaced) != 0 ? 1 : 0) | (not_finite != 0 ? 2 : 0);
             }
         }
         __syncthreads();
@@ -210,6 +227,11 @@ __device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes 
     PivotOutcome out = {0, 0};
 #pragma unroll
     for (int w = 0; w < kCholWaves; ++w) { out.dropped |= notes.dropped[w]; out.failed |= notes.failed[w]; }
+    if ((out.failed & 2) != 0) {                 // (uniform over the workgroup)
+        spread_not_finite(a, y);
+        __syncthreads();
+    }
+    out.failed &= 1;
     return out;
 }
 

@@ -108,6 +108,32 @@ def test_64_column_factor_keeps_the_column_of_a_pivot_that_fails(X, column):
     assert column == 63 or bool((row[column + 1:] > 0).all())
 
 
+@pytest.mark.parametrize("row,column", [(0, 1), (3, 12), (3, 20), (21, 32), (21, 60), (33, 40), (50, 63), (62, 63)])
+@pytest.mark.parametrize("entry", [float("nan"), float("inf")])
+def test_64_column_inverse_of_a_factor_that_is_not_finite_is_the_column_by_column_recurrence(X, entry, row, column):
+    """Where the forward substitution meets a NaN (zero times a number that is not finite is one) the inverse has it."""
+    import numpy as np
+    gram = (torch.eye(64) + 2.0 ** -8 * torch.triu(torch.ones(64, 64), 1)).repeat(2, 1, 1)
+    gram[0, row, column] = entry
+    for floor in (2e-4, 0.0):
+        U, inv, info = torch.zeros(2, 64, 64, device="cuda"), torch.zeros(2, 64, 64, device="cuda"), torch.zeros(2, dtype=torch.int32, device="cuda")
+        X.cholesky_upper(gram.cuda(), U, inv, info, pivot_floor=floor)
+        assert info[0].item() != 0 and info[1].item() == 0 and bool(torch.isfinite(inv[1]).all())   # (an infinite entry makes a pivot of minus infinity: dropped with a floor)
+        a, s = gram[0].numpy().T.copy(), np.eye(64, dtype=np.float32)
+        with np.errstate(invalid="ignore"):
+            for k in range(64):
+                d = a[k, k]
+                dropped = bool(d <= floor) and floor > 0
+                d = np.float32(floor) if dropped else d if d > floor else np.float32(1.0)
+                r = np.float32(1.0) / np.sqrt(d)
+                L = np.where(np.arange(64) > k, 0.0, d * r).astype(np.float32) if dropped else a[:, k] * r
+                s[k] *= r
+                for j in range(k + 1, 64):
+                    a[j:, j] -= L[j:] * L[j]
+                    s[j] -= L[j] * s[k]
+        assert np.isnan(s).any() and np.array_equal(np.isnan(inv[0].cpu().numpy()), np.isnan(s.T))
+
+
 @pytest.mark.parametrize("order,blocksize", [(1, 64), (3, 64), (27, 64), (66, 64), (100, 64), (129, 128), (255, 256), (260, 2048),
                                              (1200, 64), (1201, 64), (1202, 512), (2049, 2048), (4099, 2048)])
 @pytest.mark.parametrize("bits", [4, 8])
