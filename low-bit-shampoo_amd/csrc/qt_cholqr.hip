@@ -124,7 +124,7 @@ __device__ __forceinline__ void spread_not_finite(const float *a, float *y) {
 // does not: its residual on ill-conditioned panels was up to three times as large.)
 // What bounds it is the chain of the 64 pivots (about 250 cycles each: the pivot through v_readlane, v_rsq_f32 and one
 // Newton step, the column, the next pivot, with the multiply-adds of the step before in its shadow).  Back to back a launch
-// takes 12.4 us for one matrix and 13.1 for 99; with the trailing updates and the substitution behind a block as vector
+// takes 12.5 us for one matrix and 13.1 for 99; with the trailing updates and the substitution behind a block as vector
 // multiply-adds of the waves behind (300 cycles a step on top of 300 for the pivot) it took 15.4 and 16.3, with the
 // inverse from the inverses of diagonal blocks 12.0 and 12.7.
 __device__ __forceinline__ PivotOutcome factor64(float *a, float *y, PivotNotes &notes, float pivot_floor) {
