@@ -318,8 +318,8 @@ def test_threshold_tables_of_unusual_code_tables(X, bits, order, table):
 @pytest.mark.parametrize("k", [32, 48, 64, 80, 96, 112, 144, 1216])
 @pytest.mark.parametrize("m,n", [(64, 64), (65, 128), (2, 3), (200, 70)])
 def test_products_of_a_few_tiles_equal_the_same_products_in_a_large_stack(X, m, n, k, trans):
-    """Loads several k tiles ahead (k ranges around the number of register sets, ragged tiles): the bits of the large stack's
-    kernels, and fp32 accuracy against float64; beta E + alpha A B over it as well."""
+    """Loads several k tiles ahead (from k = 64 on; k ranges around the number of register sets, ragged tiles): the bits of the
+    large stack's kernels, and fp32 accuracy against float64; beta E + alpha A B over it as well."""
     g = torch.Generator().manual_seed(m + n + k)
     A, B = torch.randn(m, k, generator=g), torch.randn(k, n, generator=g)
     a = (A.T if trans == "a" else A).contiguous().cuda()
