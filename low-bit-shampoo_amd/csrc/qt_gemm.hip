@@ -1,7 +1,8 @@
 // Products of fp32 matrices on the gfx950 matrix cores, with blockwise quantized operands expanded on their
 // way into LDS and the Shampoo epilogues fused in.  Two pipes: the fp32 one (v_mfma_f32_32x32x2_f32) and, by
 // default, the bf16 one on operands split into three bf16 pieces each (v_mfma_f32_32x32x16_bf16, six products
-// per fp32 product, fp32 accumulation: fp32-grade results at a multiple of the rate; see kPipeSplit below).
+// per fp32 product, fp32 accumulation: fp32-grade results at a multiple of the rate; see kPipeSplit below).  Where the
+// caller knows how large the operands' elements are, a third one on operands split into two fp16 pieces (qt_half.h).
 //
 // What the reference does with separate steps
 //   P = dequantize(Pq);  out = P @ G            (optimizers/shampoo2.py:255-268, shampoo1.py:224-237)
@@ -22,8 +23,10 @@
 // consecutive words per step.  Global loads run two tiles ahead of the MFMAs; the LDS commit sits
 // in the middle of the MFMA stream.  (Split pipe: three bf16 planes per operand tile, [half of k][row][8].)
 #include "qt_common.h"
+#include "qt_half.h"
 #include "qt_tables.h"
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstring>
@@ -97,6 +100,12 @@ struct GemmArgs {
     int pipe;                     // 0: the process-wide choice (qtensor_hip_gemm_pipe); 1: the fp32 pipe; 2: the split bf16 pipe
 };
 
+// What a launch on the half pipe takes besides.
+struct RangedArgs : GemmArgs {
+    const uint32_t *amax_a, *amax_b;    // per batch entry: bits of (a bound of) the operand's largest |element|
+    uint32_t *amax_out;                 // optional, per batch entry: raised to the bits of the result's largest |element|
+};
+
 namespace {
 
 constexpr int BK = 16;
@@ -106,7 +115,7 @@ constexpr int BK = 16;
 // a_h b_l + a_l b_h + a_m b_m, each exact in fp32, accumulated in fp32 by v_mfma_f32_32x32x16_bf16.  The terms left out
 // are below 2^-24 |a b|: the error of a dot product stays that of fp32 arithmetic, and the bf16 pipe does sixteen times
 // the multiply-adds per cycle of the fp32 pipe, six of which make one fp32 multiply-add.
-constexpr int kPipeF32 = 0, kPipeSplit = 1;
+constexpr int kPipeF32 = 0, kPipeSplit = 1, kPipeHalf = 2;          // (kPipeHalf: qt_half.h)
 constexpr uint32_t kDies = 8;          // accelerator dies (XCDs) of an MI355X
 constexpr int LDS_PAD = 4;   // k-major tiles ([k][row]): row stride = rows + 4 floats, 16-byte aligned rows
 constexpr int LDK = BK + 4;  // row-major tiles ([row][k], for sources whose k is contiguous): 20 floats per row, so
@@ -620,12 +629,14 @@ struct LoadQuant {
     }
 };
 
+// (the 256-entry tables of the 8-bit re-encoding leave LDS for two; the half pipe's two accumulators take 128 registers)
 template <int BM, int BN, int KA, int KB, int EPI, int PREC>
-constexpr int kWavesPerSimd = (PREC == kPipeSplit && BM == 128 && BN == 128 &&
-                               (KA >= kQuant4 || KB >= kQuant4 || EPI == kRequant8)) ? 2 : 3;   // (the 256-entry tables of the 8-bit re-encoding leave LDS for two)
+constexpr int kWavesPerSimd = (PREC >= kPipeSplit && BM == 128 && BN == 128 &&
+                               (KA >= kQuant4 || KB >= kQuant4 || EPI == kRequant8 || PREC == kPipeHalf)) ? 2 : 3;
+template <int PREC> using KernelArgs = typename std::conditional<PREC == kPipeHalf, RangedArgs, GemmArgs>::type;
 
 template <int BM, int BN, int KA, int KB, int EPI, int PREC = kPipeF32, bool DEEP = false>
-__global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) void gemm_kernel(const GemmArgs args) {   // three waves per SIMD mean at most 168 registers, two 256
+__global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) void gemm_kernel(const KernelArgs<PREC> args) {   // three waves per SIMD mean at most 168 registers, two 256
     constexpr int WM = BM / 2, WN = BN / 2, MI = WM / 32, NI = WN / 32;
     // Workgroups are dealt round-robin to the 8 accelerator dies, each with its own L2.  Renumber
     // them so that every die works through one contiguous run of (batch entry, tile row, tile
@@ -654,7 +665,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     const int slices = EPI == kStore && !streamed ? args.split_k : 1;
     const int slice = id % slices;
     id /= slices;
-    constexpr bool kSplit = PREC == kPipeSplit;
+    constexpr bool kSplit = PREC >= kPipeSplit;
 
     using PlainA = typename std::conditional<KA == kDense, LoadKContig<BM>,
         typename std::conditional<KA == kDenseT, LoadRowContig<BM>,
@@ -678,7 +689,9 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     // a 32 x 32 staging square per wave that turns accumulator blocks around for the mirrored stores
     constexpr bool kRequant = EPI == kRequant4 || EPI == kRequant8;
     constexpr int SPLIT_A = SplitLayout<BM>::kOperand, SPLIT_STAGE = SPLIT_A + SplitLayout<BN>::kOperand;     // bytes
-    constexpr int STAGE_LD = 36, REQUANT_LD = 68, SIZE_MAIN = kSplit ? 2 * SPLIT_STAGE / 4 : 2 * SIZE_A + 2 * SIZE_B;
+    constexpr int HALF_STAGE = HalfLayout<BM>::kOperand + HalfLayout<BN>::kOperand;
+    constexpr int SPLIT_MAIN = 2 * (PREC == kPipeHalf && HALF_STAGE > SPLIT_STAGE ? HALF_STAGE : SPLIT_STAGE) / 4;
+    constexpr int STAGE_LD = 36, REQUANT_LD = 68, SIZE_MAIN = kSplit ? SPLIT_MAIN : 2 * SIZE_A + 2 * SIZE_B;
     constexpr int SIZE_STAGE = kRequant ? 4 * 32 * REQUANT_LD : 4 * 32 * STAGE_LD;
     __shared__ __attribute__((aligned(16))) float s_mem[SIZE_MAIN > SIZE_STAGE ? SIZE_MAIN : SIZE_STAGE];
     float (*s_a)[SIZE_A] = reinterpret_cast<float (*)[SIZE_A]>(s_mem);
@@ -871,6 +884,46 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
             }
         }
     } else {
+    bool again = true;                         // half pipe: the tile is left to the bf16 split
+    if constexpr (PREC == kPipeHalf) {
+        __shared__ uint32_t s_top[BM + BN];
+        float sa, sb, ia, ib;
+        // (rows that are not 16-byte aligned inside a list of pointers are only seen here)
+        if (half_scale(args.amax_a[b], sa, ia) && half_scale(args.amax_b[b], sb, ib) && (KA != kDense || a_vec) && (KB != kDenseT || b_vec)) {
+            constexpr int SETS = BM == 128 && BN == 128 ? 1 : 2;           // smaller tiles: less to do per tile to hide a load behind, and registers to spare
+            typename std::conditional<KA == kDense, HalfKContig<BM, SETS>, HalfRowContig<BM, SETS>>::type ha;
+            typename std::conditional<KB == kDenseT, HalfKContig<BN, SETS>, HalfRowContig<BN, SETS>>::type hb;
+            f32x16 rest[MI][NI];
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) rest[i][j][r] = 0.0f;
+            for (int i = threadIdx.x; i < BM + BN; i += 256) s_top[i] = 0;
+            ha.prepare(args.lda, m0, args.M);
+            hb.prepare(args.ldb, n0, args.N);
+            const int half_tiles = n_tiles * BK / HK;
+            auto at_k = [&](int t) { return (long long)(k_begin + min(t, half_tiles - 1) * HK); };
+            auto src_a = [&](int t) { return whole_range(A + (KA == kDense ? (long long)m0 * args.lda + at_k(t) : at_k(t) * args.lda + m0)); };
+            auto src_b = [&](int t) { return whole_range(B + (KB == kDenseT ? (long long)n0 * args.ldb + at_k(t) : at_k(t) * args.ldb + n0)); };
+            half_main_loop<BM, BN, SETS>(reinterpret_cast<unsigned char *>(s_mem), ha, hb, src_a, src_b, half_tiles, sa, sb, acc, rest);
+            ha.tops(s_top);
+            hb.tops(s_top + BM);
+            __syncthreads();
+            bool fine = true;
+            for (int i = threadIdx.x; i < BM + BN; i += 256) fine &= half_row_fine(s_top[i]);
+            again = __syncthreads_or(!fine) != 0;
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        acc[i][j][r] = again ? 0.0f : __builtin_fmaf(rest[i][j][r], 1.0f / kRestScale, acc[i][j][r]) * ia * ib;
+        }
+    }
+    if (again) {
     fetch(k_begin);
     commit(0);
     if (n_tiles > 1) fetch(k_begin + BK);
@@ -980,6 +1033,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                 }
         }
         __syncthreads();
+    }
     }
     }
 
@@ -1135,7 +1189,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         }
         return;
     }
-    float local_err = 0.0f;
+    float local_err = 0.0f, local_top = 0.0f;
     // Each wave passes its accumulator blocks (32 x 32) through a staging square of its own in LDS, so that a
     // lane ends up with four consecutive elements of one output row: 16-byte stores, eight lanes per 128-byte
     // line, and one packed load per four elements of a quantized addend.
@@ -1182,6 +1236,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                         }
                         gstore4(T + (long long)row * args.ldt + col4, t);
                     }
+                    if constexpr (PREC == kPipeHalf) local_top = fmaxf(fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3]))), local_top);
                     gstore4(C + (long long)row * ldc + col4, y);
                 }
                 wave_lds_sync();
@@ -1204,6 +1259,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                         local_err = fmaxf(local_err, fabsf(y - eye));
                         gstore(T + (long long)row * args.ldt + col, (1.0f - args.newton_w) * eye + args.newton_w * y);
                     }
+                    if constexpr (PREC == kPipeHalf) local_top = fmaxf(fabsf(y), local_top);
                     gstore(C + (long long)row * ldc + col, y);
                 }
             }
@@ -1240,6 +1296,8 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                     else if (kQuantAddend) y[q] = __builtin_fmaf(args.alpha, a[q], args.beta * e[q]);
                     else y[q] = a[q];
                 }
+                // (past the end of a row: a repeated row's products, elements of the result like the others)
+                if constexpr (PREC == kPipeHalf) local_top = fmaxf(fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3]))), local_top);
                 float *cm = C + (long long)mrow * ldc + mcol;
                 if (whole) gstore4(cm, y);
                 else
@@ -1261,6 +1319,12 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     if (EPI == kNewton) {
         uint32_t e = group_max_u32<64>(__float_as_uint(local_err));   // non-negative floats order like their bits
         if (lane == 0) atomicMax(reinterpret_cast<unsigned int *>(args.err) + b, e);
+    }
+    if constexpr (PREC == kPipeHalf) {
+        if (args.amax_out != nullptr) {
+            const uint32_t e = group_max_u32<64>(__float_as_uint(local_top));
+            if (lane == 0) atomicMax(args.amax_out + b, e);
+        }
     }
     if (!streamed) return;
     run_at += seg_tiles;
@@ -1381,8 +1445,37 @@ __global__ __launch_bounds__(256) void reduce_slices_kernel(const float *workspa
     }
 }
 
+// out[b] = max(out[b], max |element|) as bits (infinities and NaN above everything finite), over the rows x cols matrices
+// of a batch; grid (pieces of `rows_per` rows, batch).  Bound by memory: 415 MB in 0.08 ms.
+__global__ __launch_bounds__(256) void amax_kernel(BatchPtr mats, int ld, int rows, int cols, int rows_per, int inner, long long inner_stride,
+                                                   uint32_t *out) {
+    const int b = blockIdx.y, r0 = blockIdx.x * rows_per, r1 = min(rows, r0 + rows_per);
+    const float *base = dense_ptr(mats, b, inner, inner_stride);
+    uint32_t top = 0;
+    if ((ld & 3) == 0 && (cols & 3) == 0 && is_aligned16(base)) {
+        const int quads = cols >> 2;
+        for (int q = threadIdx.x; q < (r1 - r0) * quads; q += 256) {
+            const float4 x = gload4(base + (long long)(r0 + q / quads) * ld + (q % quads << 2));
+            top = max(max(max(__float_as_uint(x.x) & 0x7fffffffu, __float_as_uint(x.y) & 0x7fffffffu),
+                          max(__float_as_uint(x.z) & 0x7fffffffu, __float_as_uint(x.w) & 0x7fffffffu)), top);
+        }
+    } else {
+        for (int q = threadIdx.x; q < (r1 - r0) * cols; q += 256)
+            top = max(__float_as_uint(gload(base + (long long)(r0 + q / cols) * ld + q % cols)) & 0x7fffffffu, top);
+    }
+    top = group_max_u32<64>(top);
+    if ((threadIdx.x & 63) == 0 && top != 0) atomicMax(out + b, top);
+}
+
+void launch_amax(const BatchPtr &mats, int ld, int rows, int cols, int batch, int inner, long long inner_stride, uint32_t *out, hipStream_t stream) {
+    // 16 K elements a workgroup: 64 a thread
+    const int rows_per = (int)std::max(1ll, std::min((long long)rows, 16384ll / cols));
+    hipLaunchKernelGGL(amax_kernel, dim3((unsigned)((rows + rows_per - 1) / rows_per), (unsigned)batch), dim3(256), 0, stream, mats, ld, rows,
+                       cols, rows_per, inner, inner_stride, out);
+}
+
 template <int BM, int BN, int KA, int KB, int EPI, int PREC = kPipeF32>
-void launch_gemm(const GemmArgs &a, int batch, hipStream_t stream) {
+void launch_gemm(const RangedArgs &a, int batch, hipStream_t stream) {
     const long long tn = (a.N + BN - 1) / BN, tm = (a.M + BM - 1) / BM;
     if (a.symmetric && BM != BN) { set_error(kBadArgument, "gemm: symmetric products need square tiles"); return; }
     long long blocks = (a.symmetric ? tn * (tn + 1) / 2 : tn * tm) * batch * (EPI == kStore ? a.split_k : 1);
@@ -1497,7 +1590,11 @@ StaticScratch *static_scratch() {
     return &slot;
 }
 
-void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint = -1);
+struct Ranges {                          // qtensor_gemm_ranges
+    const float *amax_a, *amax_b;
+    float *amax_out;
+};
+void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint = -1, const Ranges *ranges = nullptr);
 
 // Process-wide choice of the matrix pipe (qtensor_hip_gemm_pipe); starts from the
 // environment variable QT_GEMM_PIPE ("f32" or "split"), else the split pipe.
@@ -1538,6 +1635,24 @@ extern "C" int qtensor_hip_gemm_pipe(int mode) {
 extern "C" void qtensor_hip_gemm(const qtensor_gemm_desc *d, void *stream_v) {
     qt::clear_error();
     gemm_dispatch(d, (hipStream_t)stream_v);
+}
+
+extern "C" void qtensor_hip_gemm_ranged(const qtensor_gemm_desc *d, const void *ranges, void *stream_v) {
+    qt::clear_error();
+    gemm_dispatch(d, (hipStream_t)stream_v, -1, static_cast<const Ranges *>(ranges));
+}
+
+extern "C" void qtensor_hip_amax_batched(const void *mats, int ld, int rows, int cols, int batch, float *out, void *stream_v) {
+    using namespace qt;
+    clear_error();
+    if (mats == nullptr || out == nullptr) { set_error(kNullPointer, "amax: null pointer"); return; }
+    const BatchPtr &p = *static_cast<const BatchPtr *>(mats);
+    if (rows < 1 || cols < 1 || ld < cols || batch < 1 || batch > 65535 || !has_host_ptr(p)) {
+        set_error(kBadArgument, "amax: need rows, cols >= 1, ld >= cols, 1 <= batch <= 65535 and a matrix (got %d x %d, ld %d, batch %d)", rows, cols, ld, batch);
+        return;
+    }
+    launch_amax(p, ld, rows, cols, batch, 1, 0, reinterpret_cast<uint32_t *>(out), (hipStream_t)stream_v);
+    launch_ok("amax");
 }
 
 extern "C" void qtensor_hip_gemm_static(const qtensor_gemm_desc *d, void *stream_v) {
@@ -1598,10 +1713,11 @@ void qt::gemm_with_tile(const qtensor_gemm_desc *d, hipStream_t stream, int tile
 }
 
 namespace {
-void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint) {
+void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint, const Ranges *ranges) {
     using namespace qt;
     if (!d) { set_error(kNullPointer, "gemm: null descriptor"); return; }
-    GemmArgs a = d->args;
+    RangedArgs a = {};
+    static_cast<GemmArgs &>(a) = d->args;
     a.M = d->M; a.N = d->N; a.K = d->K;
     if (d->M < 1 || d->N < 1 || d->K < 1 || d->batch < 1 || d->batch > 65535) {
         set_error(kBadArgument, "gemm: need M, N, K >= 1 and 1 <= batch <= 65535 (got %d %d %d, batch %d)", d->M, d->N, d->K, d->batch);
@@ -1635,6 +1751,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         if (requant && a.Eq.bs_shift != 6) { set_error(kBadArgument, "gemm: the requantizing epilogue needs blocksize 64"); return; }
     }
     if (ep == kNewton && (!has_host_ptr(a.T) || a.ldt < d->N || !a.err)) { set_error(kBadArgument, "gemm: Newton epilogue needs T and err"); return; }
+    if (ranges != nullptr && ranges->amax_out != nullptr && requant) { set_error(kBadArgument, "gemm: a re-encoded result has no amax_out"); return; }
     a.symmetric = a.symmetric != 0;
     a.batch_count = d->batch;
     a.stream_per = a.stream_lcm = 0;
@@ -1654,9 +1771,9 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
     // share its matrix pipes, so the time is (most tiles on one unit) x (tile area) / (efficiency of
     // that shape: smaller tiles read more LDS words per multiply).
     // (measured with thousands of tiles, 99 x 1024^3: 189 / 163 / 166 / 146 TFLOP/s on the split pipe -- a smaller tile splits
-    // more operand elements per product -- and 126 / 119 / 123 / 117 on the fp32 pipe)
-    struct Shape { int bm, bn; double eff, eff_split; };
-    static const Shape shapes[4] = {{128, 128, 1.0, 1.0}, {128, 64, 0.95, 0.87}, {64, 128, 0.97, 0.88}, {64, 64, 0.93, 0.77}};
+    // more operand elements per product -- 126 / 119 / 123 / 117 on the fp32 pipe and 279 / 239 / 234 / 206 on the half pipe)
+    struct Shape { int bm, bn; double eff, eff_split, eff_half; };
+    static const Shape shapes[4] = {{128, 128, 1.0, 1.0, 1.0}, {128, 64, 0.95, 0.87, 0.85}, {64, 128, 0.97, 0.88, 0.84}, {64, 64, 0.93, 0.77, 0.74}};
     // The split pipe: for whole k tiles, where the offsets of the dense operands' loads fit 31 bits -- whatever the tile
     // shape, so that the bits of a product do not depend on how it is tiled.
     bool split_pipe = false;
@@ -1669,6 +1786,16 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         const bool near_a = ka >= kQuant4 || a.lda < (1 << 22), near_b = kb >= kQuant4 || a.ldb < (1 << 22);
         split_pipe = reach_a < 0x7fffffffLL && reach_b < 0x7fffffffLL && near_a && near_b;
     }
+    // The half pipe: dense operands of known size, whole lines of k, and k long enough for its fewer roundings to outweigh
+    // the bit it does not keep (qt_half.h).  A rule on one product's own extents alone: the bits of a matrix's result
+    // depend neither on the batch it is in nor on the tile shape (save for tiles with rows of extreme size).
+    if (ranges != nullptr) {
+        a.amax_a = reinterpret_cast<const uint32_t *>(ranges->amax_a);
+        a.amax_b = reinterpret_cast<const uint32_t *>(ranges->amax_b);
+        a.amax_out = reinterpret_cast<uint32_t *>(ranges->amax_out);
+    }
+    const bool half_pipe = split_pipe && a.amax_a != nullptr && a.amax_b != nullptr && ka < kQuant4 && kb < kQuant4 && d->K % HK == 0 &&
+                           d->K >= kHalfLeastK && (ka != kDense || a.lda % 4 == 0) && (kb != kDenseT || a.ldb % 4 == 0);
     int pick = 0;
     static const char *forced = QT_KNOB("QT_GEMM_TILE");
     if (forced != nullptr) {
@@ -1689,7 +1816,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
             // another one's products: measured 0.56 of the rate reached with three per unit, 0.92 with two
             const double most = ceil(tiles / units);
             const double overlap = most <= 1.0 ? 0.56 : most <= 2.0 ? 0.92 : 1.0;
-            const double cost = most * sh.bm * sh.bn / ((split_pipe ? sh.eff_split : sh.eff) * overlap);
+            const double cost = most * sh.bm * sh.bn / ((half_pipe ? sh.eff_half : split_pipe ? sh.eff_split : sh.eff) * overlap);
             if (i == 0 || cost < best) { best = cost; pick = i; }
         }
     }
@@ -1729,7 +1856,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         int best_split = 1;
         static const char *forced_split = QT_KNOB("QT_GEMM_SPLIT");
         for (int sp = 2; sp <= 8; ++sp) {
-            if (k_tiles % sp != 0 || k_tiles / sp < 8) continue;
+            if (k_tiles % sp != 0 || k_tiles / sp < 8 || (half_pipe && k_tiles / sp % 2 != 0)) continue;
             if ((long long)sp * d->batch * d->M * d->N > a.workspace_floats) continue;
             const double cost = cost_of(sp);
             if (forced_split != nullptr) { if (sp == atoi(forced_split)) best_split = sp; }
@@ -1768,10 +1895,19 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
             }
         }
     }
+    // (a product that is not made by one launch on the half pipe has its largest element looked up afterwards)
+    uint32_t *const amax_later = half_pipe && a.split_k == 1 ? nullptr : a.amax_out;
+    if (amax_later != nullptr) a.amax_out = nullptr;
     const int combo = ka * 100 + kb * 10 + ep;
 #define QT_GEMM_CASE_DENSE(KA, KB, EP)                                                                       \
     case (KA) * 100 + (KB) * 10 + (EP):                                                                      \
-        if (split_pipe) {                                                                                    \
+        if (half_pipe) {                                                                                     \
+            if (pick == 0) launch_gemm<128, 128, KA, KB, EP, kPipeHalf>(a, d->batch, stream);                \
+            else if (pick == 1) launch_gemm<128, 64, KA, KB, EP, kPipeHalf>(a, d->batch, stream);            \
+            else if (pick == 2) launch_gemm<64, 128, KA, KB, EP, kPipeHalf>(a, d->batch, stream);            \
+            else launch_gemm<64, 64, KA, KB, EP, kPipeHalf>(a, d->batch, stream);                            \
+        }                                                                                                    \
+        else if (split_pipe) {                                                                               \
             if (pick == 0) launch_gemm<128, 128, KA, KB, EP, kPipeSplit>(a, d->batch, stream);               \
             else if (pick == 1) launch_gemm<128, 64, KA, KB, EP, kPipeSplit>(a, d->batch, stream);           \
             else if (pick == 2) launch_gemm<64, 128, KA, KB, EP, kPipeSplit>(a, d->batch, stream);           \
@@ -1824,6 +1960,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
             set_error(kBadArgument, "gemm: combination A kind %d, B kind %d, epilogue %d is not built", ka, kb, ep);
             return;
     }
+    if (amax_later != nullptr) launch_amax(a.C, a.ldc, a.M, a.N, d->batch, a.batch_inner, a.inner_c, amax_later, stream);
 #undef QT_GEMM_CASE_DENSE
 #undef QT_GEMM_CASE_REQUANT
 #undef QT_GEMM_CASE_QUANT

@@ -161,6 +161,12 @@ def ComputePowerBatched(mats, p=4, iter_count=10, error_tolerance=1e-6, ridge_ep
 
     R_ptr, M_ptr, T_ptr = table(R), table(M), table(T)
     side = torch.zeros(B, dtype=torch.bool, device=dev)                     # False: buffer 0 holds the state
+    # How large the iterates' elements are, for the pipe that wants to know: |M| and |T| follow from err = max |M - I|
+    # (T = I + w (M - I)), the roots and the powers of T are looked at by the launches that write them.
+    squarings = p.bit_length() - 1
+    tops = torch.zeros(iter_count, 1 + squarings, B, device=dev)
+    top_m, top_t = 1 + err, 1 + abs(w) * err
+    top_r = first_root * top_t                                               # of the root after the first round
     for round_number in range(iter_count):
         skip = done.to(torch.int32)
         cur = lambda tab: torch.where(side, tab[1], tab[0])                   # noqa: E731
@@ -172,16 +178,17 @@ def ComputePowerBatched(mats, p=4, iter_count=10, error_tolerance=1e-6, ridge_ep
             torch.mul(T[0], first_root.view(B, 1, 1), out=R[1])
         else:
             X.gemm(X.PtrList(Rc, shape), X.PtrList(Tc, shape), out=X.PtrList(Ro, shape), skip=skip,
-                   symmetric=symmetric)                                      # candidate root
-        power = X.PtrList(Tc, shape)                                         # T^p by repeated squaring
-        done_p = 1
-        while done_p < p:
+                   symmetric=symmetric, amax=(top_r, top_t), amax_out=tops[round_number, 0])     # candidate root
+            top_r = tops[round_number, 0]                                    # (a rejected candidate ends its matrix's iteration)
+        power, top = X.PtrList(Tc, shape), top_t                             # T^p by repeated squaring
+        for square in range(1, 1 + squarings):
             dst = Tp if power is T2 else T2
-            X.gemm(power, power, out=dst, skip=skip, symmetric=symmetric)
-            power, done_p = dst, done_p * 2
+            X.gemm(power, power, out=dst, skip=skip, symmetric=symmetric, amax=(top, top), amax_out=tops[round_number, square])
+            power, top = dst, tops[round_number, square]
         new_err = torch.zeros(B, device=dev)
         X.gemm(power, X.PtrList(Mc, shape), out=X.PtrList(Mo, shape), newton=(X.PtrList(To, shape), w, new_err),
-               skip=skip, symmetric=symmetric)
+               skip=skip, symmetric=symmetric, amax=(top, top_m))
+        top_m, top_t = 1 + new_err, 1 + abs(w) * new_err
         accept = (~done) & ~(new_err > err * 1.2)
         side = side ^ accept
         err = torch.where(accept, new_err, err)

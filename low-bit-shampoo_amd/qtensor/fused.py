@@ -50,7 +50,15 @@ class GemmDesc(ct.Structure):
                 ("kind_a", ct.c_int), ("kind_b", ct.c_int), ("epilogue", ct.c_int), ("args", GemmArgs)]
 
 
+class GemmRanges(ct.Structure):
+    _fields_ = [("amax_a", ct.c_void_p), ("amax_b", ct.c_void_p), ("amax_out", ct.c_void_p)]
+
+
 if F.lib is not None:
+    F.lib.qtensor_hip_gemm_ranged.restype = None
+    F.lib.qtensor_hip_gemm_ranged.argtypes = [ct.POINTER(GemmDesc), ct.POINTER(GemmRanges), ct.c_void_p]
+    F.lib.qtensor_hip_amax_batched.restype = None
+    F.lib.qtensor_hip_amax_batched.argtypes = [ct.POINTER(BatchPtr), ct.c_int, ct.c_int, ct.c_int, ct.c_int, ct.c_void_p, ct.c_void_p]
     F.lib.qtensor_hip_gemm_pipe.restype = ct.c_int
     F.lib.qtensor_hip_gemm_pipe.argtypes = [ct.c_int]
     F.lib.qtensor_hip_gemm.restype = None
@@ -153,10 +161,23 @@ def _workspace(device: torch.device, floats: int) -> Tensor:
     return torch.empty(min(_WORKSPACE_FLOATS, floats), dtype=torch.float32, device=device)
 
 
-def _launch(desc: GemmDesc, device: torch.device) -> None:
+def _launch(desc: GemmDesc, device: torch.device, ranges: Optional[GemmRanges] = None) -> None:
     if F.lib is None:
         raise RuntimeError("libqtensor_hip.so is not available")
+    if ranges is not None:
+        F._call(lambda d, r, s: F.lib.qtensor_hip_gemm_ranged(d, r, s), device, ct.byref(desc), ct.byref(ranges))
+        return
     F._call(lambda d, s: F.lib.qtensor_hip_gemm(d, s), device, ct.byref(desc))
+
+
+def amax(t, out: Optional[Tensor] = None) -> Tensor:
+    """fp32 [batch]: the largest |element| of every matrix of t ([rows, cols], [batch, rows, cols] or a PtrList), one
+    launch.  out: an existing vector to raise (zeroed here otherwise)."""
+    ptr, ld, batch, rows, cols = _dense(t)
+    if out is None:
+        out = torch.zeros(batch, device=t.device)
+    F._call(F.lib.qtensor_hip_amax_batched, t.device, ct.byref(ptr), ld, rows, cols, batch, out.data_ptr())
+    return out
 
 
 def gemm_pipe(mode: Optional[str] = None) -> str:
@@ -176,7 +197,8 @@ _PIPES = {None: 0, "f32": 1, "split": 2}
 
 def gemm(A, B, *, trans_a=False, trans_b=False, out: Optional[Tensor] = None, alpha=1.0, beta=0.0,
          addend=None, newton=None, skip: Optional[Tensor] = None, symmetric: bool = False,
-         upper_a: bool = False, upper_b: bool = False, requantize: bool = False, pipe: Optional[str] = None):
+         upper_a: bool = False, upper_b: bool = False, requantize: bool = False, pipe: Optional[str] = None,
+         amax=None, amax_out: Optional[Tensor] = None):
     """out[b] = epilogue(op(A[b]) @ op(B[b])).
 
     A, B: fp32 tensors ([m,k] / [batch,m,k]; with trans_x the stored matrix is the transpose; trans_a together
@@ -194,7 +216,12 @@ def gemm(A, B, *, trans_a=False, trans_b=False, out: Optional[Tensor] = None, al
     the fp32 matrix never reaches memory; returns E.
     upper_a / upper_b: op(A) / op(B) is upper triangular (zero below the diagonal, square in its k
     index, dense): the part of the k range where it is zero is skipped.
-    pipe: None (the process-wide choice, gemm_pipe), "f32" or "split" for this product alone."""
+    pipe: None (the process-wide choice, gemm_pipe), "f32" or "split" for this product alone.
+    amax: optional pair of fp32 [batch] vectors, the largest |element| of A[b] and of B[b] or bounds of them: large
+    enough products of dense operands then run on the half pipe (two fp16 pieces per element, three products per fp32
+    product: errors no larger than those of "split", 1.4 times its rate).  A bound that is wrong costs time, not
+    precision: include/qtensor_hip.h, qtensor_hip_gemm_ranged.
+    amax_out: optional fp32 [batch], raised to the largest |element| of out[b] (zeroed by the caller)."""
     d = GemmDesc()
     a = d.args
     if pipe not in _PIPES:
@@ -288,7 +315,17 @@ def gemm(A, B, *, trans_a=False, trans_b=False, out: Optional[Tensor] = None, al
         scratch = _workspace(dev, max(8 * batch * m * n, (tiles + 520) * 128 * 128 if quantized and tiles < 1024 else 0))
         a.workspace, a.workspace_floats = scratch.data_ptr(), scratch.numel()
         keep.append(scratch)
-    _launch(d, dev)
+    ranges = None
+    if amax is not None or amax_out is not None:
+        ranges = GemmRanges()
+        for t in (amax or ()) + ((amax_out,) if amax_out is not None else ()):
+            if t.dtype != torch.float32 or t.numel() != batch or not t.is_cuda or not t.is_contiguous():
+                raise ValueError("amax and amax_out are contiguous fp32 GPU vectors with one entry per batch entry")
+        if amax is not None:
+            ranges.amax_a, ranges.amax_b = amax[0].data_ptr(), amax[1].data_ptr()
+        if amax_out is not None:
+            ranges.amax_out = amax_out.data_ptr()
+    _launch(d, dev, ranges)
     return addend if requantize else out
 
 

@@ -1,0 +1,177 @@
+"""Products with known operand sizes (qtensor.fused.gemm(amax=...) -> qtensor_hip_gemm_ranged): the half pipe, where it
+hands a tile back to the bf16 split, and the largest elements it reports.  Compared with float64 products of the same
+operands.
+
+Bound of an element's error, relative to (|A| |B|)[i][j]: an operand is kept to 2^-23 (22 bits and the sign of the rest),
+the product of the rests (2^-24) is left out, and 3 k / 16 + 2 additions round to 2^-24 of sums that stay below (|A| |B|),
+in blocks of 16 whose own order is the matrix instruction's: twice that is allowed for."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def X():
+    import qtensor.functional as F
+    import qtensor.fused as X
+    assert torch.cuda.is_available() and F.lib is not None
+    return X
+
+
+def check(got, A, B, k):
+    bound = (2 * 2.0 ** -23 + 2.0 ** -24) + 2 * (3 * k / 16 + 2) * 2.0 ** -24
+    err = (got.double() - A.double() @ B.double()).abs()
+    assert bool((err <= bound * (A.double().abs() @ B.double().abs()) + 1e-300).all())
+
+
+@pytest.mark.parametrize("m,n,k,batch", [(64, 64, 256, 1), (2, 3, 256, 3), (129, 127, 288, 2), (128, 256, 256, 2), (257, 64, 512, 1),
+                                         (100, 300, 576, 5), (1030, 520, 512, 1), (256, 256, 2048, 1), (384, 384, 544, 60)])
+def test_half_pipe_against_float64_all_layouts(X, m, n, k, batch):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A = torch.randn(batch, m, k, device="cuda", generator=g)
+    B = torch.randn(batch, k, n, device="cuda", generator=g) * 1e-6
+    top = (X.amax(A), X.amax(B))
+    none = torch.zeros(batch, dtype=torch.int32, device="cuda")         # (skip flags: keeps the products from being cut along k)
+    assert torch.equal(top[0], A.abs().amax((1, 2))) and torch.equal(top[1], B.abs().amax((1, 2)))
+    for kw, a, b in ((dict(), A, B), (dict(trans_a=True), A.transpose(1, 2).contiguous(), B), (dict(trans_b=True), A, B.transpose(1, 2).contiguous())):
+        tops = torch.zeros(batch, device="cuda")
+        got = X.gemm(a, b, amax=top, amax_out=tops, **kw)
+        check(got, A, B, k)
+        assert torch.equal(tops, got.abs().amax((1, 2)))
+        # rows that are not aligned take the bf16 split: the very same bits as without amax
+        if kw.get("trans_a"):
+            continue
+        wide = torch.zeros(batch, m, k + 5, device="cuda")
+        wide[:, :, 1:k + 1] = A
+        assert torch.equal(X.gemm(wide[:, :, 1:k + 1], b, amax=top, skip=none, **kw), X.gemm(A, b, skip=none, **kw))
+    for short in (224, 240):                             # below the least k, and not whole lines
+        assert torch.equal(X.gemm(A[:, :, :short], B[:, :short], amax=top, skip=none), X.gemm(A[:, :, :short], B[:, :short], skip=none))
+
+
+@pytest.mark.parametrize("n", [128, 192])
+def test_tiles_the_half_pipe_hands_back_have_the_bits_of_the_split(X, n):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.randn(2, n, 544, device="cuda", generator=g)
+    B = torch.randn(2, 544, n, device="cuda", generator=g)
+    ones = torch.ones(2, device="cuda")
+    none = torch.zeros(2, dtype=torch.int32, device="cuda")             # (skip flags: keeps the products from being cut along k)
+    product = lambda *args, **kw: X.gemm(*args, skip=none, **kw)           # noqa: E731
+    split = product(A, B)
+    top = (X.amax(A), X.amax(B))
+    assert not torch.equal(product(A, B, amax=top), split)
+    # bounds that are far too small or of no use: the whole product
+    for bad in (1e-3, 0.0, float("inf"), float("nan"), 1e25, 1e-25):
+        assert torch.equal(product(A, B, amax=(bad * ones, top[1])), split)
+        assert torch.equal(product(A, B, amax=(top[0], bad * ones)), split)
+    # a bound that is too large by 2^10 is still near enough
+    check(product(A, B, amax=(1024 * top[0], top[1])), A, B, 544)
+    # a row of an operand that is tiny, not finite, or above the bound: its tile; elsewhere, and for zero rows, the half pipe.
+    # 64 covers every tile shape's rows
+    for value in (1e-12, float("inf"), 1e6):
+        C = A.clone()
+        C[1, 3, :] = value
+        C[0, 5, :] = 0.0
+        got, want = product(C, B, amax=top), product(C, B)
+        assert np.array_equal(got[1, :64].cpu().numpy(), want[1, :64].cpu().numpy(), equal_nan=True)
+        check(got[0], C[0], B[0], 544)
+        D = B.clone()
+        D[1, :, n - 2] = value
+        got, want = product(A, D, amax=top), product(A, D)
+        assert np.array_equal(got[1, :, n - 64:].cpu().numpy(), want[1, :, n - 64:].cpu().numpy(), equal_nan=True)
+        check(got[0], A[0], B[0], 544)
+    # NaN makes its row NaN, as on the other pipes, and leaves the others alone
+    C = A.clone()
+    C[1, 3, 7] = float("nan")
+    got = product(C, B, amax=top)
+    assert bool(got[1, 3].isnan().all())
+    got[1, 3], C[1, 3] = 0.0, 0.0
+    check(got, C, B, 544)
+
+
+def test_half_pipe_epilogues_skip_flags_and_pointer_lists(X):
+    g = torch.Generator(device="cuda").manual_seed(5)
+    n, batch = 576, 3
+    A = torch.randn(batch, n, n, device="cuda", generator=g) / n ** 0.5
+    E = torch.randn(batch, n, n, device="cuda", generator=g)
+    top, ones = X.amax(A), torch.ones(batch, device="cuda")
+    P = A.double() @ A.double()
+    # addend, in place, an odd width
+    got = E[:, :, :575].clone()
+    tops = torch.zeros(batch, device="cuda")
+    X.gemm(A, A[:, :, :575], addend=got, out=got, alpha=-0.5, beta=1.5, amax=(top, top), amax_out=tops)
+    assert float((got.double() - (1.5 * E.double() - 0.5 * P)[:, :, :575]).abs().max()) <= 1e-5
+    assert torch.equal(tops, got.abs().amax((1, 2)))
+    # Newton epilogue with a skipped entry, operands through lists of which one entry is not aligned
+    flat = torch.zeros(n * n + 4, device="cuda")
+    shifted = flat[1:1 + n * n].view(n, n)
+    shifted.copy_(A[2])
+    ptrs = torch.tensor([A[0].data_ptr(), A[1].data_ptr(), shifted.data_ptr()], dtype=torch.int64, device="cuda")
+    C, T = torch.full_like(A, 7.0), torch.full_like(A, 7.0)
+    err, tops = torch.zeros(batch, device="cuda"), torch.zeros(batch, device="cuda")
+    skip = torch.tensor([0, 1, 0], dtype=torch.int32, device="cuda")
+    X.gemm(X.PtrList(ptrs, (batch, n, n)), A, out=C, newton=(T, -0.25, err), skip=skip, amax=(top, top), amax_out=tops)
+    eye = torch.eye(n, device="cuda", dtype=torch.float64)
+    for b in (0, 2):
+        check(C[b], A[b], A[b], n)
+        assert float((T[b].double() - (1.25 * eye - 0.25 * P[b])).abs().max()) <= 1e-5
+        assert abs(float(err[b]) - float((P[b] - eye).abs().max())) <= 1e-5 and float(tops[b]) == float(C[b].abs().max())
+    assert torch.equal(C[2], X.gemm(A, A, skip=skip)[2]) and bool((C[1] == 7.0).all()) and float(err[1]) == float(tops[1]) == 0.0
+    # symmetric: exactly mirrored
+    S = X.gemm(A, A, trans_b=True, symmetric=True, amax=(top, top))
+    assert torch.equal(S, S.transpose(1, 2))
+    check(S[0], A[0], A[0].T, n)
+    # few tiles, long k: cut along k, with and without an upper triangular factor
+    L = torch.randn(1, 64, 4096, device="cuda", generator=g)
+    R = torch.randn(1, 4096, 64, device="cuda", generator=g)
+    tops = torch.zeros(1, device="cuda")
+    got = X.gemm(L, R, amax=(X.amax(L), X.amax(R)), amax_out=tops)
+    check(got, L, R, 4096)
+    assert float(tops) == float(got.abs().max())
+    U = torch.triu(A)
+    check(X.gemm(E, U, upper_b=True, amax=(X.amax(E), top)), E, U, n)
+    with pytest.raises(ValueError):
+        X.gemm(A, A, amax=(top, ones[:2]))
+    assert float(X.amax(torch.full((3, 5), -2.0, device="cuda"))) == 2.0
+
+
+def test_half_pipe_errors_against_those_of_the_split(X):
+    """2-norm against float64 over kinds of operands that the optimizers multiply: no larger than the bf16 split's.  In
+    near-identities one pair of elements makes most of a sum and shows the bit that is not kept: 2^-23 of either at most."""
+    g = torch.Generator(device="cuda").manual_seed(7)
+    for k in (256, 512, 768, 1024):
+        graded = torch.exp(0.25 * torch.randn(k, 1, device="cuda", generator=g))
+        kinds = [torch.randn(k, k, device="cuda", generator=g), graded * torch.randn(k, k, device="cuda", generator=g) * graded.T,
+                 torch.rand(k, k, device="cuda", generator=g), torch.eye(k, device="cuda") + 1e-3 * torch.randn(k, k, device="cuda", generator=g)]
+        for kind, A in enumerate(kinds):
+            B = A.T.contiguous()
+            want, top = A.double() @ B.double(), (X.amax(A), X.amax(B))
+            half = float((X.gemm(A, B, amax=top).double() - want).norm())
+            split = float((X.gemm(A, B).double() - want).norm())
+            assert half <= split + (2.0 ** -22 * float(want.norm()) if kind == 3 else 0.0), (k, kind, half, split)
+
+
+def test_inverse_roots_on_the_half_pipe_are_no_further_from_float64(X):
+    """The iteration on the half pipe against the same iteration on the bf16 split (whose products take no amax)."""
+    import optimizers.matrix_functions as MF
+    for n in (256, 320, 768):
+        errors = {"half": 0.0, "split": 0.0}
+        for seed in range(4):
+            g = torch.Generator().manual_seed(n + seed)
+            q, _ = torch.linalg.qr(torch.randn(n, n, generator=g, dtype=torch.float64))
+            lam = torch.logspace(0, -1.3, n, dtype=torch.float64)
+            A = ((q * lam) @ q.T).float()
+            A = (A + A.T) / 2
+            value, vectors = torch.linalg.eigh(A.double())
+            want = (vectors * (value + 1e-6 * float(value[-1])) ** -0.25) @ vectors.T
+            plain = X.gemm
+            for name in errors:
+                if name == "split":
+                    X.gemm = lambda *a, amax=None, amax_out=None, **kw: plain(*a, **kw)
+                try:
+                    root = MF.ComputePowerBatched(A[None].cuda(), 4, v0=torch.ones(1, n, device="cuda"))[0].cpu().double()
+                finally:
+                    X.gemm = plain
+                errors[name] += float((root - want).norm() / want.norm()) / 4
+        assert errors["half"] <= errors["split"], (n, errors)
