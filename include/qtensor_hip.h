@@ -212,8 +212,9 @@ typedef struct {
 } qtensor_gemm_ranges;
 
 /* qtensor_hip_gemm for callers that know how large the operands are (no counterpart in the reference).  Where the split
- * bf16 pipe would multiply two dense operands and K is a multiple of 32 and at least 256 (and operands whose k is
- * contiguous have a leading dimension that is a multiple of 4), the product runs on the half pipe instead: every
+ * bf16 pipe would multiply and K is a multiple of 32 and at least 256 (and dense operands whose k is contiguous have a
+ * leading dimension that is a multiple of 4, and a quantized left operand's codes are a strided batch on 16-byte
+ * boundaries), the product runs on the half pipe instead: every
  * element is scaled by a power of two taken from amax and written as the sum of two fp16 numbers (22 to 23 bits), three
  * fp16 products per fp32 product, the leading terms and the rests in fp32 accumulators of their own.  Errors against
  * float64 are those of the bf16 split or smaller (half of them for Gaussian matrices of order 1024) at 1.4 times its rate.
@@ -221,9 +222,15 @@ typedef struct {
  * it -- and every tile where a bound is zero, not finite or outside 2^-60 .. 2^61 -- is multiplied out by the bf16 split.
  * ranges may be null (then this is qtensor_hip_gemm); amax_out is served on every pipe. */
 void qtensor_hip_gemm_ranged(const qtensor_gemm_desc *desc, const qtensor_gemm_ranges *ranges, qtensor_stream_t stream);
-/* out[b] = max(out[b], largest |element| of the rows x cols matrix b) for a batch of fp32 matrices (leading dimension ld;
- * NaN counts as larger than infinity), one pass; the caller zeroes out. */
-void qtensor_hip_amax_batched(const qtensor_batch_ptr *mats, int ld, int rows, int cols, int batch, float *out, qtensor_stream_t stream);
+/* out[b] = max(out[b], largest |element| of the rows x cols matrix b) for up to eight batches of fp32 matrices in one
+ * launch (leading dimension ld; NaN counts as larger than infinity); the caller zeroes out.  Two sources may raise the
+ * same out: the maxima and the exact diagonal of quantized matrices bound their elements (code tables within +-1). */
+typedef struct {
+    qtensor_batch_ptr mats;
+    int ld, rows, cols, batch;
+    float *out;
+} qtensor_amax_source;
+void qtensor_hip_amax_batched(const qtensor_amax_source *sources, int count, qtensor_stream_t stream);
 
 /* qtensor_hip_gemm for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc); it has no counterpart in the reference.  The partial

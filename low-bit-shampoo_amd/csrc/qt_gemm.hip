@@ -655,7 +655,8 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     // products of the big stacks, which never need it, a percent)
     constexpr bool kCanStream = QT_STREAMK && EPI == kStore && (KA >= kQuant4 || KB >= kQuant4);
     const bool streamed = kCanStream && args.stream_per > 0;
-    const int k_tiles_all = args.K / BK;                 // (only used when streamed: K is then a multiple of BK)
+    constexpr int UNIT = PREC == kPipeHalf ? HK : BK;
+    const int k_tiles_all = args.K / UNIT;               // (only used when streamed: K is then a multiple of UNIT)
     long long run_at = 0, run_end = 0;                   // streamed: this workgroup's run of k tiles, [run_at, run_end)
     if (streamed) {
         run_at = (long long)id * args.stream_per;
@@ -756,14 +757,18 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     // offsets inside 31 bits: the loads of the main loop then need no predicates at all
     const bool whole_k = args.K % BK == 0;
     bool a_fast = false, b_fast = false;
-    if constexpr (kSplit) {                    // the host only picks this pipe where the fast loads apply
-        if constexpr (KA >= kQuant4) la.prepare(args.Aq, b, m0);
-        else la.prepare(args.lda, m0, args.M);
-        if constexpr (KB >= kQuant4) lb.prepare(args.Bq, b, n0);
-        else lb.prepare(args.ldb, n0, args.N);
-        if constexpr (KA == kDense) la.vec = a_vec;
-        if constexpr (KB == kDenseT) lb.vec = b_vec;
-    } else {
+    auto prepare_split = [&]() {               // the host only picks this pipe where the fast loads apply
+        if constexpr (kSplit) {
+            if constexpr (KA >= kQuant4) la.prepare(args.Aq, b, m0);
+            else la.prepare(args.lda, m0, args.M);
+            if constexpr (KB >= kQuant4) lb.prepare(args.Bq, b, n0);
+            else lb.prepare(args.ldb, n0, args.N);
+            if constexpr (KA == kDense) la.vec = a_vec;
+            if constexpr (KB == kDenseT) lb.vec = b_vec;
+        }
+    };
+    if constexpr (PREC == kPipeSplit) prepare_split();
+    if constexpr (!kSplit) {
         if constexpr (KA < kQuant4) {
             a_fast = whole_k && a_vec && (KA == kDense || (args.M & 3) == 0) &&
                      (long long)(KA == kDense ? args.M : args.K) * args.lda < 0x7fffffffLL;
@@ -822,8 +827,8 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     // (a triangular operand shortens the range to where it is not zero: tile origins are multiples of BK)
     const int k_first = (args.triangular & 1) ? min(m0, args.K) : 0;
     const int k_last = (args.triangular & 2) ? min(n0 + BN, args.K) : args.K;
-    const int n_tiles = streamed ? seg_tiles : max((k_last - k_first + BK - 1) / BK, 1) / slices;
-    const int k_begin = streamed ? seg_first * BK : k_first + slice * n_tiles * BK;
+    const int n_tiles = streamed ? seg_tiles * (UNIT / BK) : max((k_last - k_first + BK - 1) / BK, 1) / slices;
+    const int k_begin = streamed ? seg_first * UNIT : k_first + slice * n_tiles * BK;
     // DEEP (dense 64 x 64 tiles, few workgroups and four k tiles or more: launch_gemm).  A k tile is then 192 cycles of
     // matrix instructions against a load latency of several times that with next to nothing else on the unit to hide
     // it, so the loads are kept kAhead tiles ahead in as many sets of registers (eight words a set).  Loads and commits
@@ -891,8 +896,11 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         // (rows that are not 16-byte aligned inside a list of pointers are only seen here)
         if (half_scale(args.amax_a[b], sa, ia) && half_scale(args.amax_b[b], sb, ib) && (KA != kDense || a_vec) && (KB != kDenseT || b_vec)) {
             constexpr int SETS = BM == 128 && BN == 128 ? 1 : 2;           // smaller tiles: less to do per tile to hide a load behind, and registers to spare
-            typename std::conditional<KA == kDense, HalfKContig<BM, SETS>, HalfRowContig<BM, SETS>>::type ha;
-            typename std::conditional<KB == kDenseT, HalfKContig<BN, SETS>, HalfRowContig<BN, SETS>>::type hb;
+            constexpr bool QA = KA >= kQuant4, QB = KB >= kQuant4;
+            typename std::conditional<QA, HalfQuantLeft<BM, KA == kQuant4 ? 4 : 8, SETS>,
+                typename std::conditional<KA == kDense, HalfKContig<BM, SETS>, HalfRowContig<BM, SETS>>::type>::type ha;
+            typename std::conditional<QB, HalfQuantRight<BN, KB == kQuant4 ? 4 : 8, SETS>,
+                typename std::conditional<KB == kDenseT, HalfKContig<BN, SETS>, HalfRowContig<BN, SETS>>::type>::type hb;
             f32x16 rest[MI][NI];
 #pragma unroll
             for (int i = 0; i < MI; ++i)
@@ -901,13 +909,38 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
 #pragma unroll
                     for (int r = 0; r < 16; ++r) rest[i][j][r] = 0.0f;
             for (int i = threadIdx.x; i < BM + BN; i += 256) s_top[i] = 0;
-            ha.prepare(args.lda, m0, args.M);
-            hb.prepare(args.ldb, n0, args.N);
             const int half_tiles = n_tiles * BK / HK;
             auto at_k = [&](int t) { return (long long)(k_begin + min(t, half_tiles - 1) * HK); };
-            auto src_a = [&](int t) { return whole_range(A + (KA == kDense ? (long long)m0 * args.lda + at_k(t) : at_k(t) * args.lda + m0)); };
-            auto src_b = [&](int t) { return whole_range(B + (KB == kDenseT ? (long long)n0 * args.ldb + at_k(t) : at_k(t) * args.ldb + n0)); };
-            half_main_loop<BM, BN, SETS>(reinterpret_cast<unsigned char *>(s_mem), ha, hb, src_a, src_b, half_tiles, sa, sb, acc, rest);
+            const QuantRef &q = QA ? args.Aq : args.Bq;                    // (only used where one operand is quantized)
+            const float *q_codes = QA || QB ? wave_uniform(reinterpret_cast<const float *>(batch_ptr<uint8_t>(q.codes, b))) : nullptr;
+            const float *q_absmax = QA || QB ? wave_uniform(batch_ptr<float>(q.absmax, b)) : nullptr;
+            auto source = [&](long long k0) {
+                const long long step = QA ? k0 : k0 * q.order;
+                const uint8_t *codes = reinterpret_cast<const uint8_t *>(q_codes) + (KA == kQuant4 || KB == kQuant4 ? step >> 1 : step);
+                return QuantSource{whole_range(reinterpret_cast<const float *>(codes)), whole_range(q_absmax + (step >> q.bs_shift))};
+            };
+            auto src_a = [&](int t) {
+                if constexpr (QA) return source(at_k(t));
+                else return DenseSource{whole_range(A + (KA == kDense ? (long long)m0 * args.lda + at_k(t) : at_k(t) * args.lda + m0))};
+            };
+            auto src_b = [&](int t) {
+                if constexpr (QB) return source(at_k(t));
+                else return DenseSource{whole_range(B + (KB == kDenseT ? (long long)n0 * args.ldb + at_k(t) : at_k(t) * args.ldb + n0))};
+            };
+            int diag_k = 1 << 30, diag_rows = 0;
+            if constexpr (QA || QB) {
+                const float *diag = has_ptr(q.diag) ? batch_ptr<float>(q.diag, b) : nullptr;
+                if constexpr (QA) ha.prepare(s_code, diag, q.order, q.bs_shift, m0, sa);
+                else hb.prepare(s_code, diag, q.order, q.bs_shift, n0, sb);
+                if (diag != nullptr) {
+                    diag_k = QA ? m0 : n0;
+                    diag_rows = QA ? BM : BN;
+                }
+            }
+            if constexpr (!QA) ha.prepare(args.lda, m0, args.M);
+            if constexpr (!QB) hb.prepare(args.ldb, n0, args.N);
+            half_main_loop<BM, BN, SETS, QA || QB>(reinterpret_cast<unsigned char *>(s_mem), ha, hb, src_a, src_b, half_tiles, k_begin, diag_k, diag_rows,
+                                                   sa, sb, acc, rest);
             ha.tops(s_top);
             hb.tops(s_top + BM);
             __syncthreads();
@@ -924,6 +957,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         }
     }
     if (again) {
+    if constexpr (PREC == kPipeHalf) prepare_split();
     fetch(k_begin);
     commit(0);
     if (n_tiles > 1) fetch(k_begin + BK);
@@ -1321,9 +1355,12 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         if (lane == 0) atomicMax(reinterpret_cast<unsigned int *>(args.err) + b, e);
     }
     if constexpr (PREC == kPipeHalf) {
-        if (args.amax_out != nullptr) {
+        if (args.amax_out != nullptr) {            // one atomic a workgroup: they come one after the other, 10 ns each (an atomic a wave: 56 us
+            __shared__ uint32_t s_out[4];          // where the 576 tiles of one 768 x 3072 product by itself take 34)
             const uint32_t e = group_max_u32<64>(__float_as_uint(local_top));
-            if (lane == 0) atomicMax(args.amax_out + b, e);
+            if (lane == 0) s_out[wave] = e;
+            __syncthreads();
+            if (threadIdx.x == 0) atomicMax(args.amax_out + b, max(max(s_out[0], s_out[1]), max(s_out[2], s_out[3])));
         }
     }
     if (!streamed) return;
@@ -1446,32 +1483,81 @@ __global__ __launch_bounds__(256) void reduce_slices_kernel(const float *workspa
 }
 
 // out[b] = max(out[b], max |element|) as bits (infinities and NaN above everything finite), over the rows x cols matrices
-// of a batch; grid (pieces of `rows_per` rows, batch).  Bound by memory: 415 MB in 0.08 ms.
-__global__ __launch_bounds__(256) void amax_kernel(BatchPtr mats, int ld, int rows, int cols, int rows_per, int inner, long long inner_stride,
-                                                   uint32_t *out) {
-    const int b = blockIdx.y, r0 = blockIdx.x * rows_per, r1 = min(rows, r0 + rows_per);
-    const float *base = dense_ptr(mats, b, inner, inner_stride);
+// of up to kAmaxSources batches in one launch; a workgroup takes `rows_per` rows of one matrix: large pieces and one atomic
+// each, because the atomics on a batch's few cache lines come one after the other (36 x 768 x 1024, 16 K elements a
+// workgroup and an atomic a wave: 66 us, now 21).
+constexpr int kAmaxSources = 8;
+struct AmaxSource {
+    BatchPtr mats;
+    int ld, rows, cols, batch;
+    float *out;
+    long long inner_stride;                      // (the library's own use: two-level batches, see GemmArgs::batch_inner)
+    int inner, rows_per;
+    unsigned first_block;
+};
+struct AmaxArgs { AmaxSource source[kAmaxSources]; int count; };
+__global__ __launch_bounds__(256) void amax_kernel(const AmaxArgs args) {
+    int i = 0;
+    while (i + 1 < args.count && blockIdx.x >= args.source[i + 1].first_block) ++i;
+    const AmaxSource &m = args.source[i];
+    const unsigned pieces = (m.rows + m.rows_per - 1) / m.rows_per, block = blockIdx.x - m.first_block;
+    const int b = block / pieces, r0 = (int)(block % pieces) * m.rows_per, r1 = min(m.rows, r0 + m.rows_per);
+    const float *base = dense_ptr(m.mats, b, m.inner, m.inner_stride);
     uint32_t top = 0;
-    if ((ld & 3) == 0 && (cols & 3) == 0 && is_aligned16(base)) {
-        const int quads = cols >> 2;
-        for (int q = threadIdx.x; q < (r1 - r0) * quads; q += 256) {
-            const float4 x = gload4(base + (long long)(r0 + q / quads) * ld + (q % quads << 2));
-            top = max(max(max(__float_as_uint(x.x) & 0x7fffffffu, __float_as_uint(x.y) & 0x7fffffffu),
-                          max(__float_as_uint(x.z) & 0x7fffffffu, __float_as_uint(x.w) & 0x7fffffffu)), top);
+    auto see = [&](float4 x) {
+        top = max(max(max(__float_as_uint(x.x) & 0x7fffffffu, __float_as_uint(x.y) & 0x7fffffffu),
+                      max(__float_as_uint(x.z) & 0x7fffffffu, __float_as_uint(x.w) & 0x7fffffffu)), top);
+    };
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool wide = (m.ld & 3) == 0 && (m.cols & 3) == 0 && is_aligned16(base);
+    if (wide && m.ld == m.cols) {                    // a run of memory: eight loads of a thread in flight
+        const float *run = base + (long long)r0 * m.ld;
+        const int quads = (r1 - r0) * (m.cols >> 2);
+        int q = threadIdx.x;
+        for (; q + 7 * 256 < quads; q += 8 * 256) {
+            float4 x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = gload4(run + 4 * (q + j * 256));
+#pragma unroll
+            for (int j = 0; j < 8; ++j) see(x[j]);
+        }
+        for (; q < quads; q += 256) see(gload4(run + 4 * q));
+    } else if (wide) {                               // a wave takes a row, two rows at a time
+        const int quads = m.cols >> 2;
+        for (int r = r0 + wave; r < r1; r += 8) {
+            const float *x0 = base + (long long)r * m.ld, *x1 = base + (long long)min(r + 4, r1 - 1) * m.ld;
+            for (int q = lane; q < quads; q += 64) {
+                const float4 u = gload4(x0 + 4 * q), v = gload4(x1 + 4 * q);
+                see(u);
+                see(v);
+            }
         }
     } else {
-        for (int q = threadIdx.x; q < (r1 - r0) * cols; q += 256)
-            top = max(__float_as_uint(gload(base + (long long)(r0 + q / cols) * ld + q % cols)) & 0x7fffffffu, top);
+        for (int r = r0 + wave; r < r1; r += 4)
+            for (int c = lane; c < m.cols; c += 64) top = max(__float_as_uint(gload(base + (long long)r * m.ld + c)) & 0x7fffffffu, top);
     }
+    __shared__ uint32_t s_top[4];
     top = group_max_u32<64>(top);
-    if ((threadIdx.x & 63) == 0 && top != 0) atomicMax(out + b, top);
+    if (lane == 0) s_top[wave] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned int *>(m.out) + b, max(max(s_top[0], s_top[1]), max(s_top[2], s_top[3])));
 }
 
-void launch_amax(const BatchPtr &mats, int ld, int rows, int cols, int batch, int inner, long long inner_stride, uint32_t *out, hipStream_t stream) {
-    // 16 K elements a workgroup: 64 a thread
-    const int rows_per = (int)std::max(1ll, std::min((long long)rows, 16384ll / cols));
-    hipLaunchKernelGGL(amax_kernel, dim3((unsigned)((rows + rows_per - 1) / rows_per), (unsigned)batch), dim3(256), 0, stream, mats, ld, rows,
-                       cols, rows_per, inner, inner_stride, out);
+// False (error slot) if the sources have more pieces than a grid takes.
+bool launch_amax(AmaxArgs &args, hipStream_t stream) {
+    long long blocks = 0, elements = 0;
+    for (int i = 0; i < args.count; ++i) elements += (long long)args.source[i].rows * args.source[i].cols * args.source[i].batch;
+    // a workgroup a unit, of 8 to 256 elements a thread (a thousand workgroups: 11 us for 768 x 3072, most of it atomics)
+    const long long piece = std::max(2048ll, std::min(65536ll, elements / 256));
+    for (int i = 0; i < args.count; ++i) {
+        AmaxSource &m = args.source[i];
+        m.rows_per = (int)std::max(1ll, std::min((long long)m.rows, piece / m.cols));
+        m.first_block = (unsigned)blocks;
+        blocks += (long long)((m.rows + m.rows_per - 1) / m.rows_per) * m.batch;
+    }
+    if (blocks > 0x7fffffffLL) { set_error(kBadArgument, "amax: too many rows (%lld pieces)", blocks); return false; }
+    hipLaunchKernelGGL(amax_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, args);
+    return true;
 }
 
 template <int BM, int BN, int KA, int KB, int EPI, int PREC = kPipeF32>
@@ -1480,7 +1566,7 @@ void launch_gemm(const RangedArgs &a, int batch, hipStream_t stream) {
     if (a.symmetric && BM != BN) { set_error(kBadArgument, "gemm: symmetric products need square tiles"); return; }
     long long blocks = (a.symmetric ? tn * (tn + 1) / 2 : tn * tm) * batch * (EPI == kStore ? a.split_k : 1);
     if (EPI == kStore && a.stream_per > 0) {
-        const long long runs = tn * tm * batch * (a.K / BK);
+        const long long runs = tn * tm * batch * (a.K / (PREC == kPipeHalf ? HK : BK));
         blocks = (runs + a.stream_per - 1) / a.stream_per;
     }
     if (blocks > 0x7fffffffLL) { set_error(kBadArgument, "gemm: too many tiles (%lld)", blocks); return; }
@@ -1503,7 +1589,7 @@ void launch_gemm(const RangedArgs &a, int batch, hipStream_t stream) {
         hipLaunchKernelGGL((gemm_kernel<BM, BN, KA, KB, EPI, PREC>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
     if (EPI == kStore && a.stream_per > 0) {
         hipLaunchKernelGGL(reduce_pieces_kernel, dim3((unsigned)(tn * tm * batch), 4), dim3(256), 0, stream, a.workspace, a.C, a.ldc,
-                           a.M, a.N, BM, BN, (int)tm, (int)tn, a.K / BK, a.stream_per, a.stream_lcm);
+                           a.M, a.N, BM, BN, (int)tm, (int)tn, a.K / (PREC == kPipeHalf ? HK : BK), a.stream_per, a.stream_lcm);
         return;
     }
     if (EPI == kStore && a.split_k > 1) {
@@ -1642,17 +1728,30 @@ extern "C" void qtensor_hip_gemm_ranged(const qtensor_gemm_desc *d, const void *
     gemm_dispatch(d, (hipStream_t)stream_v, -1, static_cast<const Ranges *>(ranges));
 }
 
-extern "C" void qtensor_hip_amax_batched(const void *mats, int ld, int rows, int cols, int batch, float *out, void *stream_v) {
+namespace {
+struct PublicAmaxSource {                        // qtensor_amax_source
+    qt::BatchPtr mats;
+    int ld, rows, cols, batch;
+    float *out;
+};
+}  // namespace
+extern "C" void qtensor_hip_amax_batched(const void *sources_v, int count, void *stream_v) {
     using namespace qt;
     clear_error();
-    if (mats == nullptr || out == nullptr) { set_error(kNullPointer, "amax: null pointer"); return; }
-    const BatchPtr &p = *static_cast<const BatchPtr *>(mats);
-    if (rows < 1 || cols < 1 || ld < cols || batch < 1 || batch > 65535 || !has_host_ptr(p)) {
-        set_error(kBadArgument, "amax: need rows, cols >= 1, ld >= cols, 1 <= batch <= 65535 and a matrix (got %d x %d, ld %d, batch %d)", rows, cols, ld, batch);
-        return;
+    const PublicAmaxSource *sources = static_cast<const PublicAmaxSource *>(sources_v);
+    if (sources == nullptr || count < 1 || count > kAmaxSources) { set_error(kBadArgument, "amax: 1 to %d sources (got %d)", kAmaxSources, count); return; }
+    AmaxArgs args = {};
+    args.count = count;
+    for (int i = 0; i < count; ++i) {
+        const PublicAmaxSource &m = sources[i];
+        if (m.out == nullptr || !has_host_ptr(m.mats)) { set_error(kNullPointer, "amax: null pointer"); return; }
+        if (m.rows < 1 || m.cols < 1 || m.ld < m.cols || m.batch < 1) {
+            set_error(kBadArgument, "amax: need rows, cols, batch >= 1 and ld >= cols (got %d x %d, ld %d, batch %d)", m.rows, m.cols, m.ld, m.batch);
+            return;
+        }
+        args.source[i] = {m.mats, m.ld, m.rows, m.cols, m.batch, m.out, 0, 1, 0, 0};
     }
-    launch_amax(p, ld, rows, cols, batch, 1, 0, reinterpret_cast<uint32_t *>(out), (hipStream_t)stream_v);
-    launch_ok("amax");
+    if (launch_amax(args, (hipStream_t)stream_v)) launch_ok("amax");
 }
 
 extern "C" void qtensor_hip_gemm_static(const qtensor_gemm_desc *d, void *stream_v) {
@@ -1794,8 +1893,10 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         a.amax_b = reinterpret_cast<const uint32_t *>(ranges->amax_b);
         a.amax_out = reinterpret_cast<uint32_t *>(ranges->amax_out);
     }
-    const bool half_pipe = split_pipe && a.amax_a != nullptr && a.amax_b != nullptr && ka < kQuant4 && kb < kQuant4 && d->K % HK == 0 &&
-                           d->K >= kHalfLeastK && (ka != kDense || a.lda % 4 == 0) && (kb != kDenseT || a.ldb % 4 == 0);
+    // (codes are read in words of up to 16 bytes: a left factor's have to lie that way)
+    const bool codes_lie = ka < kQuant4 || (a.Aq.codes.list == nullptr && is_aligned(a.Aq.codes.base, 16) && a.Aq.codes.stride % 16 == 0);
+    const bool half_pipe = split_pipe && a.amax_a != nullptr && a.amax_b != nullptr && d->K % HK == 0 && d->K >= kHalfLeastK &&
+                           (ka != kDense || a.lda % 4 == 0) && (kb != kDenseT || a.ldb % 4 == 0) && codes_lie;
     int pick = 0;
     static const char *forced = QT_KNOB("QT_GEMM_TILE");
     if (forced != nullptr) {
@@ -1831,14 +1932,16 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
     // (nor a quantized left factor with k up to 1024: measured on 36 to 144 output tiles, the product that is not cut
     // -- smaller tiles, three workgroups per unit -- takes 31-55 us where runs of k tiles and the launch that sums the
     // pieces take 35-57; from k = 1536 on the cut wins by a quarter and more, and so it does for a quantized right factor)
-    const bool short_left = ka >= kQuant4 && d->K <= 1024;
+    // (on the half pipe a quantized right factor neither: 12 x 768 x 768 by 768 58 against 85 us, 1024 x 1024 by 1024 29 and 44,
+    // 2 x 256 x 1024 by 1024 15 and 42)
+    const bool short_quant = (ka >= kQuant4 || (kb >= kQuant4 && half_pipe)) && d->K <= 1024;
     if (ep == kStore && !a.symmetric && a.batch_inner <= 1 && a.triangular == 0 && a.workspace != nullptr && d->K % 16 == 0 &&
-        is_aligned(a.workspace, 16) && a.skip == nullptr && !short_left) {
+        is_aligned(a.workspace, 16) && a.skip == nullptr && !short_quant) {
         const Shape &sh = shapes[pick];
         const double units = compute_units();
         const long long tm = (d->M + sh.bm - 1) / sh.bm, tn = (d->N + sh.bn - 1) / sh.bn;
         const double tiles = (double)tm * tn * d->batch;
-        const int k_tiles = d->K / 16;
+        const int unit = half_pipe ? HK : BK, k_tiles = d->K / unit;
         // Cost of a way to cut, in k steps of one workgroup that has its unit to itself: the workgroups of a launch run
         // three to a unit side by side, each at its own pace while the unit's matrix pipe has room (a lone workgroup
         // uses about half of it) -- so the time is the longer of (rounds of resident workgroups) x (k range + a fixed
@@ -1856,7 +1959,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         int best_split = 1;
         static const char *forced_split = QT_KNOB("QT_GEMM_SPLIT");
         for (int sp = 2; sp <= 8; ++sp) {
-            if (k_tiles % sp != 0 || k_tiles / sp < 8 || (half_pipe && k_tiles / sp % 2 != 0)) continue;
+            if (k_tiles % sp != 0 || k_tiles / sp < 128 / unit) continue;
             if ((long long)sp * d->batch * d->M * d->N > a.workspace_floats) continue;
             const double cost = cost_of(sp);
             if (forced_split != nullptr) { if (sp == atoi(forced_split)) best_split = sp; }
@@ -1873,11 +1976,11 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         const Shape &bs = shapes[big];
         const long long btm = (d->M + bs.bm - 1) / bs.bm, btn = (d->N + bs.bn - 1) / bs.bn;
         const long long big_tiles = btm * btn * d->batch, runs = big_tiles * k_tiles;
-        if (stream_wgs > 0 && (ka >= kQuant4 || kb >= kQuant4) && a.skip == nullptr && k_tiles >= 16 && big_tiles < 2 * (long long)units) {
+        if (stream_wgs > 0 && (ka >= kQuant4 || kb >= kQuant4) && a.skip == nullptr && k_tiles >= 256 / unit && big_tiles < 2 * (long long)units) {
             long long groups = (long long)units * stream_wgs;
-            static const int min_run = QT_KNOB("QT_GEMM_STREAM_MIN") != nullptr ? atoi(QT_KNOB("QT_GEMM_STREAM_MIN")) : 24;
-            if (groups > runs / min_run) {                                // at least that many k tiles per workgroup,
-                groups = runs / min_run;                                  // and no unit with one workgroup more than another
+            static const int min_run = QT_KNOB("QT_GEMM_STREAM_MIN") != nullptr ? atoi(QT_KNOB("QT_GEMM_STREAM_MIN")) : 384;        // of k
+            if (groups > runs * unit / min_run) {                         // at least that much of k per workgroup,
+                groups = runs * unit / min_run;                                  // and no unit with one workgroup more than another
                 if (groups > (long long)units) groups -= groups % (long long)units;
             }
             const long long per_group = groups > 0 ? (runs + groups - 1) / groups : 0;
@@ -1896,7 +1999,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         }
     }
     // (a product that is not made by one launch on the half pipe has its largest element looked up afterwards)
-    uint32_t *const amax_later = half_pipe && a.split_k == 1 ? nullptr : a.amax_out;
+    uint32_t *const amax_later = half_pipe && a.split_k == 1 && a.stream_per == 0 ? nullptr : a.amax_out;
     if (amax_later != nullptr) a.amax_out = nullptr;
     const int combo = ka * 100 + kb * 10 + ep;
 #define QT_GEMM_CASE_DENSE(KA, KB, EP)                                                                       \
@@ -1925,7 +2028,13 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         break;
 #define QT_GEMM_CASE_QUANT(KA, KB, EP)                                                                        \
     case (KA) * 100 + (KB) * 10 + (EP):                                                                      \
-        if (split_pipe) {                                                                                    \
+        if (half_pipe) {                                                                                     \
+            if (pick == 0) launch_gemm<128, 128, KA, KB, EP, kPipeHalf>(a, d->batch, stream);                \
+            else if (pick == 1) launch_gemm<128, 64, KA, KB, EP, kPipeHalf>(a, d->batch, stream);            \
+            else if (pick == 2) launch_gemm<64, 128, KA, KB, EP, kPipeHalf>(a, d->batch, stream);            \
+            else launch_gemm<64, 64, KA, KB, EP, kPipeHalf>(a, d->batch, stream);                            \
+        }                                                                                                    \
+        else if (split_pipe) {                                                                               \
             if (pick == 0) launch_gemm<128, 128, KA, KB, EP, kPipeSplit>(a, d->batch, stream);               \
             else if (pick == 1) launch_gemm<128, 64, KA, KB, EP, kPipeSplit>(a, d->batch, stream);           \
             else if (pick == 2) launch_gemm<64, 128, KA, KB, EP, kPipeSplit>(a, d->batch, stream);           \
@@ -1960,7 +2069,12 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
             set_error(kBadArgument, "gemm: combination A kind %d, B kind %d, epilogue %d is not built", ka, kb, ep);
             return;
     }
-    if (amax_later != nullptr) launch_amax(a.C, a.ldc, a.M, a.N, d->batch, a.batch_inner, a.inner_c, amax_later, stream);
+    if (amax_later != nullptr) {
+        AmaxArgs after = {};
+        after.count = 1;
+        after.source[0] = {a.C, a.ldc, a.M, a.N, d->batch, reinterpret_cast<float *>(amax_later), a.inner_c, a.batch_inner, 0, 0};
+        if (!launch_amax(after, stream)) return;
+    }
 #undef QT_GEMM_CASE_DENSE
 #undef QT_GEMM_CASE_REQUANT
 #undef QT_GEMM_CASE_QUANT

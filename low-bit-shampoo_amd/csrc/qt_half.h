@@ -53,8 +53,12 @@ __device__ __forceinline__ void halve_pair(float a, float b, float s, uint32_t &
 }
 
 // Loaders.  `prepare` fixes a thread's place; `fetch` issues part q of four of a k tile's loads into one of SETS register
-// sets; `pair` splits two elements of a set and stores to LDS whenever a store's worth is together; `tops` folds the
-// largest (scaled) elements seen into one word per tile row.  Rows beyond the matrix are clamped into it.
+// sets; `pair` splits two elements of a set and stores to LDS whenever a store's worth is together (`ahead` starts the table
+// look-ups of a pair of codes); `tops` folds the largest (scaled) elements seen into one word per tile row.  Rows beyond
+// the matrix are clamped into it.
+// Source of a k tile: base addresses in scalar registers.
+struct DenseSource { __amdgpu_buffer_rsrc_t at; };
+struct QuantSource { __amdgpu_buffer_rsrc_t codes, absmax; };
 
 // k contiguous (element (row, k) at base[row * ld + k], rows 16-byte aligned): eight lanes take the 128 bytes of a row,
 // a thread the rows t / 8 + 32 i.
@@ -72,10 +76,12 @@ struct HalfKContig {
             top[i] = 0.0f;
         }
     }
-    __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t src, int set, int q) {
+    __device__ __forceinline__ void ahead(int, int) {}
+    __device__ __forceinline__ void patch(unsigned char *, int, float) const {}
+    __device__ __forceinline__ void fetch(const DenseSource &src, int set, int q) {
 #pragma unroll
         for (int i = q * VEC / 4; i < (q + 1) * VEC / 4; ++i) {
-            const qt_u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(src, (int)off[i], 0, 0);
+            const qt_u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(src.at, (int)off[i], 0, 0);
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[set][4 * i + e] = __uint_as_float(x[e]);
         }
@@ -111,10 +117,12 @@ struct HalfRowContig {
         step = (uint32_t)ld * 4u;
         top = 0.0f;
     }
-    __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t src, int set, int q) {
+    __device__ __forceinline__ void ahead(int, int) {}
+    __device__ __forceinline__ void patch(unsigned char *, int, float) const {}
+    __device__ __forceinline__ void fetch(const DenseSource &src, int set, int q) {
 #pragma unroll
         for (int j = q * PER / 4; j < (q + 1) * PER / 4; ++j)
-            v[set][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(src, (int)off, (int)(j * step), 0));
+            v[set][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(src.at, (int)off, (int)(j * step), 0));
     }
     __device__ __forceinline__ void pair(unsigned char *operand, int set, float s, int p) {
         using L = HalfLayout<ROWS>;
@@ -127,6 +135,173 @@ struct HalfRowContig {
         }
     }
     __device__ __forceinline__ void tops(uint32_t *s_top) const { atomicMax(s_top + (threadIdx.x & (ROWS - 1)), __float_as_uint(top)); }
+};
+
+// Quantized square matrices (order x order, flat layout), expanded while they are split.  A pair costs the look-ups of two
+// codes (issued one pair ahead: their latency lies behind a matrix instruction) and two products besides its split.
+// `patch` writes the exact diagonal over what the codes gave, on the few k tiles that hold a part of it: by the thread that
+// wrote those elements, behind all its pairs (a branch that touches neither loads nor accumulators; a loop body of its own
+// for those tiles had the compiler spill the accumulators).
+__device__ __forceinline__ void patch_element(unsigned char *at, int plane, float x) {
+    const _Float16 h = (_Float16)x;
+    *reinterpret_cast<_Float16 *>(at) = h;
+    *reinterpret_cast<_Float16 *>(at + plane) = (_Float16)((x - (float)h) * kRestScale);
+}
+
+// Left factor, k along the matrix rows: a thread takes 16 (128 tile rows) or 8 consecutive codes of one row.
+template <int ROWS, int BITS, int SETS>
+struct HalfQuantLeft {
+    static constexpr int PER = ROWS * HK / 256, PARTS = HK / PER, kPairs = PER / 2, WORDS = PER * BITS / 32;
+    uint32_t w[SETS][WORDS];
+    float amax[SETS];
+    float dval, top;
+    uint32_t code_off, amax_off;
+    int row;                                           // the tile row's matrix row less this thread's first k
+    const float *table;
+    float c[2][2];
+    uint32_t h[4], r[4];
+    __device__ __forceinline__ void prepare(const float *code, const float *diag, int order, int bs_shift, int row0, float s) {
+        const int part = threadIdx.x % PARTS;
+        table = code;
+        row = min(row0 + (int)(threadIdx.x / PARTS), order - 1);
+        code_off = (uint32_t)((row * order + part * PER) * BITS / 8);      // order^2 < 2^31: checked on the host
+        amax_off = (uint32_t)(row * (order >> bs_shift)) * 4u;
+        dval = diag != nullptr ? diag[row] : 0.0f;
+        row -= part * PER;
+        top = fabsf(dval) * s;
+    }
+    __device__ __forceinline__ void fetch(const QuantSource &src, int set, int q) {
+        if (q == 0) {
+            if constexpr (WORDS == 1) w[set][0] = __builtin_amdgcn_raw_buffer_load_b32(src.codes, (int)code_off, 0, 0);
+            else if constexpr (WORDS == 2) {
+                const qt_u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(src.codes, (int)code_off, 0, 0);
+                w[set][0] = x.x; w[set][1] = x.y;
+            } else {
+                const qt_u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(src.codes, (int)code_off, 0, 0);
+                w[set][0] = x.x; w[set][1] = x.y; w[set][2] = x.z; w[set][3] = x.w;
+            }
+            amax[set] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(src.absmax, (int)amax_off, 0, 0));
+        }
+    }
+    __device__ __forceinline__ void ahead(int set, int p) {
+        if (p >= kPairs) return;
+        if constexpr (BITS == 4) {
+            const uint32_t byte = w[set][p >> 2] >> (8 * (p & 3));
+            c[p & 1][0] = table[(byte >> 4) & 15u];
+            c[p & 1][1] = table[byte & 15u];
+        } else {
+            const uint32_t two = w[set][p >> 1] >> (16 * (p & 1));
+            c[p & 1][0] = table[two & 255u];
+            c[p & 1][1] = table[(two >> 8) & 255u];
+        }
+    }
+    __device__ __forceinline__ void pair(unsigned char *operand, int set, float s, int p) {
+        using L = HalfLayout<ROWS>;
+        float a = c[p & 1][0] * amax[set], b = c[p & 1][1] * amax[set];
+        ahead(set, p + 1);
+        halve_pair(a, b, s, h[p & 3], r[p & 3], top);
+        if ((p & 3) == 3) {
+            const int eight = threadIdx.x % PARTS * (PER / 8) + (p >> 2);
+            unsigned char *at = operand + (eight >> 1) * L::kSub + (eight & 1) * L::kEight + threadIdx.x / PARTS * 16;
+            *reinterpret_cast<qt_u32x4 *>(at) = qt_u32x4{h[0], h[1], h[2], h[3]};
+            *reinterpret_cast<qt_u32x4 *>(at + L::kPlane) = qt_u32x4{r[0], r[1], r[2], r[3]};
+        }
+    }
+    __device__ __forceinline__ void patch(unsigned char *operand, int k0, float s) const {
+        using L = HalfLayout<ROWS>;
+        const int d = row - k0;                        // the element on the diagonal, if in 0 .. PER - 1
+        if ((unsigned)d < (unsigned)PER) {
+            const int eight = threadIdx.x % PARTS * (PER / 8) + (d >> 3);
+            patch_element(operand + (eight >> 1) * L::kSub + (eight & 1) * L::kEight + threadIdx.x / PARTS * 16 + (d & 7) * 2, L::kPlane, dval * s);
+        }
+    }
+    __device__ __forceinline__ void tops(uint32_t *s_top) const { atomicMax(s_top + threadIdx.x / PARTS, __float_as_uint(top)); }
+};
+
+// Right factor, k along the matrix columns: a thread takes the codes of two neighbouring columns (one byte, or two) of 8
+// (128 tile rows) or 4 consecutive matrix rows, so that nothing has to be turned around.  (It reads the whole word they lie
+// in, as two or four lanes do: what a byte load returns the compiler masks again, at once, and waits for it.)  Of every eight lanes four begin with the even column and four with the odd one: their 16-byte stores then
+// fall into different banks.
+template <int ROWS, int BITS, int SETS>
+struct HalfQuantRight {
+    static constexpr int LANES = ROWS / 2, GROUPS = 256 / LANES, PER = HK / GROUPS, kPairs = PER;      // k per thread; pairs: first column's, then the second's
+    uint32_t w[SETS][PER];
+    float amax[SETS][PER];
+    float dval[2], top[2];
+    uint32_t code_off, amax_off, code_step, amax_step, at[2];
+    int column, way;                                   // the first column less this thread's first k, and how far the second is (1 or -1)
+    const float *table;
+    float c[2][2];
+    uint32_t h[4], r[4];
+    __device__ __forceinline__ void prepare(const float *code, const float *diag, int order, int bs_shift, int row0, float s) {
+        const int lane = threadIdx.x % LANES, group = threadIdx.x / LANES;
+        const int even = min(row0 + 2 * lane, order - 2);
+        table = code;
+        way = (lane >> 2) & 1 ? -1 : 1;
+        column = even + (way < 0 ? 1 : 0);
+        code_step = (uint32_t)(order * BITS / 8);
+        amax_step = (uint32_t)(order >> bs_shift) * 4u;
+        code_off = (uint32_t)(group * PER) * code_step + ((uint32_t)(even * BITS / 8) & ~3u);
+        // a column's place in the word: 4 bits: the even column in the high half of its byte
+        const uint32_t first = ((uint32_t)(even * BITS / 8) & 3u) * 8;
+        at[0] = first + (BITS == 4 ? (way > 0 ? 4 : 0) : (way > 0 ? 0 : 8));
+        at[1] = first + (BITS == 4 ? (way > 0 ? 0 : 4) : (way > 0 ? 8 : 0));
+        amax_off = (uint32_t)(group * PER) * amax_step + (uint32_t)(even >> bs_shift) * 4u;
+        dval[0] = diag != nullptr ? diag[column] : 0.0f;
+        dval[1] = diag != nullptr ? diag[column + way] : 0.0f;
+        column -= group * PER;
+        top[0] = fabsf(dval[0]) * s;
+        top[1] = fabsf(dval[1]) * s;
+    }
+    __device__ __forceinline__ void fetch(const QuantSource &src, int set, int q) {
+#pragma unroll
+        for (int j = q * PER / 4; j < (q + 1) * PER / 4; ++j) {
+            w[set][j] = __builtin_amdgcn_raw_buffer_load_b32(src.codes, (int)code_off, (int)(j * code_step), 0);
+            amax[set][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(src.absmax, (int)amax_off, (int)(j * amax_step), 0));
+        }
+    }
+    __device__ __forceinline__ void ahead(int set, int p) {
+        if (p >= kPairs) return;
+        const int second = p / (PER / 2), j = p % (PER / 2) * 2;
+        c[p & 1][0] = table[(w[set][j] >> at[second]) & ((1u << BITS) - 1)];
+        c[p & 1][1] = table[(w[set][j + 1] >> at[second]) & ((1u << BITS) - 1)];
+    }
+    __device__ __forceinline__ void pair(unsigned char *operand, int set, float s, int p) {
+        using L = HalfLayout<ROWS>;
+        constexpr int HALF = PER / 2, WORDS = PER / 2;                       // packed words per column
+        const int second = p / HALF, j = p % HALF * 2;
+        float a = c[p & 1][0] * amax[set][j], b = c[p & 1][1] * amax[set][j + 1];
+        ahead(set, p + 1);
+        halve_pair(a, b, s, h[p % WORDS], r[p % WORDS], top[second]);
+        if (p % WORDS == WORDS - 1) {
+            const int lane = threadIdx.x % LANES, group = threadIdx.x / LANES, k8 = group * PER / 8;
+            const int tile_row = 2 * lane + ((way < 0) != (second != 0) ? 1 : 0);
+            unsigned char *at = operand + (k8 >> 1) * L::kSub + (k8 & 1) * L::kEight + tile_row * 16 + (PER == 4 ? (group & 1) * 8 : 0);
+            if constexpr (WORDS == 4) {
+                *reinterpret_cast<qt_u32x4 *>(at) = qt_u32x4{h[0], h[1], h[2], h[3]};
+                *reinterpret_cast<qt_u32x4 *>(at + L::kPlane) = qt_u32x4{r[0], r[1], r[2], r[3]};
+            } else {
+                *reinterpret_cast<uint2 *>(at) = make_uint2(h[0], h[1]);
+                *reinterpret_cast<uint2 *>(at + L::kPlane) = make_uint2(r[0], r[1]);
+            }
+        }
+    }
+    __device__ __forceinline__ void patch(unsigned char *operand, int k0, float s) const {
+        using L = HalfLayout<ROWS>;
+        const int lane = threadIdx.x % LANES, group = threadIdx.x / LANES, k8 = group * PER / 8;
+#pragma unroll
+        for (int second = 0; second < 2; ++second) {
+            const int d = column + (second ? way : 0) - k0;
+            if ((unsigned)d < (unsigned)PER)
+                patch_element(operand + (k8 >> 1) * L::kSub + (k8 & 1) * L::kEight + (2 * lane + ((way < 0) != (second != 0) ? 1 : 0)) * 16 +
+                              ((PER == 4 ? (group & 1) * 4 : 0) + d) * 2, L::kPlane, dval[second] * s);
+        }
+    }
+    __device__ __forceinline__ void tops(uint32_t *s_top) const {
+        const int lane = threadIdx.x % LANES;
+        atomicMax(s_top + 2 * lane + (way < 0 ? 1 : 0), __float_as_uint(top[0]));
+        atomicMax(s_top + 2 * lane + (way < 0 ? 0 : 1), __float_as_uint(top[1]));
+    }
 };
 
 // The scale of an operand whose largest element has the bits `amax`, and its inverse.  False where a scale, its inverse or
@@ -153,9 +328,10 @@ __device__ __forceinline__ bool half_row_fine(uint32_t top) {
 // left to the compiler 830 us, matrix pipes busy 0.43; this 775, 0.50.  What bounds it from there on is power: the same
 // launch on zeros takes 500 us, at 2.3 instead of 1.6 GHz.)  Loads past the last tile repeat it instead of being left
 // out: a branch around a load makes the next wait one for all loads in flight.
-template <int BM, int BN, int SETS, typename LA, typename LB, typename SrcA, typename SrcB, typename Acc>
-__device__ __forceinline__ void half_main_loop(unsigned char *mem, LA &la, LB &lb, SrcA src_a, SrcB src_b, int tiles, float sa, float sb,
-                                               Acc &acc, Acc &rest) {
+// k_begin: the first k; diag_k, diag_rows: the exact diagonal of a quantized operand is met by k in diag_k .. diag_k + diag_rows - 1.
+template <int BM, int BN, int SETS, bool DIAG, typename LA, typename LB, typename SrcA, typename SrcB, typename Acc>
+__device__ __forceinline__ void half_main_loop(unsigned char *mem, LA &la, LB &lb, SrcA src_a, SrcB src_b, int tiles, int k_begin, int diag_k,
+                                               int diag_rows, float sa, float sb, Acc &acc, Acc &rest) {
     using HA = HalfLayout<BM>;
     using HB = HalfLayout<BN>;
     constexpr int MI = BM / 64, NI = BN / 64, STAGE = HA::kOperand + HB::kOperand;
@@ -168,12 +344,24 @@ __device__ __forceinline__ void half_main_loop(unsigned char *mem, LA &la, LB &l
 #pragma unroll
         for (int q = 0; q < 4; ++q) { la.fetch(src_a(s), s, q); lb.fetch(src_b(s), s, q); }
     __builtin_amdgcn_sched_barrier(0);
+    la.ahead(0, 0);
+    lb.ahead(0, 0);
 #pragma unroll
     for (int p = 0; p < LA::kPairs; ++p) la.pair(mem, 0, sa, p);
 #pragma unroll
     for (int p = 0; p < LB::kPairs; ++p) lb.pair(mem + HA::kOperand, 0, sb, p);
 #pragma unroll
     for (int q = 0; q < 4; ++q) { la.fetch(src_a(SETS), 0, q); lb.fetch(src_b(SETS), 0, q); }
+    auto patch = [&](unsigned char *stage, int t) {
+        if constexpr (DIAG) {
+            const int k0 = k_begin + t * HK;
+            if (k0 + HK > diag_k && k0 < diag_k + diag_rows) {
+                la.patch(stage, k0, sa);
+                lb.patch(stage + HA::kOperand, k0, sb);
+            }
+        }
+    };
+    patch(mem, 0);
     __syncthreads();
     auto tile = [&](int t, int cur, int set) {          // multiplies tile t; `set` holds tile t + 1
         const unsigned char *pa = mem + cur * STAGE + eight * HA::kEight + row_a * 16;
@@ -188,9 +376,11 @@ __device__ __forceinline__ void half_main_loop(unsigned char *mem, LA &la, LB &l
             else fb[u][1][n - 2 * MI - NI] = *reinterpret_cast<const qt_f16x8 *>(pb + u * HB::kSub + HB::kPlane + (n - 2 * MI - NI) * 32 * 16);
         };
         constexpr int READS = 2 * (MI + NI);
-        const auto from_a = src_a(t + 1 + SETS), from_b = src_b(t + 1 + SETS);
+        const auto from_a = src_a(t + 1 + SETS);
+        const auto from_b = src_b(t + 1 + SETS);
 #pragma unroll
         for (int n = 0; n < READS; ++n) read(0, n);
+        la.ahead(set, 0);
 #pragma unroll
         for (int g = 0; g < STEPS; ++g) {
             const int u = g / (3 * BLOCKS), c = g % (3 * BLOCKS) / BLOCKS, i = g % BLOCKS / NI, j = g % NI;
@@ -199,8 +389,10 @@ __device__ __forceinline__ void half_main_loop(unsigned char *mem, LA &la, LB &l
 #pragma unroll
             for (int w = g * WORK / STEPS; w < (g + 1) * WORK / STEPS; ++w) {
                 if (w < LA::kPairs) la.pair(next, set, sa, w);
-                else if (w < LA::kPairs + 4) la.fetch(from_a, set, w - LA::kPairs);
-                else if (w < LA::kPairs + 4 + LB::kPairs) lb.pair(next + HA::kOperand, set, sb, w - LA::kPairs - 4);
+                else if (w < LA::kPairs + 4) {
+                    la.fetch(from_a, set, w - LA::kPairs);
+                    if (w == LA::kPairs + 3) lb.ahead(set, 0);
+                } else if (w < LA::kPairs + 4 + LB::kPairs) lb.pair(next + HA::kOperand, set, sb, w - LA::kPairs - 4);
                 else lb.fetch(from_b, set, w - LA::kPairs - 4 - LB::kPairs);
             }
             // the other half's fragments, from the middle of this half's products on
@@ -209,6 +401,7 @@ __device__ __forceinline__ void half_main_loop(unsigned char *mem, LA &la, LB &l
                 if (g == 2 * BLOCKS + n * BLOCKS / READS - (BLOCKS == 1 ? 1 : 0)) read(1, n);
             __builtin_amdgcn_sched_barrier(0);
         }
+        patch(next, t + 1);
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
     };

@@ -434,8 +434,15 @@ class ShampooBank:
                 left = left if left.flat else X.load_stack(left)         # read inside the product, or dequantized first
                 right = right if right.flat else X.load_stack(right)
                 half = torch.empty(len(g), g.bm, g.bn, device=self.device)
-                X.gemm(left, self._grad_list(g, grads), out=half, skip=skip)
-                X.gemm(half, right, out=self._out_list(g), skip=skip)
+                G = self._grad_list(g, grads)
+                if not X.worth_measuring(left, G, right):
+                    X.gemm(left, G, out=half, skip=skip)
+                    X.gemm(half, right, out=self._out_list(g), skip=skip)
+                    return
+                tops = torch.zeros(4, len(g), device=self.device)
+                X.amax_into((left, tops[0]), (G, tops[1]), (right, tops[2]))
+                X.gemm(left, G, out=half, skip=skip, amax=(tops[0], tops[1]), amax_out=tops[3])
+                X.gemm(half, right, out=self._out_list(g), skip=skip, amax=(tops[3], tops[2]))
             return run
 
         for g in self.groups:

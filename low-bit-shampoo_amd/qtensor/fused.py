@@ -54,11 +54,15 @@ class GemmRanges(ct.Structure):
     _fields_ = [("amax_a", ct.c_void_p), ("amax_b", ct.c_void_p), ("amax_out", ct.c_void_p)]
 
 
+class AmaxSource(ct.Structure):
+    _fields_ = [("mats", BatchPtr), ("ld", ct.c_int), ("rows", ct.c_int), ("cols", ct.c_int), ("batch", ct.c_int), ("out", ct.c_void_p)]
+
+
 if F.lib is not None:
     F.lib.qtensor_hip_gemm_ranged.restype = None
     F.lib.qtensor_hip_gemm_ranged.argtypes = [ct.POINTER(GemmDesc), ct.POINTER(GemmRanges), ct.c_void_p]
     F.lib.qtensor_hip_amax_batched.restype = None
-    F.lib.qtensor_hip_amax_batched.argtypes = [ct.POINTER(BatchPtr), ct.c_int, ct.c_int, ct.c_int, ct.c_int, ct.c_void_p, ct.c_void_p]
+    F.lib.qtensor_hip_amax_batched.argtypes = [ct.POINTER(AmaxSource), ct.c_int, ct.c_void_p]
     F.lib.qtensor_hip_gemm_pipe.restype = ct.c_int
     F.lib.qtensor_hip_gemm_pipe.argtypes = [ct.c_int]
     F.lib.qtensor_hip_gemm.restype = None
@@ -170,13 +174,31 @@ def _launch(desc: GemmDesc, device: torch.device, ranges: Optional[GemmRanges] =
     F._call(lambda d, s: F.lib.qtensor_hip_gemm(d, s), device, ct.byref(desc))
 
 
-def amax(t, out: Optional[Tensor] = None) -> Tensor:
-    """fp32 [batch]: the largest |element| of every matrix of t ([rows, cols], [batch, rows, cols] or a PtrList), one
-    launch.  out: an existing vector to raise (zeroed here otherwise)."""
-    ptr, ld, batch, rows, cols = _dense(t)
-    if out is None:
-        out = torch.zeros(batch, device=t.device)
-    F._call(F.lib.qtensor_hip_amax_batched, t.device, ct.byref(ptr), ld, rows, cols, batch, out.data_ptr())
+def amax_into(*pairs) -> None:
+    """Each pair (t, out): fp32 [batch] out raised to the largest |element| of every matrix of t ([rows, cols], [batch,
+    rows, cols], a PtrList) or to a bound of it (a `Quantized`: its maxima and exact diagonal; code tables hold nothing
+    beyond +-1).  All of them in one launch (up to eight tensors; a `Quantized` with a diagonal counts as two)."""
+    sources = []
+    for t, out in pairs:
+        if isinstance(t, Quantized):
+            per_row = t.absmax.shape[1] // t.order
+            parts = [(BatchPtr(t.absmax.data_ptr(), None, t.absmax.stride(0)), per_row, t.batch, t.order, per_row)]
+            if t.diag is not None:
+                parts.append((BatchPtr(t.diag.data_ptr(), None, t.diag.stride(0)), t.order, t.batch, 1, t.order))
+        else:
+            parts = [_dense(t)]
+        for ptr, ld, batch, rows, cols in parts:
+            if out.dtype != torch.float32 or out.numel() != batch or not out.is_cuda or not out.is_contiguous():
+                raise ValueError("out must be a contiguous fp32 GPU vector with one entry per batch entry")
+            sources.append(AmaxSource(ptr, ld, rows, cols, batch, out.data_ptr()))
+    F._call(F.lib.qtensor_hip_amax_batched, pairs[0][1].device, (AmaxSource * len(sources))(*sources), len(sources))
+
+
+def amax(t) -> Tensor:
+    """fp32 [batch]: the largest |element| of every matrix of t, or a bound of it (see amax_into)."""
+    out = torch.zeros(t.batch if isinstance(t, Quantized) else 1 if t.dim() == 2 else t.shape[0],
+                      device=t.codes.device if isinstance(t, Quantized) else t.device)
+    amax_into((t, out))
     return out
 
 
@@ -354,8 +376,26 @@ def matvec(mats: Tensor, v: Tensor) -> Tensor:
 def precondition(G: Tensor, left, right, out: Optional[Tensor] = None) -> Tensor:
     """deq(left) @ G @ deq(right) with both factors expanded inside the products.
     left / right: `Quantized` or dense fp32 matrices."""
-    tmp = gemm(left, G)
-    return gemm(tmp, right, out=out)
+    if not worth_measuring(left, G, right):
+        tmp = gemm(left, G)
+        return gemm(tmp, right, out=out)
+    tops = torch.zeros(4, 1 if G.dim() == 2 else G.shape[0], device=G.device)
+    amax_into((left, tops[0]), (G, tops[1]), (right, tops[2]))
+    tmp = gemm(left, G, amax=(tops[0], tops[1]), amax_out=tops[3])
+    return gemm(tmp, right, out=out, amax=(tops[3], tops[2]))
+
+
+def worth_measuring(left, G, right) -> bool:
+    """Whether the largest elements of the operands of deq(left) @ G @ deq(right) are worth looking up: both products on the
+    half pipe (whole lines of k, 256 at least) save more than the look-up and the clearing of its results take: two launches,
+    8 us of the device and 20 of the host (768 x 3072 by itself 145 -> 133 us; half as much work gains nothing)."""
+    m, n = G.shape[-2:]
+    batch = 1 if G.dim() == 2 else G.shape[0]
+    return min(m, n) >= 256 and m % 32 == n % 32 == 0 and batch * m * n * (m + n) >= MEASURE_FROM and gemm_pipe() == "split" and all(
+        q.flat if isinstance(q, Quantized) else q.stride(-1) == 1 for q in (left, right))
+
+
+MEASURE_FROM = 1 << 33           # multiply-adds
 
 
 def gram(G: Tensor, axis: int, *, stat=None, beta=0.0, alpha=1.0, out: Optional[Tensor] = None) -> Tensor:

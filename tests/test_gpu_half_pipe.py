@@ -175,3 +175,59 @@ def test_inverse_roots_on_the_half_pipe_are_no_further_from_float64(X):
                     X.gemm = plain
                 errors[name] += float((root - want).norm() / want.norm()) / 4
         assert errors["half"] <= errors["split"], (n, errors)
+
+
+@pytest.mark.parametrize("bits,bs,name", [(4, 64, "linear-2"), (8, 256, "dynamic"), (8, 64, "linear-2"), (4, 128, "dynamic")])
+@pytest.mark.parametrize("diag", [False, True])
+def test_half_pipe_with_a_quantized_factor(X, code_maps, bits, bs, name, diag):
+    """Either factor, sizes that take every tile shape, the cut along k and partners that end inside a tile; the operand is
+    what the stack dequantizer (pinned to the oracle elsewhere) writes."""
+    code = torch.from_numpy(code_maps[(name, bits)]).cuda()
+    g = torch.Generator(device="cuda").manual_seed(bits + bs)
+    for n, other, batch in ((256, 100, 2), (768, 320, 1), (1024, 64, 1), (256, 200, 40), (512, 132, 24), (320, 96, 60), (1536, 256, 1), (2304, 768, 1)):
+        if n % bs:
+            continue
+        mats = torch.randn(batch, n, n, device="cuda", generator=g)
+        mats[:, 3, :64] = 0.0                                  # a segment of zeros
+        mats[0, n - 1] *= 1e-3
+        q = X.quantize_stack(mats, X.empty_quantized(batch, n, bs, bits, code, diag))
+        if diag:
+            q.diag[0, 5] = 0.0
+        deq = X.dequantize_stack(q)
+        left, right = torch.randn(batch, n, other, device="cuda", generator=g), torch.randn(batch, other, n, device="cuda", generator=g)
+        top = X.amax(q)
+        assert bool((top >= deq.abs().amax((1, 2))).all())
+        tops = torch.zeros(batch, device="cuda")
+        got = X.gemm(q, left, amax=(top, X.amax(left)), amax_out=tops)
+        check(got, deq, left, n)
+        assert torch.equal(tops, got.abs().amax((1, 2)))
+        tops.zero_()
+        got = X.gemm(right, q, amax=(X.amax(right), top), amax_out=tops)
+        check(got, right, deq, n)
+        assert torch.equal(tops, got.abs().amax((1, 2)))
+        if n > 1024:
+            continue
+        none = torch.zeros(batch, dtype=torch.int32, device="cuda")
+        zero = torch.zeros(batch, device="cuda")               # a bound of no use: the bf16 split
+        assert torch.equal(X.gemm(q, left, amax=(zero, top), skip=none), X.gemm(q, left, skip=none))
+        assert torch.equal(X.gemm(right, q, amax=(top, zero), skip=none), X.gemm(right, q, skip=none))
+        # maxima that are not finite or beyond the bound make their tile the split's
+        q.absmax[0, 2 * (n // bs)] = float("inf")
+        for product in (lambda **kw: X.gemm(q, left, **kw)[0, :64], lambda **kw: X.gemm(right, q, **kw)[0, :, :64]):
+            a, b = product(amax=(top, top), skip=none), product(skip=none)
+            assert np.array_equal(a.cpu().numpy(), b.cpu().numpy(), equal_nan=True)
+
+
+def test_preconditioned_gradients_look_their_operands_up_where_it_pays(X, code_maps):
+    code = torch.from_numpy(code_maps[("linear-2", 4)]).cuda()
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for m, n, batch in ((768, 3072, 1), (256, 256, 3)):
+        made = [torch.randn(batch, k, k, device="cuda", generator=g) * 0.02 + torch.eye(k, device="cuda") for k in (m, n)]
+        left, right = (X.quantize_stack(t, X.empty_quantized(batch, t.shape[1], 64, 4, code, True)) for t in made)
+        G = torch.randn(batch, m, n, device="cuda", generator=g)
+        assert X.worth_measuring(left, G, right) == (m == 768)
+        want = X.dequantize_stack(left).double() @ G.double() @ X.dequantize_stack(right).double()
+        assert float((X.precondition(G, left, right).double() - want).norm() / want.norm()) <= 1e-6
+    left = X.quantize_stack(made[0], X.empty_quantized(batch, 256, 64, 4, code, True))
+    flat = X.precondition(G[0], X.Quantized(left.codes[:1], left.absmax[:1], left.diag[:1], 256, 64, 4, code), right.rows(0, 1))
+    assert flat.shape == (256, 256)
