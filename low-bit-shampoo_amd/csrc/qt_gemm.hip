@@ -2023,7 +2023,8 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         break;
 #define QT_GEMM_CASE_REQUANT(KA, KB, EP)                                                                     \
     case (KA) * 100 + (KB) * 10 + (EP):                                                                      \
-        if (split_pipe) launch_gemm<128, 128, KA, KB, EP, kPipeSplit>(a, d->batch, stream);                  \
+        if (half_pipe) launch_gemm<128, 128, KA, KB, EP, kPipeHalf>(a, d->batch, stream);                    \
+        else if (split_pipe) launch_gemm<128, 128, KA, KB, EP, kPipeSplit>(a, d->batch, stream);             \
         else launch_gemm<128, 128, KA, KB, EP>(a, d->batch, stream);                                         \
         break;
 #define QT_GEMM_CASE_QUANT(KA, KB, EP)                                                                        \

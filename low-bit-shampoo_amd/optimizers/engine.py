@@ -342,12 +342,13 @@ class ShampooBank:
         w1 = self.stat_decay
         w2 = 1.0 if w1 == 1.0 else 1.0 - w1
 
-        def job(g, side):
+        def job(g, side, top=None):
             def run():
                 G = self._grad_list(g, grads)
                 seg = self._segment(self.stats, g, side)
                 skip = self._skip(g, only)
-                kw = dict(trans_a=side == 1, trans_b=side == 0, alpha=w2, beta=w1, symmetric=True)
+                kw = dict(trans_a=side == 1, trans_b=side == 0, alpha=w2, beta=w1, symmetric=True,
+                          amax=None if top is None else (top, top))
                 if seg.flat and self.blocksize == 64:
                     # dequantize, update and requantize in one launch: the fp32 statistic never reaches memory
                     X.gemm(G, G, addend=seg, requantize=True, skip=skip, **kw)
@@ -363,6 +364,8 @@ class ShampooBank:
                     return
                 # some blocks are left out: the others are gathered, updated and put back
                 take = torch.nonzero(skip == 0).squeeze(1)
+                if top is not None:
+                    kw["amax"] = (top.index_select(0, take),) * 2
                 sub = seg.select(take)
                 dense = X.load_stack(sub)
                 X.gemm(X.PtrList(G.ptrs.index_select(0, take), (take.numel(), g.bm, g.bn), ld=g.ld),
@@ -371,10 +374,23 @@ class ShampooBank:
                 seg.put(take, X.store_stack(dense, sub))
             return run
 
+        def both(g):
+            def run():                  # the gradients' largest elements serve both sides
+                top = X.amax(self._grad_list(g, grads))
+                for side in (0, 1):
+                    job(g, side, top)()
+            return run
+
+        jobs = []
         for g in self.groups:           # address tables are written on the current stream, before the fan-out
             self._grad_list(g, grads)
-        self._fan_out([job(g, side) for g in self.groups for side in (0, 1)
-                       if only is None or any(pi in only for pi in g.param_index)])
+            if only is not None and not any(pi in only for pi in g.param_index):
+                continue
+            if X.worth_measuring_for(len(g) * g.bm * g.bn * (g.bm + g.bn) // 2, g.bm, g.bn):
+                jobs.append(both(g))
+            else:
+                jobs += [job(g, 0), job(g, 1)]
+        self._fan_out(jobs)
 
     @torch.no_grad()
     def compute_preconditioners(self, v0=None, only=None):

@@ -391,11 +391,16 @@ def worth_measuring(left, G, right) -> bool:
     8 us of the device and 20 of the host (768 x 3072 by itself 145 -> 133 us; half as much work gains nothing)."""
     m, n = G.shape[-2:]
     batch = 1 if G.dim() == 2 else G.shape[0]
-    return min(m, n) >= 256 and m % 32 == n % 32 == 0 and batch * m * n * (m + n) >= MEASURE_FROM and gemm_pipe() == "split" and all(
+    return worth_measuring_for(batch * m * n * (m + n), m, n) and all(
         q.flat if isinstance(q, Quantized) else q.stride(-1) == 1 for q in (left, right))
 
 
-MEASURE_FROM = 1 << 33           # multiply-adds
+def worth_measuring_for(multiply_adds: int, *k: int) -> bool:
+    """The same for products of so much work in all, over sums of these lengths."""
+    return multiply_adds >= MEASURE_FROM and all(x >= 256 and x % 32 == 0 for x in k) and gemm_pipe() == "split"
+
+
+MEASURE_FROM = 1 << 33
 
 
 def gram(G: Tensor, axis: int, *, stat=None, beta=0.0, alpha=1.0, out: Optional[Tensor] = None) -> Tensor:
