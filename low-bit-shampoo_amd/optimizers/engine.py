@@ -26,6 +26,7 @@ so the parameters of a bank may be due for different things at one call.
 import threading
 from collections import defaultdict
 
+import numpy as np
 import torch
 
 from optimizers.matrix_functions import ComputePowerBatched
@@ -40,7 +41,7 @@ class _Group:
         self.bm, self.bn, self.ld = bm, bn, ld
         self.param_index, self.offset = [], []       # which parameter, element offset of the block
         self.slot = [None, None]                     # (order, first row in that order's stack) per side
-        self.grad_key, self.grad_ptrs, self.out_ptrs = None, None, None
+        self.grad_ptrs, self.out_ptrs = None, None
 
     def __len__(self):
         return len(self.param_index)
@@ -140,6 +141,9 @@ class ShampooBank:
         # Independent groups run on a few side streams so that the tail of one launch overlaps the
         # head of the next; biggest first.
         self.groups.sort(key=lambda g: -len(g) * g.bm * g.bn * (g.bm + g.bn))
+        self.grad_key = None
+        self.table_params = np.concatenate([np.asarray(g.param_index, dtype=np.int64) for g in self.groups])
+        self.table_offsets = 4 * np.concatenate([np.asarray(g.offset, dtype=np.int64) for g in self.groups])
         streams = self.DEFAULT_STREAMS if streams is None else streams
         self.streams = [shared_stream(self.device, i) for i in range(min(streams, len(self.groups), 8))]
 
@@ -242,13 +246,23 @@ class ShampooBank:
         order, first = g.slot[side]
         return table[order].rows(first, len(g))
 
-    def _grad_list(self, g, grads):
+    def _write_grad_tables(self, grads):
+        """The device table of all groups' block addresses, written on the current stream if a gradient has moved: one
+        copy for all groups, through pinned memory and without blocking (a pageable copy per group made the host wait
+        for what was queued, fourteen times in a step over the convolution weights)."""
         # (a parameter that is left out of this call has no gradient: its own storage stands in, never read)
-        key = tuple((self.params[pi] if grads[pi] is None else grads[pi]).data_ptr() for pi in g.param_index)
-        if key != g.grad_key:
-            g.grad_ptrs = torch.tensor([base + 4 * off for base, off in zip(key, g.offset)], dtype=torch.int64,
-                                       device=self.device)
-            g.grad_key = key
+        bases = tuple([(p if grad is None else grad).data_ptr() for p, grad in zip(self.params, grads)])
+        if bases == self.grad_key:
+            return
+        host = torch.from_numpy(np.asarray(bases, dtype=np.int64)[self.table_params] + self.table_offsets)
+        table = host.pin_memory().to(self.device, non_blocking=True)
+        first = 0
+        for g in self.groups:
+            g.grad_ptrs = table[first:first + len(g)]
+            first += len(g)
+        self.grad_key = bases
+
+    def _grad_list(self, g):
         return X.PtrList(g.grad_ptrs, (len(g), g.bm, g.bn), ld=g.ld)
 
     def _out_list(self, g):
@@ -312,8 +326,7 @@ class ShampooBank:
         started afterwards from several threads only read them."""
         only = self._only(only, len(self.params))
         self._check(grads, only)
-        for g in self.groups:
-            self._grad_list(g, grads)
+        self._write_grad_tables(grads)
 
     # The coupled Newton iteration holds ten fp32 stacks of what it works on (two copies each of the root, the
     # iterate and the iteration matrix, two powers, the input, the result): a stack goes through it in parts of
@@ -344,7 +357,7 @@ class ShampooBank:
 
         def job(g, side, top=None):
             def run():
-                G = self._grad_list(g, grads)
+                G = self._grad_list(g)
                 seg = self._segment(self.stats, g, side)
                 skip = self._skip(g, only)
                 kw = dict(trans_a=side == 1, trans_b=side == 0, alpha=w2, beta=w1, symmetric=True,
@@ -376,14 +389,14 @@ class ShampooBank:
 
         def both(g):
             def run():                  # the gradients' largest elements serve both sides
-                top = X.amax(self._grad_list(g, grads))
+                top = X.amax(self._grad_list(g))
                 for side in (0, 1):
                     job(g, side, top)()
             return run
 
         jobs = []
-        for g in self.groups:           # address tables are written on the current stream, before the fan-out
-            self._grad_list(g, grads)
+        self._write_grad_tables(grads)  # on the current stream, before the fan-out
+        for g in self.groups:
             if only is not None and not any(pi in only for pi in g.param_index):
                 continue
             if X.worth_measuring_for(len(g) * g.bm * g.bn * (g.bm + g.bn) // 2, g.bm, g.bn):
@@ -450,7 +463,7 @@ class ShampooBank:
                 left = left if left.flat else X.load_stack(left)         # read inside the product, or dequantized first
                 right = right if right.flat else X.load_stack(right)
                 half = torch.empty(len(g), g.bm, g.bn, device=self.device)
-                G = self._grad_list(g, grads)
+                G = self._grad_list(g)
                 if not X.worth_measuring(left, G, right):
                     X.gemm(left, G, out=half, skip=skip)
                     X.gemm(half, right, out=self._out_list(g), skip=skip)
@@ -461,8 +474,8 @@ class ShampooBank:
                 X.gemm(half, right, out=self._out_list(g), skip=skip, amax=(tops[3], tops[2]))
             return run
 
+        self._write_grad_tables(grads)
         for g in self.groups:
-            self._grad_list(g, grads)
             self._out_list(g)
         self._fan_out([job(g) for g in self.groups if only is None or any(pi in only for pi in g.param_index)], inline=inline)
         return [out.view(p.shape) if only is None or pi in only else None

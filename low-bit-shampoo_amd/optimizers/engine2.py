@@ -197,11 +197,11 @@ class ShampooBank2(ShampooBank):
         top_stat = {o: self._tops(o, self.per_order[o]) for o in orders}               # largest elements, where they are looked up
         ones = torch.ones(max(self.per_order.values()), device=self.device)
         top_grad = {}                                                                  # group -> its gradients' largest elements
+        self._write_grad_tables(grads)
         for g in self.groups:
-            G = self._grad_list(g, grads)
             if (only is None or any(pi in only for pi in g.param_index)) and X.worth_measuring_for(
                     len(g) * g.bm * g.bn * (g.bm + g.bn) // 2, g.bm, g.bn):
-                top_grad[id(g)] = X.amax(G)
+                top_grad[id(g)] = X.amax(self._grad_list(g))
 
         solver, redone, tick, begun = {}, {}, {}, {}
         # (a stack starts with the replacing sweep when most of it needed that sweep lately, or when it holds many
@@ -223,7 +223,7 @@ class ShampooBank2(ShampooBank):
             def run():
                 order, first = g.slot[side]
                 seg = stat[order][first:first + len(g)]
-                G = self._grad_list(g, grads)
+                G = self._grad_list(g)
                 top_out = None if top_stat[order] is None else top_stat[order][first:first + len(g)]
                 X.gemm(G, G, trans_a=side == 1, trans_b=side == 0, addend=seg, alpha=w2, beta=w1, out=seg, symmetric=True,
                        skip=self._skip(g, only), amax=(top_grad[id(g)],) * 2 if id(g) in top_grad else None, amax_out=top_out)

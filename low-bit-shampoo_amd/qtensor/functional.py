@@ -163,13 +163,23 @@ def _check_common(code: Tensor, order: int, blocksize: int, bits: int, device: t
     _check_buffer(code, "code", 2 ** bits, torch.float32, device)
 
 
+def _raw_stream(index: int) -> int:
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# (what current_stream looks up, without the Stream object around it: 0.2 of 3 us per call, where a call is 8 us)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _raw_stream)
+_this_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 def _call(fn, device: torch.device, *args) -> None:
-    stream = torch.cuda.current_stream(device).cuda_stream
-    if device.index is not None and device.index != torch.cuda.current_device():
-        with torch.cuda.device(device):
-            fn(*args, stream)
+    here = _this_device()
+    index = here if device.index is None else device.index
+    if index != here:
+        with torch.cuda.device(index):
+            fn(*args, _raw_stream(index))
     else:
-        fn(*args, stream)
+        fn(*args, _raw_stream(index))
     if lib.qtensor_hip_last_error():
         raise RuntimeError("libqtensor_hip: " + lib.qtensor_hip_last_error_string().decode())
 

@@ -169,9 +169,9 @@ def _launch(desc: GemmDesc, device: torch.device, ranges: Optional[GemmRanges] =
     if F.lib is None:
         raise RuntimeError("libqtensor_hip.so is not available")
     if ranges is not None:
-        F._call(lambda d, r, s: F.lib.qtensor_hip_gemm_ranged(d, r, s), device, ct.byref(desc), ct.byref(ranges))
+        F._call(F.lib.qtensor_hip_gemm_ranged, device, ct.byref(desc), ct.byref(ranges))
         return
-    F._call(lambda d, s: F.lib.qtensor_hip_gemm(d, s), device, ct.byref(desc))
+    F._call(F.lib.qtensor_hip_gemm, device, ct.byref(desc))
 
 
 def amax_into(*pairs) -> None:
