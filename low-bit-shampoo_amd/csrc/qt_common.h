@@ -61,6 +61,16 @@ __device__ __forceinline__ uint16_t float_to_bf16_bits(float x) {
     return (uint16_t)(u >> 16);
 }
 
+// Two floats to packed bf16, the bits of float_to_bf16_bits: the conversion instruction rounds the same way (checked for all
+// 2^32 values) and only its NaN differ.
+__device__ __forceinline__ uint32_t floats_to_bf16_pair(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    if (__builtin_expect(__builtin_isunordered(a, b), 0)) return (uint32_t)float_to_bf16_bits(a) | ((uint32_t)float_to_bf16_bits(b) << 16);
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
 // 16-byte global accesses with an optional streaming (nontemporal) hint: data that is touched
 // once should not displace what the caches hold.  On MI355X the hint lifts a pure read stream
 // from about 6.4 to 7.2 TB/s.

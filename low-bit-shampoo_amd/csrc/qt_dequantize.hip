@@ -15,15 +15,11 @@ namespace {
 #ifndef QT_D_THREADS
 #define QT_D_THREADS 128
 #endif
-#ifndef QT_D_BLOCKS_PER_CU
-#define QT_D_BLOCKS_PER_CU 3
-#endif
 #ifndef QT_D_CHUNKED
 #define QT_D_CHUNKED 0
 #endif
 constexpr int kThreads = 256;             // general-path kernel
 constexpr int kFlatThreads = QT_D_THREADS;
-constexpr int kFlatBlocksPerCU = QT_D_BLOCKS_PER_CU;
 constexpr int kSuper = 2048;              // elements a wave turns around per step
 
 template <typename T> struct Vec4Store;
@@ -38,8 +34,8 @@ template <> struct Vec4Store<uint16_t> {
     template <bool STREAM>
     static __device__ __forceinline__ void store(uint16_t *base, uint32_t k, float4 y) {
         uint2 w;
-        w.x = (uint32_t)float_to_bf16_bits(y.x) | ((uint32_t)float_to_bf16_bits(y.y) << 16);
-        w.y = (uint32_t)float_to_bf16_bits(y.z) | ((uint32_t)float_to_bf16_bits(y.w) << 16);
+        w.x = floats_to_bf16_pair(y.x, y.y);
+        w.y = floats_to_bf16_pair(y.z, y.w);
         store_u32x2<STREAM>(base + k, w);
     }
     static __device__ __forceinline__ void store1(uint16_t *base, size_t k, float y) { base[k] = float_to_bf16_bits(y); }
@@ -52,9 +48,17 @@ template <> struct Vec4Store<uint16_t> {
 // The loads of the next step are issued before the stores of the current one.  Big outputs are written
 // with the streaming hint, but the codes are always read with plain loads: on an MI355X the hint on this
 // thin read stream beside the wide write stream costs a tenth of the bandwidth (0.224 -> 0.199 ms for the
-// 16384^2 tensor), and six waves per compute unit in workgroups of two do better than twelve in
+// 16384^2 tensor), and six waves per compute unit in workgroups of two do better there than twelve in
 // workgroups of four (0.199 -> 0.185 ms).
-template <typename T, int BITS, bool DIAG, bool STREAM>
+//
+// The exact diagonal.  kDiagFew: orders of 2048 and more, where a step's elements lie in two rows at most: the places of
+// their diagonal entries are the same for the whole wave and cost a scalar comparison per store.  kDiagAny: every lane
+// walks along rows and columns, work that waits beside the loads: 8192 x 8192 with codes that come from memory, 4 bits to
+// fp32 97 us, few 61 (without a diagonal 58), to bf16 54 us at best, few 34.  With codes that the last-level cache still
+// holds the slower walk paces the stores, any 45 us and few 46 (12032 x 12032: 93 and 96, 8 bits 100 and 108): the codes of a
+// preconditioner that is used once per step come from memory.
+enum DiagKind : int { kDiagNone = 0, kDiagAny = 1, kDiagFew = 2 };
+template <typename T, int BITS, int DIAG, bool STREAM>
 __global__ __launch_bounds__(kFlatThreads) void dequantize_flat_kernel(
     const uint8_t *__restrict__ q, const float *__restrict__ code, uint32_t n_super, uint32_t bs_shift,
     FastDiv row_div, FastDiv order_div, const float *__restrict__ absmax, const float *__restrict__ diag, T *__restrict__ out) {
@@ -105,7 +109,18 @@ __global__ __launch_bounds__(kFlatThreads) void dequantize_flat_kernel(
 
         const uint32_t k4_0 = st * (uint32_t)(kSuper / 4) + lane;   // index of this lane's first 4-vector
         uint32_t row = 0, col4 = 0, lrow = 0;                        // row of the stack, and inside its matrix
-        if (DIAG) {
+        // kDiagFew: where the two rows' diagonal entries lie, counted from the step's first element (beyond the step: none)
+        uint32_t at0 = 0xffffffffu, at1 = 0xffffffffu;
+        float d0 = 0.0f, d1 = 0.0f;
+        if (DIAG == kDiagFew) {
+            const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)st) * (uint32_t)kSuper, order = order_div.divisor;
+            const uint32_t r = fastdiv(first >> 2, row_div), in = r - fastdiv(r, order_div) * order, next = in + 1u == order ? 0u : in + 1u;
+            at0 = r * order + in - first;                            // (wraps around where the entry lies before the step)
+            at1 = (r + 1u) * order + next - first;
+            if (at0 < (uint32_t)kSuper) d0 = diag[r];
+            if (at1 < (uint32_t)kSuper) d1 = diag[r + 1u];
+        }
+        if (DIAG == kDiagAny) {
             row = fastdiv(k4_0, row_div);
             col4 = k4_0 - row * row_div.divisor;
             lrow = row - fastdiv(row, order_div) * order_div.divisor;
@@ -128,7 +143,17 @@ __global__ __launch_bounds__(kFlatThreads) void dequantize_flat_kernel(
             } else {
                 y = make_float4(s_code[id0] * scale, s_code[id1] * scale, s_code[id2] * scale, s_code[id3] * scale);
             }
-            if (DIAG) {
+            if (DIAG == kDiagFew) {
+                if (at0 >> 8 == j && (at0 >> 2 & 63u) == lane) {
+                    const uint32_t e = at0 & 3u;
+                    if (e == 0) y.x = d0; else if (e == 1) y.y = d0; else if (e == 2) y.z = d0; else y.w = d0;
+                }
+                if (at1 >> 8 == j && (at1 >> 2 & 63u) == lane) {
+                    const uint32_t e = at1 & 3u;
+                    if (e == 0) y.x = d1; else if (e == 1) y.y = d1; else if (e == 2) y.z = d1; else y.w = d1;
+                }
+            }
+            if (DIAG == kDiagAny) {
                 if ((lrow >> 2) == col4) {
                     const float d = diag[row];
                     const uint32_t e = lrow & 3u;
@@ -198,8 +223,7 @@ template <> struct AnyAligned4<float> {
 template <> struct AnyAligned4<uint16_t> {
     typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
     static __device__ __forceinline__ void store(uint16_t *p, const float y[4]) {
-        const u32x2_any v = {(uint32_t)float_to_bf16_bits(y[0]) | ((uint32_t)float_to_bf16_bits(y[1]) << 16),
-                             (uint32_t)float_to_bf16_bits(y[2]) | ((uint32_t)float_to_bf16_bits(y[3]) << 16)};
+        const u32x2_any v = {floats_to_bf16_pair(y[0], y[1]), floats_to_bf16_pair(y[2], y[3])};
         *reinterpret_cast<u32x2_any *>(p) = v;
     }
 };
@@ -321,15 +345,24 @@ void dequantize_dispatch(const uint8_t *q, const float *code, int order_i, const
         constexpr uint32_t kWaves = kFlatThreads / 64;
         const uint32_t n_super = total / kSuper;
         const uint32_t blocks = (n_super + kWaves - 1) / kWaves;
-        const dim3 grid(capped_grid(blocks, kFlatBlocksPerCU));
+        // Workgroups of two waves per unit.  An fp32 output that streams to memory is bound by its stores and takes the fewest
+        // that keep them coming (8192 x 8192: 47 us with three, 49.5 with six); one that the last-level cache takes, and
+        // bf16, whose look-ups per byte written are twice as many, want more waves to hide them behind: 4096 x 4096 fp32
+        // with its diagonal 15.4 us with three, 13.9 with six; bf16 8 bits 14.6 with three, 11.0 with six and with ten, 4
+        // bits 14.6, 10.2, 9.5; 12032 x 12032 bf16 80, 59, 61.
+        const bool streams = total >= (1u << 25);
+        const dim3 grid(capped_grid(blocks, sizeof(T) == 2 ? (streams ? 6 : 10) : streams ? 3 : 6));
+        constexpr int ANY = DIAG ? kDiagAny : kDiagNone, FEW = DIAG ? kDiagFew : kDiagNone;
         // Outputs far beyond the 256 MB last-level cache are written with the streaming hint.
-        if (total >= (1u << 25)) {
-            hipLaunchKernelGGL((dequantize_flat_kernel<T, BITS, DIAG, true>), grid, dim3(kFlatThreads), 0, stream,
-                               q, code, n_super, (uint32_t)bs_shift, make_fastdiv(order / 4), make_fastdiv(order), absmax, diag, out);
-        } else {
-            hipLaunchKernelGGL((dequantize_flat_kernel<T, BITS, DIAG, false>), grid, dim3(kFlatThreads), 0, stream,
-                               q, code, n_super, (uint32_t)bs_shift, make_fastdiv(order / 4), make_fastdiv(order), absmax, diag, out);
-        }
+#define QT_DEQUANT_FLAT(KIND, STREAM)                                                                                                   \
+        hipLaunchKernelGGL((dequantize_flat_kernel<T, BITS, KIND, STREAM>), grid, dim3(kFlatThreads), 0, stream, q, code, n_super,       \
+                           (uint32_t)bs_shift, make_fastdiv(order / 4), make_fastdiv(order), absmax, diag, out)
+        if (order >= (uint32_t)kSuper) {
+            if (streams) QT_DEQUANT_FLAT(FEW, true);
+            else QT_DEQUANT_FLAT(FEW, false);
+        } else if (streams) QT_DEQUANT_FLAT(ANY, true);
+        else QT_DEQUANT_FLAT(ANY, false);
+#undef QT_DEQUANT_FLAT
     } else {
         const uint32_t nb = (order + bs - 1) / bs;
         const uint32_t one = order * order;

@@ -388,3 +388,30 @@ def test_launches_on_either_side_of_the_lines_of_the_loads_far_ahead_have_the_sa
         want[flags.bool().cpu()] = -7.0
     # dropped pieces 2^-24 |a b| each and k fp32 additions, plus the last sum's rounding
     assert bool(((b.cpu().double() - want).abs() <= (k + 4) * 2 ** -24 * size + 1e-30).all())
+
+
+@pytest.mark.parametrize("order,batch,bits,blocksize", [(1984, 1, 4, 64), (2048, 3, 4, 64), (2048, 1, 8, 2048), (2112, 2, 8, 64), (4096, 1, 4, 256), (5888, 1, 8, 256)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_flat_dequantizer_puts_the_diagonal_where_it_belongs_in_wide_matrices(order, batch, bits, blocksize, dtype):
+    """Orders on either side of the step's 2048 elements, launches on either side of the streaming one, segments that are zero
+    or not finite and NaN on the diagonal (bf16: the same NaN): against the oracle's dequantizer, bit for bit."""
+    import numpy as np
+    import qtensor.functional as F
+    from oracle import quant_np as Q
+    from qtensor import fused
+    code = F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)
+    g = torch.Generator().manual_seed(order)
+    q = fused.empty_quantized(batch, order, blocksize, bits, code.cuda(), True)
+    q.codes.copy_(torch.randint(0, 256, q.codes.shape, generator=g, dtype=torch.uint8))
+    q.absmax.copy_(torch.rand(q.absmax.shape, generator=g))
+    q.diag.copy_(torch.randn(q.diag.shape, generator=g))
+    q.absmax[0, 5], q.absmax[0, 6], q.absmax[0, 7] = 0.0, float("inf"), float("nan")
+    q.diag[0, 9], q.diag[batch - 1, order - 1] = float("nan"), -float("nan")
+    got = fused.dequantize_stack(q, outdtype=dtype)
+    for b in range(batch):
+        want = Q.dequantize_c(q.codes[b].cpu().numpy(), code.numpy(), order, q.absmax[b].cpu().numpy(), blocksize, bits,
+                              diag=q.diag[b].cpu().numpy(), to_bf16=dtype == torch.bfloat16)
+        assert np.array_equal(got[b].float().cpu().numpy(), np.asarray(want).reshape(order, order), equal_nan=True)
+        if dtype == torch.bfloat16:
+            bad = got[b].isnan()
+            assert bool((got[b].view(torch.int16)[bad] == 0x7FC0).all())
