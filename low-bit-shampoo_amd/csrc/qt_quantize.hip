@@ -246,25 +246,27 @@ __device__ __forceinline__ void load_upto_four(const T *p, uint32_t n, float x[4
 }
 
 constexpr uint32_t kChunkIds = 8192;     // codes of the largest chunk (four segments of 2048)
-__host__ __device__ inline uint32_t chunk_segments(uint32_t bs_shift) { return bs_shift < 9 ? 2048u >> bs_shift : 4u; }
+// Segments of a chunk: places for 2048 elements, or for 8192 where there are chunks enough all the same (LARGE).
+inline uint32_t chunk_segments(uint32_t bs_shift, bool large) { return large ? kChunkIds >> bs_shift : bs_shift < 9 ? 2048u >> bs_shift : 4u; }
 
-template <typename T, int BITS, bool DIAG, bool WHOLE>
+template <typename T, int BITS, bool DIAG, bool WHOLE, bool LARGE>
 __global__ __launch_bounds__(kThreads) void quantize_general_kernel(
     const T *__restrict__ A, const float *__restrict__ code, uint32_t order, uint32_t bs_shift, uint32_t nb, FastDiv nb_div,
-    uint32_t n_segments, uint32_t chunks_per_matrix, uint32_t n_chunks, float *__restrict__ absmax, float *__restrict__ diag,
-    uint8_t *__restrict__ out) {
+    uint32_t n_segments, uint32_t per_chunk, uint32_t chunks_per_matrix, uint32_t n_chunks, float *__restrict__ absmax,
+    float *__restrict__ diag, uint8_t *__restrict__ out) {
     constexpr int NCODE = 1 << BITS;
     constexpr uint32_t EPB = 8 / BITS;
     __shared__ CodeTables<NCODE> tab;
     __shared__ uint8_t ids[WHOLE ? 1 : kChunkIds + 1];               // (the shared byte's second code behind them)
-    build_code_tables<NCODE>(code, tab, nullptr);
+    __shared__ uint2 lut_mem[LARGE ? kLutEntries : 1];
+    uint2 *lut = LARGE ? lut_mem : nullptr;
+    build_code_tables<NCODE>(code, tab, lut);
     const bool fast_ok = (tab.flags & kFlagLut) != 0, ascending = (tab.flags & kFlagAscending) != 0;
     const uint32_t bs = 1u << bs_shift;
     const uint32_t g_shift = min(bs_shift - 2u, 6u);                  // log2 of the lanes per segment
     const uint32_t in_group = (threadIdx.x & ((1u << g_shift) - 1u)) * 4u, group = threadIdx.x >> g_shift;
     const uint32_t n_groups = (uint32_t)kThreads >> g_shift;
     const uint32_t total = order * order, n_bytes = (total + EPB - 1) / EPB;
-    const uint32_t per_chunk = chunk_segments(bs_shift);
 
     for (uint32_t chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
         const uint32_t b = chunk / chunks_per_matrix;
@@ -321,7 +323,7 @@ __global__ __launch_bounds__(kThreads) void quantize_general_kernel(
                 for (int e = 0; e < 4; ++e) {
                     if (exact) idx[e] = exact_index<NCODE>(x[e], m, tab);
                     else {
-                        idx[e] = fast_index<NCODE, false>(x[e], a, recip, tab, nullptr);
+                        idx[e] = fast_index<NCODE, LARGE>(x[e], a, recip, tab, lut);
                         if (!ascending) idx[e] = tab.perm[idx[e]];
                     }
                 }
@@ -472,16 +474,24 @@ void launch_general(const T *A, const float *code, uint32_t order, uint32_t bs, 
     const uint32_t bs_shift = (uint32_t)__builtin_ctz(bs);
     const uint32_t nb = (order + bs - 1) / bs;
     const uint32_t n_segments = order * nb;
-    const uint32_t per_chunk = chunk_segments(bs_shift), per_matrix = (n_segments + per_chunk - 1) / per_chunk;
+    // 8-bit codes of many elements: the index from the bucket table instead of a search of eight dependent LDS reads, chunks
+    // four times as large.  One matrix, us with the search and with the table: 2001 x 2001 16.8 and 16.6, 3001 x 3001 29.7
+    // and 26.6, 5001 x 5001 in segments of 128 75.9 and 45.9, 9001 x 9001 258 and 141.  4-bit codes, whose search is one
+    // dependent read, gain nothing (5001 x 5001 41.4 and 46.8).
+    const bool large = BITS == 8 && (uint64_t)order * order * batch >= (1u << 23);
+    const uint32_t per_chunk = chunk_segments(bs_shift, large), per_matrix = (n_segments + per_chunk - 1) / per_chunk;
     const uint32_t n_chunks = per_matrix * batch;      // (batch * order * order < 2^31 and batch <= 65535: fits)
     const FastDiv nbd = make_fastdiv(nb);
-    const dim3 grid(grid_for(n_chunks, 8));
-    if (order % 4 == 0 && is_aligned(out, BITS == 4 ? 2 : 4))
-        hipLaunchKernelGGL((quantize_general_kernel<T, BITS, DIAG, true>), grid, dim3(kThreads), 0, stream,
-                           A, code, order, bs_shift, nb, nbd, n_segments, per_matrix, n_chunks, absmax, diag, out);
-    else
-        hipLaunchKernelGGL((quantize_general_kernel<T, BITS, DIAG, false>), grid, dim3(kThreads), 0, stream,
-                           A, code, order, bs_shift, nb, nbd, n_segments, per_matrix, n_chunks, absmax, diag, out);
+    const dim3 grid(grid_for(n_chunks, large ? 4 : 8));
+    const bool whole = order % 4 == 0 && is_aligned(out, BITS == 4 ? 2 : 4);
+    constexpr bool TABLE = BITS == 8;
+#define QT_QUANT_GENERAL(WHOLE, LARGE)                                                                                               \
+    hipLaunchKernelGGL((quantize_general_kernel<T, BITS, DIAG, WHOLE, LARGE>), grid, dim3(kThreads), 0, stream, A, code, order, bs_shift, \
+                       nb, nbd, n_segments, per_chunk, per_matrix, n_chunks, absmax, diag, out)
+    if (whole) { if (large) QT_QUANT_GENERAL(true, TABLE); else QT_QUANT_GENERAL(true, false); }
+    else if (large) QT_QUANT_GENERAL(false, TABLE);
+    else QT_QUANT_GENERAL(false, false);
+#undef QT_QUANT_GENERAL
 }
 
 template <typename T, int BITS, bool DIAG>

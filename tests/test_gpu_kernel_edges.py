@@ -390,6 +390,25 @@ def test_launches_on_either_side_of_the_lines_of_the_loads_far_ahead_have_the_sa
     assert bool(((b.cpu().double() - want).abs() <= (k + 4) * 2 ** -24 * size + 1e-30).all())
 
 
+@pytest.mark.parametrize("order,batch,blocksize", [(2896, 1, 512), (2900, 1, 64), (2897, 1, 128), (102, 807, 64), (4100, 1, 2048)])
+def test_general_quantizer_on_either_side_of_the_size_from_which_it_has_a_bucket_table(order, batch, blocksize):
+    """8-bit codes, 2^23 elements: the first and the last matrix against the oracle, bit for bit."""
+    import numpy as np
+    import qtensor.functional as F
+    from oracle import quant_np as Q
+    from qtensor import fused
+    code = F.create_dynamic_map(True, 8, 1)
+    mats = torch.randn(batch, order, order, generator=torch.Generator().manual_seed(order))
+    mats[0, order // 2] = 0.0
+    mats[0, 3, 5] = float("nan")
+    mats[batch - 1, order - 1] *= 1e-30                                    # maxima outside the fast division's range
+    q = fused.quantize_stack(mats.cuda(), fused.empty_quantized(batch, order, blocksize, 8, code.cuda(), True))
+    for b in {0, batch - 1}:
+        want = Q.quantize_c(mats[b].numpy(), code.numpy(), order, blocksize, 8, True)
+        assert np.array_equal(q.codes[b].cpu().numpy(), want[0])
+        assert np.array_equal(q.absmax[b].cpu().numpy(), want[1], equal_nan=True) and np.array_equal(q.diag[b].cpu().numpy(), want[2], equal_nan=True)
+
+
 @pytest.mark.parametrize("order,batch,bits,blocksize", [(1984, 1, 4, 64), (2048, 3, 4, 64), (2048, 1, 8, 2048), (2112, 2, 8, 64), (4096, 1, 4, 256), (5888, 1, 8, 256)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_flat_dequantizer_puts_the_diagonal_where_it_belongs_in_wide_matrices(order, batch, bits, blocksize, dtype):
