@@ -162,11 +162,14 @@ def ComputePowerBatched(mats, p=4, iter_count=10, error_tolerance=1e-6, ridge_ep
     R_ptr, M_ptr, T_ptr = table(R), table(M), table(T)
     side = torch.zeros(B, dtype=torch.bool, device=dev)                     # False: buffer 0 holds the state
     # How large the iterates' elements are, for the pipe that wants to know: |M| and |T| follow from err = max |M - I|
-    # (T = I + w (M - I)), the roots and the powers of T are looked at by the launches that write them.
+    # (T = I + w (M - I)), the roots and the powers of T are looked at by the launches that write them.  Small stacks are
+    # bound by the host, which this costs 40 us a round (statistics of convolutions of width 32: 29 ms without, 33 with).
+    measured = X.worth_measuring_for(B * n ** 3, n)
     squarings = p.bit_length() - 1
-    tops = torch.zeros(iter_count, 1 + squarings, B, device=dev)
-    top_m, top_t = 1 + err, 1 + abs(w) * err
-    top_r = first_root * top_t                                               # of the root after the first round
+    if measured:
+        tops = torch.zeros(iter_count, 1 + squarings, B, device=dev)
+        top_m, top_t = 1 + err, 1 + abs(w) * err
+        top_r = first_root * top_t                                           # of the root after the first round
     for round_number in range(iter_count):
         skip = done.to(torch.int32)
         cur = lambda tab: torch.where(side, tab[1], tab[0])                   # noqa: E731
@@ -178,17 +181,22 @@ def ComputePowerBatched(mats, p=4, iter_count=10, error_tolerance=1e-6, ridge_ep
             torch.mul(T[0], first_root.view(B, 1, 1), out=R[1])
         else:
             X.gemm(X.PtrList(Rc, shape), X.PtrList(Tc, shape), out=X.PtrList(Ro, shape), skip=skip,
-                   symmetric=symmetric, amax=(top_r, top_t), amax_out=tops[round_number, 0])     # candidate root
-            top_r = tops[round_number, 0]                                    # (a rejected candidate ends its matrix's iteration)
-        power, top = X.PtrList(Tc, shape), top_t                             # T^p by repeated squaring
+                   symmetric=symmetric,                                      # candidate root
+                   **(dict(amax=(top_r, top_t), amax_out=tops[round_number, 0]) if measured else {}))
+            if measured:
+                top_r = tops[round_number, 0]                                # (a rejected candidate ends its matrix's iteration)
+        power = X.PtrList(Tc, shape)                                         # T^p by repeated squaring
+        top = top_t if measured else None
         for square in range(1, 1 + squarings):
             dst = Tp if power is T2 else T2
-            X.gemm(power, power, out=dst, skip=skip, symmetric=symmetric, amax=(top, top), amax_out=tops[round_number, square])
-            power, top = dst, tops[round_number, square]
+            after = tops[round_number, square] if measured else None
+            X.gemm(power, power, out=dst, skip=skip, symmetric=symmetric, amax=(top, top) if measured else None, amax_out=after)
+            power, top = dst, after
         new_err = torch.zeros(B, device=dev)
         X.gemm(power, X.PtrList(Mc, shape), out=X.PtrList(Mo, shape), newton=(X.PtrList(To, shape), w, new_err),
-               skip=skip, symmetric=symmetric, amax=(top, top_m))
-        top_m, top_t = 1 + new_err, 1 + abs(w) * new_err
+               skip=skip, symmetric=symmetric, amax=(top, top_m) if measured else None)
+        if measured:
+            top_m, top_t = 1 + new_err, 1 + abs(w) * new_err
         accept = (~done) & ~(new_err > err * 1.2)
         side = side ^ accept
         err = torch.where(accept, new_err, err)

@@ -152,9 +152,10 @@ def test_half_pipe_errors_against_those_of_the_split(X):
             assert half <= split + (2.0 ** -22 * float(want.norm()) if kind == 3 else 0.0), (k, kind, half, split)
 
 
-def test_inverse_roots_on_the_half_pipe_are_no_further_from_float64(X):
+def test_inverse_roots_on_the_half_pipe_are_no_further_from_float64(X, monkeypatch):
     """The iteration on the half pipe against the same iteration on the bf16 split (whose products take no amax)."""
     import optimizers.matrix_functions as MF
+    monkeypatch.setattr(X, "MEASURE_FROM", 0)                              # (these stacks are below the size that is measured)
     for n in (256, 320, 768):
         errors = {"half": 0.0, "split": 0.0}
         for seed in range(4):
