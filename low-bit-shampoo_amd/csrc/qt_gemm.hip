@@ -1153,12 +1153,15 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     const bool direct_vec = vec_ok && (args.N & 3) == 0;
     if constexpr (kRequant) {
         // beta * deq(E) + alpha * acc goes straight back into E's codes, maxima and exact diagonal: the fp32
-        // statistic never reaches memory.  A wave's 64 x 64 quadrant holds whole segments (blocksize 64) of 64
-        // rows -- and, mirrored, of 64 rows of the transposed tile -- so it encodes them alone: 32 rows at a
-        // time go through its staging area, 16 lanes take one row (four consecutive elements each), and the
-        // maximum, the division and the table search are those of the flat quantizer.  Each element of E is
+        // statistic never reaches memory.  A wave's 64 x 64 quadrant of a 128 x 128 tile holds whole segments
+        // (blocksize 64) of 64 rows -- and, mirrored, of 64 rows of the transposed tile -- so it encodes them alone: 32
+        // rows at a time go through its staging area, 16 lanes take one row (four consecutive elements each), and the
+        // maximum, the division and the table search are those of the flat quantizer.  A 64 x 64 tile, whose quadrants
+        // are half a segment wide, is staged as a whole, and each wave encodes 16 of its rows.  Each element of E is
         // read and rewritten by the same wave, all reads of a row before its writes.
-        float *stage = s_mem + wave * (32 * REQUANT_LD);
+        constexpr bool SMALL = BN == 64;
+        constexpr int ROWS = SMALL ? 16 : 32;                        // rows that a wave encodes at a time
+        float *stage = s_mem + wave * (ROWS * REQUANT_LD);
         uint8_t *o_codes = const_cast<uint8_t *>(e_codes);
         float *o_absmax = const_cast<float *>(e_absmax), *o_diag = const_cast<float *>(e_diag);
         const bool fast_ok = (tab.flags & kFlagLut) != 0, ascending = (tab.flags & kFlagAscending) != 0;
@@ -1166,7 +1169,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         auto encode_rows = [&](int row_base, int col_base) {
             if (col_base >= order) return;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
+            for (int q = 0; q < ROWS / 4; ++q) {
                 const int rl = q * 4 + (lane >> 4), c4 = (lane & 15) * 4;
                 const float4 a4 = *reinterpret_cast<const float4 *>(stage + rl * REQUANT_LD + c4);
                 const float a[4] = {a4.x, a4.y, a4.z, a4.w};
@@ -1197,6 +1200,22 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                     *(QT_GLOBAL uint32_t *)(o_codes + k0) = idx[0] | (idx[1] << 8) | (idx[2] << 16) | (idx[3] << 24);
             }
         };
+        if constexpr (SMALL) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                s_mem[(wm + 8 * (r / 4) + 4 * (lane >> 5) + r % 4) * REQUANT_LD + wn + (lane & 31)] = acc[0][0][r];
+            __syncthreads();
+            encode_rows(m0 + wave * ROWS, n0);
+            if (mirror) {                                            // (the same for the whole workgroup)
+                __syncthreads();
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    s_mem[(wn + (lane & 31)) * REQUANT_LD + wm + 8 * (r / 4) + 4 * (lane >> 5) + r % 4] = acc[0][0][r];
+                __syncthreads();
+                encode_rows(n0 + wave * ROWS, m0);
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
 #pragma unroll
@@ -1570,7 +1589,8 @@ void launch_gemm(const RangedArgs &a, int batch, hipStream_t stream) {
         blocks = (runs + a.stream_per - 1) / a.stream_per;
     }
     if (blocks > 0x7fffffffLL) { set_error(kBadArgument, "gemm: too many tiles (%lld)", blocks); return; }
-    if constexpr (PREC == kPipeSplit && BM == 64 && BN == 64 && KA < kQuant4 && KB < kQuant4 && EPI <= kAxpbyDense) {
+    if constexpr (PREC == kPipeSplit && BM == 64 && BN == 64 && KA < kQuant4 && KB < kQuant4 &&
+                  (EPI <= kAxpbyDense || EPI == kRequant4 || EPI == kRequant8)) {
         // Loads far ahead where the launch's own workgroups have a unit each and half of the units stay free: a per-parameter
         // optimizer step over convolution weights, chains of products of 2 to 38 tiles, 34.1 -> 32.3 ms.  Both lines are
         // measured.  Workgroups: at one or two per unit the step is the same to the noise, and for every launch the
@@ -1910,7 +1930,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         double best = 0.0;
         for (int i = 0; i < 4; ++i) {
             const Shape &sh = shapes[i];
-            if (a.symmetric && sh.bm != sh.bn) continue;
+            if ((a.symmetric || requant) && sh.bm != sh.bn) continue;
             const long long tm = (d->M + sh.bm - 1) / sh.bm, tn = (d->N + sh.bn - 1) / sh.bn;
             const double tiles = (double)(a.symmetric ? tn * (tn + 1) / 2 : tm * tn) * d->batch;
             // a workgroup alone on its unit hides none of its load latencies, prologue and epilogue behind
@@ -1922,7 +1942,10 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         }
     }
     if (a.symmetric && shapes[pick].bm != shapes[pick].bn) pick = 0;
-    if (requant) pick = 0;          // a wave's quadrant must hold whole 64-element segments
+    // Re-encoding tiles hold whole 64-element segments: 128 x 128, or 64 x 64 where the model above finds them the sooner done
+    // (statistics of convolutions, one to ten 128 x 128 tiles of up to 75 k tiles, us on average 105 and 43, their step's
+    // kernels 2.2 and 1.72 ms) -- not on the half pipe, whose callers' products have tiles for every unit.
+    if (requant && (half_pipe || shapes[pick].bm != shapes[pick].bn)) pick = 0;
     // Few tiles and a long k range: cut k into equal slices (whole k tiles each) that write partial products
     // to the caller's workspace and are summed in order afterwards.  Same cost model, with a fixed cost per
     // workgroup (prologue, epilogue, the extra pass over the output) worth about 64 k steps.
@@ -2024,8 +2047,12 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
 #define QT_GEMM_CASE_REQUANT(KA, KB, EP)                                                                     \
     case (KA) * 100 + (KB) * 10 + (EP):                                                                      \
         if (half_pipe) launch_gemm<128, 128, KA, KB, EP, kPipeHalf>(a, d->batch, stream);                    \
-        else if (split_pipe) launch_gemm<128, 128, KA, KB, EP, kPipeSplit>(a, d->batch, stream);             \
-        else launch_gemm<128, 128, KA, KB, EP>(a, d->batch, stream);                                         \
+        else if (split_pipe) {                                                                               \
+            if (pick == 0) launch_gemm<128, 128, KA, KB, EP, kPipeSplit>(a, d->batch, stream);               \
+            else launch_gemm<64, 64, KA, KB, EP, kPipeSplit>(a, d->batch, stream);                           \
+        }                                                                                                    \
+        else if (pick == 0) launch_gemm<128, 128, KA, KB, EP>(a, d->batch, stream);                          \
+        else launch_gemm<64, 64, KA, KB, EP>(a, d->batch, stream);                                           \
         break;
 #define QT_GEMM_CASE_QUANT(KA, KB, EP)                                                                        \
     case (KA) * 100 + (KB) * 10 + (EP):                                                                      \

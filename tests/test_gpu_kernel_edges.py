@@ -434,3 +434,29 @@ def test_flat_dequantizer_puts_the_diagonal_where_it_belongs_in_wide_matrices(or
         if dtype == torch.bfloat16:
             bad = got[b].isnan()
             assert bool((got[b].view(torch.int16)[bad] == 0x7FC0).all())
+
+
+@pytest.mark.parametrize("bits,n,k,batch", [(4, 64, 48, 1), (4, 64, 64, 1), (8, 192, 80, 3), (4, 448, 1024, 2), (4, 1216, 2400, 1),
+                                            (4, 768, 128, 40), (8, 256, 64, 400)])
+@pytest.mark.parametrize("left,symmetric", [(True, True), (False, True), (True, False)])
+def test_reencoding_products_with_tiles_of_either_size_equal_update_then_quantize(bits, n, k, batch, left, symmetric):
+    """Few workgroups of 64 x 64 tiles (loads far ahead from four k tiles on), more of them, and stacks that keep 128 x 128:
+    codes, maxima and diagonal are those of the fused product to fp32 and the stack quantizer after it, bit for bit."""
+    import qtensor.functional as F
+    from qtensor import fused
+    code = (F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)).cuda()
+    g = torch.Generator().manual_seed(n + k)
+    G = 0.1 * torch.randn(batch, *((n, k) if left else (k, n)), generator=g)
+    G[batch - 1, 3] = 0.0
+    G[0, n - 1 if left else 0, 1] = float("nan")
+    G = G.cuda()
+    start = torch.randn(batch, n, n, generator=g).cuda()
+    start = start + start.transpose(1, 2)
+    one = fused.quantize_stack(start, fused.empty_quantized(batch, n, 64, bits, code, True))
+    two = fused.quantize_stack(start, fused.empty_quantized(batch, n, 64, bits, code, True))
+    kw = dict(alpha=0.05, beta=0.95, symmetric=symmetric, trans_a=not left, trans_b=left)
+    fused.quantize_stack(fused.gemm(G, G, addend=two, **kw), two)
+    fused.gemm(G, G, addend=one, requantize=True, **kw)
+    assert torch.equal(one.codes, two.codes)
+    assert torch.equal(one.absmax.view(torch.int32), two.absmax.view(torch.int32))
+    assert torch.equal(one.diag.nan_to_num(7.0), two.diag.nan_to_num(7.0))
