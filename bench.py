@@ -169,7 +169,8 @@ def precond_step_gpu(torch, variant="shampoo1"):
         more["subspace_iteration_updates"] = 30 * sum(bank.per_order.values())
     import qtensor.fused as X
     more["gemm_pipe"] = ("products on the %s matrix pipe" %
-                         ("bf16 (operands split into three bf16 pieces, six products per fp32 product, fp32 accumulation)"
+                         ("fp16 (operands of known size split into two scaled fp16 pieces, three products per fp32 product, fp32 "
+                          "accumulation) and, for the others, bf16 (three bf16 pieces, six products)"
                           if X.gemm_pipe() == "split" else "fp32"))
     return {
         **more,
