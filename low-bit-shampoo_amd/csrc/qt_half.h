@@ -21,6 +21,7 @@
 // multiplied out again by the bf16 split.  Neither a wrong bound nor rows of very different size cost precision.
 #pragma once
 #include "qt_common.h"
+#include "qt_offsets.h"
 
 namespace qt {
 namespace {
@@ -164,8 +165,8 @@ struct HalfQuantLeft {
         const int part = threadIdx.x % PARTS;
         table = code;
         row = min(row0 + (int)(threadIdx.x / PARTS), order - 1);
-        code_off = (uint32_t)((row * order + part * PER) * BITS / 8);      // order^2 < 2^31: checked on the host
-        amax_off = (uint32_t)(row * (order >> bs_shift)) * 4u;
+        code_off = code_offset<BITS>(row, part * PER, order);
+        amax_off = absmax_offset(row, order, bs_shift);
         dval = diag != nullptr ? diag[row] : 0.0f;
         row -= part * PER;
         top = fabsf(dval) * s;
@@ -239,8 +240,8 @@ struct HalfQuantRight {
         table = code;
         way = (lane >> 2) & 1 ? -1 : 1;
         column = even + (way < 0 ? 1 : 0);
-        code_step = (uint32_t)(order * BITS / 8);
-        amax_step = (uint32_t)(order >> bs_shift) * 4u;
+        code_step = code_offset<BITS>(1, 0, order);
+        amax_step = absmax_offset(1, order, bs_shift);
         code_off = (uint32_t)(group * PER) * code_step + ((uint32_t)(even * BITS / 8) & ~3u);
         // a column's place in the word: 4 bits: the even column in the high half of its byte
         const uint32_t first = ((uint32_t)(even * BITS / 8) & 3u) * 8;

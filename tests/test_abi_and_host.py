@@ -163,3 +163,20 @@ def test_bench_refuses_more_than_one_gpu_and_names_its_sections():
     helptext = subprocess.run([sys.executable, str(bench), "--help"], capture_output=True, text=True, check=True).stdout
     for flag in ("--gpus", "--steps", "--warmup", "--section", "--no-cpu-baseline"):
         assert flag in helptext
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_offsets_into_the_largest_quantized_matrices(tmp_path, bits):
+    """The arithmetic that the products' loaders share, compiled for the host with overflow checks, against Python's integers:
+    orders on either side of where order * order * bits passes 31 bits, up to the largest that is accepted."""
+    source = tmp_path / "offsets.cpp"
+    source.write_text('#include "qt_offsets.h"\n#include <cstdio>\n#include <cstdlib>\nint main(int, char **v) {\n'
+                      "    const int row = atoi(v[1]), col = atoi(v[2]), order = atoi(v[3]), shift = atoi(v[4]);\n"
+                      f'    printf("%u %u\\n", qt::code_offset<{bits}>(row, col, order), qt::absmax_offset(row, order, shift));\n}}\n')
+    program = tmp_path / "offsets"
+    subprocess.run(["g++", "-std=c++17", "-fsanitize=undefined", "-fno-sanitize-recover=all", f"-I{ROOT / 'low-bit-shampoo_amd' / 'csrc'}",
+                    str(source), "-o", str(program)], check=True)
+    for order, shift in ((64, 6), (16320, 6), (16448, 6), (23104, 7), (23232, 6), (46336, 8)):
+        for row, col in ((0, 0), (1, 0), (order // 2, 16), (order - 1, 0), (order - 1, order - 8)):
+            out = subprocess.run([str(program)] + [str(x) for x in (row, col, order, shift)], capture_output=True, text=True, check=True).stdout
+            assert [int(x) for x in out.split()] == [(row * order + col) * bits // 8, 4 * row * (order >> shift)], (order, row, col)
