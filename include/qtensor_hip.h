@@ -231,6 +231,15 @@ typedef struct {
     float *out;
 } qtensor_amax_source;
 void qtensor_hip_amax_batched(const qtensor_amax_source *sources, int count, qtensor_stream_t stream);
+/* The same for stacks of which some entries are left out: skip (optional, device, int32 [batch]): a matrix with a nonzero
+ * flag is not read -- its address need not hold one -- and its out not raised. */
+typedef struct {
+    qtensor_batch_ptr mats;
+    int ld, rows, cols, batch;
+    float *out;
+    const int *skip;
+} qtensor_measure_source;
+void qtensor_hip_measure_batched(const qtensor_measure_source *sources, int count, qtensor_stream_t stream);
 
 /* qtensor_hip_gemm for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc); it has no counterpart in the reference.  The partial

@@ -1510,6 +1510,7 @@ struct AmaxSource {
     BatchPtr mats;
     int ld, rows, cols, batch;
     float *out;
+    const int *skip;                             // optional: skip[b] != 0 -> matrix b is not read
     long long inner_stride;                      // (the library's own use: two-level batches, see GemmArgs::batch_inner)
     int inner, rows_per;
     unsigned first_block;
@@ -1521,6 +1522,7 @@ __global__ __launch_bounds__(256) void amax_kernel(const AmaxArgs args) {
     const AmaxSource &m = args.source[i];
     const unsigned pieces = (m.rows + m.rows_per - 1) / m.rows_per, block = blockIdx.x - m.first_block;
     const int b = block / pieces, r0 = (int)(block % pieces) * m.rows_per, r1 = min(m.rows, r0 + m.rows_per);
+    if (m.skip != nullptr && m.skip[b] != 0) return;
     const float *base = dense_ptr(m.mats, b, m.inner, m.inner_stride);
     uint32_t top = 0;
     auto see = [&](float4 x) {
@@ -1754,24 +1756,33 @@ struct PublicAmaxSource {                        // qtensor_amax_source
     int ld, rows, cols, batch;
     float *out;
 };
-}  // namespace
-extern "C" void qtensor_hip_amax_batched(const void *sources_v, int count, void *stream_v) {
+struct PublicMeasureSource : PublicAmaxSource { const int *skip; };        // qtensor_measure_source
+
+template <typename Source>
+void measure(const char *what, const Source *sources, int count, hipStream_t stream) {
     using namespace qt;
     clear_error();
-    const PublicAmaxSource *sources = static_cast<const PublicAmaxSource *>(sources_v);
-    if (sources == nullptr || count < 1 || count > kAmaxSources) { set_error(kBadArgument, "amax: 1 to %d sources (got %d)", kAmaxSources, count); return; }
+    if (sources == nullptr || count < 1 || count > kAmaxSources) { set_error(kBadArgument, "%s: 1 to %d sources (got %d)", what, kAmaxSources, count); return; }
     AmaxArgs args = {};
     args.count = count;
     for (int i = 0; i < count; ++i) {
-        const PublicAmaxSource &m = sources[i];
-        if (m.out == nullptr || !has_host_ptr(m.mats)) { set_error(kNullPointer, "amax: null pointer"); return; }
+        const Source &m = sources[i];
+        if (m.out == nullptr || !has_host_ptr(m.mats)) { set_error(kNullPointer, "%s: null pointer", what); return; }
         if (m.rows < 1 || m.cols < 1 || m.ld < m.cols || m.batch < 1) {
-            set_error(kBadArgument, "amax: need rows, cols, batch >= 1 and ld >= cols (got %d x %d, ld %d, batch %d)", m.rows, m.cols, m.ld, m.batch);
+            set_error(kBadArgument, "%s: need rows, cols, batch >= 1 and ld >= cols (got %d x %d, ld %d, batch %d)", what, m.rows, m.cols, m.ld, m.batch);
             return;
         }
-        args.source[i] = {m.mats, m.ld, m.rows, m.cols, m.batch, m.out, 0, 1, 0, 0};
+        args.source[i] = {m.mats, m.ld, m.rows, m.cols, m.batch, m.out, nullptr, 0, 1, 0, 0};
+        if constexpr (std::is_same<Source, PublicMeasureSource>::value) args.source[i].skip = m.skip;
     }
-    if (launch_amax(args, (hipStream_t)stream_v)) launch_ok("amax");
+    if (launch_amax(args, stream)) launch_ok(what);
+}
+}  // namespace
+extern "C" void qtensor_hip_amax_batched(const void *sources, int count, void *stream) {
+    measure("amax", static_cast<const PublicAmaxSource *>(sources), count, (hipStream_t)stream);
+}
+extern "C" void qtensor_hip_measure_batched(const void *sources, int count, void *stream) {
+    measure("measure", static_cast<const PublicMeasureSource *>(sources), count, (hipStream_t)stream);
 }
 
 extern "C" void qtensor_hip_gemm_static(const qtensor_gemm_desc *d, void *stream_v) {
@@ -2100,7 +2111,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
     if (amax_later != nullptr) {
         AmaxArgs after = {};
         after.count = 1;
-        after.source[0] = {a.C, a.ldc, a.M, a.N, d->batch, reinterpret_cast<float *>(amax_later), a.inner_c, a.batch_inner, 0, 0};
+        after.source[0] = {a.C, a.ldc, a.M, a.N, d->batch, reinterpret_cast<float *>(amax_later), a.skip, a.inner_c, a.batch_inner, 0, 0};
         if (!launch_amax(after, stream)) return;
     }
 #undef QT_GEMM_CASE_DENSE

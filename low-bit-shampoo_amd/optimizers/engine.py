@@ -250,7 +250,8 @@ class ShampooBank:
         """The device table of all groups' block addresses, written on the current stream if a gradient has moved: one
         copy for all groups, through pinned memory and without blocking (a pageable copy per group made the host wait
         for what was queued, fourteen times in a step over the convolution weights)."""
-        # (a parameter that is left out of this call has no gradient: its own storage stands in, never read)
+        # (a parameter that is left out of this call has no gradient, or one that nobody has checked: its address, or the
+        # parameter's own, stands in and is never read -- every launch on these tables takes the skip flags)
         bases = tuple([(p if grad is None else grad).data_ptr() for p, grad in zip(self.params, grads)])
         if bases == self.grad_key:
             return
@@ -389,7 +390,7 @@ class ShampooBank:
 
         def both(g):
             def run():                  # the gradients' largest elements serve both sides
-                top = X.amax(self._grad_list(g))
+                top = X.amax(self._grad_list(g), skip=self._skip(g, only))
                 for side in (0, 1):
                     job(g, side, top)()
             return run
@@ -469,7 +470,7 @@ class ShampooBank:
                     X.gemm(half, right, out=self._out_list(g), skip=skip)
                     return
                 tops = torch.zeros(4, len(g), device=self.device)
-                X.amax_into((left, tops[0]), (G, tops[1]), (right, tops[2]))
+                X.amax_into((left, tops[0]), (G, tops[1]), (right, tops[2]), skip=skip)
                 X.gemm(left, G, out=half, skip=skip, amax=(tops[0], tops[1]), amax_out=tops[3])
                 X.gemm(half, right, out=self._out_list(g), skip=skip, amax=(tops[3], tops[2]))
             return run

@@ -201,7 +201,7 @@ class ShampooBank2(ShampooBank):
         for g in self.groups:
             if (only is None or any(pi in only for pi in g.param_index)) and X.worth_measuring_for(
                     len(g) * g.bm * g.bn * (g.bm + g.bn) // 2, g.bm, g.bn):
-                top_grad[id(g)] = X.amax(self._grad_list(g))
+                top_grad[id(g)] = X.amax(self._grad_list(g), skip=self._skip(g, only))
 
         solver, redone, tick, begun = {}, {}, {}, {}
         # (a stack starts with the replacing sweep when most of it needed that sweep lately, or when it holds many

@@ -54,15 +54,16 @@ class GemmRanges(ct.Structure):
     _fields_ = [("amax_a", ct.c_void_p), ("amax_b", ct.c_void_p), ("amax_out", ct.c_void_p)]
 
 
-class AmaxSource(ct.Structure):
-    _fields_ = [("mats", BatchPtr), ("ld", ct.c_int), ("rows", ct.c_int), ("cols", ct.c_int), ("batch", ct.c_int), ("out", ct.c_void_p)]
+class MeasureSource(ct.Structure):
+    _fields_ = [("mats", BatchPtr), ("ld", ct.c_int), ("rows", ct.c_int), ("cols", ct.c_int), ("batch", ct.c_int), ("out", ct.c_void_p),
+                ("skip", ct.c_void_p)]
 
 
 if F.lib is not None:
     F.lib.qtensor_hip_gemm_ranged.restype = None
     F.lib.qtensor_hip_gemm_ranged.argtypes = [ct.POINTER(GemmDesc), ct.POINTER(GemmRanges), ct.c_void_p]
-    F.lib.qtensor_hip_amax_batched.restype = None
-    F.lib.qtensor_hip_amax_batched.argtypes = [ct.POINTER(AmaxSource), ct.c_int, ct.c_void_p]
+    F.lib.qtensor_hip_measure_batched.restype = None
+    F.lib.qtensor_hip_measure_batched.argtypes = [ct.POINTER(MeasureSource), ct.c_int, ct.c_void_p]
     F.lib.qtensor_hip_gemm_pipe.restype = ct.c_int
     F.lib.qtensor_hip_gemm_pipe.argtypes = [ct.c_int]
     F.lib.qtensor_hip_gemm.restype = None
@@ -174,10 +175,11 @@ def _launch(desc: GemmDesc, device: torch.device, ranges: Optional[GemmRanges] =
     F._call(F.lib.qtensor_hip_gemm, device, ct.byref(desc))
 
 
-def amax_into(*pairs) -> None:
+def amax_into(*pairs, skip: Optional[Tensor] = None) -> None:
     """Each pair (t, out): fp32 [batch] out raised to the largest |element| of every matrix of t ([rows, cols], [batch,
     rows, cols], a PtrList) or to a bound of it (a `Quantized`: its maxima and exact diagonal; code tables hold nothing
-    beyond +-1).  All of them in one launch (up to eight tensors; a `Quantized` with a diagonal counts as two)."""
+    beyond +-1).  All of them in one launch (up to eight tensors; a `Quantized` with a diagonal counts as two).
+    skip: optional int32 [batch]; matrices with a nonzero flag are not read and their entries of out not raised."""
     sources = []
     for t, out in pairs:
         if isinstance(t, Quantized):
@@ -190,15 +192,17 @@ def amax_into(*pairs) -> None:
         for ptr, ld, batch, rows, cols in parts:
             if out.dtype != torch.float32 or out.numel() != batch or not out.is_cuda or not out.is_contiguous():
                 raise ValueError("out must be a contiguous fp32 GPU vector with one entry per batch entry")
-            sources.append(AmaxSource(ptr, ld, rows, cols, batch, out.data_ptr()))
-    F._call(F.lib.qtensor_hip_amax_batched, pairs[0][1].device, (AmaxSource * len(sources))(*sources), len(sources))
+            if skip is not None and (skip.dtype != torch.int32 or skip.numel() != batch):
+                raise ValueError("skip must be int32 [batch]")
+            sources.append(MeasureSource(ptr, ld, rows, cols, batch, out.data_ptr(), None if skip is None else skip.data_ptr()))
+    F._call(F.lib.qtensor_hip_measure_batched, pairs[0][1].device, (MeasureSource * len(sources))(*sources), len(sources))
 
 
-def amax(t) -> Tensor:
+def amax(t, skip: Optional[Tensor] = None) -> Tensor:
     """fp32 [batch]: the largest |element| of every matrix of t, or a bound of it (see amax_into)."""
     out = torch.zeros(t.batch if isinstance(t, Quantized) else 1 if t.dim() == 2 else t.shape[0],
                       device=t.codes.device if isinstance(t, Quantized) else t.device)
-    amax_into((t, out))
+    amax_into((t, out), skip=skip)
     return out
 
 

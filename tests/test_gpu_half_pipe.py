@@ -232,3 +232,38 @@ def test_preconditioned_gradients_look_their_operands_up_where_it_pays(X, code_m
     left = X.quantize_stack(made[0], X.empty_quantized(batch, 256, 64, 4, code, True))
     flat = X.precondition(G[0], X.Quantized(left.codes[:1], left.absmax[:1], left.diag[:1], 256, 64, 4, code), right.rows(0, 1))
     assert flat.shape == (256, 256)
+
+
+def test_matrices_that_are_left_out_are_not_looked_at(X, monkeypatch):
+    """Skip flags of the look-up itself, and a bank with a parameter whose gradient is missing: its storage (here 512 floats
+    for a 512 x 512 matrix) stands in the address tables and must not be read."""
+    import qtensor.functional as F
+    from optimizers.engine import ShampooBank
+    from optimizers.engine2 import ShampooBank2
+    skip = torch.tensor([0, 1, 0], dtype=torch.int32, device="cuda")
+    A = torch.randn(3, 64, 96, device="cuda")
+    assert torch.equal(X.amax(A, skip=skip), A.abs().amax((1, 2)) * (1 - skip))
+    nowhere = torch.tensor([A[0].data_ptr(), 0, A[2].data_ptr()], dtype=torch.int64, device="cuda")
+    assert torch.equal(X.amax(X.PtrList(nowhere, (3, 64, 96)), skip=skip), A.abs().amax((1, 2)) * (1 - skip))
+    monkeypatch.setattr(X, "MEASURE_FROM", 0)
+    code = F.create_linear_map(True, 4, 2)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    present = torch.randn(512, 512, device="cuda", generator=g)
+    absent = torch.nn.Parameter(torch.randn(1, 512, device="cuda", generator=g).expand(512, 512))
+    assert absent.untyped_storage().nbytes() == 4 * 512
+    grad = torch.randn(512, 512, device="cuda", generator=g)
+    for kind in (ShampooBank, ShampooBank2):
+        banks = [kind(params, {"linear-2": code}, "linear-2", prec_maxorder=1024)
+                 for params in ([torch.nn.Parameter(present), absent], [torch.nn.Parameter(present)])]
+        for bank, grads in zip(banks, ([grad, None], [grad])):
+            bank.add_statistics(grads, only=[0])
+        if kind is ShampooBank:                          # the statistics of the parameter that is there: rows 0, 2 and 0, 1
+            for part in ("codes", "absmax", "diag"):
+                both, alone = (getattr(bank.stats[512], part) for bank in banks)
+                assert torch.equal(both[[0, 2]], alone)
+        # both with the same roots, so that the directions can be compared (products without skip flags are cut along k)
+        for bank in banks:
+            for at in range(0, bank.precs[512].batch, bank.precs[512].batch // 2):
+                X.quantize_stack(torch.eye(512, device="cuda")[None] + 0.01 * present[None], bank.precs[512].rows(at, 1))
+        got, want = (bank.preconditioned_grads(grads, only=[0]) for bank, grads in zip(banks, ([grad, None], [grad])))
+        assert got[1] is None and float((got[0] - want[0]).norm() / want[0].norm()) <= 1e-6
