@@ -12,7 +12,6 @@
 //            two launches for all pairs of all matrices -- then, for each 256-wide column panel j,
 //            X_j = (Q_j - X_<j U_<j,j) U_jj^-1; products with a triangular factor skip its zero part.
 // All launches go to the caller's stream; nothing is allocated or synchronised here.
-#include <algorithm>
 #include "qt_common.h"
 
 #include "qtensor_hip.h"
@@ -21,7 +20,7 @@
 #include <initializer_list>
 
 namespace qt {
-void gemm_with_tile(const qtensor_gemm_desc *d, hipStream_t stream, int tile, const void *ranges);     // qt_gemm.hip
+void gemm_with_tile(const qtensor_gemm_desc *d, hipStream_t stream, int tile);     // qt_gemm.hip
 namespace {
 
 constexpr int NB = 64;
@@ -548,15 +547,9 @@ bool run(qtensor_gemm_desc &d, hipStream_t stream) {
 
 // The same with the tile shape chosen here (0 = 128 x 128, 2 = 64 x 128): for the sweep's projections, where measured
 // times and the product kernel's cost model part ways.
-bool run_tiled(qtensor_gemm_desc &d, hipStream_t stream, int tile, const qtensor_gemm_ranges *ranges) {
-    gemm_with_tile(&d, stream, tile, ranges);
+bool run_tiled(qtensor_gemm_desc &d, hipStream_t stream, int tile) {
+    gemm_with_tile(&d, stream, tile);
     return qtensor_hip_last_error() == 0;
-}
-
-// What the sweep tells the product kernel about the size of its operands: `batch` ones (columns of unit length hold nothing
-// beyond 1), then zeroes that the launches which write coefficients raise.
-__global__ __launch_bounds__(256) void sweep_tops_kernel(float *tops, int batch, int count) {
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < count; i += gridDim.x * 256) tops[i] = i < batch ? 1.0f : 0.0f;
 }
 
 bool stack_args_ok(const char *what, int n, int batch, std::initializer_list<const void *> ptrs) {
@@ -654,19 +647,11 @@ struct Sweep {
     long long mat() const { return (long long)n * n; }
     // With stand-in columns the tail of w holds, per matrix and 64-column panel of the current outer panel, which
     // columns the pass before set aside (w_cols / 64 words of 64 bits per matrix)
-    // and in front of it `batch` words per outer panel and pass, and `batch` more: the largest coefficient (sweep_tops_kernel).
-    // (The coefficients of an outer panel take n - w_cols of the n rows of w at most: the tail is theirs alone.)
-    bool wide() const { return (long long)batch * n >= 49152; }
-    long long projections() const { return (long long)(replace ? 3 : 2) * (n / w_cols); }
-    long long tops_floats() const { return wide() ? (projections() + 1) * batch : 0; }
-    long long aside_floats() const { return fill != nullptr ? 2LL * batch * (w_cols / NB) : 0; }
-    long long w_floats() const { return (long long)batch * n * w_cols - aside_floats() - tops_floats(); }
-    float *tops() const { return w + w_floats(); }
-    unsigned long long *aside_words() const { return reinterpret_cast<unsigned long long *>(w + (long long)batch * n * w_cols - aside_floats()); }
+    long long w_floats() const { return (long long)batch * n * w_cols - (fill != nullptr ? 2LL * batch * (w_cols / NB) : 0); }
+    unsigned long long *aside_words() const { return reinterpret_cast<unsigned long long *>(w + w_floats()); }
 
     // columns [c0, c0 + width) -= Q[:, a0:c0] (Q[:, a0:c0]^T columns): the columns a0..c0 are orthonormal
-    // (number >= 0: which of the sweep's projections of outer panels this is)
-    bool project(int a0, int c0, int width, int number = -1) {
+    bool project(int a0, int c0, int width) {
         const int k = c0 - a0;
         if (k <= 0) return true;
         // The coefficients of matrix b sit k * width floats apart; what is left of w behind them takes the partial
@@ -689,13 +674,8 @@ struct Sweep {
         // idle) against 773 with what the product's cost model picks; the application 771 us with tiles of 64 rows and the
         // panel's full width against 800 (136 of order 768: 389 against 441 and 424 against 448; 50 of order 1024: 384
         // against 419 and 388 against 435).  Smaller stacks are left to the model, which is as good or better there.
-        // The half pipe takes them (columns of unit length: no element above 1; the coefficients of a second pass are rounding
-        // noise, so the launch that writes them says how large they are): coefficients of seven panels 564 -> 440 us, an
-        // application 104 -> 99, the step over a ViT-B/32's weights 17.1 -> 16.4 ms; tiles of 128 x 128 for the application as
-        // well: the same to the noise.
-        const bool tiled = width == 2 * NB && number >= 0 && wide();
-        const qtensor_gemm_ranges finding = {tops(), tops(), tops() + (long long)(number + 1) * batch};
-        if (!(tiled ? run_tiled(p, stream, 0, &finding) : run(p, stream))) return false;
+        const bool wide = width == 2 * NB && (long long)batch * n >= 49152;
+        if (!(wide ? run_tiled(p, stream, 0) : run(p, stream))) return false;
         qtensor_gemm_desc r = {};                             // Y -= Q_a W
         r.M = n; r.N = width; r.K = k; r.batch = batch;
         r.kind_a = QTENSOR_DENSE; r.kind_b = QTENSOR_DENSE; r.epilogue = QTENSOR_EPI_AXPBY_DENSE;
@@ -704,8 +684,7 @@ struct Sweep {
         r.args.C = strided(q + c0, mat()); r.args.ldc = n;
         r.args.E = strided(q + c0, mat()); r.args.lde = n;
         r.args.alpha = -1.0f; r.args.beta = 1.0f;
-        const qtensor_gemm_ranges found = {tops(), finding.amax_out, nullptr};
-        return tiled ? run_tiled(r, stream, 2, &found) : run(r, stream);
+        return wide ? run_tiled(r, stream, 2) : run(r, stream);
     }
 
     // The 64 columns from c0 on, in pass `pass` of `passes` over their outer panel (which starts at column a0): take the
@@ -814,12 +793,6 @@ extern "C" void qtensor_hip_block_gram_schmidt_replacing_batched(float *q, float
     // less than half.  Every stand-in column is orthogonalised against everything before it at least once after it
     // came in, every other column three times.
     const int passes = s.replace ? 3 : 2;
-    if (s.wide()) {
-        const int count = (int)s.tops_floats();
-        hipLaunchKernelGGL(sweep_tops_kernel, dim3(std::min(64, (count + 255) / 256)), dim3(256), 0, s.stream, s.tops(), batch, count);
-        if (!launch_ok("block_gram_schmidt_batched (bounds)")) return;
-    }
-    int number = 0;
     for (int o0 = 0; o0 < n; o0 += outer) {
         const int width = n - o0 < outer ? n - o0 : outer;
         for (int pass = 0; pass < passes; ++pass) {
@@ -829,7 +802,7 @@ extern "C" void qtensor_hip_block_gram_schmidt_replacing_batched(float *q, float
                                    outer / NB, s.aside_words(), fill + o0, n, info);
                 if (!launch_ok("block_gram_schmidt_batched (stand-in columns)")) return;
             }
-            if (!s.project(0, o0, width, o0 > 0 ? number++ : -1)) return;
+            if (!s.project(0, o0, width)) return;
             for (int c0 = o0; c0 < o0 + width; c0 += NB)
                 if (!s.panel(o0, c0, pass, passes)) return;
         }

@@ -1835,11 +1835,11 @@ extern "C" void qtensor_hip_gemm_static(const qtensor_gemm_desc *d, void *stream
 // projections): the product with the tile shape given, 0..3 = 128 x 128, 128 x 64, 64 x 128, 64 x 64.  The bits of a
 // product do not depend on its tiles, only on whether k is cut, which is still decided for that shape.
 namespace qt {
-void gemm_with_tile(const qtensor_gemm_desc *d, hipStream_t stream, int tile, const void *ranges);
+void gemm_with_tile(const qtensor_gemm_desc *d, hipStream_t stream, int tile);
 }
-void qt::gemm_with_tile(const qtensor_gemm_desc *d, hipStream_t stream, int tile, const void *ranges) {
+void qt::gemm_with_tile(const qtensor_gemm_desc *d, hipStream_t stream, int tile) {
     qt::clear_error();
-    gemm_dispatch(d, stream, tile, static_cast<const Ranges *>(ranges));
+    gemm_dispatch(d, stream, tile);
 }
 
 namespace {
