@@ -155,7 +155,9 @@ enum { QTENSOR_EPI_STORE = 0, QTENSOR_EPI_AXPBY_DENSE = 1, QTENSOR_EPI_AXPBY_QUA
         * not used): the statistics update L <- beta L + (1 - beta) G G^T of optimizers/shampoo1.py:164-178
         * (dequantize, update, quantize) in one launch.  Blocksize 64; bit-identical to AXPBY_QUANT* followed
         * by the stack quantizer. */
-       QTENSOR_EPI_REQUANT4 = 5, QTENSOR_EPI_REQUANT8 = 6 };
+       QTENSOR_EPI_REQUANT4 = 5, QTENSOR_EPI_REQUANT8 = 6,
+       /* NEWTON for an iteration that multiplies deviations from I: C = beta * E + alpha * (A B), T = C - I, err = max |T|. */
+       QTENSOR_EPI_DEVIATION = 7 };
 
 typedef struct {
     int M, N, K, batch;
@@ -168,12 +170,12 @@ typedef struct {
         qtensor_batch_ptr B; int ldb;
         qtensor_quant_ref Aq, Bq;
         qtensor_batch_ptr C; int ldc;
-        float alpha, beta;      /* AXPBY: C = beta * E + alpha * (A B)                          */
+        float alpha, beta;      /* AXPBY, DEVIATION: C = beta * E + alpha * (A B)               */
         qtensor_batch_ptr E; int lde;
         qtensor_quant_ref Eq;   /* AXPBY_QUANT*: E is this quantized M x M matrix               */
-        qtensor_batch_ptr T; int ldt;   /* NEWTON: T = (1 - w) I + w (A B), besides C = A B     */
+        qtensor_batch_ptr T; int ldt;   /* NEWTON: T = (1 - w) I + w (A B), besides C = A B; DEVIATION: T = C - I */
         float newton_w;
-        float *err;             /* NEWTON: err[b] = max(err[b], max |A B - I|); caller zeroes   */
+        float *err;             /* NEWTON: err[b] = max(err[b], max |C - I|); caller zeroes (DEVIATION too) */
         const int *skip;        /* optional device array: skip[b] != 0 leaves entry b untouched */
         const float *code;      /* code table of the quantized operands / addend               */
         int symmetric;          /* != 0: A B is known to be symmetric (M == N, dense operands): only the tiles
@@ -200,7 +202,7 @@ typedef struct {
 } qtensor_gemm_desc;
 
 /* Combinations built: (QUANT*, DENSE, STORE), (DENSE, QUANT*, STORE), (DENSE, DENSE_T, STORE|AXPBY_*),
- * (DENSE_T, DENSE, STORE|AXPBY_*), (DENSE, DENSE, STORE|AXPBY_DENSE|NEWTON), and REQUANT* with
+ * (DENSE_T, DENSE, STORE|AXPBY_*), (DENSE, DENSE, STORE|AXPBY_DENSE|NEWTON|DEVIATION), and REQUANT* with
  * (DENSE, DENSE_T) or (DENSE_T, DENSE); anything else is an error. */
 void qtensor_hip_gemm(const qtensor_gemm_desc *desc, qtensor_stream_t stream);
 
@@ -208,7 +210,7 @@ void qtensor_hip_gemm(const qtensor_gemm_desc *desc, qtensor_stream_t stream);
 typedef struct {
     const float *amax_a, *amax_b;   /* largest |element| of A[b] and B[b], or a bound of it; either null: not known    */
     float *amax_out;                /* optional: raised to the largest |element| of C[b] (caller zeroes); plain store,
-                                     * AXPBY and NEWTON (C, not T)                                                    */
+                                     * AXPBY, NEWTON and DEVIATION (C, not T)                                         */
 } qtensor_gemm_ranges;
 
 /* qtensor_hip_gemm for callers that know how large the operands are (no counterpart in the reference).  Where the split

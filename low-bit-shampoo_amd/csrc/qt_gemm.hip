@@ -53,7 +53,7 @@
 namespace qt {
 
 enum OperandKind : int { kDense = 0, kDenseT = 1, kQuant4 = 2, kQuant8 = 3 };
-enum EpilogueKind : int { kStore = 0, kAxpbyDense = 1, kAxpbyQuant4 = 2, kAxpbyQuant8 = 3, kNewton = 4, kRequant4 = 5, kRequant8 = 6 };
+enum EpilogueKind : int { kStore = 0, kAxpbyDense = 1, kAxpbyQuant4 = 2, kAxpbyQuant8 = 3, kNewton = 4, kRequant4 = 5, kRequant8 = 6, kDeviation = 7 };
 
 // One matrix argument over the batch: either base + b * stride, or list[b] when list != nullptr.
 struct BatchPtr {
@@ -77,11 +77,11 @@ struct GemmArgs {
     QuantRef Aq, Bq;              // used when the operand kind is quantized
     BatchPtr C; int ldc;
     float alpha, beta;
-    BatchPtr E; int lde;          // dense addend for kAxpbyDense
+    BatchPtr E; int lde;          // dense addend for kAxpbyDense and kDeviation
     QuantRef Eq;                  // quantized addend for kAxpbyQuant*
-    BatchPtr T; int ldt;          // kNewton: second output
+    BatchPtr T; int ldt;          // kNewton, kDeviation (T = C - I): second output
     float newton_w;               // kNewton: T = (1 - w) I + w acc
-    float *err;                   // kNewton: err[b] = max |acc - I| (must be zeroed by the caller)
+    float *err;                   // kNewton, kDeviation: err[b] = max |C - I| (must be zeroed by the caller)
     const int *skip;              // optional: skip[b] != 0 -> this batch entry is left untouched
     const float *code;            // code table for quantized operands / addend
     int symmetric;                // != 0: the product is symmetric (M == N); only tiles on or above the
@@ -1136,8 +1136,9 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         C = args.workspace + seg_slot * (BM * BN) - ((long long)m0 * BN + n0);
         ldc = BN;
     }
-    float *T = EPI == kNewton ? const_cast<float *>(batch_ptr<float>(args.T, b)) : nullptr;
-    const float *E = EPI == kAxpbyDense ? dense_ptr(args.E, b, args.batch_inner, args.inner_e) : nullptr;
+    constexpr bool kSecond = EPI == kNewton || EPI == kDeviation, kDenseAddend = EPI == kAxpbyDense || EPI == kDeviation;
+    float *T = kSecond ? const_cast<float *>(batch_ptr<float>(args.T, b)) : nullptr;
+    const float *E = kDenseAddend ? dense_ptr(args.E, b, args.batch_inner, args.inner_e) : nullptr;
     constexpr bool kQuantAddend = EPI == kAxpbyQuant4 || EPI == kAxpbyQuant8 || kRequant;
     constexpr int EBITS = (EPI == kAxpbyQuant8 || EPI == kRequant8) ? 8 : 4;
     const uint8_t *e_codes = kQuantAddend ? batch_ptr<uint8_t>(args.Eq.codes, b) : nullptr;
@@ -1147,8 +1148,8 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     // read at the mirrored position, so an addend that is not exactly symmetric is honoured
     const bool mirror = args.symmetric != 0 && tile_n != tile_m;
     const bool vec_ok = (ldc & 3) == 0 && is_aligned16(C) &&
-                        (EPI != kNewton || ((args.ldt & 3) == 0 && is_aligned16(T))) &&
-                        (EPI != kAxpbyDense || ((args.lde & 3) == 0 && is_aligned16(E)));
+                        (!kSecond || ((args.ldt & 3) == 0 && is_aligned16(T))) &&
+                        (!kDenseAddend || ((args.lde & 3) == 0 && is_aligned16(E)));
     const bool mirror_vec = vec_ok && (args.M & 3) == 0;
     const bool direct_vec = vec_ok && (args.N & 3) == 0;
     if constexpr (kRequant) {
@@ -1263,7 +1264,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                     float y[4] = {a4.x, a4.y, a4.z, a4.w};
                     const int row = m0 + wm + i * 32 + ml, col4 = n0 + wn + j * 32 + nl;
                     if (row >= args.M || col4 >= args.N) continue;           // N % 4 == 0: col4 + 3 < N
-                    if (EPI == kAxpbyDense) {
+                    if (kDenseAddend) {
                         const float4 x = gload4(E + (long long)row * args.lde + col4);
                         const float e[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
@@ -1279,13 +1280,14 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                         // same two roundings as tensor.mul_(beta).add_(S, alpha=1-beta)
 #pragma unroll
                         for (int q = 0; q < 4; ++q) y[q] = __builtin_fmaf(args.alpha, y[q], args.beta * e[q]);
-                    } else if (EPI == kNewton) {
+                    }
+                    if (kSecond) {
                         float t[4];
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
                             const float eye = row == col4 + q ? 1.0f : 0.0f;
                             local_err = fmaxf(local_err, fabsf(y[q] - eye));
-                            t[q] = (1.0f - args.newton_w) * eye + args.newton_w * y[q];
+                            t[q] = EPI == kDeviation ? y[q] - eye : (1.0f - args.newton_w) * eye + args.newton_w * y[q];
                         }
                         gstore4(T + (long long)row * args.ldt + col4, t);
                     }
@@ -1301,16 +1303,18 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                     const int row = m0 + wm + i * 32 + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
                     if (row >= args.M || col >= args.N) continue;
                     float y = acc[i][j][r];
-                    if (EPI == kAxpbyDense) {
+                    if (kDenseAddend) {
                         y = args.beta * gload(E + (long long)row * args.lde + col) + args.alpha * y;
                     } else if (kQuantAddend) {
                         const float e = dequant_element<EBITS>(e_codes, e_absmax, e_diag, s_code, args.Eq.order,
                                                                args.Eq.bs_shift, row, col);
                         y = __builtin_fmaf(args.alpha, y, args.beta * e);
-                    } else if (EPI == kNewton) {
+                    }
+                    if (kSecond) {
                         const float eye = row == col ? 1.0f : 0.0f;
                         local_err = fmaxf(local_err, fabsf(y - eye));
-                        gstore(T + (long long)row * args.ldt + col, (1.0f - args.newton_w) * eye + args.newton_w * y);
+                        gstore(T + (long long)row * args.ldt + col,
+                               EPI == kDeviation ? y - eye : (1.0f - args.newton_w) * eye + args.newton_w * y);
                     }
                     if constexpr (PREC == kPipeHalf) local_top = fmaxf(fabsf(y), local_top);
                     gstore(C + (long long)row * ldc + col, y);
@@ -1334,7 +1338,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                 // elements (mrow, mcol .. mcol+3), never on the diagonal
                 float y[4], e[4] = {0.f, 0.f, 0.f, 0.f};
                 const bool whole = mirror_vec;                  // M % 4 == 0: mcol + 3 < M
-                if (EPI == kAxpbyDense) {
+                if (kDenseAddend) {
                     if (whole) { const float4 x = gload4(E + (long long)mrow * args.lde + mcol); e[0] = x.x; e[1] = x.y; e[2] = x.z; e[3] = x.w; }
                     else
 #pragma unroll
@@ -1345,7 +1349,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                 }
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    if (EPI == kAxpbyDense) y[q] = args.beta * e[q] + args.alpha * a[q];
+                    if (kDenseAddend) y[q] = args.beta * e[q] + args.alpha * a[q];
                     else if (kQuantAddend) y[q] = __builtin_fmaf(args.alpha, a[q], args.beta * e[q]);
                     else y[q] = a[q];
                 }
@@ -1356,10 +1360,13 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                 else
 #pragma unroll
                     for (int q = 0; q < 4; ++q) if (mcol + q < args.M) gstore(cm + q, y[q]);
-                if (EPI == kNewton) {
+                if (kSecond) {
                     float t[4];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) t[q] = args.newton_w * y[q];
+                    for (int q = 0; q < 4; ++q) {
+                        t[q] = EPI == kDeviation ? y[q] : args.newton_w * y[q];
+                        if (EPI == kDeviation && mcol + q < args.M) local_err = fmaxf(local_err, fabsf(y[q]));
+                    }
                     float *tm = T + (long long)mrow * args.ldt + mcol;
                     if (whole) gstore4(tm, t);
                     else
@@ -1369,7 +1376,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
             }
             wave_lds_sync();
         }
-    if (EPI == kNewton) {
+    if (kSecond) {
         uint32_t e = group_max_u32<64>(__float_as_uint(local_err));   // non-negative floats order like their bits
         if (lane == 0) atomicMax(reinterpret_cast<unsigned int *>(args.err) + b, e);
     }
@@ -1854,7 +1861,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         return;
     }
     const int ka = d->kind_a, kb = d->kind_b, ep = d->epilogue;
-    if (ka < kDense || ka > kQuant8 || kb < kDense || kb > kQuant8 || ep < kStore || ep > kRequant8) {
+    if (ka < kDense || ka > kQuant8 || kb < kDense || kb > kQuant8 || ep < kStore || ep > kDeviation) {
         set_error(kBadArgument, "gemm: unknown operand or epilogue kind (%d, %d, %d)", ka, kb, ep);
         return;
     }
@@ -1874,13 +1881,16 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         if (!valid_quant(a.Bq, kb == kQuant4 ? 4 : 8, "B")) return;
         if (a.Bq.order != d->N || d->K != d->N) { set_error(kBadArgument, "gemm: quantized B must be square with K == N == order"); return; }
     }
-    if (ep == kAxpbyDense && (!has_host_ptr(a.E) || a.lde < d->N)) { set_error(kBadArgument, "gemm: bad dense addend"); return; }
+    if ((ep == kAxpbyDense || ep == kDeviation) && (!has_host_ptr(a.E) || a.lde < d->N)) { set_error(kBadArgument, "gemm: bad dense addend"); return; }
     if (ep == kAxpbyQuant4 || ep == kAxpbyQuant8 || requant) {
         if (!valid_quant(a.Eq, ep == kAxpbyQuant4 || ep == kRequant4 ? 4 : 8, "addend")) return;
         if (a.Eq.order != d->M || d->M != d->N) { set_error(kBadArgument, "gemm: quantized addend must be M x N square of its order"); return; }
         if (requant && a.Eq.bs_shift != 6) { set_error(kBadArgument, "gemm: the requantizing epilogue needs blocksize 64"); return; }
     }
-    if (ep == kNewton && (!has_host_ptr(a.T) || a.ldt < d->N || !a.err)) { set_error(kBadArgument, "gemm: Newton epilogue needs T and err"); return; }
+    if ((ep == kNewton || ep == kDeviation) && (!has_host_ptr(a.T) || a.ldt < d->N || !a.err)) {
+        set_error(kBadArgument, "gemm: Newton and deviation epilogues need T and err");
+        return;
+    }
     if (ranges != nullptr && ranges->amax_out != nullptr && requant) { set_error(kBadArgument, "gemm: a re-encoded result has no amax_out"); return; }
     a.symmetric = a.symmetric != 0;
     a.batch_count = d->batch;
@@ -2104,6 +2114,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         QT_GEMM_CASE_DENSE(kDense, kDense, kStore)
         QT_GEMM_CASE_DENSE(kDense, kDense, kAxpbyDense)
         QT_GEMM_CASE_DENSE(kDense, kDense, kNewton)
+        QT_GEMM_CASE_DENSE(kDense, kDense, kDeviation)
         default:
             set_error(kBadArgument, "gemm: combination A kind %d, B kind %d, epilogue %d is not built", ka, kb, ep);
             return;

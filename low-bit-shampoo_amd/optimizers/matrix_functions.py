@@ -6,9 +6,19 @@ accept CPU or GPU tensors and then behave like the reference, sync for sync.
 
 ComputePowerBatched is the MI355X form of ComputePower for a whole stack of equally sized
 matrices: every product runs on the matrix cores through qtensor.fused.gemm (4 launches per
-iteration for the whole stack), max|M - I| and the next iteration matrix come out of the last
-product's epilogue, and the per-matrix stopping rules are evaluated on the device, so the host
-never waits inside the iteration.
+iteration for the whole stack), max|M - I| and M - I come out of the last product's epilogue, and
+the per-matrix stopping rules are evaluated on the device, so the host never waits inside the
+iteration.  Beside M it keeps E = M - I, and it multiplies deviations from the identity out:
+
+    T = I + w E (w = -1/p),  R T = R + w R E,  F = T^2 - I = 2 w E + w^2 E E,  F <- 2 F + F F for
+    every further squaring,  T^p M = M + F M
+
+-- in exact arithmetic the reference's iteration.  Products of M and T themselves are products of
+near-identities: one pair of elements makes most of every sum, and what its operands lose when
+they are split, and the sum when it is rounded, is a part of the identity.  Relative error of the
+root against the same iteration in float64 (4-bit statistics of condition 20, half pipe; the bf16
+split for order 128): order 128 3.6e-7 -> 1.2e-7, 256 6.9e-7 -> 1.5e-7, 768 9.1e-7 -> 2.3e-7,
+1024 1.1e-6 -> 2.8e-7; on the bf16 split the same but for 4 % (from 4.8e-7 at 256, 9.5e-7 at 1024).
 """
 from typing import Optional
 
@@ -146,57 +156,57 @@ def ComputePowerBatched(mats, p=4, iter_count=10, error_tolerance=1e-6, ridge_ep
     first_root = torch.pow(z, 1.0 / p)                                       # the root starts as this multiple of the identity
     R[0].diagonal(dim1=1, dim2=2).copy_(first_root.unsqueeze(1).expand(B, n))
     M = [mats * z.view(B, 1, 1), torch.empty(B, n, n, device=dev)]
-    T = [(1 - w) * eye + w * M[0], torch.empty(B, n, n, device=dev)]
-    T2 = torch.empty(B, n, n, device=dev)
-    Tp = torch.empty(B, n, n, device=dev)
-    err = (M[0] - eye).abs().amax(dim=(1, 2))
+    E = [M[0] - eye, torch.empty(B, n, n, device=dev)]
+    F = [torch.empty(B, n, n, device=dev) for _ in range(2)]                  # T^2 - I, T^4 - I, ... in turn
+    err = E[0].abs().amax(dim=(1, 2))
     rounds = torch.zeros(B, dtype=torch.int32, device=dev)
     done = (err <= error_tolerance)
 
-    # which of the two buffers currently holds matrix b's accepted R / M / T: pointer tables on
+    # which of the two buffers currently holds matrix b's accepted R / M / E: pointer tables on
     # the device, swapped per matrix when a round is accepted
     def table(pair):
         step = pair[0].stride(0) * 4
         return [torch.arange(B, device=dev, dtype=torch.int64) * step + t.data_ptr() for t in pair]
 
-    R_ptr, M_ptr, T_ptr = table(R), table(M), table(T)
+    R_ptr, M_ptr, E_ptr = table(R), table(M), table(E)
     side = torch.zeros(B, dtype=torch.bool, device=dev)                     # False: buffer 0 holds the state
-    # How large the iterates' elements are, for the pipe that wants to know: |M| and |T| follow from err = max |M - I|
-    # (T = I + w (M - I)), the roots and the powers of T are looked at by the launches that write them.  Small stacks are
+    # How large the iterates' elements are, for the pipe that wants to know: |E| and |M| follow from err = max |E|, the roots
+    # and the powers of T are looked at by the launches that write them.  Small stacks are
     # bound by the host, which this costs 40 us a round (statistics of convolutions of width 32: 29 ms without, 33 with).
     measured = X.worth_measuring_for(B * n ** 3, n)
     squarings = p.bit_length() - 1
     if measured:
         tops = torch.zeros(iter_count, 1 + squarings, B, device=dev)
-        top_m, top_t = 1 + err, 1 + abs(w) * err
-        top_r = first_root * top_t                                           # of the root after the first round
+        top_e, top_m = err, 1 + err
+        top_r = first_root * (1 + abs(w) * err)                              # of the root after the first round
     for round_number in range(iter_count):
         skip = done.to(torch.int32)
         cur = lambda tab: torch.where(side, tab[1], tab[0])                   # noqa: E731
         oth = lambda tab: torch.where(side, tab[0], tab[1])                   # noqa: E731
-        Rc, Ro, Mc, Mo, Tc, To = cur(R_ptr), oth(R_ptr), cur(M_ptr), oth(M_ptr), cur(T_ptr), oth(T_ptr)
         shape = (B, n, n)
+        Rc, Ro, Mc, Mo, Ec, Eo = [X.PtrList(which(tab), shape) for tab in (R_ptr, M_ptr, E_ptr) for which in (cur, oth)]
         if round_number == 0:
-            # candidate root of the first round: (c I) T = c T, every matrix still in its first buffer
-            torch.mul(T[0], first_root.view(B, 1, 1), out=R[1])
+            # candidate root of the first round: c (I + w E), every matrix still in its first buffer
+            torch.mul(E[0], (w * first_root).view(B, 1, 1), out=R[1])
+            R[1].diagonal(dim1=1, dim2=2).add_(first_root.unsqueeze(1))
         else:
-            X.gemm(X.PtrList(Rc, shape), X.PtrList(Tc, shape), out=X.PtrList(Ro, shape), skip=skip,
-                   symmetric=symmetric,                                      # candidate root
-                   **(dict(amax=(top_r, top_t), amax_out=tops[round_number, 0]) if measured else {}))
+            X.gemm(Rc, Ec, addend=Rc, alpha=w, beta=1.0, out=Ro, skip=skip, symmetric=symmetric,        # candidate root
+                   **(dict(amax=(top_r, top_e), amax_out=tops[round_number, 0]) if measured else {}))
             if measured:
                 top_r = tops[round_number, 0]                                # (a rejected candidate ends its matrix's iteration)
-        power = X.PtrList(Tc, shape)                                         # T^p by repeated squaring
-        top = top_t if measured else None
+        power, scale = Ec, w                                                 # T^p = I + scale * power by repeated squaring
+        top = top_e if measured else None
         for square in range(1, 1 + squarings):
-            dst = Tp if power is T2 else T2
+            dst = F[square % 2]
             after = tops[round_number, square] if measured else None
-            X.gemm(power, power, out=dst, skip=skip, symmetric=symmetric, amax=(top, top) if measured else None, amax_out=after)
-            power, top = dst, after
+            X.gemm(power, power, addend=power, alpha=scale * scale, beta=2 * scale, out=dst, skip=skip, symmetric=symmetric,
+                   amax=(top, top) if measured else None, amax_out=after)
+            power, scale, top = dst, 1.0, after
         new_err = torch.zeros(B, device=dev)
-        X.gemm(power, X.PtrList(Mc, shape), out=X.PtrList(Mo, shape), newton=(X.PtrList(To, shape), w, new_err),
-               skip=skip, symmetric=symmetric, amax=(top, top_m) if measured else None)
+        X.gemm(power, Mc, addend=Mc, alpha=scale, beta=1.0, out=Mo, deviation=(Eo, new_err), skip=skip, symmetric=symmetric,
+               amax=(top, top_m) if measured else None)
         if measured:
-            top_m, top_t = 1 + new_err, 1 + abs(w) * new_err
+            top_e, top_m = new_err, 1 + new_err
         accept = (~done) & ~(new_err > err * 1.2)
         side = side ^ accept
         err = torch.where(accept, new_err, err)

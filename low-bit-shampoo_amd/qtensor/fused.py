@@ -15,7 +15,7 @@ from torch import Tensor
 import qtensor.functional as F
 
 DENSE, DENSE_T, QUANT4, QUANT8 = 0, 1, 2, 3
-EPI_STORE, EPI_AXPBY_DENSE, EPI_AXPBY_QUANT4, EPI_AXPBY_QUANT8, EPI_NEWTON, EPI_REQUANT4, EPI_REQUANT8 = 0, 1, 2, 3, 4, 5, 6
+EPI_STORE, EPI_AXPBY_DENSE, EPI_AXPBY_QUANT4, EPI_AXPBY_QUANT8, EPI_NEWTON, EPI_REQUANT4, EPI_REQUANT8, EPI_DEVIATION = range(8)
 
 
 class BatchPtr(ct.Structure):
@@ -224,7 +224,7 @@ _PIPES = {None: 0, "f32": 1, "split": 2}
 def gemm(A, B, *, trans_a=False, trans_b=False, out: Optional[Tensor] = None, alpha=1.0, beta=0.0,
          addend=None, newton=None, skip: Optional[Tensor] = None, symmetric: bool = False,
          upper_a: bool = False, upper_b: bool = False, requantize: bool = False, pipe: Optional[str] = None,
-         amax=None, amax_out: Optional[Tensor] = None):
+         amax=None, amax_out: Optional[Tensor] = None, deviation=None):
     """out[b] = epilogue(op(A[b]) @ op(B[b])).
 
     A, B: fp32 tensors ([m,k] / [batch,m,k]; with trans_x the stored matrix is the transpose; trans_a together
@@ -233,6 +233,7 @@ def gemm(A, B, *, trans_a=False, trans_b=False, out: Optional[Tensor] = None, al
     addend: None, a dense tensor E or a `Quantized` E: out = beta*E + alpha*product.
     newton: None or (T_out, w, err): also writes T_out = (1-w) I + w*product and folds
     max|product - I| into err[b] (fp32 [batch], zeroed by the caller).
+    deviation: None or (T_out, err), with a dense addend: also writes T_out = out - I and folds max|out - I| into err[b].
     skip: optional int32 [batch]; entries with a nonzero flag are not touched.
     symmetric: the caller knows the product to be symmetric (a Gram matrix, a product of commuting
     symmetric matrices): only the tiles on and above the diagonal are multiplied out and mirrored,
@@ -309,16 +310,18 @@ def gemm(A, B, *, trans_a=False, trans_b=False, out: Optional[Tensor] = None, al
                 raise ValueError("dense addend must have the shape of the result")
             d.epilogue = EPI_AXPBY_DENSE
     keep = [out]
-    if newton is not None:
-        if addend is not None:
-            raise ValueError("the Newton epilogue takes no addend")
-        t_out, w, err = newton
+    if newton is not None and (addend is not None or deviation is not None):
+        raise ValueError("the Newton epilogue takes no addend")
+    if deviation is not None and d.epilogue != EPI_AXPBY_DENSE:
+        raise ValueError("the deviation epilogue takes a dense addend")
+    if newton is not None or deviation is not None:
+        t_out, w, err = newton if newton is not None else (deviation[0], 0.0, deviation[1])
         a.T, a.ldt, bt, mt, nt = _dense(t_out)
         if (bt, mt, nt) != (batch, m, n) or err.numel() != batch or err.dtype != torch.float32:
             raise ValueError("Newton outputs must match the result")
         a.newton_w = w
         a.err = err.data_ptr()
-        d.epilogue = EPI_NEWTON
+        d.epilogue = EPI_NEWTON if newton is not None else EPI_DEVIATION
     if skip is not None:
         if skip.dtype != torch.int32 or skip.numel() != batch:
             raise ValueError("skip must be int32 [batch]")

@@ -103,3 +103,71 @@ def test_stack_matrix_vector_product(n, batch):
     view = torch.zeros(batch, n, n + 4, device="cuda")[:, :, 1:n + 1]            # not contiguous: refused
     with pytest.raises(ValueError):
         X.matvec(view, v.cuda())
+
+
+@pytest.mark.parametrize("n,batch", [(288, 3), (150, 2), (77, 1), (33, 4), (1024, 2)])
+@pytest.mark.parametrize("pipe", ["f32", "split", "half"])
+def test_deviation_epilogue(n, batch, pipe):
+    """C = beta M + alpha F M, T = C - I, err = max |T|: plain and mirrored, whole and ragged tiles, a skipped entry, an output
+    that is not aligned.  Bound of an element: a sum of n products in fp32 and two more roundings."""
+    import qtensor.fused as X
+    g = torch.Generator(device="cuda").manual_seed(n)
+    F = torch.randn(batch, n, n, device="cuda", generator=g) / n
+    F = F + F.transpose(1, 2)
+    P = F @ F + torch.eye(n, device="cuda")                                # commutes with F
+    P = ((P + P.transpose(1, 2)) / 2).contiguous()
+    skip = torch.zeros(batch, dtype=torch.int32, device="cuda")
+    skip[-1] = 1 if batch > 1 else 0
+    eye = torch.eye(n, device="cuda", dtype=torch.float64)
+    want = P.double() + 0.5 * F.double() @ P.double()
+    size = P.double().abs() + 0.5 * F.double().abs() @ P.double().abs()
+    kw = dict(pipe="f32") if pipe == "f32" else dict(amax=(X.amax(F), X.amax(P))) if pipe == "half" else {}
+    for symmetric in (False, True):
+        for shift in (0, 1):
+            C = torch.full((batch, n, n + shift), 7.0, device="cuda")[:, :, shift:]
+            T, err = torch.full((batch, n, n), 7.0, device="cuda"), torch.zeros(batch, device="cuda")
+            X.gemm(F, P, addend=P, alpha=0.5, beta=1.0, out=C, deviation=(T, err), skip=skip, symmetric=symmetric, **kw)
+            for b in range(batch):
+                if int(skip[b]):
+                    assert bool((C[b] == 7.0).all()) and bool((T[b] == 7.0).all()) and float(err[b]) == 0.0
+                    continue
+                # (the mirrored product takes F P for P F, which agree but for the rounding of P)
+                assert bool(((C[b].double() - want[b]).abs() <= (n + 8) * 2.0 ** -23 * size[b]).all())
+                assert torch.equal(T[b], (C[b].double() - eye).float()) and float(err[b]) == float(T[b].abs().max())
+                if symmetric:                                              # outside the diagonal tiles: an exact mirror
+                    tile = torch.arange(n, device="cuda") // 128
+                    off = tile[:, None] != tile[None, :]
+                    assert torch.equal(C[b][off], C[b].T[off])
+    with pytest.raises(ValueError):
+        X.gemm(F, P, deviation=(T, err))
+    with pytest.raises(ValueError):
+        X.gemm(F, P, addend=P, deviation=(T, err), newton=(T, -0.25, err))
+
+
+@pytest.mark.parametrize("n", [128, 256, 320, 512, 768, 1024])
+@pytest.mark.parametrize("measured", [False, True])
+def test_inverse_roots_against_the_same_iteration_in_float64(n, measured, monkeypatch):
+    """Eigenvalues over a factor of twenty.  Every round rounds R (relative 2^-24) and M (of which the root sees a quarter):
+    ten rounds of independent roundings make 2^-24 sqrt(10 (1 + 1/16) / 3) = 1.1e-7; three times that is allowed for, the rest
+    being the products of deviations.  On either pipe (the half pipe from order 256 on)."""
+    import qtensor.fused as X
+    from optimizers import matrix_functions
+    monkeypatch.setattr(X, "MEASURE_FROM", 0 if measured else 1 << 62)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    q, _ = torch.linalg.qr(torch.randn(2, n, n, device="cuda", generator=g, dtype=torch.float64))
+    lam = torch.exp(-3.0 * torch.rand(2, 1, n, device="cuda", generator=g, dtype=torch.float64))
+    mats = torch.bmm(q * lam, q.transpose(1, 2).contiguous())
+    mats = ((mats + mats.transpose(1, 2)) / 2).float()
+    v0 = torch.rand(2, n, device="cuda", generator=g) * 2 - 1
+    got = ComputePowerBatched(mats.clone(), 4, v0=v0)
+    rounds = matrix_functions._LAST_ROUNDS[n].tolist()
+    top = PowerIterBatched(mats, v0=v0).double()
+    A = mats.double()
+    A.diagonal(dim1=1, dim2=2).add_((1e-6 * top).unsqueeze(1))
+    z, eye = 5 / (2 * torch.linalg.matrix_norm(A)), torch.eye(n, device="cuda", dtype=torch.float64)
+    for b in range(2):
+        M, R = A[b] * z[b], eye * z[b] ** 0.25
+        for _ in range(rounds[b]):
+            T = 1.25 * eye - 0.25 * M
+            R, M = R @ T, (T @ T) @ (T @ T) @ M
+        assert float((got[b].double() - R).norm() / R.norm()) <= 3.3e-7, n
