@@ -218,12 +218,31 @@ typedef struct {
  * leading dimension that is a multiple of 4, and a quantized left operand's codes are a strided batch on 16-byte
  * boundaries), the product runs on the half pipe instead: every
  * element is scaled by a power of two taken from amax and written as the sum of two fp16 numbers (22 to 23 bits), three
- * fp16 products per fp32 product, the leading terms and the rests in fp32 accumulators of their own.  Errors against
- * float64 are those of the bf16 split or smaller (half of them for Gaussian matrices of order 1024) at 1.4 times its rate.
+ * fp16 products per fp32 product, the leading terms and the rests in fp32 accumulators of their own, at 1.4 times the
+ * split's rate.  Relative errors against float64 for Gaussian matrices of order 1024: 2.2e-7, the split 4.9e-7.  Where one
+ * pair of elements makes most of a sum the bit that is not kept shows: with a multiple of the identity as one operand
+ * 5.4e-8, the split 3.5e-8.
  * A bound need not be sharp: a tile with a row of an operand that exceeds its bound, is not finite or lies below 2^-24 of
  * it -- and every tile where a bound is zero, not finite or outside 2^-60 .. 2^61 -- is multiplied out by the bf16 split.
+ * What bounds alone do not tell is whether rows and columns hold small elements beside large ones: below 2^-28 of the
+ * bound an element loses bits, below 2^-51 it counts as zero.  A caller that gives bounds alone vouches that such elements
+ * do not matter; qtensor_hip_gemm_measured looks after them.
  * ranges may be null (then this is qtensor_hip_gemm); amax_out is served on every pipe. */
 void qtensor_hip_gemm_ranged(const qtensor_gemm_desc *desc, const qtensor_gemm_ranges *ranges, qtensor_stream_t stream);
+/* The same with what else the half pipe wants to know of its operands: how small their smallest piece is.  Pieces are four
+ * elements next to each other in a row and up to eight in a column (of the result of a product four, eight rows apart), the
+ * largest of them counts, and pieces of zeroes do not; a fineness is the largest reciprocal of a piece.  A product with an
+ * operand whose smallest piece lies below 2^-13 of what its scale makes of its bound (between 2^-28 and 2^-27 of the bound)
+ * is multiplied out by the bf16 split: on the half pipe an element is kept to 2^-23 of the largest next to it in its row
+ * and in its column.  fine_a, fine_b: as found by qtensor_hip_measure_batched or a product before, or larger; null: the
+ * caller vouches.  fine_out: raised to that of C[b] (and of T[b]);
+ * caller zeroes; with the epilogues that serve amax_out. */
+typedef struct {
+    const float *fine_a, *fine_b;
+    float *fine_out;
+} qtensor_gemm_fineness;
+void qtensor_hip_gemm_measured(const qtensor_gemm_desc *desc, const qtensor_gemm_ranges *ranges, const qtensor_gemm_fineness *fineness,
+                               qtensor_stream_t stream);
 /* out[b] = max(out[b], largest |element| of the rows x cols matrix b) for up to eight batches of fp32 matrices in one
  * launch (leading dimension ld; NaN counts as larger than infinity); the caller zeroes out.  Two sources may raise the
  * same out: the maxima and the exact diagonal of quantized matrices bound their elements (code tables within +-1). */
@@ -234,12 +253,19 @@ typedef struct {
 } qtensor_amax_source;
 void qtensor_hip_amax_batched(const qtensor_amax_source *sources, int count, qtensor_stream_t stream);
 /* The same for stacks of which some entries are left out: skip (optional, device, int32 [batch]): a matrix with a nonzero
- * flag is not read -- its address need not hold one -- and its out not raised. */
+ * flag is not read -- its address need not hold one -- and its out not raised.  fine (optional, caller zeroes): raised to
+ * the fineness of the matrix (see qtensor_gemm_fineness); each != 0: every element is a piece by itself: a quantized matrix
+ * is measured as its maxima, with its code table (code, n_code = 16 or 256 entries, of which the smallest that is not zero
+ * counts; else null), and its diagonal. */
 typedef struct {
     qtensor_batch_ptr mats;
     int ld, rows, cols, batch;
     float *out;
     const int *skip;
+    float *fine;
+    int each;
+    const float *code;
+    int n_code;
 } qtensor_measure_source;
 void qtensor_hip_measure_batched(const qtensor_measure_source *sources, int count, qtensor_stream_t stream);
 

@@ -104,6 +104,8 @@ struct GemmArgs {
 struct RangedArgs : GemmArgs {
     const uint32_t *amax_a, *amax_b;    // per batch entry: bits of (a bound of) the operand's largest |element|
     uint32_t *amax_out;                 // optional, per batch entry: raised to the bits of the result's largest |element|
+    const float *fine_a, *fine_b;       // optional, per batch entry: 1 / the smallest of the operand's pieces (qt_half.h)
+    uint32_t *fine_out;                 // optional, per batch entry: raised to the bits of that of the result (and of T)
 };
 
 namespace {
@@ -894,7 +896,8 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         __shared__ uint32_t s_top[BM + BN];
         float sa, sb, ia, ib;
         // (rows that are not 16-byte aligned inside a list of pointers are only seen here)
-        if (half_scale(args.amax_a[b], sa, ia) && half_scale(args.amax_b[b], sb, ib) && (KA != kDense || a_vec) && (KB != kDenseT || b_vec)) {
+        if (half_scale(args.amax_a, args.fine_a, b, sa, ia) && half_scale(args.amax_b, args.fine_b, b, sb, ib) && (KA != kDense || a_vec) &&
+            (KB != kDenseT || b_vec)) {
             constexpr int SETS = BM == 128 && BN == 128 ? 1 : 2;           // smaller tiles: less to do per tile to hide a load behind, and registers to spare
             constexpr bool QA = KA >= kQuant4, QB = KB >= kQuant4;
             typename std::conditional<QA, HalfQuantLeft<BM, KA == kQuant4 ? 4 : 8, SETS>,
@@ -1244,6 +1247,12 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         return;
     }
     float local_err = 0.0f, local_top = 0.0f;
+    // How large the result's elements are.  (Not with a quantized right factor, whose kernels have no registers left for it:
+    // looked up afterwards.)
+    constexpr bool kSized = PREC == kPipeHalf && KB < kQuant4;
+    bool pieces = false;
+    if constexpr (kSized) pieces = args.fine_out != nullptr;
+    Pieces seen, seen_t;
     // Each wave passes its accumulator blocks (32 x 32) through a staging square of its own in LDS, so that a
     // lane ends up with four consecutive elements of one output row: 16-byte stores, eight lanes per 128-byte
     // line, and one packed load per four elements of a quantized addend.
@@ -1289,13 +1298,17 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                             local_err = fmaxf(local_err, fabsf(y[q] - eye));
                             t[q] = EPI == kDeviation ? y[q] - eye : (1.0f - args.newton_w) * eye + args.newton_w * y[q];
                         }
+                        if (kSized && pieces) seen_t.row(t);
                         gstore4(T + (long long)row * args.ldt + col4, t);
                     }
-                    if constexpr (PREC == kPipeHalf) local_top = fmaxf(fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3]))), local_top);
+                    if (kSized && pieces) seen.row(y);
+                    if constexpr (kSized) local_top = fmaxf(fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3]))), local_top);
                     gstore4(C + (long long)row * ldc + col4, y);
                 }
                 wave_lds_sync();
+                if (kSized && pieces) { seen.end(); if (kSecond) seen_t.end(); }
             } else {
+                seen.low = 0;                      // (not looked at piece by piece: holds nothing)
                 // accumulator register r of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32 of the block
                 const int col = n0 + wn + j * 32 + (lane & 31);
 #pragma unroll
@@ -1316,7 +1329,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                         gstore(T + (long long)row * args.ldt + col,
                                EPI == kDeviation ? y - eye : (1.0f - args.newton_w) * eye + args.newton_w * y);
                     }
-                    if constexpr (PREC == kPipeHalf) local_top = fmaxf(fabsf(y), local_top);
+                    if constexpr (kSized) local_top = fmaxf(fabsf(y), local_top);
                     gstore(C + (long long)row * ldc + col, y);
                 }
             }
@@ -1354,7 +1367,8 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                     else y[q] = a[q];
                 }
                 // (past the end of a row: a repeated row's products, elements of the result like the others)
-                if constexpr (PREC == kPipeHalf) local_top = fmaxf(fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3]))), local_top);
+                if constexpr (kSized) local_top = fmaxf(fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3]))), local_top);
+                if (kSized && pieces) seen.row(y);
                 float *cm = C + (long long)mrow * ldc + mcol;
                 if (whole) gstore4(cm, y);
                 else
@@ -1367,6 +1381,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                         t[q] = EPI == kDeviation ? y[q] : args.newton_w * y[q];
                         if (EPI == kDeviation && mcol + q < args.M) local_err = fmaxf(local_err, fabsf(y[q]));
                     }
+                    if (kSized && pieces) seen_t.row(t);
                     float *tm = T + (long long)mrow * args.ldt + mcol;
                     if (whole) gstore4(tm, t);
                     else
@@ -1375,18 +1390,22 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                 }
             }
             wave_lds_sync();
+            if (kSized && pieces) { seen.end(); if (kSecond) seen_t.end(); }
         }
     if (kSecond) {
         uint32_t e = group_max_u32<64>(__float_as_uint(local_err));   // non-negative floats order like their bits
         if (lane == 0) atomicMax(reinterpret_cast<unsigned int *>(args.err) + b, e);
     }
-    if constexpr (PREC == kPipeHalf) {
-        if (args.amax_out != nullptr) {            // one atomic a workgroup: they come one after the other, 10 ns each (an atomic a wave: 56 us
-            __shared__ uint32_t s_out[4];          // where the 576 tiles of one 768 x 3072 product by itself take 34)
-            const uint32_t e = group_max_u32<64>(__float_as_uint(local_top));
-            if (lane == 0) s_out[wave] = e;
+    if constexpr (kSized) {
+        if (args.amax_out != nullptr || pieces) {  // once a workgroup (an atomic a wave: 56 us where the 576 tiles of a 768 x 3072
+            __shared__ uint32_t s_out[8];          // product by itself take 34)
+            const uint32_t e = group_max_u32<64>(__float_as_uint(local_top)), f = group_max_u32<64>(~min(seen.low, seen_t.low));
+            if (lane == 0) { s_out[wave] = e; s_out[4 + wave] = f; }
             __syncthreads();
-            if (threadIdx.x == 0) atomicMax(args.amax_out + b, max(max(s_out[0], s_out[1]), max(s_out[2], s_out[3])));
+            if (threadIdx.x == 0) {
+                if (args.amax_out != nullptr) raise_word(args.amax_out + b, max(max(s_out[0], s_out[1]), max(s_out[2], s_out[3])));
+                if (pieces) raise_fineness(args.fine_out + b, ~max(max(s_out[4], s_out[5]), max(s_out[6], s_out[7])));
+            }
         }
     }
     if (!streamed) return;
@@ -1508,82 +1527,105 @@ __global__ __launch_bounds__(256) void reduce_slices_kernel(const float *workspa
     }
 }
 
-// out[b] = max(out[b], max |element|) as bits (infinities and NaN above everything finite), over the rows x cols matrices
-// of up to kAmaxSources batches in one launch; a workgroup takes `rows_per` rows of one matrix: large pieces and one atomic
-// each, because the atomics on a batch's few cache lines come one after the other (36 x 768 x 1024, 16 K elements a
-// workgroup and an atomic a wave: 66 us, now 21).
+// out[b] = max(out[b], max |element|) as bits (infinities and NaN above everything finite), and fine[b] raised to 1 / the
+// smallest piece (qt_half.h), over the rows x cols matrices of up to kAmaxSources batches in one launch.  A thread takes
+// squares of 8 rows by 4 columns, neighbours neighbouring columns: eight 16-byte loads in flight, and the pieces of four
+// elements of a row and of eight of a column lie inside one thread.  A workgroup takes `squares` of them, many where there
+// is much to read, and raises a word or two.
+// 99 x 1024 x 1024 99 us with the clearing of its results (4.2 TB/s), without pieces 77 us; 768 x 3072 12 us either way.
 constexpr int kAmaxSources = 8;
 struct AmaxSource {
     BatchPtr mats;
     int ld, rows, cols, batch;
-    float *out;
+    float *out;                                  // optional
     const int *skip;                             // optional: skip[b] != 0 -> matrix b is not read
-    long long inner_stride;                      // (the library's own use: two-level batches, see GemmArgs::batch_inner)
-    int inner, rows_per;
-    unsigned first_block;
+    float *fine;                                 // optional
+    int each;                                    // != 0: every element is a piece by itself (maxima of segments, diagonals)
+    const float *code;                           // optional: maxima of segments of these codes (16 or 256): a piece is the
+    int n_code;                                  // smallest entry that is not zero times the maximum
+    int inner;                                   // (the library's own use: two-level batches, see GemmArgs::batch_inner)
+    long long inner_stride;
+    unsigned groups, first_block;                // workgroups per matrix, first workgroup of this source
+    FastDiv quads;                               // by the four-column pieces of a row
 };
-struct AmaxArgs { AmaxSource source[kAmaxSources]; int count; };
+struct AmaxArgs { AmaxSource source[kAmaxSources]; int count; unsigned squares; };
 __global__ __launch_bounds__(256) void amax_kernel(const AmaxArgs args) {
     int i = 0;
     while (i + 1 < args.count && blockIdx.x >= args.source[i + 1].first_block) ++i;
     const AmaxSource &m = args.source[i];
-    const unsigned pieces = (m.rows + m.rows_per - 1) / m.rows_per, block = blockIdx.x - m.first_block;
-    const int b = block / pieces, r0 = (int)(block % pieces) * m.rows_per, r1 = min(m.rows, r0 + m.rows_per);
+    const unsigned block = blockIdx.x - m.first_block;
+    const int b = block / m.groups;
     if (m.skip != nullptr && m.skip[b] != 0) return;
     const float *base = dense_ptr(m.mats, b, m.inner, m.inner_stride);
-    uint32_t top = 0;
-    auto see = [&](float4 x) {
-        top = max(max(max(__float_as_uint(x.x) & 0x7fffffffu, __float_as_uint(x.y) & 0x7fffffffu),
-                      max(__float_as_uint(x.z) & 0x7fffffffu, __float_as_uint(x.w) & 0x7fffffffu)), top);
-    };
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const bool wide = (m.ld & 3) == 0 && (m.cols & 3) == 0 && is_aligned16(base);
-    if (wide && m.ld == m.cols) {                    // a run of memory: eight loads of a thread in flight
-        const float *run = base + (long long)r0 * m.ld;
-        const int quads = (r1 - r0) * (m.cols >> 2);
-        int q = threadIdx.x;
-        for (; q + 7 * 256 < quads; q += 8 * 256) {
-            float4 x[8];
+    const bool wide = (m.ld & 3) == 0 && (m.cols & 3) == 0 && is_aligned16(base), each = m.each != 0;
+    const unsigned quads = m.quads.divisor, all = ((unsigned)(m.rows + 7) / 8) * quads;
+    const unsigned first = (block % m.groups) * args.squares, last = min(all, first + args.squares);
+    uint32_t top = 0, low = 0xffffffffu;
+    for (unsigned at = first + threadIdx.x; at < last; at += 256) {
+        const unsigned band = fastdiv(at, m.quads);
+        const int r0 = (int)band * 8, c0 = (int)(at - band * quads) * 4;
+        float4 x[8];                                 // past the end: the last row and column again
+        if (wide) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) x[j] = gload4(run + 4 * (q + j * 256));
+            for (int r = 0; r < 8; ++r) x[r] = gload4(base + (long long)min(r0 + r, m.rows - 1) * m.ld + c0);
+        } else {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) see(x[j]);
-        }
-        for (; q < quads; q += 256) see(gload4(run + 4 * q));
-    } else if (wide) {                               // a wave takes a row, two rows at a time
-        const int quads = m.cols >> 2;
-        for (int r = r0 + wave; r < r1; r += 8) {
-            const float *x0 = base + (long long)r * m.ld, *x1 = base + (long long)min(r + 4, r1 - 1) * m.ld;
-            for (int q = lane; q < quads; q += 64) {
-                const float4 u = gload4(x0 + 4 * q), v = gload4(x1 + 4 * q);
-                see(u);
-                see(v);
+            for (int r = 0; r < 8; ++r) {
+                const float *row = base + (long long)min(r0 + r, m.rows - 1) * m.ld;
+                const int end = m.cols - 1;
+                x[r] = make_float4(gload(row + c0), gload(row + min(c0 + 1, end)), gload(row + min(c0 + 2, end)), gload(row + min(c0 + 3, end)));
             }
         }
-    } else {
-        for (int r = r0 + wave; r < r1; r += 4)
-            for (int c = lane; c < m.cols; c += 64) top = max(__float_as_uint(gload(base + (long long)r * m.ld + c)) & 0x7fffffffu, top);
+        Pieces seen;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const float y[4] = {x[r].x, x[r].y, x[r].z, x[r].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) top = max(top, __float_as_uint(y[e]) & 0x7fffffffu);
+            if (each)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) seen.see(fabsf(y[e]));
+            else seen.row(y);
+        }
+        seen.end();
+        low = min(low, seen.low);
     }
-    __shared__ uint32_t s_top[4];
+    if (m.code != nullptr) {
+        uint32_t entry = 0xffffffffu;
+        for (int e = threadIdx.x & 63; e < m.n_code; e += 64) entry = min(entry, (__float_as_uint(gload(m.code + e)) & 0x7fffffffu) - 1u);
+        entry = ~group_max_u32<64>(~entry);
+        if (entry == 0xffffffffu) low = entry;                       // nothing but zeroes
+        else if (low != 0xffffffffu) low = max(__float_as_uint(__uint_as_float(low + 1u) * __uint_as_float(entry + 1u)), 1u) - 1u;
+    }
+    __shared__ uint32_t s_top[4], s_low[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     top = group_max_u32<64>(top);
-    if (lane == 0) s_top[wave] = top;
+    low = group_max_u32<64>(~low);
+    if (lane == 0) { s_top[wave] = top; s_low[wave] = low; }
     __syncthreads();
-    if (threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned int *>(m.out) + b, max(max(s_top[0], s_top[1]), max(s_top[2], s_top[3])));
+    if (threadIdx.x == 0) {
+        if (m.out != nullptr) raise_word(reinterpret_cast<uint32_t *>(m.out) + b, max(max(s_top[0], s_top[1]), max(s_top[2], s_top[3])));
+        if (m.fine != nullptr)
+            raise_fineness(reinterpret_cast<uint32_t *>(m.fine) + b, ~max(max(s_low[0], s_low[1]), max(s_low[2], s_low[3])));
+    }
 }
 
-// False (error slot) if the sources have more pieces than a grid takes.
+// False (error slot) if the sources have more squares than a grid takes.
 bool launch_amax(AmaxArgs &args, hipStream_t stream) {
     long long blocks = 0, elements = 0;
     for (int i = 0; i < args.count; ++i) elements += (long long)args.source[i].rows * args.source[i].cols * args.source[i].batch;
-    // a workgroup a unit, of 8 to 256 elements a thread (a thousand workgroups: 11 us for 768 x 3072, most of it atomics)
-    const long long piece = std::max(2048ll, std::min(65536ll, elements / 256));
+    // a workgroup a unit, of one to eight squares a thread
+    args.squares = 256u * (unsigned)std::max(1ll, std::min(8ll, elements / (256 * 8192)));
     for (int i = 0; i < args.count; ++i) {
         AmaxSource &m = args.source[i];
-        m.rows_per = (int)std::max(1ll, std::min((long long)m.rows, piece / m.cols));
+        const long long all = ((long long)m.rows + 7) / 8 * (((long long)m.cols + 3) / 4);
+        if (all + args.squares > 0x7fffffffLL) { set_error(kBadArgument, "amax: too large a matrix (%d x %d)", m.rows, m.cols); return false; }
+        m.groups = (unsigned)((all + args.squares - 1) / args.squares);
+        m.quads = make_fastdiv((unsigned)((m.cols + 3LL) / 4));
         m.first_block = (unsigned)blocks;
-        blocks += (long long)((m.rows + m.rows_per - 1) / m.rows_per) * m.batch;
+        blocks += (long long)m.groups * m.batch;
+        if (blocks > 0x7fffffffLL) { set_error(kBadArgument, "amax: too many matrices (%lld pieces)", blocks); return false; }
     }
-    if (blocks > 0x7fffffffLL) { set_error(kBadArgument, "amax: too many rows (%lld pieces)", blocks); return false; }
     hipLaunchKernelGGL(amax_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, args);
     return true;
 }
@@ -1709,7 +1751,12 @@ struct Ranges {                          // qtensor_gemm_ranges
     const float *amax_a, *amax_b;
     float *amax_out;
 };
-void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint = -1, const Ranges *ranges = nullptr);
+struct Fineness {                        // qtensor_gemm_fineness
+    const float *fine_a, *fine_b;
+    float *fine_out;
+};
+void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint = -1, const Ranges *ranges = nullptr,
+                   const Fineness *fineness = nullptr);
 
 // Process-wide choice of the matrix pipe (qtensor_hip_gemm_pipe); starts from the
 // environment variable QT_GEMM_PIPE ("f32" or "split"), else the split pipe.
@@ -1757,13 +1804,24 @@ extern "C" void qtensor_hip_gemm_ranged(const qtensor_gemm_desc *d, const void *
     gemm_dispatch(d, (hipStream_t)stream_v, -1, static_cast<const Ranges *>(ranges));
 }
 
+extern "C" void qtensor_hip_gemm_measured(const qtensor_gemm_desc *d, const void *ranges, const void *fineness, void *stream_v) {
+    qt::clear_error();
+    gemm_dispatch(d, (hipStream_t)stream_v, -1, static_cast<const Ranges *>(ranges), static_cast<const Fineness *>(fineness));
+}
+
 namespace {
 struct PublicAmaxSource {                        // qtensor_amax_source
     qt::BatchPtr mats;
     int ld, rows, cols, batch;
     float *out;
 };
-struct PublicMeasureSource : PublicAmaxSource { const int *skip; };        // qtensor_measure_source
+struct PublicMeasureSource : PublicAmaxSource {  // qtensor_measure_source
+    const int *skip;
+    float *fine;
+    int each;
+    const float *code;
+    int n_code;
+};
 
 template <typename Source>
 void measure(const char *what, const Source *sources, int count, hipStream_t stream) {
@@ -1779,8 +1837,18 @@ void measure(const char *what, const Source *sources, int count, hipStream_t str
             set_error(kBadArgument, "%s: need rows, cols, batch >= 1 and ld >= cols (got %d x %d, ld %d, batch %d)", what, m.rows, m.cols, m.ld, m.batch);
             return;
         }
-        args.source[i] = {m.mats, m.ld, m.rows, m.cols, m.batch, m.out, nullptr, 0, 1, 0, 0};
-        if constexpr (std::is_same<Source, PublicMeasureSource>::value) args.source[i].skip = m.skip;
+        args.source[i] = {m.mats, m.ld, m.rows, m.cols, m.batch, m.out, nullptr, nullptr, 0, nullptr, 0, 1, 0, 0, 0};
+        if constexpr (std::is_same<Source, PublicMeasureSource>::value) {
+            args.source[i].skip = m.skip;
+            args.source[i].fine = m.fine;
+            args.source[i].each = m.each;
+            args.source[i].code = m.code;
+            args.source[i].n_code = m.n_code;
+            if (m.code != nullptr && (m.each == 0 || (m.n_code != 16 && m.n_code != 256))) {
+                set_error(kBadArgument, "%s: a code table has 16 or 256 entries and goes with maxima (got %d entries)", what, m.n_code);
+                return;
+            }
+        }
     }
     if (launch_amax(args, stream)) launch_ok(what);
 }
@@ -1850,7 +1918,7 @@ void qt::gemm_with_tile(const qtensor_gemm_desc *d, hipStream_t stream, int tile
 }
 
 namespace {
-void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint, const Ranges *ranges) {
+void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint, const Ranges *ranges, const Fineness *fineness) {
     using namespace qt;
     if (!d) { set_error(kNullPointer, "gemm: null descriptor"); return; }
     RangedArgs a = {};
@@ -1891,7 +1959,7 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         set_error(kBadArgument, "gemm: Newton and deviation epilogues need T and err");
         return;
     }
-    if (ranges != nullptr && ranges->amax_out != nullptr && requant) { set_error(kBadArgument, "gemm: a re-encoded result has no amax_out"); return; }
+    if (requant && ((ranges != nullptr && ranges->amax_out != nullptr) || (fineness != nullptr && fineness->fine_out != nullptr))) { set_error(kBadArgument, "gemm: a re-encoded result has no amax_out"); return; }
     a.symmetric = a.symmetric != 0;
     a.batch_count = d->batch;
     a.stream_per = a.stream_lcm = 0;
@@ -1933,6 +2001,11 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         a.amax_a = reinterpret_cast<const uint32_t *>(ranges->amax_a);
         a.amax_b = reinterpret_cast<const uint32_t *>(ranges->amax_b);
         a.amax_out = reinterpret_cast<uint32_t *>(ranges->amax_out);
+    }
+    if (fineness != nullptr) {
+        a.fine_a = fineness->fine_a;
+        a.fine_b = fineness->fine_b;
+        a.fine_out = reinterpret_cast<uint32_t *>(fineness->fine_out);
     }
     // (codes are read in words of up to 16 bytes: a left factor's have to lie that way)
     const bool codes_lie = ka < kQuant4 || (a.Aq.codes.list == nullptr && is_aligned(a.Aq.codes.base, 16) && a.Aq.codes.stride % 16 == 0);
@@ -2043,8 +2116,8 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
         }
     }
     // (a product that is not made by one launch on the half pipe has its largest element looked up afterwards)
-    uint32_t *const amax_later = half_pipe && a.split_k == 1 && a.stream_per == 0 ? nullptr : a.amax_out;
-    if (amax_later != nullptr) a.amax_out = nullptr;
+    uint32_t *amax_later = nullptr, *fine_later = nullptr;
+    if (!(half_pipe && kb < kQuant4 && a.split_k == 1 && a.stream_per == 0)) { std::swap(amax_later, a.amax_out); std::swap(fine_later, a.fine_out); }
     const int combo = ka * 100 + kb * 10 + ep;
 #define QT_GEMM_CASE_DENSE(KA, KB, EP)                                                                       \
     case (KA) * 100 + (KB) * 10 + (EP):                                                                      \
@@ -2119,10 +2192,12 @@ void gemm_dispatch(const qtensor_gemm_desc *d, hipStream_t stream, int tile_hint
             set_error(kBadArgument, "gemm: combination A kind %d, B kind %d, epilogue %d is not built", ka, kb, ep);
             return;
     }
-    if (amax_later != nullptr) {
+    if (amax_later != nullptr || fine_later != nullptr) {
         AmaxArgs after = {};
-        after.count = 1;
-        after.source[0] = {a.C, a.ldc, a.M, a.N, d->batch, reinterpret_cast<float *>(amax_later), a.skip, a.inner_c, a.batch_inner, 0, 0};
+        after.source[after.count++] = {a.C, a.ldc, a.M, a.N, d->batch, reinterpret_cast<float *>(amax_later), a.skip,
+                                       reinterpret_cast<float *>(fine_later), 0, nullptr, 0, a.batch_inner, a.inner_c, 0, 0};
+        if (fine_later != nullptr && (ep == kNewton || ep == kDeviation))
+            after.source[after.count++] = {a.T, a.ldt, a.M, a.N, d->batch, nullptr, a.skip, reinterpret_cast<float *>(fine_later), 0, nullptr, 0, 1, 0, 0, 0};
         if (!launch_amax(after, stream)) return;
     }
 #undef QT_GEMM_CASE_DENSE

@@ -17,8 +17,18 @@
 // The scale needs the largest element beforehand (qtensor_gemm_ranges): a bound that the caller knows, what the launch
 // that wrote the matrix found (amax_out), or a pass over it.  It only has to be near: while the tiles are split the
 // kernel keeps the largest element of every tile row it reads, and a tile with a row that overflows its scale, is not finite,
-// or is so small against the scale (below 2^-24 of the largest element) that its elements might have lost bits is
-// multiplied out again by the bf16 split.  Neither a wrong bound nor rows of very different size cost precision.
+// or is small against the scale (below 2^-24 of the largest element) is multiplied out again by the bf16 split.
+//
+// That does not see small elements in a row that holds large ones as well -- a small row of B or column of A, all rows of
+// which are fine: with a diagonal A a row of B at 2^-40 of the others is a row of the result with 11 bits, at 2^-52 it is
+// zero.  So the launches that look for the largest element look for the smallest *piece* too: four elements of a row or
+// up to eight of a column next to each other (of the result of a product: four, eight rows apart), of which the largest
+// counts, and only pieces that are not zero.  Where every piece is at least 2^-28 of the bound an element is kept to 2^-23
+// of the largest next to it, in its row and in its column; a matrix with a smaller one is left to the bf16 split as a
+// whole (half_scale).  A piece, not an element, because some element of a matrix of noise is always that small: of a
+// Gaussian one of 768 x 3072 every eighth has one, of one with elements of 1e-6 of its diagonal all do.  Launches hand the
+// reciprocal on, the largest over the pieces ("fineness"), so that vectors of zeroes are what to begin with.  A caller that
+// gives bounds alone vouches for the pieces.
 #pragma once
 #include "qt_common.h"
 #include "qt_offsets.h"
@@ -305,14 +315,41 @@ struct HalfQuantRight {
     }
 };
 
-// The scale of an operand whose largest element has the bits `amax`, and its inverse.  False where a scale, its inverse or
-// the product of two could leave the fp32 range (the bf16 split takes such a product; an infinite or zero bound too).
-__device__ __forceinline__ bool half_scale(uint32_t amax, float &s, float &inverse) {
-    const uint32_t e = amax >> 23;                     // the largest element lies in [2^(e - 127), 2^(e - 126))
+// The scale of an operand whose largest element has the bits amax[b], and its inverse.  False where a scale, its inverse or
+// the product of two could leave the fp32 range (an infinite or zero bound too), and where the smallest piece of the
+// operand, scaled, lies below 2^-13: the bf16 split takes such a product.  (Nothing but two words and their comparison here:
+// with a look at the code table as well the compiler spilled inside the loops with a quantized operand, 84 -> 96 us for
+// a product by a quantized 3072 x 3072.)
+__device__ __forceinline__ bool half_scale(const uint32_t *amax, const float *fine, int b, float &s, float &inverse) {
+    const uint32_t e = amax[b] >> 23;                  // the largest element lies in [2^(e - 127), 2^(e - 126))
     if (e < 67 || e > 187) return false;
     s = __uint_as_float((127 + 14 + 127 - e) << 23);
     inverse = __uint_as_float((e - 14) << 23);
-    return true;
+    return fine == nullptr || fine[b] * 0x1p-13f <= s;
+}
+
+// The smallest piece of what is shown to it, four elements of a row at a time (minus one, as bits: zero counts as the largest).
+struct Pieces {
+    uint32_t low = 0xffffffffu;
+    float column[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    __device__ __forceinline__ void see(float piece) { low = min(low, __float_as_uint(piece) - 1u); }
+    __device__ __forceinline__ void row(const float y[4]) {
+        see(fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3]))));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) column[e] = fmaxf(column[e], fabsf(y[e]));
+    }
+    __device__ __forceinline__ void end() {              // of a run of rows: their columns' pieces
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { see(column[e]); column[e] = 0.0f; }
+    }
+};
+// *word = max(*word, value) for a word that only ever rises.  Atomics on one line come one after the other, 10 ns each, so a
+// look at the word first leaves out those that change nothing, all but a few.
+__device__ __forceinline__ void raise_word(uint32_t *word, uint32_t value) {
+    if (value > __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(word, value);
+}
+__device__ __forceinline__ void raise_fineness(uint32_t *fine, uint32_t low) {
+    if (low != 0xffffffffu) raise_word(fine, __float_as_uint(1.0f / __uint_as_float(low + 1u)));
 }
 
 // A tile row is fine if its largest scaled element is zero or in [2^-10, 2^15).

@@ -379,7 +379,7 @@ class ShampooBank:
                 # some blocks are left out: the others are gathered, updated and put back
                 take = torch.nonzero(skip == 0).squeeze(1)
                 if top is not None:
-                    kw["amax"] = (top.index_select(0, take),) * 2
+                    kw["amax"] = (top.index_select(1, take),) * 2
                 sub = seg.select(take)
                 dense = X.load_stack(sub)
                 X.gemm(X.PtrList(G.ptrs.index_select(0, take), (take.numel(), g.bm, g.bn), ld=g.ld),
@@ -389,8 +389,8 @@ class ShampooBank:
             return run
 
         def both(g):
-            def run():                  # the gradients' largest elements serve both sides
-                top = X.amax(self._grad_list(g), skip=self._skip(g, only))
+            def run():                  # how large the gradients' elements are serves both sides
+                top = X.measure(self._grad_list(g), skip=self._skip(g, only))
                 for side in (0, 1):
                     job(g, side, top)()
             return run
@@ -469,7 +469,7 @@ class ShampooBank:
                     X.gemm(left, G, out=half, skip=skip)
                     X.gemm(half, right, out=self._out_list(g), skip=skip)
                     return
-                tops = torch.zeros(4, len(g), device=self.device)
+                tops = torch.zeros(4, 2, len(g), device=self.device)
                 X.amax_into((left, tops[0]), (G, tops[1]), (right, tops[2]), skip=skip)
                 X.gemm(left, G, out=half, skip=skip, amax=(tops[0], tops[1]), amax_out=tops[3])
                 X.gemm(half, right, out=self._out_list(g), skip=skip, amax=(tops[3], tops[2]))

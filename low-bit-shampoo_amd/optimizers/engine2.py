@@ -139,29 +139,28 @@ class ShampooBank2(ShampooBank):
         rule on the whole stack, so that the bits do not depend on the part of it that is worked on."""
         return self.lowbit(order) and X.worth_measuring_for(self.per_order[order] * order ** 3, order, max(1, order // 2))
 
-    def _tops(self, order, count):
-        return torch.zeros(count, device=self.device) if self._measured(order) else None
-
     @staticmethod
-    def _rectify(vt, steps, top):
-        """`steps` Bjorck steps vt <- 1.5 vt - 0.5 (vt vt^T) vt and the largest elements (top: those of vt, None: not
-        looked at) of the result."""
+    def _rectify(vt, steps, size):
+        """`steps` Bjorck steps vt <- 1.5 vt - 0.5 (vt vt^T) vt = vt - 0.5 (vt vt^T - I) vt and how large the elements (size:
+        those of vt, None: not looked at) of the result are.  (The deviation from the identity: its elements are of one
+        size to the last step, where vt vt^T itself ends as the identity and rounding noise.)"""
+        eye = torch.eye(vt.shape[1], device=vt.device).expand(vt.shape[0], -1, -1) if steps > 0 else None
         for _ in range(steps):
-            square, after = (None, None) if top is None else torch.zeros(2, vt.shape[0], device=vt.device)
-            vvt = X.gemm(vt, vt, trans_b=True, symmetric=True, amax=None if top is None else (top, top), amax_out=square)
-            vt = X.gemm(vvt, vt, addend=vt, alpha=-0.5, beta=1.5, amax=None if top is None else (square, top), amax_out=after)
-            top = after
-        return vt, top
+            square, after = (None, None) if size is None else torch.zeros(2, 2, vt.shape[0], device=vt.device)
+            gram = X.gemm(vt, vt, trans_b=True, symmetric=True, addend=eye, beta=-1.0, amax=None if size is None else (size, size),
+                          amax_out=square)
+            vt = X.gemm(gram, vt, addend=vt, alpha=-0.5, amax=None if size is None else (square, size), beta=1.0, amax_out=after)
+            size = after
+        return vt, size
 
-    def _rectified_basis(self, order, rows=None, with_top=False):
+    def _rectified_basis(self, order, rows=None, with_size=False):
         """Dequantized Vt after rect_t1 Bjorck steps (utils.py:194-198; a basis held in fp32 is used as it is);
-        with_top: and its matrices' largest elements (None where they are not looked up)."""
+        with_size: and how large its elements are (None where that is not looked up)."""
         basis = self._pick(order, rows)[0]
-        vt, top = X.load_stack(basis), None
+        vt, size = X.load_stack(basis), None
         if not isinstance(basis, X.DenseStack):
-            top = X.amax(basis) if self._measured(order) else None
-            vt, top = self._rectify(vt, self.rect_t1, top)
-        return (vt, top) if with_top else vt
+            vt, size = self._rectify(vt, self.rect_t1, X.measure(basis) if self._measured(order) else None)
+        return (vt, size) if with_size else vt
 
     @staticmethod
     def _gather_rows(vt, keep):
@@ -171,12 +170,11 @@ class ShampooBank2(ShampooBank):
     def _kept_rows(self, order, vt, rows=None):
         return self._gather_rows(vt, self._pick(order, rows)[1])
 
-    def _statistic(self, order, vt, out=None, rows=None, top=None, top_out=None):
-        """Vt[keep]^T diag(S) Vt[keep] (utils.py:200-203).  top: Vt's largest elements, top_out: raised to the result's."""
+    def _statistic(self, order, vt, out=None, rows=None):
+        """Vt[keep]^T diag(S) Vt[keep] (utils.py:200-203)."""
         _, keep, svalue, _ = self._pick(order, rows)
         kept = self._gather_rows(vt, keep)
-        amax = None if top is None else (top * svalue.abs().amax(dim=1), top)
-        return X.gemm(kept * svalue.unsqueeze(2), kept, trans_a=True, symmetric=True, out=out, amax=amax, amax_out=top_out)
+        return X.gemm(kept * svalue.unsqueeze(2), kept, trans_a=True, symmetric=True, out=out)
 
     # ---- the operations of the reference's Preconditioner ----------------------------------------
     @torch.no_grad()
@@ -193,15 +191,16 @@ class ShampooBank2(ShampooBank):
             return
         # buffers that cross the phases below belong to the current stream
         stat = {o: torch.empty(self.per_order[o], o, o, device=self.device) for o in orders}
-        basis, top_vt = {}, {}
-        top_stat = {o: self._tops(o, self.per_order[o]) for o in orders}               # largest elements, where they are looked up
-        ones = torch.ones(max(self.per_order.values()), device=self.device)
-        top_grad = {}                                                                  # group -> its gradients' largest elements
+        basis = {}
+        # How large elements are, where that is looked up.  The statistics': with every block's gradient term by the launches that
+        # add them, else by a pass over the stack.
+        size_vt, size_grad = {}, {}                            # (the gradients' by group)
+        size_stat = {o: torch.zeros(2, self.per_order[o], device=self.device) for o in orders if only is None and self._measured(o)}
         self._write_grad_tables(grads)
         for g in self.groups:
             if (only is None or any(pi in only for pi in g.param_index)) and X.worth_measuring_for(
                     len(g) * g.bm * g.bn * (g.bm + g.bn) // 2, g.bm, g.bn):
-                top_grad[id(g)] = X.amax(self._grad_list(g), skip=self._skip(g, only))
+                size_grad[id(g)] = X.measure(self._grad_list(g), skip=self._skip(g, only))
 
         solver, redone, tick, begun = {}, {}, {}, {}
         # (a stack starts with the replacing sweep when most of it needed that sweep lately, or when it holds many
@@ -215,8 +214,8 @@ class ShampooBank2(ShampooBank):
 
         def rebuild(order):
             def run():
-                basis[order], top_vt[order] = self._rectified_basis(order, with_top=True)
-                self._statistic(order, basis[order], out=stat[order], top=top_vt[order], top_out=top_stat[order])
+                basis[order], size_vt[order] = self._rectified_basis(order, with_size=True)
+                self._statistic(order, basis[order], out=stat[order])
             return run
 
         def accumulate(g, side):
@@ -224,9 +223,9 @@ class ShampooBank2(ShampooBank):
                 order, first = g.slot[side]
                 seg = stat[order][first:first + len(g)]
                 G = self._grad_list(g)
-                top_out = None if top_stat[order] is None else top_stat[order][first:first + len(g)]
+                found = tuple(row[first:first + len(g)] for row in size_stat[order]) if order in size_stat else None
                 X.gemm(G, G, trans_a=side == 1, trans_b=side == 0, addend=seg, alpha=w2, beta=w1, out=seg, symmetric=True,
-                       skip=self._skip(g, only), amax=(top_grad[id(g)],) * 2 if id(g) in top_grad else None, amax_out=top_out)
+                       skip=self._skip(g, only), amax=(size_grad[id(g)],) * 2 if id(g) in size_grad else None, amax_out=found)
             return run
 
         def project(order):
@@ -237,8 +236,12 @@ class ShampooBank2(ShampooBank):
                 def remake(ids):
                     return X.gemm(stat[order].index_select(0, ids), self._rectified_basis(order, ids), trans_b=True)
 
-                product = X.gemm(stat[order], basis[order], trans_b=True,
-                                 amax=None if top_stat[order] is None else (top_stat[order], top_vt[order]))
+                sizes = None
+                if size_vt[order] is not None:
+                    if order not in size_stat:
+                        size_stat[order] = X.measure(stat[order])
+                    sizes = (size_stat[order], size_vt[order])
+                product = X.gemm(stat[order], basis[order], trans_b=True, amax=sizes)
                 begun[order] = torch.cuda.Event()
                 begun[order].record(torch.cuda.current_stream(self.device))
                 if apart[order]:
@@ -269,8 +272,10 @@ class ShampooBank2(ShampooBank):
                 per = max(1, self.QUOTIENT_PART_BYTES // (4 * order * order))
                 for first in range(0, Q.shape[0], per):
                     q = Q[first:first + per]
-                    # (columns of unit length: nothing beyond 1)
-                    lq = X.gemm(L[first:first + per], q, amax=None if top_stat[order] is None else (top_stat[order][first:first + per], ones[:q.shape[0]]))
+                    sizes = None
+                    if order in size_stat:
+                        sizes = (tuple(row[first:first + per] for row in size_stat[order]), X.measure(q))
+                    lq = X.gemm(L[first:first + per], q, amax=sizes)
                     quotients[first:first + per] = X.column_dots(q, lq) if order % 64 == 0 else (q * lq).sum(dim=1)
                 del lq
                 ascending, where = torch.sort(quotients, dim=1)
@@ -467,14 +472,13 @@ class ShampooBank2(ShampooBank):
                     whole = rows is None and part[1] == self.per_order[order]
                     basis, keep, svalue, max_eig = self._pick(order, None if whole else index)
                     if self.inv_root_mode == 0:
-                        kept, top = self._gather_rows(X.load_stack(basis), keep), None
+                        kept, size = self._gather_rows(X.load_stack(basis), keep), None
                         if not isinstance(basis, X.DenseStack):          # (a basis held in fp32 is not rectified: utils.py:205-227)
-                            top = X.amax(basis) if self._measured(order) else None
-                            kept, top = self._rectify(kept, self.rect_t2, top)
+                            kept, size = self._rectify(kept, self.rect_t2, X.measure(basis) if self._measured(order) else None)
                         ridge = self.matrix_eps * max_eig
                         weights = 1 / (svalue + ridge.unsqueeze(1)).pow(1 / 4)
                         roots = X.gemm(kept * weights.unsqueeze(2), kept, trans_a=True, symmetric=True,
-                                       amax=None if top is None else (top * weights.amax(dim=1), top))
+                                       amax=None if size is None else ((size[0] * weights.amax(dim=1), size[1] / weights.amin(dim=1)), size))
                     else:
                         L = self._statistic(order, self._rectified_basis(order, None if whole else index), rows=None if whole else index)
                         start = starts[order] if whole else starts[order].index_select(0, index)

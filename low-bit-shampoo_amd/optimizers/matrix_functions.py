@@ -170,15 +170,18 @@ def ComputePowerBatched(mats, p=4, iter_count=10, error_tolerance=1e-6, ridge_ep
 
     R_ptr, M_ptr, E_ptr = table(R), table(M), table(E)
     side = torch.zeros(B, dtype=torch.bool, device=dev)                     # False: buffer 0 holds the state
-    # How large the iterates' elements are, for the pipe that wants to know: |E| and |M| follow from err = max |E|, the roots
-    # and the powers of T are looked at by the launches that write them.  Small stacks are
+    # How large the iterates' elements are, for the pipe that wants to know: the bounds of E and M follow from err = max |E|,
+    # the rest is looked at by the launches that write them (both of E and M by one).  Small stacks are
     # bound by the host, which this costs 40 us a round (statistics of convolutions of width 32: 29 ms without, 33 with).
     measured = X.worth_measuring_for(B * n ** 3, n)
     squarings = p.bit_length() - 1
     if measured:
-        tops = torch.zeros(iter_count, 1 + squarings, B, device=dev)
-        top_e, top_m = err, 1 + err
-        top_r = first_root * (1 + abs(w) * err)                              # of the root after the first round
+        first = torch.zeros(2, B, device=dev)
+        X.amax_into((M[0], first), (E[0], first))
+        found = torch.zeros(iter_count, 2 + squarings, 2, B, device=dev)     # per round: root, powers, E with M
+        top_e, top_m = (err, first[1]), (1 + err, first[1])
+        # of the root after the first round, c (I + w E): small pieces are c w times those of E
+        top_r = (first_root * (1 + abs(w) * err), first[1] / (abs(w) * first_root))
     for round_number in range(iter_count):
         skip = done.to(torch.int32)
         cur = lambda tab: torch.where(side, tab[1], tab[0])                   # noqa: E731
@@ -191,22 +194,23 @@ def ComputePowerBatched(mats, p=4, iter_count=10, error_tolerance=1e-6, ridge_ep
             R[1].diagonal(dim1=1, dim2=2).add_(first_root.unsqueeze(1))
         else:
             X.gemm(Rc, Ec, addend=Rc, alpha=w, beta=1.0, out=Ro, skip=skip, symmetric=symmetric,        # candidate root
-                   **(dict(amax=(top_r, top_e), amax_out=tops[round_number, 0]) if measured else {}))
+                   **(dict(amax=(top_r, top_e), amax_out=found[round_number, 0]) if measured else {}))
             if measured:
-                top_r = tops[round_number, 0]                                # (a rejected candidate ends its matrix's iteration)
+                top_r = found[round_number, 0]                               # (a rejected candidate ends its matrix's iteration)
         power, scale = Ec, w                                                 # T^p = I + scale * power by repeated squaring
         top = top_e if measured else None
         for square in range(1, 1 + squarings):
             dst = F[square % 2]
-            after = tops[round_number, square] if measured else None
+            after = found[round_number, square] if measured else None
             X.gemm(power, power, addend=power, alpha=scale * scale, beta=2 * scale, out=dst, skip=skip, symmetric=symmetric,
                    amax=(top, top) if measured else None, amax_out=after)
             power, scale, top = dst, 1.0, after
         new_err = torch.zeros(B, device=dev)
         X.gemm(power, Mc, addend=Mc, alpha=scale, beta=1.0, out=Mo, deviation=(Eo, new_err), skip=skip, symmetric=symmetric,
-               amax=(top, top_m) if measured else None)
+               amax=(top, top_m) if measured else None, amax_out=found[round_number, 1 + squarings] if measured else None)
         if measured:
-            top_e, top_m = new_err, 1 + new_err
+            fine = found[round_number, 1 + squarings, 1]
+            top_e, top_m = (new_err, fine), (1 + new_err, fine)
         accept = (~done) & ~(new_err > err * 1.2)
         side = side ^ accept
         err = torch.where(accept, new_err, err)

@@ -56,12 +56,16 @@ class GemmRanges(ct.Structure):
 
 class MeasureSource(ct.Structure):
     _fields_ = [("mats", BatchPtr), ("ld", ct.c_int), ("rows", ct.c_int), ("cols", ct.c_int), ("batch", ct.c_int), ("out", ct.c_void_p),
-                ("skip", ct.c_void_p)]
+                ("skip", ct.c_void_p), ("fine", ct.c_void_p), ("each", ct.c_int), ("code", ct.c_void_p), ("n_code", ct.c_int)]
+
+
+class GemmFineness(ct.Structure):
+    _fields_ = [("fine_a", ct.c_void_p), ("fine_b", ct.c_void_p), ("fine_out", ct.c_void_p)]
 
 
 if F.lib is not None:
-    F.lib.qtensor_hip_gemm_ranged.restype = None
-    F.lib.qtensor_hip_gemm_ranged.argtypes = [ct.POINTER(GemmDesc), ct.POINTER(GemmRanges), ct.c_void_p]
+    F.lib.qtensor_hip_gemm_measured.restype = None
+    F.lib.qtensor_hip_gemm_measured.argtypes = [ct.POINTER(GemmDesc), ct.POINTER(GemmRanges), ct.POINTER(GemmFineness), ct.c_void_p]
     F.lib.qtensor_hip_measure_batched.restype = None
     F.lib.qtensor_hip_measure_batched.argtypes = [ct.POINTER(MeasureSource), ct.c_int, ct.c_void_p]
     F.lib.qtensor_hip_gemm_pipe.restype = ct.c_int
@@ -166,42 +170,70 @@ def _workspace(device: torch.device, floats: int) -> Tensor:
     return torch.empty(min(_WORKSPACE_FLOATS, floats), dtype=torch.float32, device=device)
 
 
-def _launch(desc: GemmDesc, device: torch.device, ranges: Optional[GemmRanges] = None) -> None:
+def _launch(desc: GemmDesc, device: torch.device, ranges: Optional[GemmRanges] = None, fineness: Optional[GemmFineness] = None) -> None:
     if F.lib is None:
         raise RuntimeError("libqtensor_hip.so is not available")
     if ranges is not None:
-        F._call(F.lib.qtensor_hip_gemm_ranged, device, ct.byref(desc), ct.byref(ranges))
+        F._call(F.lib.qtensor_hip_gemm_measured, device, ct.byref(desc), ct.byref(ranges), ct.byref(fineness))
         return
     F._call(F.lib.qtensor_hip_gemm, device, ct.byref(desc))
+
+
+def _pair(what, batch: int, name: str):
+    """(address of the largest elements, address of the finenesses or None) of what `amax` and `amax_out` take: an fp32
+    vector [batch], both in one tensor [2, batch] (`measure`), or a tuple of two vectors."""
+    if isinstance(what, Tensor):
+        both = what.numel() == 2 * batch and what.shape[0] == 2
+        fits = (both or what.numel() == batch) and what.dtype == torch.float32 and what.is_cuda and what.is_contiguous()
+        if not fits:
+            raise ValueError(f"{name}: contiguous fp32 GPU vectors with one entry per batch entry, one or two of them")
+        return what.data_ptr(), what.data_ptr() + 4 * batch if both else None
+    top, fine = what
+    return _pair(top, batch, name)[0], _pair(fine, batch, name)[0]
 
 
 def amax_into(*pairs, skip: Optional[Tensor] = None) -> None:
     """Each pair (t, out): fp32 [batch] out raised to the largest |element| of every matrix of t ([rows, cols], [batch,
     rows, cols], a PtrList) or to a bound of it (a `Quantized`: its maxima and exact diagonal; code tables hold nothing
-    beyond +-1).  All of them in one launch (up to eight tensors; a `Quantized` with a diagonal counts as two).
+    beyond +-1).  All of them in one launch (up to eight tensors; a `Quantized` with a diagonal counts as two).  An out of
+    [2, batch] has its second row raised to the finenesses (`measure`).
     skip: optional int32 [batch]; matrices with a nonzero flag are not read and their entries of out not raised."""
     sources = []
     for t, out in pairs:
-        if isinstance(t, Quantized):
+        each = isinstance(t, Quantized)
+        if each:
             per_row = t.absmax.shape[1] // t.order
-            parts = [(BatchPtr(t.absmax.data_ptr(), None, t.absmax.stride(0)), per_row, t.batch, t.order, per_row)]
+            parts = [(BatchPtr(t.absmax.data_ptr(), None, t.absmax.stride(0)), per_row, t.batch, t.order, per_row, t.code.data_ptr())]
             if t.diag is not None:
-                parts.append((BatchPtr(t.diag.data_ptr(), None, t.diag.stride(0)), t.order, t.batch, 1, t.order))
+                parts.append((BatchPtr(t.diag.data_ptr(), None, t.diag.stride(0)), t.order, t.batch, 1, t.order, None))
         else:
-            parts = [_dense(t)]
-        for ptr, ld, batch, rows, cols in parts:
-            if out.dtype != torch.float32 or out.numel() != batch or not out.is_cuda or not out.is_contiguous():
-                raise ValueError("out must be a contiguous fp32 GPU vector with one entry per batch entry")
+            parts = [_dense(t) + (None,)]
+        for ptr, ld, batch, rows, cols, code in parts:
+            top, fine = _pair(out, batch, "out")
             if skip is not None and (skip.dtype != torch.int32 or skip.numel() != batch):
                 raise ValueError("skip must be int32 [batch]")
-            sources.append(MeasureSource(ptr, ld, rows, cols, batch, out.data_ptr(), None if skip is None else skip.data_ptr()))
+            sources.append(MeasureSource(ptr, ld, rows, cols, batch, top, None if skip is None else skip.data_ptr(), fine, each,
+                                         code, 0 if code is None else t.code.numel()))
     F._call(F.lib.qtensor_hip_measure_batched, pairs[0][1].device, (MeasureSource * len(sources))(*sources), len(sources))
+
+
+def _batch_of(t) -> int:
+    return t.batch if isinstance(t, Quantized) else 1 if t.dim() == 2 else t.shape[0]
 
 
 def amax(t, skip: Optional[Tensor] = None) -> Tensor:
     """fp32 [batch]: the largest |element| of every matrix of t, or a bound of it (see amax_into)."""
-    out = torch.zeros(t.batch if isinstance(t, Quantized) else 1 if t.dim() == 2 else t.shape[0],
-                      device=t.codes.device if isinstance(t, Quantized) else t.device)
+    out = torch.zeros(_batch_of(t), device=t.codes.device if isinstance(t, Quantized) else t.device)
+    amax_into((t, out), skip=skip)
+    return out
+
+
+def measure(t, skip: Optional[Tensor] = None) -> Tensor:
+    """fp32 [2, batch]: the largest |element| of every matrix of t, or a bound of it, and its fineness: the reciprocal of its
+    smallest piece, four elements of a row or up to eight of a column, of which the largest counts (of a `Quantized`: of a
+    bound of its smallest element, the smallest code times the smallest maximum, or of its diagonal).  Products on the half pipe take no matrix with a piece below 2^-28 of its
+    bound, and so lose no bits of rows or columns that are small beside others (qtensor_hip_gemm_measured)."""
+    out = torch.zeros(2, _batch_of(t), device=t.codes.device if isinstance(t, Quantized) else t.device)
     amax_into((t, out), skip=skip)
     return out
 
@@ -244,11 +276,12 @@ def gemm(A, B, *, trans_a=False, trans_b=False, out: Optional[Tensor] = None, al
     upper_a / upper_b: op(A) / op(B) is upper triangular (zero below the diagonal, square in its k
     index, dense): the part of the k range where it is zero is skipped.
     pipe: None (the process-wide choice, gemm_pipe), "f32" or "split" for this product alone.
-    amax: optional pair of fp32 [batch] vectors, the largest |element| of A[b] and of B[b] or bounds of them: large
-    enough products of dense operands then run on the half pipe (two fp16 pieces per element, three products per fp32
-    product: errors no larger than those of "split", 1.4 times its rate).  A bound that is wrong costs time, not
-    precision: include/qtensor_hip.h, qtensor_hip_gemm_ranged.
-    amax_out: optional fp32 [batch], raised to the largest |element| of out[b] (zeroed by the caller)."""
+    amax: optional pair, how large the elements of A[b] and of B[b] are: for either what `measure` returns, or a pair of
+    fp32 [batch] vectors (a bound of the largest |element|, a fineness), or a bound alone: large enough products then run
+    on the half pipe (two fp16 pieces per element, three products per fp32 product, 1.4 times the rate of "split").
+    A bound that is wrong costs time, not precision; a caller that gives a bound alone vouches that elements below
+    2^-28 of it do not matter (include/qtensor_hip.h, qtensor_hip_gemm_ranged and qtensor_hip_gemm_measured).
+    amax_out: optional, raised to the same of out[b] (zeroed by the caller): fp32 [batch], [2, batch] or a pair."""
     d = GemmDesc()
     a = d.args
     if pipe not in _PIPES:
@@ -344,17 +377,15 @@ def gemm(A, B, *, trans_a=False, trans_b=False, out: Optional[Tensor] = None, al
         scratch = _workspace(dev, max(8 * batch * m * n, (tiles + 520) * 128 * 128 if quantized and tiles < 1024 else 0))
         a.workspace, a.workspace_floats = scratch.data_ptr(), scratch.numel()
         keep.append(scratch)
-    ranges = None
+    ranges = fineness = None
     if amax is not None or amax_out is not None:
-        ranges = GemmRanges()
-        for t in (amax or ()) + ((amax_out,) if amax_out is not None else ()):
-            if t.dtype != torch.float32 or t.numel() != batch or not t.is_cuda or not t.is_contiguous():
-                raise ValueError("amax and amax_out are contiguous fp32 GPU vectors with one entry per batch entry")
+        ranges, fineness = GemmRanges(), GemmFineness()
         if amax is not None:
-            ranges.amax_a, ranges.amax_b = amax[0].data_ptr(), amax[1].data_ptr()
+            ranges.amax_a, fineness.fine_a = _pair(amax[0], batch, "amax")
+            ranges.amax_b, fineness.fine_b = _pair(amax[1], batch, "amax")
         if amax_out is not None:
-            ranges.amax_out = amax_out.data_ptr()
-    _launch(d, dev, ranges)
+            ranges.amax_out, fineness.fine_out = _pair(amax_out, batch, "amax_out")
+    _launch(d, dev, ranges, fineness)
     return addend if requantize else out
 
 
@@ -386,7 +417,7 @@ def precondition(G: Tensor, left, right, out: Optional[Tensor] = None) -> Tensor
     if not worth_measuring(left, G, right):
         tmp = gemm(left, G)
         return gemm(tmp, right, out=out)
-    tops = torch.zeros(4, 1 if G.dim() == 2 else G.shape[0], device=G.device)
+    tops = torch.zeros(4, 2, 1 if G.dim() == 2 else G.shape[0], device=G.device)
     amax_into((left, tops[0]), (G, tops[1]), (right, tops[2]))
     tmp = gemm(left, G, amax=(tops[0], tops[1]), amax_out=tops[3])
     return gemm(tmp, right, out=out, amax=(tops[3], tops[2]))

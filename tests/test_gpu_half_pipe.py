@@ -267,3 +267,141 @@ def test_matrices_that_are_left_out_are_not_looked_at(X, monkeypatch):
                 X.quantize_stack(torch.eye(512, device="cuda")[None] + 0.01 * present[None], bank.precs[512].rows(at, 1))
         got, want = (bank.preconditioned_grads(grads, only=[0]) for bank, grads in zip(banks, ([grad, None], [grad])))
         assert got[1] is None and float((got[0] - want[0]).norm() / want[0].norm()) <= 1e-6
+
+
+def two_products_bound(L, G, R):
+    """Elementwise bound of deq(L) G deq(R) by the rule above for either product, and for what the first one's error becomes."""
+    one = lambda k: (2 * 2.0 ** -23 + 2.0 ** -24) + 2 * (3 * k / 16 + 2) * 2.0 ** -24        # noqa: E731
+    return 1.01 * (one(L.shape[-1]) + one(R.shape[-1])) * (L.double().abs() @ G.double().abs() @ R.double().abs())
+
+
+@pytest.mark.parametrize("down", [20, 28, 32, 36, 40, 44, 52, 60, 100])
+@pytest.mark.parametrize("factors", ["diagonal", "roots"])
+def test_preconditioned_gradients_keep_small_rows_and_columns(X, code_maps, monkeypatch, down, factors):
+    """Rows and columns of a gradient that are 2^-down of the others (units that hardly learn), with factors that keep them
+    apart: element by element against float64.  Small rows are lines of the first product's k, small columns of the second's."""
+    monkeypatch.setattr(X, "MEASURE_FROM", 0)
+    code = torch.from_numpy(code_maps[("linear-2", 4)]).cuda()
+    g = torch.Generator(device="cuda").manual_seed(down)
+    m, n = 512, 768
+    for bits in (4, 8):
+        code = torch.from_numpy(code_maps[("linear-2", 4) if bits == 4 else ("dynamic", 8)]).cuda()
+        made = []
+        for k in (m, n):
+            mats = torch.diag_embed(1 + torch.rand(2, k, device="cuda", generator=g))
+            if factors == "roots":
+                half = torch.arange(k, device="cuda") % 2                # units of two kinds that have nothing to do with each other
+                mats = mats + 0.02 * torch.randn(2, k, k, device="cuda", generator=g) * (half[:, None] == half[None, :])
+            made.append(X.quantize_stack(mats.contiguous(), X.empty_quantized(2, k, 64, bits, code, True)))
+        L, R = (X.dequantize_stack(q) for q in made)
+        for which in ("row", "column", "rows and columns"):
+            G = torch.randn(2, m, n, device="cuda", generator=g)
+            small = 2.0 ** -down
+            if which == "row":
+                G[0, 3] *= small
+            elif which == "column":
+                G[1, :, 5] *= small
+            else:
+                G[:, 1::2] *= small
+                G[:, :, 1::2] *= small
+            want = L.double() @ G.double() @ R.double()
+            err = (X.precondition(G, *made).double() - want).abs()
+            # (2^-120: below 2^-110 the pieces of the bf16 split reach the end of the exponents)
+            assert bool((err <= two_products_bound(L, G, R) + 2.0 ** -120).all()), (bits, which)
+
+
+@pytest.mark.parametrize("k,m,n", [(512, 130, 200), (768, 384, 256), (4096, 64, 64)])
+def test_products_of_measured_operands_keep_small_pieces(X, k, m, n):
+    """Either operand with one small line of k, small lines all along one half of k, or small elements everywhere beside one
+    large row and one large column (all layouts, the cut along k): element by element against float64."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    for down in (30, 45, 70):
+        small = 2.0 ** -down
+        for kind in ("line", "half", "cross"):
+            A, B = torch.randn(2, m, k, device="cuda", generator=g), torch.randn(2, k, n, device="cuda", generator=g)
+            for side in (0, 1):
+                a, b = A.clone(), B.clone()
+                t = a if side == 0 else b.transpose(1, 2)               # [batch, rows, k]
+                if kind == "line":
+                    t[0, :, 7] *= small
+                    (b[0, 8:] if side == 0 else a[0, :, 8:]).zero_()     # so that the line makes a part of every sum ...
+                    (b[0, :7] if side == 0 else a[0, :, :7]).zero_()     # ... which nothing else does
+                elif kind == "half":
+                    t[:, :, 1::2] *= small
+                    (b[:, ::2, ::2] if side == 0 else a[:, ::2, ::2]).zero_()
+                else:
+                    t[:, 1:, 1:] *= small
+                    (b[:, 0, 1:] if side == 0 else a[:, 1:, 0]).zero_()
+                for kw, x, y in ((dict(), a, b), (dict(trans_a=True), a.transpose(1, 2).contiguous(), b),
+                                 (dict(trans_b=True), a, b.transpose(1, 2).contiguous())):
+                    check(X.gemm(x, y, amax=(X.measure(x), X.measure(y)), **kw), a, b, k)
+
+
+def test_measures_of_matrices_and_results(X):
+    """The largest element and the fineness (1 / the smallest piece) against those counted piece by piece, of matrices of
+    whole and ragged sizes and of results on every route; ordinary operands stay on the half pipe."""
+    def fineness(t, rows):                                               # t [n, n]; column pieces of `rows` at these places
+        a = t.abs()
+        c = torch.nn.functional.pad(a, (0, -a.shape[1] % 4, 0, -a.shape[0] % rows))
+        tops = torch.cat([c.reshape(c.shape[0], -1, 4).amax(2).flatten(), c.reshape(-1, rows, c.shape[1]).amax(1).flatten()])
+        return 1 / tops[tops > 0].min()
+    g = torch.Generator(device="cuda").manual_seed(2)
+    for rows, cols in ((64, 64), (9, 4), (1, 7), (130, 33), (1000, 516)):
+        t = torch.randn(3, rows, cols, device="cuda", generator=g)
+        t[1] *= (torch.rand(rows, cols, device="cuda", generator=g) < 0.3)
+        t[2] = 0.0
+        size = X.measure(t)
+        assert torch.equal(size[0], t.abs().amax((1, 2))) and float(size[1, 2]) == 0.0
+        if cols % 4 == 0 or cols < 4:
+            for b in (0, 1):
+                assert float(size[1, b]) == float(fineness(t[b], 8))
+    t[0, 3, 5] = float("nan")
+    assert bool(X.measure(t)[0, 0].isnan())
+    code = torch.linspace(-1, 1, 16, device="cuda")
+    q = X.quantize_stack(torch.randn(2, 128, 128, device="cuda", generator=g), X.empty_quantized(2, 128, 64, 4, code, True))
+    q.absmax[0, 3], q.absmax[0, 4], q.diag[1, 7] = 1e-5, 0.0, 1e-7
+    assert torch.allclose(X.measure(q)[1], torch.tensor([1e5 * 15, 1e7], device="cuda"), rtol=1e-6)        # (codes of 1/15 and up)
+    A = torch.randn(2, 544, 544, device="cuda", generator=g)
+    A[0, 1::2, 1::2] *= 1e-3
+    size = X.measure(A)
+    none = torch.zeros(2, dtype=torch.int32, device="cuda")
+    split, half = X.gemm(A, A, skip=none), X.gemm(A, A, amax=(size[0], size[0]), skip=none)
+    assert not torch.equal(split, half)
+    for kw, want in ((dict(amax=(size, size), skip=none), half), (dict(amax=(size, 1e6 * size), skip=none), split),
+                     (dict(amax=(size, size), pipe="f32", skip=none), X.gemm(A, A, pipe="f32", skip=none))):
+        found = torch.zeros(2, 2, device="cuda")
+        got = X.gemm(A, A, amax_out=found, **kw)
+        assert torch.equal(got, want) and torch.equal(found[0], got.abs().amax((1, 2)))
+        for b in (0, 1):                                                 # pieces of four or eight rows: between the smallest elements ...
+            assert float(1 / got[b].abs()[got[b] != 0].min()) >= float(found[1, b]) >= float(fineness(got[b], 32))     # ... and rows
+    # second outputs are looked at as well
+    found, T, err = torch.zeros(2, 2, device="cuda"), torch.empty_like(A), torch.zeros(2, device="cuda")
+    C = torch.empty_like(A)
+    X.gemm(A, A, addend=A, out=C, deviation=(T, err), amax=(size, size), amax_out=found)
+    assert torch.equal(found[0], C.abs().amax((1, 2))) and torch.equal(T, C - torch.eye(544, device="cuda"))
+
+
+def test_inverse_roots_keep_units_that_hardly_learn(X, monkeypatch):
+    """A statistic with 64 units at 2^-40 of the others' gradients (their diagonal is the ridge's): the blocks of the root
+    that tie them to the others, against the same iteration in float64.  Every round rounds them like the rest."""
+    import optimizers.matrix_functions as MF
+    monkeypatch.setattr(X, "MEASURE_FROM", 0)
+    n = 512
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, _ = torch.linalg.qr(torch.randn(n, n, device="cuda", generator=g, dtype=torch.float64))
+    d = torch.ones(n, device="cuda", dtype=torch.float64)
+    d[-64:] = 2.0 ** -40
+    mat = (d[:, None] * (q * torch.exp(-3 * torch.rand(n, device="cuda", generator=g, dtype=torch.float64))) @ q.T * d).float()
+    mat = ((mat + mat.T) / 2)[None].contiguous()
+    v0 = torch.ones(1, n, device="cuda")
+    got = MF.ComputePowerBatched(mat.clone(), 4, v0=v0)[0].double()
+    A, eye = mat[0].double(), torch.eye(n, device="cuda", dtype=torch.float64)
+    A = A + 1e-6 * MF.PowerIterBatched(mat, v0=v0).double() * eye
+    z = 5 / (2 * A.norm())
+    M, R = A * z, eye * z ** 0.25
+    for _ in range(int(MF._LAST_ROUNDS[n])):
+        T = 1.25 * eye - 0.25 * M
+        R, M = R @ T, (T @ T) @ (T @ T) @ M
+    for block in (got[:-64, -64:] - R[:-64, -64:], got[-64:, :-64] - R[-64:, :-64]):
+        assert float(block.norm() / R[:-64, -64:].norm()) <= 3e-6
+    assert float((got - R).norm() / R.norm()) <= 3.3e-7
