@@ -202,10 +202,12 @@ def amax_into(*pairs, skip: Optional[Tensor] = None) -> None:
     for t, out in pairs:
         each = isinstance(t, Quantized)
         if each:
-            per_row = t.absmax.shape[1] // t.order
-            parts = [(BatchPtr(t.absmax.data_ptr(), None, t.absmax.stride(0)), per_row, t.batch, t.order, per_row, t.code.data_ptr())]
+            # (one matrix may have its buffers as vectors, as quantize_blockwise writes them)
+            per_row = t.absmax.shape[-1] // t.order
+            stacked = [BatchPtr(x.data_ptr(), None, x.stride(0) if x.dim() == 2 else 0) for x in (t.absmax, t.diag) if x is not None]
+            parts = [(stacked[0], per_row, t.batch, t.order, per_row, t.code.data_ptr())]
             if t.diag is not None:
-                parts.append((BatchPtr(t.diag.data_ptr(), None, t.diag.stride(0)), t.order, t.batch, 1, t.order, None))
+                parts.append((stacked[1], t.order, t.batch, 1, t.order, None))
         else:
             parts = [_dense(t) + (None,)]
         for ptr, ld, batch, rows, cols, code in parts:
@@ -430,7 +432,7 @@ def worth_measuring(left, G, right) -> bool:
     m, n = G.shape[-2:]
     batch = 1 if G.dim() == 2 else G.shape[0]
     return worth_measuring_for(batch * m * n * (m + n), m, n) and all(
-        q.flat if isinstance(q, Quantized) else q.stride(-1) == 1 for q in (left, right))
+        q.flat if isinstance(q, Quantized) else isinstance(q, PtrList) or q.stride(-1) == 1 for q in (left, right))
 
 
 def worth_measuring_for(multiply_adds: int, *k: int) -> bool:

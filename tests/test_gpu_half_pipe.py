@@ -405,3 +405,28 @@ def test_inverse_roots_keep_units_that_hardly_learn(X, monkeypatch):
     for block in (got[:-64, -64:] - R[:-64, -64:], got[-64:, :-64] - R[-64:, :-64]):
         assert float(block.norm() / R[:-64, -64:].norm()) <= 3e-6
     assert float((got - R).norm() / R.norm()) <= 3.3e-7
+
+
+def test_preconditioned_gradients_take_every_form_of_their_factors_where_they_are_measured(X, code_maps, monkeypatch):
+    """One matrix in vectors, as quantize_blockwise_diagreal returns it, with and without a diagonal, and factors given by
+    addresses: the same bits as stacks and tensors."""
+    import qtensor.functional as F
+    monkeypatch.setattr(X, "MEASURE_FROM", 0)
+    code = torch.from_numpy(code_maps[("linear-2", 4)]).cuda()
+    g = torch.Generator(device="cuda").manual_seed(8)
+    G, left, right = (torch.randn(*s, device="cuda", generator=g) for s in ((512, 768), (512, 512), (768, 768)))
+    for diag in (True, False):
+        flat, stacked = [], []
+        for mat in (left, right):
+            made = (F.quantize_blockwise_diagreal if diag else F.quantize_blockwise)(mat, code, mat.shape[0], blocksize=64, bits=4)
+            codes, absmax, d = made if diag else made + (None,)
+            assert absmax.dim() == 1
+            flat.append(X.Quantized(codes, absmax, d, mat.shape[0], 64, 4, code))
+            stacked.append(X.Quantized(codes[None], absmax[None], None if d is None else d[None], mat.shape[0], 64, 4, code))
+        want = X.precondition(G, *stacked)
+        assert torch.equal(X.precondition(G, *flat), want) and torch.equal(X.measure(flat[0]), X.measure(stacked[0]))
+        half = X.Quantized(flat[0].codes[None], flat[0].absmax, flat[0].diag, 512, 64, 4, code)          # (codes stacked, the rest not)
+        assert torch.equal(X.precondition(G, half, flat[1]), want)
+    listed = [X.PtrList(torch.tensor([t.data_ptr()], dtype=torch.int64, device="cuda"), (1,) + tuple(t.shape)) for t in (G, left, right)]
+    want = X.precondition(G[None], left[None], right[None])
+    assert torch.equal(X.precondition(*listed), want) and torch.equal(X.precondition(G[None], listed[1], right[None]), want)
