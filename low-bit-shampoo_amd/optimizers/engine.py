@@ -426,7 +426,7 @@ class ShampooBank:
                     # (an fp32 statistic is handed over as it is and keeps the ridge that the iteration adds in
                     # place, as in the reference: optimizers/shampoo1.py:198)
                     dense = X.load_stack(stat)
-                    roots = ComputePowerBatched(dense, 4, ridge_epsilon=self.matrix_eps, v0=start)
+                    roots = ComputePowerBatched(dense, 4, ridge_epsilon=self.matrix_eps, v0=start, stack=self.per_order[order])
                     X.store_stack(roots, target)
                     if rows is not None:
                         if isinstance(stat, X.DenseStack):

@@ -483,7 +483,8 @@ class ShampooBank2(ShampooBank):
                         L = self._statistic(order, self._rectified_basis(order, None if whole else index), rows=None if whole else index)
                         start = starts[order] if whole else starts[order].index_select(0, index)
                         # L is symmetric up to the rounding inside its diagonal tiles: half products are fine
-                        roots = ComputePowerBatched(L, 4, ridge_epsilon=self.matrix_eps, v0=start, symmetric=True)
+                        roots = ComputePowerBatched(L, 4, ridge_epsilon=self.matrix_eps, v0=start, symmetric=True,
+                                                    stack=self.per_order[order])
                     if rows is None:
                         X.store_stack(roots, self.precs[order].rows(part[0], part[1]))
                     else:

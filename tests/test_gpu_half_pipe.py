@@ -430,3 +430,26 @@ def test_preconditioned_gradients_take_every_form_of_their_factors_where_they_ar
     listed = [X.PtrList(torch.tensor([t.data_ptr()], dtype=torch.int64, device="cuda"), (1,) + tuple(t.shape)) for t in (G, left, right)]
     want = X.precondition(G[None], left[None], right[None])
     assert torch.equal(X.precondition(*listed), want) and torch.equal(X.precondition(G[None], listed[1], right[None]), want)
+
+
+@pytest.mark.parametrize("variant", [1, 2])
+def test_inverse_roots_of_a_part_have_the_bits_of_the_whole_stack(X, monkeypatch, variant):
+    """Ten matrices of order 512, measured as a stack and not in parts of four, or of the two of one parameter."""
+    import qtensor.functional as F
+    from optimizers.engine import ShampooBank
+    from optimizers.engine2 import ShampooBank2
+    monkeypatch.setattr(X, "MEASURE_FROM", 6 * 512 ** 3)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    grads = [torch.randn(512, 512, device="cuda", generator=g) for _ in range(5)]
+    v0 = {512: torch.rand(10, 512, device="cuda", generator=g) * 2 - 1}
+    make = ShampooBank if variant == 1 else lambda *a, **kw: ShampooBank2(*a, inv_root_mode=1, **kw)
+    code = F.create_linear_map(True, 4, 2)
+    roots = {}
+    for name, part, only in (("whole", 10, None), ("parts", 4, None), ("chosen", 10, [1])):
+        bank = make([torch.nn.Parameter(p) for p in grads], {"linear-2": code}, "linear-2", prec_maxorder=1024)
+        bank.NEWTON_PART_BYTES = part * 4 * 512 * 512
+        bank.add_statistics(grads)
+        bank.compute_preconditioners(v0=v0, only=only)
+        roots[name] = X.load_stack(bank.precs[512])
+    assert torch.equal(roots["parts"], roots["whole"])
+    assert torch.equal(roots["chosen"][[1, 6]], roots["whole"][[1, 6]])
