@@ -55,20 +55,19 @@ template <> struct Vec4Store<uint16_t> {
 // their diagonal entries are the same for the whole wave and cost a scalar comparison per store.  kDiagAny: every lane
 // walks along rows and columns, work that waits beside the loads: 8192 x 8192 with codes that come from memory, 4 bits to
 // fp32 97 us, few 61 (without a diagonal 58), to bf16 54 us at best, few 34.  With codes that the last-level cache still
-// holds the slower walk paces the stores, any 45 us and few 46 (12032 x 12032: 93 and 96, 8 bits 100 and 108): the codes of a
-// preconditioner that is used once per step come from memory.
+// holds, as right behind their quantizer, the walk of kDiagAny costs nothing (see the launch).
 enum DiagKind : int { kDiagNone = 0, kDiagAny = 1, kDiagFew = 2 };
-template <typename T, int BITS, int DIAG, bool STREAM>
-__global__ __launch_bounds__(kFlatThreads) void dequantize_flat_kernel(
+template <typename T, int BITS, int DIAG, bool STREAM, int THREADS = kFlatThreads>
+__global__ __launch_bounds__(THREADS) void dequantize_flat_kernel(
     const uint8_t *__restrict__ q, const float *__restrict__ code, uint32_t n_super, uint32_t bs_shift,
     FastDiv row_div, FastDiv order_div, const float *__restrict__ absmax, const float *__restrict__ diag, T *__restrict__ out) {
     constexpr int NCODE = 1 << BITS;
-    constexpr int kWaves = kFlatThreads / 64;
+    constexpr int kWaves = THREADS / 64;
     constexpr int CODE_VECS = BITS == 4 ? 1 : 2;            // uint4 loads per lane per step
     __shared__ float s_code[NCODE];
     __shared__ uint4 s_stage[kWaves][CODE_VECS * 64];
     __shared__ float s_scale[kWaves][32];
-    for (int i = threadIdx.x; i < NCODE; i += kFlatThreads) s_code[i] = code[i];
+    for (int i = threadIdx.x; i < NCODE; i += THREADS) s_code[i] = code[i];
     __syncthreads();
 
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
@@ -350,6 +349,11 @@ void dequantize_dispatch(const uint8_t *q, const float *code, int order_i, const
         // bf16, whose look-ups per byte written are twice as many, want more waves to hide them behind: 4096 x 4096 fp32
         // with its diagonal 15.4 us with three, 13.9 with six; bf16 8 bits 14.6 with three, 11.0 with six and with ten, 4
         // bits 14.6, 10.2, 9.5; 12032 x 12032 bf16 80, 59, 61.
+        // With the exact diagonal by wave-uniform places (kDiagFew) 4-bit codes do best with five waves per unit, each a workgroup
+        // of its own.  us for codes from memory and right behind their quantizer, any place with 3 x 2 waves, few with 3 x 2, few
+        // with 5 x 1: 8192 x 8192 104 70 68 and 48 50 47, 10240 x 10240 157 106 108 and 70 74 70, 12032 x 12032 217 147 141 and 95 100
+        // 93.  8 bits the same to the noise for both of few, 8192 x 8192 114 81 82 and 51 54 54, 10240 x 10240 169 126 132 and 76 81 80,
+        // 12032 x 12032 233 174 178 and 180 117 115: two to seven percent lost where 64 to 110 MB of codes have just been written.
         const bool streams = total >= (1u << 25);
         const dim3 grid(capped_grid(blocks, sizeof(T) == 2 ? (streams ? 6 : 10) : streams ? 3 : 6));
         constexpr int ANY = DIAG ? kDiagAny : kDiagNone, FEW = DIAG ? kDiagFew : kDiagNone;
@@ -357,8 +361,12 @@ void dequantize_dispatch(const uint8_t *q, const float *code, int order_i, const
 #define QT_DEQUANT_FLAT(KIND, STREAM)                                                                                                   \
         hipLaunchKernelGGL((dequantize_flat_kernel<T, BITS, KIND, STREAM>), grid, dim3(kFlatThreads), 0, stream, q, code, n_super,       \
                            (uint32_t)bs_shift, make_fastdiv(order / 4), make_fastdiv(order), absmax, diag, out)
+        constexpr bool ONE = DIAG && BITS == 4 && sizeof(T) == 4;
         if (order >= (uint32_t)kSuper) {
-            if (streams) QT_DEQUANT_FLAT(FEW, true);
+            if (streams)
+                hipLaunchKernelGGL((dequantize_flat_kernel<T, BITS, FEW, true, ONE ? 64 : kFlatThreads>), ONE ? dim3(capped_grid(n_super, 5)) : grid,
+                                   dim3(ONE ? 64 : kFlatThreads), 0, stream, q, code, n_super, (uint32_t)bs_shift, make_fastdiv(order / 4),
+                                   make_fastdiv(order), absmax, diag, out);
             else QT_DEQUANT_FLAT(FEW, false);
         } else if (streams) QT_DEQUANT_FLAT(ANY, true);
         else QT_DEQUANT_FLAT(ANY, false);

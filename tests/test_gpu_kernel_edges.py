@@ -409,7 +409,8 @@ def test_general_quantizer_on_either_side_of_the_size_from_which_it_has_a_bucket
         assert np.array_equal(q.absmax[b].cpu().numpy(), want[1], equal_nan=True) and np.array_equal(q.diag[b].cpu().numpy(), want[2], equal_nan=True)
 
 
-@pytest.mark.parametrize("order,batch,bits,blocksize", [(1984, 1, 4, 64), (2048, 3, 4, 64), (2048, 1, 8, 2048), (2112, 2, 8, 64), (4096, 1, 4, 256), (5888, 1, 8, 256)])
+@pytest.mark.parametrize("order,batch,bits,blocksize", [(1984, 1, 4, 64), (2048, 3, 4, 64), (2048, 1, 8, 2048), (2112, 2, 8, 64), (4096, 1, 4, 256), (5888, 1, 8, 256),
+                                                       (5824, 1, 4, 64), (2112, 8, 4, 64)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_flat_dequantizer_puts_the_diagonal_where_it_belongs_in_wide_matrices(order, batch, bits, blocksize, dtype):
     """Orders on either side of the step's 2048 elements, launches on either side of the streaming one, segments that are zero
