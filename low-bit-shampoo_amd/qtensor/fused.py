@@ -416,7 +416,7 @@ def matvec(mats: Tensor, v: Tensor) -> Tensor:
 def precondition(G: Tensor, left, right, out: Optional[Tensor] = None) -> Tensor:
     """deq(left) @ G @ deq(right) with both factors expanded inside the products.
     left / right: `Quantized` or dense fp32 matrices."""
-    if not worth_measuring(left, G, right):
+    if not worth_measuring(left, G, right, LONE_CALL):
         tmp = gemm(left, G)
         return gemm(tmp, right, out=out)
     tops = torch.zeros(4, 2, 1 if G.dim() == 2 else G.shape[0], device=G.device)
@@ -425,22 +425,30 @@ def precondition(G: Tensor, left, right, out: Optional[Tensor] = None) -> Tensor
     return gemm(tmp, right, out=out, amax=(tops[3], tops[2]))
 
 
-def worth_measuring(left, G, right) -> bool:
+def worth_measuring(left, G, right, times: float = 1.0) -> bool:
     """Whether the largest elements of the operands of deq(left) @ G @ deq(right) are worth looking up: both products on the
-    half pipe (whole lines of k, 256 at least) save more than the look-up and the clearing of its results take: two launches,
-    8 us of the device and 20 of the host (768 x 3072 by itself 145 -> 133 us; half as much work gains nothing)."""
+    half pipe save more than the look-up and the clearing of its results take: two launches, 8 us of the device and
+    20 of the host.  times: by how much the caller's line lies above
+    `worth_measuring_for`'s, which is that of callers who queue their launches (a bank's groups: what the host does is
+    hidden there)."""
     m, n = G.shape[-2:]
     batch = 1 if G.dim() == 2 else G.shape[0]
-    return worth_measuring_for(batch * m * n * (m + n), m, n) and all(
+    return worth_measuring_for(batch * m * n * (m + n) / times, m, n) and all(
         q.flat if isinstance(q, Quantized) else isinstance(q, PtrList) or q.stride(-1) == 1 for q in (left, right))
 
 
-def worth_measuring_for(multiply_adds: int, *k: int) -> bool:
-    """The same for products of so much work in all, over sums of these lengths."""
+def worth_measuring_for(multiply_adds: float, *k: int) -> bool:
+    """The same for products of so much work in all, over sums of these lengths (256 at least)."""
     return multiply_adds >= MEASURE_FROM and all(x >= 256 and x % 32 == 0 for x in k) and gemm_pipe() == "split"
 
 
 MEASURE_FROM = 1 << 33
+# A call that finds the device idle has nothing to hide the look-up and the host behind.  us on the split and measured,
+# operands out of the caches, multiply-adds in 2^33: 1.05 768 x 3072 182 and 191; 1.5 1024 x 3072 225 and 215; 2.0 1024 x 1024 by
+# 8 250 and 226; 2.5 1536 x 3072 332 and 304, 512 x 2048 by 8 291 and 260; 6.75 3072 x 3072 926 and 711.  Between 1.2 and 2 it is
+# one or the other by shape, and with 20 us less on the host (a look-up's sources packed by hand) it still was: 1.5 512 x
+# 512 by 48 215 and 224, 2.0 2048 x 2048 270 and 235.
+LONE_CALL = 2.5
 
 
 def gram(G: Tensor, axis: int, *, stat=None, beta=0.0, alpha=1.0, out: Optional[Tensor] = None) -> Tensor:

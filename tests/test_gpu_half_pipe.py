@@ -220,13 +220,16 @@ def test_half_pipe_with_a_quantized_factor(X, code_maps, bits, bs, name, diag):
 
 
 def test_preconditioned_gradients_look_their_operands_up_where_it_pays(X, code_maps):
+    """Whole products on either side of the line, which is a higher one for a call by itself than inside a bank."""
     code = torch.from_numpy(code_maps[("linear-2", 4)]).cuda()
     g = torch.Generator(device="cuda").manual_seed(1)
-    for m, n, batch in ((768, 3072, 1), (256, 256, 3)):
+    for m, n, batch in ((1536, 3072, 1), (768, 3072, 1), (256, 256, 3)):
         made = [torch.randn(batch, k, k, device="cuda", generator=g) * 0.02 + torch.eye(k, device="cuda") for k in (m, n)]
         left, right = (X.quantize_stack(t, X.empty_quantized(batch, t.shape[1], 64, 4, code, True)) for t in made)
         G = torch.randn(batch, m, n, device="cuda", generator=g)
-        assert X.worth_measuring(left, G, right) == (m == 768)
+        assert X.worth_measuring(left, G, right) == (m >= 768) and X.worth_measuring(left, G, right, X.LONE_CALL) == (m == 1536)
+        if m == 768:                                     # not looked up: the very bits of the products without amax
+            assert torch.equal(X.precondition(G, left, right), X.gemm(X.gemm(left, G), right))
         want = X.dequantize_stack(left).double() @ G.double() @ X.dequantize_stack(right).double()
         assert float((X.precondition(G, left, right).double() - want).norm() / want.norm()) <= 1e-6
     left = X.quantize_stack(made[0], X.empty_quantized(batch, 256, 64, 4, code, True))
