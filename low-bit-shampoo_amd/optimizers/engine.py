@@ -400,7 +400,9 @@ class ShampooBank:
         for g in self.groups:
             if only is not None and not any(pi in only for pi in g.param_index):
                 continue
-            if X.worth_measuring_for(len(g) * g.bm * g.bn * (g.bm + g.bn) // 2, g.bm, g.bn):
+            # (re-encoding tiles are 128 x 128 on the half pipe: order 320 135 us on the split, with 64 x 64 tiles, and 190, 512
+            # 120 and 117, 640 120 and 126, 768 106 and 82, before a look-up of 23 for both sides)
+            if X.worth_measuring_for(len(g) * g.bm * g.bn * (g.bm + g.bn) // 2, g.bm, g.bn, least=768):
                 jobs.append(both(g))
             else:
                 jobs += [job(g, 0), job(g, 1)]

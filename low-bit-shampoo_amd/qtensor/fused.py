@@ -427,19 +427,24 @@ def precondition(G: Tensor, left, right, out: Optional[Tensor] = None) -> Tensor
 
 def worth_measuring(left, G, right, times: float = 1.0) -> bool:
     """Whether the largest elements of the operands of deq(left) @ G @ deq(right) are worth looking up: both products on the
-    half pipe save more than the look-up and the clearing of its results take: two launches, 8 us of the device and
-    20 of the host.  times: by how much the caller's line lies above
+    half pipe save more than the look-up and the clearing of its results take: two launches, 8 us of the device and more
+    where there are more matrices, and 20 of the host.  times: by how much the caller's line lies above
     `worth_measuring_for`'s, which is that of callers who queue their launches (a bank's groups: what the host does is
-    hidden there)."""
+    hidden there).
+
+    Only where sums are long: what a product saves grows with rows + columns, the look-up with the elements.  1.2 2^33
+    multiply-adds a product, us on the split and on the half pipe, left and right: order 256 168 and 149, 170 and 194
+    (look-ups 70); 384 162 and 131, 164 and 170; 512 147 and 107, 141 and 125 (58: nothing gained); 640 175 and 122, 170 and
+    139; 768 159 and 109, 174 and 119."""
     m, n = G.shape[-2:]
     batch = 1 if G.dim() == 2 else G.shape[0]
-    return worth_measuring_for(batch * m * n * (m + n) / times, m, n) and all(
+    return m + n > 1024 and worth_measuring_for(batch * m * n * (m + n) / times, m, n, least=512) and all(
         q.flat if isinstance(q, Quantized) else isinstance(q, PtrList) or q.stride(-1) == 1 for q in (left, right))
 
 
-def worth_measuring_for(multiply_adds: float, *k: int) -> bool:
-    """The same for products of so much work in all, over sums of these lengths (256 at least)."""
-    return multiply_adds >= MEASURE_FROM and all(x >= 256 and x % 32 == 0 for x in k) and gemm_pipe() == "split"
+def worth_measuring_for(multiply_adds: float, *k: int, least: int = 256) -> bool:
+    """The same for products of so much work in all, over sums of these lengths, of which the shortest has to be `least`."""
+    return multiply_adds >= MEASURE_FROM and all(x >= least and x % 32 == 0 for x in k) and gemm_pipe() == "split"
 
 
 MEASURE_FROM = 1 << 33

@@ -237,9 +237,33 @@ def test_preconditioned_gradients_look_their_operands_up_where_it_pays(X, code_m
     assert flat.shape == (256, 256)
 
 
+def test_short_sums_are_not_looked_up(X, code_maps, monkeypatch):
+    """Products over short sums gain less than the look-up takes, whatever the number of matrices: preconditioned gradients
+    up to 512 x 512, statistics below order 768 (re-encoded) and 512 (added to in fp32)."""
+    import qtensor.functional as F
+    from optimizers.engine import ShampooBank
+    from optimizers.engine2 import ShampooBank2
+    monkeypatch.setattr(X, "MEASURE_FROM", 0)
+    code = torch.from_numpy(code_maps[("linear-2", 4)]).cuda()
+    looked = []
+    into = X.amax_into
+    monkeypatch.setattr(X, "amax_into", lambda *a, **kw: (looked.append(a), into(*a, **kw)))
+    for m, n, expect in ((256, 256, False), (512, 512, False), (384, 1024, False), (512, 576, True)):
+        left, right = (X.quantize_stack(torch.eye(k, device="cuda")[None], X.empty_quantized(1, k, 64, 4, code, True)) for k in (m, n))
+        del looked[:]
+        X.precondition(torch.randn(1, m, n, device="cuda"), left, right)
+        assert bool(looked) == expect
+    for kind, order, expect in ((ShampooBank, 512, False), (ShampooBank, 768, True), (ShampooBank2, 448, False), (ShampooBank2, 512, True)):
+        bank = kind([torch.nn.Parameter(torch.randn(order, order, device="cuda"))], {"linear-2": F.create_linear_map(True, 4, 2)}, "linear-2",
+                    prec_maxorder=1024)
+        del looked[:]
+        bank.add_statistics([torch.randn(order, order, device="cuda")])
+        assert any(isinstance(t, X.PtrList) for call in looked for t, _ in call) == expect
+
+
 def test_matrices_that_are_left_out_are_not_looked_at(X, monkeypatch):
-    """Skip flags of the look-up itself, and a bank with a parameter whose gradient is missing: its storage (here 512 floats
-    for a 512 x 512 matrix) stands in the address tables and must not be read."""
+    """Skip flags of the look-up itself, and a bank with a parameter whose gradient is missing: its storage (here 768 floats
+    for a 768 x 768 matrix) stands in the address tables and must not be read."""
     import qtensor.functional as F
     from optimizers.engine import ShampooBank
     from optimizers.engine2 import ShampooBank2
@@ -251,10 +275,10 @@ def test_matrices_that_are_left_out_are_not_looked_at(X, monkeypatch):
     monkeypatch.setattr(X, "MEASURE_FROM", 0)
     code = F.create_linear_map(True, 4, 2)
     g = torch.Generator(device="cuda").manual_seed(3)
-    present = torch.randn(512, 512, device="cuda", generator=g)
-    absent = torch.nn.Parameter(torch.randn(1, 512, device="cuda", generator=g).expand(512, 512))
-    assert absent.untyped_storage().nbytes() == 4 * 512
-    grad = torch.randn(512, 512, device="cuda", generator=g)
+    present = torch.randn(768, 768, device="cuda", generator=g)
+    absent = torch.nn.Parameter(torch.randn(1, 768, device="cuda", generator=g).expand(768, 768))
+    assert absent.untyped_storage().nbytes() == 4 * 768
+    grad = torch.randn(768, 768, device="cuda", generator=g)
     for kind in (ShampooBank, ShampooBank2):
         banks = [kind(params, {"linear-2": code}, "linear-2", prec_maxorder=1024)
                  for params in ([torch.nn.Parameter(present), absent], [torch.nn.Parameter(present)])]
@@ -262,12 +286,12 @@ def test_matrices_that_are_left_out_are_not_looked_at(X, monkeypatch):
             bank.add_statistics(grads, only=[0])
         if kind is ShampooBank:                          # the statistics of the parameter that is there: rows 0, 2 and 0, 1
             for part in ("codes", "absmax", "diag"):
-                both, alone = (getattr(bank.stats[512], part) for bank in banks)
+                both, alone = (getattr(bank.stats[768], part) for bank in banks)
                 assert torch.equal(both[[0, 2]], alone)
         # both with the same roots, so that the directions can be compared (products without skip flags are cut along k)
         for bank in banks:
-            for at in range(0, bank.precs[512].batch, bank.precs[512].batch // 2):
-                X.quantize_stack(torch.eye(512, device="cuda")[None] + 0.01 * present[None], bank.precs[512].rows(at, 1))
+            for at in range(0, bank.precs[768].batch, bank.precs[768].batch // 2):
+                X.quantize_stack(torch.eye(768, device="cuda")[None] + 0.01 * present[None], bank.precs[768].rows(at, 1))
         got, want = (bank.preconditioned_grads(grads, only=[0]) for bank, grads in zip(banks, ([grad, None], [grad])))
         assert got[1] is None and float((got[0] - want[0]).norm() / want[0].norm()) <= 1e-6
 
