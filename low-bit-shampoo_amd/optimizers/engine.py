@@ -330,10 +330,10 @@ class ShampooBank:
         self._write_grad_tables(grads)
 
     # The coupled Newton iteration holds ten fp32 stacks of what it works on (two copies each of the root, the
-    # iterate and the iteration matrix, two powers, the input, the result): a stack goes through it in parts of
+    # iterate and its deviation from the identity, two powers, the input, the result): a stack goes through it in parts of
     # at most this many bytes, one after the other, so that the iteration of a whole model takes ten times this
-    # much scratch and not ten times its largest stack (ViT-B/32: 70.1 ms per step with inverse roots and 1.8 GiB of
-    # scratch, against 68.8 ms and 4.2 GiB with whole stacks).  (A part still is dozens of matrices: every product launch
+    # much scratch and not ten times its largest stack (ViT-B/32: 62.1 ms per step with inverse roots and 1.7 GiB of
+    # scratch, against 59.0 ms and 3.9 GiB with whole stacks).  (A part still is dozens of matrices: every product launch
     # has thousands of tiles; the bits of a matrix's root do not depend on how its stack is cut.)
     NEWTON_PART_BYTES = 160 << 20
     NEWTON_SIDE_BY_SIDE = True                   # the orders' iterations run side by side on the side streams (False: one after the other)
