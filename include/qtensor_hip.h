@@ -394,6 +394,41 @@ void qtensor_hip_solve_upper_right_batched(const float *q, const float *u, float
  * fixed summation order: the matrix-vector product of the power iteration that scales the ridge term of the inverse
  * roots (torch.mv per matrix and round in the reference: optimizers/matrix_functions.py:42). */
 void qtensor_hip_matvec_batched(const float *a, const float *v, float *out, int n, int batch, qtensor_stream_t stream);
+/* The step of that power iteration behind a product (optimizers/matrix_functions.py:36-46): product [batch, n] = A u;
+ * quotient = u . product, change = |quotient - value|, value = quotient, u = product / |product|, for every vector whose
+ * change is above tolerance; the others are left alone.  first != 0: value = 0, change = 1, u = product / |product|, whatever
+ * they held.  Sums in double precision. */
+void qtensor_hip_power_step_batched(const float *product, float *u, float *value, float *change, int n, int batch, float tolerance,
+                                    int first, qtensor_stream_t stream);
+
+/* ---- the coupled Newton iteration between its products (optimizers/matrix_functions.py:100-141) ----
+ * Start: mats [batch, n, n] += ridge * top[b] on the diagonal, in place; z = (1 + p) / (2 |mats|_F), c = z^(1/p);
+ * M = z mats, E = M - I, R = c (I - E / p) (the root after the first round, should that be accepted), first_root = c,
+ * err (zeroed by the caller) = max |E|; fine (optional, zeroed by the caller; n a multiple of 4): raised to the fineness of
+ * E and M (qtensor_gemm_fineness).  partial: scratch of batch * ceil(n / 8) doubles. */
+void qtensor_hip_newton_first_batched(float *mats, const float *top, float ridge, int p, int n, int batch, double *partial, float *M,
+                                      float *E, float *R, float *first_root, float *err, float *fine, qtensor_stream_t stream);
+/* Stopping rules: new_err NULL before the first round, else max |E| after a round.  A round is accepted unless new_err > 1.2 err;
+ * a matrix is done once a round of it is not, at err <= tolerance, or after `iterations` rounds.  All device arrays of
+ * [batch]; rounds counts the accepted ones, side flips with each (0: the state lies in the buffers of even place).
+ * tables [6][batch]: addresses of (root, iterate, deviation) x (state, other one) of every matrix, from the six buffers'
+ * addresses (root 0, root 1, iterate 0, ...) and the bytes between two matrices.  done holds 0 or 1, as the products'
+ * skip flags.  bound_m (optional): 1 + the last error.  root_bound, root_fine (optional, written before the first round): bound
+ * and fineness of R from those of E (first_fine) and step = -1 / p. */
+typedef struct {
+    int batch, iterations;
+    float tolerance, step;
+    float *err;
+    int *done, *side, *rounds;
+    const float *first_root, *first_fine;
+    float *root_bound, *root_fine;
+    long long *tables;
+    long long buffers[6], stride;
+} qtensor_newton_state;
+void qtensor_hip_newton_decide(const qtensor_newton_state *state, const float *new_err, float *bound_m, qtensor_stream_t stream);
+/* out[b] = first_root[b] I where rounds[b] is 0, else r1[b] where side[b] is not 0, else r0[b]; out may be r0 or r1. */
+void qtensor_hip_newton_result_batched(const float *r0, const float *r1, const int *side, const int *rounds, const float *first_root,
+                                       float *out, int n, int batch, qtensor_stream_t stream);
 
 /* ---- the elementwise end of an optimizer step for all parameters at once -------------------------
  * Replaces the per-parameter torch calls of the reference's step():

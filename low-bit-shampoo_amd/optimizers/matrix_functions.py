@@ -20,6 +20,7 @@ root against the same iteration in float64 (4-bit statistics of condition 20, ha
 split for order 128): order 128 3.6e-7 -> 1.2e-7, 256 6.9e-7 -> 1.5e-7, 768 9.1e-7 -> 2.3e-7,
 1024 1.1e-6 -> 2.8e-7; on the bf16 split the same but for 4 % (from 4.8e-7 at 256, 9.5e-7 at 1024).
 """
+import ctypes as ct
 from typing import Optional
 
 import torch
@@ -106,20 +107,21 @@ def PowerIterBatched(mats, error_tolerance=1e-6, num_iters=10, v0=None):
     """PowerIter for a stack [B, n, n]; every matrix follows its own stopping rule (entries that
     have converged are frozen).  v0: optional [B, n] or [n] start vectors.  Returns the [B]
     eigenvalue estimates.  No host synchronisation.
-    Sums are taken in float64 and rounded: the order in which torch adds up depends on the number of matrices."""
+    Sums are taken in float64 and rounded, so that they do not depend on the number of matrices."""
     from qtensor import fused as X
     B, n, _ = mats.shape
     if v0 is None:
         v = torch.rand(B, n, device=mats.device) * 2 - 1
     else:
         v = v0.to(mats.device).expand(B, n).clone()
+    if X.on_matrix_cores(mats) and mats.is_contiguous():            # the library's kernels: two launches a round
+        return X.power_iteration(mats, v.contiguous(), error_tolerance, num_iters)
     value = torch.zeros(B, device=mats.device)
     change = torch.ones(B, device=mats.device)
-    own = X.on_matrix_cores(mats) and mats.is_contiguous()          # the stack-wide matrix-vector kernel of the library
     for _ in range(num_iters):
         active = change > error_tolerance
         u = v / torch.linalg.vector_norm(v, dim=1, keepdim=True, dtype=torch.float64).float()
-        w = X.matvec(mats, u.contiguous()) if own else torch.bmm(mats, u.unsqueeze(2)).squeeze(2)
+        w = torch.bmm(mats, u.unsqueeze(2)).squeeze(2)
         quotient = (u * w).sum(dim=1, dtype=torch.float64).float()
         change = torch.where(active, (quotient - value).abs(), change)
         value = torch.where(active, quotient, value)
@@ -148,58 +150,47 @@ def ComputePowerBatched(mats, p=4, iter_count=10, error_tolerance=1e-6, ridge_ep
         raise ValueError("ComputePowerBatched supports p in 1, 2, 4, ..., 32")
     B, n, _ = mats.shape
     dev = mats.device
-    eye = torch.eye(n, device=dev)
     if n == 1:
-        res = eye.expand(B, 1, 1).clone()
+        res = torch.ones(B, 1, 1, device=dev)
         return res if out is None else out.copy_(res)
     w = -1.0 / p
-    top = PowerIterBatched(mats, v0=v0)
-    mats.diagonal(dim1=1, dim2=2).add_((ridge_epsilon * top).unsqueeze(1))
-    # (the norm: column by column in the library's fixed order, 99 x 1024 x 1024 in 60 us; in float64 as a whole 650)
-    squares = X.column_dots(mats, mats) if n % 64 == 0 and mats.is_contiguous() else mats.flatten(1).square()
-    z = (1 + p) / (2 * squares.sum(dim=1, dtype=torch.float64).sqrt().float())                          # [B]
-    R = [torch.zeros(B, n, n, device=dev), torch.empty(B, n, n, device=dev)]
-    first_root = torch.pow(z, 1.0 / p)                                       # the root starts as this multiple of the identity
-    R[0].diagonal(dim1=1, dim2=2).copy_(first_root.unsqueeze(1).expand(B, n))
-    M = [mats * z.view(B, 1, 1), torch.empty(B, n, n, device=dev)]
-    E = [M[0] - eye, torch.empty(B, n, n, device=dev)]
-    F = [torch.empty(B, n, n, device=dev) for _ in range(2)]                  # T^2 - I, T^4 - I, ... in turn
-    err = E[0].abs().amax(dim=(1, 2))
-    rounds = torch.zeros(B, dtype=torch.int32, device=dev)
-    done = (err <= error_tolerance)
-
-    # which of the two buffers currently holds matrix b's accepted R / M / E: pointer tables on
-    # the device, swapped per matrix when a round is accepted
-    def table(pair):
-        step = pair[0].stride(0) * 4
-        return [torch.arange(B, device=dev, dtype=torch.int64) * step + t.data_ptr() for t in pair]
-
-    R_ptr, M_ptr, E_ptr = table(R), table(M), table(E)
-    side = torch.zeros(B, dtype=torch.bool, device=dev)                     # False: buffer 0 holds the state
+    work = mats if mats.is_contiguous() else mats.contiguous()
+    top = PowerIterBatched(work, v0=v0)
+    R, M, E, F = [[torch.empty(B, n, n, device=dev) for _ in range(2)] for _ in range(4)]     # F: T^2 - I, T^4 - I, ... in turn
     # How large the iterates' elements are, for the pipe that wants to know: the bounds of E and M follow from err = max |E|,
-    # the rest is looked at by the launches that write them (both of E and M by one).  Small stacks are
-    # bound by the host, which this costs 40 us a round (statistics of convolutions of width 32: 29 ms without, 33 with).
+    # the rest is looked at by the launches that write them (both of E and M by one).
     measured = X.worth_measuring_for((B if stack is None else stack) * n ** 3, n)
     squarings = p.bit_length() - 1
-    if measured:
-        first = torch.zeros(2, B, device=dev)
-        X.amax_into((M[0], first), (E[0], first))
-        found = torch.zeros(iter_count, 2 + squarings, 2, B, device=dev)     # per round: root, powers, E with M
-        top_e, top_m = (err, first[1]), (1 + err, first[1])
-        # of the root after the first round, c (I + w E): small pieces are c w times those of E
-        top_r = (first_root * (1 + abs(w) * err), first[1] / (abs(w) * first_root))
+    # errors before the first round and after each; what the rounds' products find (root, powers, E with M)
+    zeros = torch.zeros((iter_count + 2) * B + (2 * iter_count * (2 + squarings) * B if measured else 0), device=dev)
+    errors, first_fine = zeros[:(iter_count + 1) * B].view(-1, B), zeros[(iter_count + 1) * B:(iter_count + 2) * B]
+    found = zeros[(iter_count + 2) * B:].view(iter_count, 2 + squarings, 2, B) if measured else None
+    floats = torch.empty(5, B, device=dev)
+    first_root, err, top_m, root_bound, root_fine = floats
+    flags = torch.empty(3, B, dtype=torch.int32, device=dev)
+    done, side, rounds = flags
+    tables = torch.empty(6, B, dtype=torch.int64, device=dev)
+    X.newton_first(work, top, ridge_epsilon, p, M[0], E[0], R[1], first_root, errors[0], first_fine if measured else None)
+    if work is not mats:
+        mats.copy_(work)
+    err.copy_(errors[0])
+    state = X.NewtonState(B, iter_count, error_tolerance, w, err.data_ptr(), done.data_ptr(), side.data_ptr(), rounds.data_ptr(),
+                          first_root.data_ptr(), first_fine.data_ptr(), root_bound.data_ptr() if measured else None,
+                          root_fine.data_ptr(), tables.data_ptr(),
+                          (ct.c_longlong * 6)(*[t.data_ptr() for pair in (R, M, E) for t in pair]), 4 * n * n)
+
+    def decide(new_err):
+        X.F._call(X.F.lib.qtensor_hip_newton_decide, dev, ct.byref(state), None if new_err is None else new_err.data_ptr(),
+                  top_m.data_ptr())
+
+    # the buffer that holds matrix b's accepted R / M / E, and the other one: rewritten on the device after every round
+    Rc, Ro, Mc, Mo, Ec, Eo = [X.PtrList(table, (B, n, n)) for table in tables]
+    decide(None)
+    fine, top_r = first_fine, (root_bound, root_fine)
     for round_number in range(iter_count):
-        skip = done.to(torch.int32)
-        cur = lambda tab: torch.where(side, tab[1], tab[0])                   # noqa: E731
-        oth = lambda tab: torch.where(side, tab[0], tab[1])                   # noqa: E731
-        shape = (B, n, n)
-        Rc, Ro, Mc, Mo, Ec, Eo = [X.PtrList(which(tab), shape) for tab in (R_ptr, M_ptr, E_ptr) for which in (cur, oth)]
-        if round_number == 0:
-            # candidate root of the first round: c (I + w E), every matrix still in its first buffer
-            torch.mul(E[0], (w * first_root).view(B, 1, 1), out=R[1])
-            R[1].diagonal(dim1=1, dim2=2).add_(first_root.unsqueeze(1))
-        else:
-            X.gemm(Rc, Ec, addend=Rc, alpha=w, beta=1.0, out=Ro, skip=skip, symmetric=symmetric,        # candidate root
+        top_e = (errors[round_number], fine)
+        if round_number > 0:                       # (the first round's candidate root is there already)
+            X.gemm(Rc, Ec, addend=Rc, alpha=w, beta=1.0, out=Ro, skip=done, symmetric=symmetric,        # candidate root
                    **(dict(amax=(top_r, top_e), amax_out=found[round_number, 0]) if measured else {}))
             if measured:
                 top_r = found[round_number, 0]                               # (a rejected candidate ends its matrix's iteration)
@@ -208,20 +199,19 @@ def ComputePowerBatched(mats, p=4, iter_count=10, error_tolerance=1e-6, ridge_ep
         for square in range(1, 1 + squarings):
             dst = F[square % 2]
             after = found[round_number, square] if measured else None
-            X.gemm(power, power, addend=power, alpha=scale * scale, beta=2 * scale, out=dst, skip=skip, symmetric=symmetric,
+            X.gemm(power, power, addend=power, alpha=scale * scale, beta=2 * scale, out=dst, skip=done, symmetric=symmetric,
                    amax=(top, top) if measured else None, amax_out=after)
             power, scale, top = dst, 1.0, after
-        new_err = torch.zeros(B, device=dev)
-        X.gemm(power, Mc, addend=Mc, alpha=scale, beta=1.0, out=Mo, deviation=(Eo, new_err), skip=skip, symmetric=symmetric,
-               amax=(top, top_m) if measured else None, amax_out=found[round_number, 1 + squarings] if measured else None)
+        new_err = errors[round_number + 1]
+        X.gemm(power, Mc, addend=Mc, alpha=scale, beta=1.0, out=Mo, deviation=(Eo, new_err), skip=done, symmetric=symmetric,
+               amax=(top, (top_m, fine)) if measured else None, amax_out=found[round_number, 1 + squarings] if measured else None)
         if measured:
             fine = found[round_number, 1 + squarings, 1]
-            top_e, top_m = (new_err, fine), (1 + new_err, fine)
-        accept = (~done) & ~(new_err > err * 1.2)
-        side = side ^ accept
-        err = torch.where(accept, new_err, err)
-        rounds = rounds + accept.to(torch.int32)
-        done = done | ~accept | (err <= error_tolerance) | (rounds >= iter_count)
+        decide(new_err)
     _LAST_ROUNDS[n] = rounds                       # accepted rounds per matrix of the last stack of this order
-    res = torch.where(side.view(B, 1, 1), R[1], R[0])
-    return res if out is None else out.copy_(res)
+    res = R[0]
+    if out is not None and out.is_contiguous() and out.dtype == torch.float32 and out.device == dev and out.shape == R[0].shape:
+        res = out
+    X.F._call(X.F.lib.qtensor_hip_newton_result_batched, dev, R[0].data_ptr(), R[1].data_ptr(), side.data_ptr(), rounds.data_ptr(),
+              first_root.data_ptr(), res.data_ptr(), n, B)
+    return res if out is None or res is out else out.copy_(res)

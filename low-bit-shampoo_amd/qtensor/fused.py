@@ -413,6 +413,51 @@ def matvec(mats: Tensor, v: Tensor) -> Tensor:
     return out
 
 
+class NewtonState(ct.Structure):
+    _fields_ = [("batch", ct.c_int), ("iterations", ct.c_int), ("tolerance", ct.c_float), ("step", ct.c_float), ("err", ct.c_void_p),
+                ("done", ct.c_void_p), ("side", ct.c_void_p), ("rounds", ct.c_void_p), ("first_root", ct.c_void_p),
+                ("first_fine", ct.c_void_p), ("root_bound", ct.c_void_p), ("root_fine", ct.c_void_p), ("tables", ct.c_void_p),
+                ("buffers", ct.c_longlong * 6), ("stride", ct.c_longlong)]
+
+
+if F.lib is not None:
+    F.lib.qtensor_hip_power_step_batched.restype = None
+    F.lib.qtensor_hip_power_step_batched.argtypes = [ct.c_void_p] * 4 + [ct.c_int, ct.c_int, ct.c_float, ct.c_int, ct.c_void_p]
+    F.lib.qtensor_hip_newton_first_batched.restype = None
+    F.lib.qtensor_hip_newton_first_batched.argtypes = ([ct.c_void_p] * 2 + [ct.c_float, ct.c_int, ct.c_int, ct.c_int] + [ct.c_void_p] * 8)
+    F.lib.qtensor_hip_newton_decide.restype = None
+    F.lib.qtensor_hip_newton_decide.argtypes = [ct.POINTER(NewtonState), ct.c_void_p, ct.c_void_p, ct.c_void_p]
+    F.lib.qtensor_hip_newton_result_batched.restype = None
+    F.lib.qtensor_hip_newton_result_batched.argtypes = [ct.c_void_p] * 6 + [ct.c_int, ct.c_int, ct.c_void_p]
+
+
+def power_iteration(mats: Tensor, v0: Tensor, tolerance: float, rounds: int) -> Tensor:
+    """[B]: largest eigenvalues of the contiguous fp32 GPU stack mats [B, n, n] from the start vectors v0 [B, n]: two launches
+    a round, a matrix whose Rayleigh quotient has moved by no more than tolerance is left alone."""
+    B, n, _ = mats.shape
+    _stack(mats, "mats", (B, n, n)), _stack(v0, "v0", (B, n))
+    u, product, out = torch.empty_like(v0), v0, torch.empty(2, B, device=mats.device)
+    for r in range(rounds + 1):
+        F._call(F.lib.qtensor_hip_power_step_batched, mats.device, product.data_ptr(), u.data_ptr(), out[0].data_ptr(), out[1].data_ptr(),
+                n, B, tolerance, int(r == 0))
+        if r < rounds:
+            product = matvec(mats, u)
+    return out[0]
+
+
+def newton_first(mats: Tensor, top: Tensor, ridge: float, p: int, M: Tensor, E: Tensor, R: Tensor, first_root: Tensor, err: Tensor,
+                 fine: Optional[Tensor]) -> None:
+    """First iterates of the coupled Newton iteration (qtensor_hip_newton_first_batched); all stacks contiguous [B, n, n]."""
+    B, n, _ = mats.shape
+    for name, t in (("mats", mats), ("M", M), ("E", E), ("R", R)):
+        _stack(t, name, (B, n, n))
+    for name, t in (("top", top), ("first_root", first_root), ("err", err)) + ((("fine", fine),) if fine is not None else ()):
+        _stack(t, name, (B,))
+    partial = torch.empty(B * -(-n // 8), dtype=torch.float64, device=mats.device)
+    F._call(F.lib.qtensor_hip_newton_first_batched, mats.device, mats.data_ptr(), top.data_ptr(), ridge, p, n, B, partial.data_ptr(),
+            M.data_ptr(), E.data_ptr(), R.data_ptr(), first_root.data_ptr(), err.data_ptr(), None if fine is None else fine.data_ptr())
+
+
 def precondition(G: Tensor, left, right, out: Optional[Tensor] = None) -> Tensor:
     """deq(left) @ G @ deq(right) with both factors expanded inside the products.
     left / right: `Quantized` or dense fp32 matrices."""

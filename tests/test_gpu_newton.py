@@ -171,3 +171,33 @@ def test_inverse_roots_against_the_same_iteration_in_float64(n, measured, monkey
             T = 1.25 * eye - 0.25 * M
             R, M = R @ T, (T @ T) @ (T @ T) @ M
         assert float((got[b].double() - R).norm() / R.norm()) <= 3.3e-7, n
+
+
+@pytest.mark.parametrize("n", [2, 7, 33, 130, 288])
+@pytest.mark.parametrize("strided", [False, True])
+def test_start_stopping_rules_and_result_of_a_stack(n, strided):
+    """Orders that no band of eight rows or quad of columns divides; in one stack a matrix that goes all rounds, one that is
+    done before the first, one whose first round is rejected (indefinite: the root is then the multiple of the identity that
+    the iteration starts from) and one of NaN.  Ridge in place, `out` taken, start vectors per matrix.  Ten rounds of fp32
+    products of order n: 1e-5 as for the well-conditioned matrices above."""
+    mats, v0 = psd_stack(4, n, 1.0, seed=n)
+    mats[1] = 0.5 * torch.eye(n)
+    mats[2] = torch.diag(torch.linspace(-1.0, 1.0, n))
+    mats[3, 0, 0] = float("nan")
+    eps = 1e-6
+    given = torch.full((4, n, n + 3), 7.0)[:, :, :n].cuda() if strided else torch.empty(4, n, n, device="cuda")
+    given.copy_(mats)
+    out = torch.full((4, n, n), 7.0, device="cuda")
+    got = ComputePowerBatched(given, 4, ridge_epsilon=eps, v0=v0, out=out)
+    assert got is out
+    for b in range(3):
+        top = power_iteration(mats[b], v0[b])
+        ridged = mats[b] + eps * float(top) * torch.eye(n)
+        assert float((given[b].cpu() - ridged).abs().max()) <= 1e-6 * float(ridged.abs().max())
+        want = ComputePower(mats[b].clone(), 4, ridge_epsilon=eps, v0=v0[b])
+        assert float((got[b].cpu() - want).norm() / want.norm()) <= 1e-5, (n, b)
+    assert bool(torch.isnan(got[3]).any())
+    again = ComputePowerBatched(mats.cuda(), 4, ridge_epsilon=eps, v0=v0)
+    assert torch.equal(again[:3], got[:3])                                     # the same bits, strided or not
+    part = ComputePowerBatched(mats[1:3].cuda(), 4, ridge_epsilon=eps, v0=v0[1:3])
+    assert torch.equal(part, got[1:3])                                         # and of a part of the stack
