@@ -1,5 +1,6 @@
 #!/usr/bin/env bash
-# Builds qtensor/libqtensor_hip.so for gfx950 (cross-compiles without a GPU).
+# Builds qtensor/libqtensor_hip.so for gfx950 (cross-compiles without a GPU) and qtensor/_direct.so, the native host side
+# of a quantize or dequantize call (plain C++ against torch's headers).
 # Sources compile in parallel to objects under csrc/build/, then link.
 set -euo pipefail
 here="$(cd "$(dirname "${BASH_SOURCE[0]}")" && pwd)"
@@ -20,6 +21,14 @@ for src in "${here}"/qt_*.hip; do
   "${HIPCC}" "${FLAGS[@]}" "$@" -c "${src}" -o "${o}" &
   pids+=($!)
 done
+# (beside the library that it is bound to: none for a library built somewhere else)
+if [[ -z "${QT_OUT:-}" ]]; then
+  mapfile -t where < <(python3 -c 'import os, sysconfig, torch; print(os.path.dirname(torch.__file__)); print(sysconfig.get_paths()["include"])')
+  g++ -O2 -std=c++17 -shared -fPIC -Wall -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -I"${where[0]}/include" -I"${where[0]}/include/torch/csrc/api/include" \
+    -I"${HIP_PATH:-/opt/rocm}/include" -I"${where[1]}" "${here}/direct_call.cpp" -o "${here}/../qtensor/_direct.so" \
+    -L"${where[0]}/lib" -lc10 -lc10_hip -ltorch_cpu -ltorch_hip -ltorch -ltorch_python -Wl,-rpath,"${where[0]}/lib" &
+  pids+=($!)
+fi
 for p in "${pids[@]}"; do wait "${p}"; done
 "${HIPCC}" --offload-arch=gfx950 -shared -fPIC "${objs[@]}" -o "${out}"
 echo "built ${out}"

@@ -69,7 +69,18 @@ if lib is not None:
         return table
 
     _STREAM_FN = _bind_stream_variants()
+
+    # the same calls with their host side in native code (csrc/direct_call.cpp): what it does not take goes the way below
+    try:
+        from qtensor import _direct
+    except ImportError:
+        _direct = None                              # not built: the same launches from Python
+    if _direct is not None:
+        _direct.bind([ct.cast(fn, ct.c_void_p).value for fn in
+                      [_STREAM_FN[(kind, bits, slot, diag)] for kind in ("quantize", "dequantize") for bits in (4, 8)
+                       for slot in (0, 1) for diag in (False, True)] + [lib.qtensor_hip_last_error, lib.qtensor_hip_last_error_string]])
 else:
+    _direct = None
     lib_quan = {}
     lib_dequan = {}
     lib_quan_diagreal = {}
@@ -248,8 +259,8 @@ def quantize_blockwise(
 
     Returns (out, absmax): out uint8[ceil(order*order*bits/8)], absmax
     fp32[order*ceil(order/blocksize)].  Passed-in buffers are reused."""
-    out, absmax, _ = _quantize(A, code, order, absmax, None, out, blocksize, bits, False)
-    return out, absmax
+    done = None if _direct is None else _direct.quantize(A, code, order, absmax, None, out, blocksize, bits, False)
+    return done or _quantize(A, code, order, absmax, None, out, blocksize, bits, False)[:2]
 
 
 def dequantize_blockwise(
@@ -264,7 +275,8 @@ def dequantize_blockwise(
 ) -> Tensor:
     """Inverse of quantize_blockwise; returns an order x order tensor of `outdtype`
     (fp32 or bf16), or fills and returns `out`."""
-    return _dequantize(A, code, order, absmax, None, outdtype, out, blocksize, bits, False)
+    done = None if _direct is None else _direct.dequantize(A, code, order, absmax, None, outdtype, out, blocksize, bits, False)
+    return _dequantize(A, code, order, absmax, None, outdtype, out, blocksize, bits, False) if done is None else done
 
 
 def quantize_blockwise_diagreal(
@@ -279,7 +291,8 @@ def quantize_blockwise_diagreal(
 ) -> Tuple[Tensor, Tensor, Tensor]:
     """As quantize_blockwise, but the diagonal is kept exactly in diag (fp32[order]) and
     counts as zero for the segment maxima and the codes.  Returns (out, absmax, diag)."""
-    return _quantize(A, code, order, absmax, diag, out, blocksize, bits, True)
+    done = None if _direct is None else _direct.quantize(A, code, order, absmax, diag, out, blocksize, bits, True)
+    return done or _quantize(A, code, order, absmax, diag, out, blocksize, bits, True)
 
 
 def dequantize_blockwise_diagreal(
@@ -294,7 +307,8 @@ def dequantize_blockwise_diagreal(
     bits: int = 8,
 ) -> Tensor:
     """Inverse of quantize_blockwise_diagreal: dequantize, then put diag on the diagonal."""
-    return _dequantize(A, code, order, absmax, diag, outdtype, out, blocksize, bits, True)
+    done = None if _direct is None else _direct.dequantize(A, code, order, absmax, diag, outdtype, out, blocksize, bits, True)
+    return _dequantize(A, code, order, absmax, diag, outdtype, out, blocksize, bits, True) if done is None else done
 
 
 @torch.no_grad()

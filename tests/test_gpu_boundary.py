@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 import torch
 
+import qtensor.functional as F
 from oracle import quant_np as Q
 
 pytestmark = pytest.mark.gpu
@@ -98,3 +99,68 @@ def test_pipe_switch_and_matrix_pipe_yardstick_through_the_bare_library():
         rate = flop / (e0.elapsed_time(e1) * 1e-3)
         assert 0.1 * peak <= rate <= 1.02 * peak, (pipe, rate)
     assert float(sink[0]) == 0.0                                                              # the sink is never written
+
+
+class _Subclass(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("bits,blocksize,order", [(4, 64, 1), (4, 64, 77), (8, 256, 256), (4, 2048, 130)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("diag", [False, True])
+def test_native_host_side_takes_the_good_calls_and_no_others(bits, blocksize, order, dtype, diag, monkeypatch):
+    """The call with its host side in native code against the same call from Python, bit for bit: buffers made and buffers
+    given, on a side stream; what is not plainly good is not taken and ends as it does from Python."""
+    assert F._direct is not None
+    taken = []
+    native = F._direct
+
+    class Spy:
+        @staticmethod
+        def quantize(*args):
+            taken.append(native.quantize(*args))
+            return taken[-1]
+
+        @staticmethod
+        def dequantize(*args):
+            taken.append(native.dequantize(*args))
+            return taken[-1]
+
+    code = (F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)).cuda()
+    A = torch.randn(order, order, device="cuda").to(dtype)
+    kw = dict(blocksize=blocksize, bits=bits)
+    quantize, dequantize = ((F.quantize_blockwise_diagreal, F.dequantize_blockwise_diagreal) if diag else
+                            (F.quantize_blockwise, F.dequantize_blockwise))
+
+    def both(A, given=None, **more):
+        made = quantize(A, code, order, **kw, **({} if given is None else given), **more)
+        return made, dequantize(made[0], code, order, *made[1:], outdtype=dtype, **kw)
+
+    monkeypatch.setattr(F, "_direct", None)
+    want = both(A)
+    monkeypatch.setattr(F, "_direct", Spy)
+    got = both(A)
+    given = dict(zip(("out", "absmax", "diag"), [torch.full_like(t, 7) for t in want[0]]))
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        again = both(A, given)
+    side.synchronize()
+    assert len(taken) == 4 and all(t is not None for t in taken)
+    assert all(a is b for a, b in zip(again[0], given.values()))
+    for result in (got, again):
+        assert all(torch.equal(a, b) and a.dtype == b.dtype and a.shape == b.shape for a, b in zip(result[0] + (result[1],), want[0] + (want[1],)))
+    # not plainly good, but good: a subclass
+    taken.clear()
+    assert all(torch.equal(a, b) for a, b in zip(quantize(A.as_subclass(_Subclass), code, order, **kw), want[0]))
+    # and not good
+    wide = torch.randn(order, order + 1, device="cuda").to(dtype)
+    for error, call in ((ValueError, lambda: quantize(wide, code, order, **kw)), (ValueError, lambda: quantize(A.double(), code, order, **kw)),
+                        (ValueError, lambda: quantize(wide[:, 1:] if order > 1 else wide, code, order, **kw)),
+                        (RuntimeError, lambda: quantize(A.cpu(), code, order, **kw)), (AssertionError, lambda: quantize(A, code, order, blocksize=65, bits=bits)),
+                        (ValueError, lambda: quantize(A, code.cpu(), order, **kw)), (ValueError, lambda: quantize(A, code, order, out=A, **kw)),
+                        (ValueError, lambda: dequantize(want[0][0], code, order, want[0][1][:0], *want[0][2:], **kw)),
+                        (ValueError, lambda: dequantize(*([want[0][0], code, order] + list(want[0][1:])), outdtype=torch.float16, **kw))):
+        with pytest.raises(error):
+            call()
+    assert len(taken) == 10 and all(t is None for t in taken)
