@@ -334,12 +334,18 @@ void dequantize_dispatch(const uint8_t *q, const float *code, int order_i, const
     }
     const uint32_t order = (uint32_t)order_i, bs = (uint32_t)blocksize;
     const uint32_t total = order * order * (uint32_t)batch;
-    const bool flat = order % bs == 0 && is_aligned(out, 4 * sizeof(T)) && is_aligned(q, 16) && is_aligned(absmax, 4);
+    bool flat = order % bs == 0 && is_aligned(out, 4 * sizeof(T)) && is_aligned(q, 16) && is_aligned(absmax, 4);
     if (batch > 65535 && !flat) {
         set_error(kBadArgument, "dequantize_blockwise: a stack whose order the blocksize does not divide (or with unaligned buffers) "
                                 "takes at most 65535 matrices per launch");
         return;
     }
+    // Small outputs are bound by latency: a thread of the general kernel writes four elements and not thirty-two, and finds
+    // the diagonal without a walk.  us, flat and general, one matrix in 4 bits (8 bits the same to 0.1): fp32 256 x 256 3.0 and
+    // 2.4, with its diagonal 4.1 and 2.5; 1280 x 1280 3.9 and 3.7, 4.5 and 3.8; 1536 x 1536 4.3 and 4.5, 4.9 and 4.6; 1792 x 1792
+    // 4.8 and 5.4, 5.4 and 5.5; bf16 1536 x 1536 4.2 and 3.9, 4.9 and 4.1; 1792 x 1792 4.4 and 4.4, 5.0 and 4.7; 2048 x 2048 4.6 and
+    // 5.1, 5.0 and 5.4.
+    if (total < (DIAG || sizeof(T) == 2 ? 3u << 20 : 1u << 21)) flat = false;
     if (flat) {
         constexpr uint32_t kWaves = kFlatThreads / 64;
         const uint32_t n_super = total / kSuper;

@@ -6,9 +6,10 @@
 //    step as 8 coalesced 16-byte loads per lane, the segment maximum is a DPP butterfly, the
 //    quotient is a correctly rounded fp32 division (one exact reciprocal per segment, then the
 //    multiply / residual-fma / correction-fma sequence), and the index is a threshold count
-//    done either through a bucket table in LDS (large inputs) or a binary search in LDS.
+//    done through a bucket table in LDS.
 //  * general path -- any order/blocksize (ragged last segment, odd order with nibble pairs that
-//    straddle rows): chunks of segments, each read once by a group of lanes.
+//    straddle rows), and whatever is small: chunks of segments, each read once by a group of lanes; the
+//    threshold count through the bucket table in 8 bits, by a search in LDS in 4.
 //
 // Arithmetic follows qtensor/functional.py:526-615 and :703-735 of the reference.
 #include "qt_common.h"
@@ -26,6 +27,7 @@ namespace {
 #endif
 constexpr int kThreads = 256;            // general-path kernels
 constexpr int kFlatThreads = QT_Q_THREADS;
+static_assert(kFlatThreads == 256, "build_code_tables");
 constexpr int kFlatBlocksPerCU = QT_Q_BLOCKS_PER_CU;
 constexpr int kStep = 2048;              // elements a wave takes per step on the flat path
 
@@ -59,7 +61,7 @@ struct WaveStage {
 // lanes of one vector for BS <= 256, and JS = BS/256 whole vectors of the wave above that.  The
 // packed codes and the maxima are parked in LDS so that they leave as one contiguous 1 KiB
 // (4-bit) or 2 KiB (8-bit) run and one run of 2048/BS floats per step.
-template <typename T, int BITS, int BS, bool DIAG, bool USE_LUT, bool STREAM>
+template <typename T, int BITS, int BS, bool DIAG, bool STREAM>
 struct FlatQuantizer {
     static constexpr int NCODE = 1 << BITS;
     static constexpr int J = 8;
@@ -83,11 +85,13 @@ struct FlatQuantizer {
         float4 v[J];
     };
 
-    __device__ __forceinline__ void load(Step &s, uint32_t step) const {
-        const uint32_t k0 = step * (uint32_t)kStep + lane * 4u;
+    static __device__ __forceinline__ void load_step(const T *A, Step &s, uint32_t step) {
+        const uint32_t k0 = step * (uint32_t)kStep + (threadIdx.x & 63u) * 4u;
 #pragma unroll
         for (int j = 0; j < J; ++j) s.v[j] = ElementLoader<T>::template load4<STREAM>(A, k0 + (uint32_t)j * 256u);
     }
+
+    __device__ __forceinline__ void load(Step &s, uint32_t step) const { load_step(A, s, step); }
 
     __device__ __forceinline__ void process(Step &s, uint32_t step) const {
         if (DIAG) {
@@ -143,10 +147,8 @@ struct FlatQuantizer {
 #pragma unroll
                 for (int jj = 0; jj < JS; ++jj) {
                     const float4 v = s.v[jg + jj];
-                    idx[jj][0] = fast_index<NCODE, USE_LUT>(v.x, amax, r, tab, lut);
-                    idx[jj][1] = fast_index<NCODE, USE_LUT>(v.y, amax, r, tab, lut);
-                    idx[jj][2] = fast_index<NCODE, USE_LUT>(v.z, amax, r, tab, lut);
-                    idx[jj][3] = fast_index<NCODE, USE_LUT>(v.w, amax, r, tab, lut);
+                    const float x[4] = {v.x, v.y, v.z, v.w};
+                    fast_four(x, amax, r, lut, idx[jj]);
                 }
                 if (!ascending) {
 #pragma unroll
@@ -174,22 +176,24 @@ struct FlatQuantizer {
     }
 };
 
-template <typename T, int BITS, int BS, bool DIAG, bool USE_LUT, bool STREAM>
+template <typename T, int BITS, int BS, bool DIAG, bool STREAM>
 __global__ __launch_bounds__(kFlatThreads) void quantize_flat_kernel(
     const T *__restrict__ A, const float *__restrict__ code, uint32_t n_steps, FastDiv row_div, FastDiv order_div,
     float *__restrict__ absmax, float *__restrict__ diag, uint8_t *__restrict__ out) {
-    using Q = FlatQuantizer<T, BITS, BS, DIAG, USE_LUT, STREAM>;
+    using Q = FlatQuantizer<T, BITS, BS, DIAG, STREAM>;
     constexpr int NCODE = Q::NCODE;
     constexpr int kWaves = kFlatThreads / 64;
 
     __shared__ CodeTables<NCODE> tab;
-    __shared__ uint2 lut_mem[USE_LUT ? kLutEntries : 1];
+    __shared__ uint2 lut[kLutEntries];
     __shared__ WaveStage<BITS> stages[kWaves];
-    uint2 *lut = USE_LUT ? lut_mem : nullptr;
+    const uint32_t w = threadIdx.x >> 6;
+    typename Q::Step a, b;
+    // the first step's loads are on their way while the tables are set up
+    Q::load_step(A, a, min(blockIdx.x * kWaves + w, n_steps - 1));
     build_code_tables<NCODE>(code, tab, lut);
     const int flags = tab.flags;
 
-    const uint32_t w = threadIdx.x >> 6;
     const Q q{A, absmax, diag, out, tab, lut, stages[w], row_div, order_div, (flags & kFlagLut) != 0,
               (flags & kFlagAscending) != 0, threadIdx.x & 63u};
     const uint32_t n_waves = gridDim.x * kWaves;
@@ -198,8 +202,6 @@ __global__ __launch_bounds__(kFlatThreads) void quantize_flat_kernel(
     // Two register buffers in ping-pong: the loads of the next step are in flight while the
     // current one is processed.  Look-ahead indices are clamped so every load is unconditional.
     const uint32_t last = n_steps - 1;
-    typename Q::Step a, b;
-    q.load(a, step);
     while (true) {
         q.load(b, min(step + n_waves, last));
         q.process(a, step);
@@ -246,10 +248,10 @@ __device__ __forceinline__ void load_upto_four(const T *p, uint32_t n, float x[4
 }
 
 constexpr uint32_t kChunkIds = 8192;     // codes of the largest chunk (four segments of 2048)
-// Segments of a chunk: places for 2048 elements, or for 8192 where there are chunks enough all the same (LARGE).
-inline uint32_t chunk_segments(uint32_t bs_shift, bool large) { return large ? kChunkIds >> bs_shift : bs_shift < 9 ? 2048u >> bs_shift : 4u; }
+// Segments of a chunk: places for 2048 elements (for 8192, where there are chunks enough all the same, is no faster).
+inline uint32_t chunk_segments(uint32_t bs_shift) { return bs_shift < 9 ? 2048u >> bs_shift : 4u; }
 
-template <typename T, int BITS, bool DIAG, bool WHOLE, bool LARGE>
+template <typename T, int BITS, bool DIAG, bool WHOLE>
 __global__ __launch_bounds__(kThreads) void quantize_general_kernel(
     const T *__restrict__ A, const float *__restrict__ code, uint32_t order, uint32_t bs_shift, uint32_t nb, FastDiv nb_div,
     uint32_t n_segments, uint32_t per_chunk, uint32_t chunks_per_matrix, uint32_t n_chunks, float *__restrict__ absmax,
@@ -258,15 +260,26 @@ __global__ __launch_bounds__(kThreads) void quantize_general_kernel(
     constexpr uint32_t EPB = 8 / BITS;
     __shared__ CodeTables<NCODE> tab;
     __shared__ uint8_t ids[WHOLE ? 1 : kChunkIds + 1];               // (the shared byte's second code behind them)
-    __shared__ uint2 lut_mem[LARGE ? kLutEntries : 1];
-    uint2 *lut = LARGE ? lut_mem : nullptr;
-    build_code_tables<NCODE>(code, tab, lut);
-    const bool fast_ok = (tab.flags & kFlagLut) != 0, ascending = (tab.flags & kFlagAscending) != 0;
+    __shared__ uint2 lut_mem[BITS == 8 ? kLutEntries : 1];
+    uint2 *lut = BITS == 8 ? lut_mem : nullptr;
     const uint32_t bs = 1u << bs_shift;
     const uint32_t g_shift = min(bs_shift - 2u, 6u);                  // log2 of the lanes per segment
     const uint32_t in_group = (threadIdx.x & ((1u << g_shift) - 1u)) * 4u, group = threadIdx.x >> g_shift;
     const uint32_t n_groups = (uint32_t)kThreads >> g_shift;
     const uint32_t total = order * order, n_bytes = (total + EPB - 1) / EPB;
+    // the first segment's first loads are on their way while the tables are set up
+    float ahead[4] = {};
+    uint32_t ahead_of = 0xffffffffu;                                  // the segment (of chunk blockIdx.x) that they are of
+    {
+        const uint32_t b = blockIdx.x / chunks_per_matrix, s = (blockIdx.x - b * chunks_per_matrix) * per_chunk + group;
+        if (s < n_segments) {
+            const uint32_t r = fastdiv(s, nb_div), c = ((s - r * nb) << bs_shift) + in_group, c1 = min(c - in_group + bs, order);
+            load_upto_four<T>(A + (size_t)b * total + (size_t)r * order + c, c < c1 ? c1 - c : 0u, ahead);
+            ahead_of = s;
+        }
+    }
+    build_code_tables<NCODE>(code, tab, lut);
+    const bool fast_ok = (tab.flags & kFlagLut) != 0, ascending = (tab.flags & kFlagAscending) != 0;
 
     for (uint32_t chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
         const uint32_t b = chunk / chunks_per_matrix;
@@ -288,8 +301,8 @@ __global__ __launch_bounds__(kThreads) void quantize_general_kernel(
             const uint32_t c1 = min(c0 + bs, order);
             const T *row = src + (size_t)r * order;
             const bool own = s < s1;                                  // the shared byte's other segment is not
-            auto four = [&](uint32_t c, float x[4], bool first) {
-                load_upto_four<T>(row + c, c < c1 ? c1 - c : 0u, x);
+            auto four = [&](uint32_t c, float x[4], bool first, bool loaded = false) {
+                if (!loaded) load_upto_four<T>(row + c, c < c1 ? c1 - c : 0u, x);
                 if (DIAG && r - c < 4u && r < c1) {
                     const uint32_t e = r - c;
                     const float d = e == 0 ? x[0] : e == 1 ? x[1] : e == 2 ? x[2] : x[3];
@@ -299,7 +312,10 @@ __global__ __launch_bounds__(kThreads) void quantize_general_kernel(
                 }
             };
             float x[4];
-            four(c0 + in_group, x, true);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = ahead[e];
+            four(c0 + in_group, x, true, s == ahead_of);
+            ahead_of = 0xffffffffu;
             uint32_t m = max(max(abs_bits(x[0]), abs_bits(x[1])), max(abs_bits(x[2]), abs_bits(x[3])));
             for (uint32_t c = c0 + 256u; c < c1; c += 256u) {                 // (c1 is the same for all lanes of a segment)
                 float y[4];
@@ -319,13 +335,17 @@ __global__ __launch_bounds__(kThreads) void quantize_general_kernel(
                 const uint32_t at = c + in_group;
                 if (at >= c1) continue;
                 uint32_t idx[4];
+                if (exact) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (exact) idx[e] = exact_index<NCODE>(x[e], m, tab);
-                    else {
-                        idx[e] = fast_index<NCODE, LARGE>(x[e], a, recip, tab, lut);
-                        if (!ascending) idx[e] = tab.perm[idx[e]];
-                    }
+                    for (int e = 0; e < 4; ++e) idx[e] = exact_index<NCODE>(x[e], m, tab);
+                } else {
+                    if constexpr (BITS == 8) fast_four(x, a, recip, lut, idx);
+                    else
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) idx[e] = fast_index<NCODE>(x[e], a, recip, tab);
+                    if (!ascending)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) idx[e] = tab.perm[idx[e]];
                 }
                 const uint32_t k = r * order + at;
                 if (WHOLE) {
@@ -340,6 +360,7 @@ __global__ __launch_bounds__(kThreads) void quantize_general_kernel(
                 }
             }
         }
+        ahead_of = 0xffffffffu;                                       // (a group without a segment in the first chunk)
         if (!WHOLE) {
             __syncthreads();
             const uint32_t j0 = (k0 + EPB - 1) / EPB, j1 = (k1 + EPB - 1) / EPB;
@@ -420,7 +441,7 @@ __global__ __launch_bounds__(kThreads) void quantize_transposed_kernel(
                 const float r = exact_reciprocal(amax);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    idx[e] = fast_index<NCODE, false>(x[e], amax, r, tab, nullptr);
+                    idx[e] = fast_index<NCODE>(x[e], amax, r, tab);
                     if (!ascending) idx[e] = tab.perm[idx[e]];
                 }
             }
@@ -449,20 +470,17 @@ void launch_flat(const T *A, const float *code, uint32_t order, uint32_t batch, 
     const uint32_t n_steps = total / kStep;
     const FastDiv rd = make_fastdiv(order / 4), od = make_fastdiv(order);
     const uint32_t blocks_needed = (n_steps + kWaves - 1) / kWaves;
-    const int grid = grid_for(blocks_needed, kFlatBlocksPerCU);
-    // The bucket table costs a few microseconds of set-up per workgroup; it pays from about
-    // a million elements on.  Inputs far beyond the 256 MB last-level cache are read with the
-    // streaming hint.
-    if (total >= (1u << 25)) {
-        hipLaunchKernelGGL((quantize_flat_kernel<T, BITS, BS, DIAG, true, true>), dim3(grid), dim3(kFlatThreads), 0, stream,
+    // Inputs far beyond the 256 MB last-level cache are read with the streaming hint, by the fewest workgroups that keep the
+    // loads coming.  Below that 4-bit codes do better with five: us with three, four, five, fp32 with its diagonal 3072 x
+    // 3072 14.1 13.2 13.2, 4096 x 4096 19.4 19.4 18.6, bf16 4096 x 4096 14.2 14.1 13.0; 8 bits, bf16 4096 x 4096 15.9 16.3 17.7.
+    const bool streams = total >= (1u << 25);
+    const int grid = grid_for(blocks_needed, BITS == 4 && !streams ? 5 : kFlatBlocksPerCU);
+    if (streams)
+        hipLaunchKernelGGL((quantize_flat_kernel<T, BITS, BS, DIAG, true>), dim3(grid), dim3(kFlatThreads), 0, stream,
                            A, code, n_steps, rd, od, absmax, diag, out);
-    } else if (total >= (1u << 20)) {
-        hipLaunchKernelGGL((quantize_flat_kernel<T, BITS, BS, DIAG, true, false>), dim3(grid), dim3(kFlatThreads), 0, stream,
+    else
+        hipLaunchKernelGGL((quantize_flat_kernel<T, BITS, BS, DIAG, false>), dim3(grid), dim3(kFlatThreads), 0, stream,
                            A, code, n_steps, rd, od, absmax, diag, out);
-    } else {
-        hipLaunchKernelGGL((quantize_flat_kernel<T, BITS, BS, DIAG, false, false>), dim3(grid), dim3(kFlatThreads), 0, stream,
-                           A, code, n_steps, rd, od, absmax, diag, out);
-    }
 }
 
 template <typename T, int BITS, bool DIAG>
@@ -474,23 +492,20 @@ void launch_general(const T *A, const float *code, uint32_t order, uint32_t bs, 
     const uint32_t bs_shift = (uint32_t)__builtin_ctz(bs);
     const uint32_t nb = (order + bs - 1) / bs;
     const uint32_t n_segments = order * nb;
-    // 8-bit codes of many elements: the index from the bucket table instead of a search of eight dependent LDS reads, chunks
-    // four times as large.  One matrix, us with the search and with the table: 2001 x 2001 16.8 and 16.6, 3001 x 3001 29.7
-    // and 26.6, 5001 x 5001 in segments of 128 75.9 and 45.9, 9001 x 9001 258 and 141.  4-bit codes, whose search is one
-    // dependent read, gain nothing (5001 x 5001 41.4 and 46.8).
-    const bool large = BITS == 8 && (uint64_t)order * order * batch >= (1u << 23);
-    const uint32_t per_chunk = chunk_segments(bs_shift, large), per_matrix = (n_segments + per_chunk - 1) / per_chunk;
+    // 8 bits: the index from the bucket table instead of a search of eight dependent LDS reads, and no more workgroups than
+    // share its set-up.  us with the search, and with the table and four or eight workgroups a unit: 1024 x 1024 bf16 6.6, 6.0 and
+    // 6.7; 2048 x 2048 13.4, 9.2 and 15.0; 5001 x 5001 fp32 in segments of 128 75.9 with the search and 42.6.  (4-bit codes,
+    // whose search is one dependent read, gain nothing: 5001 x 5001 39.9 with the search, 46.8 with the table.)
+    const uint32_t per_chunk = chunk_segments(bs_shift), per_matrix = (n_segments + per_chunk - 1) / per_chunk;
     const uint32_t n_chunks = per_matrix * batch;      // (batch * order * order < 2^31 and batch <= 65535: fits)
     const FastDiv nbd = make_fastdiv(nb);
-    const dim3 grid(grid_for(n_chunks, large ? 4 : 8));
+    const dim3 grid(grid_for(n_chunks, BITS == 8 ? 4 : 8));
     const bool whole = order % 4 == 0 && is_aligned(out, BITS == 4 ? 2 : 4);
-    constexpr bool TABLE = BITS == 8;
-#define QT_QUANT_GENERAL(WHOLE, LARGE)                                                                                               \
-    hipLaunchKernelGGL((quantize_general_kernel<T, BITS, DIAG, WHOLE, LARGE>), grid, dim3(kThreads), 0, stream, A, code, order, bs_shift, \
+#define QT_QUANT_GENERAL(WHOLE)                                                                                               \
+    hipLaunchKernelGGL((quantize_general_kernel<T, BITS, DIAG, WHOLE>), grid, dim3(kThreads), 0, stream, A, code, order, bs_shift, \
                        nb, nbd, n_segments, per_chunk, per_matrix, n_chunks, absmax, diag, out)
-    if (whole) { if (large) QT_QUANT_GENERAL(true, TABLE); else QT_QUANT_GENERAL(true, false); }
-    else if (large) QT_QUANT_GENERAL(false, TABLE);
-    else QT_QUANT_GENERAL(false, false);
+    if (whole) QT_QUANT_GENERAL(true);
+    else QT_QUANT_GENERAL(false);
 #undef QT_QUANT_GENERAL
 }
 
@@ -512,12 +527,18 @@ void quantize_dispatch(const T *A, const float *code, int order_i, float *absmax
         return;
     }
     const uint32_t order = (uint32_t)order_i, bs = (uint32_t)blocksize;
-    const bool flat = order % bs == 0 && is_aligned(A, 4 * sizeof(T)) && is_aligned(out, 16) && is_aligned(absmax, 4);
+    bool flat = order % bs == 0 && is_aligned(A, 4 * sizeof(T)) && is_aligned(out, 16) && is_aligned(absmax, 4);
     if (batch > 65535 && !flat) {
         set_error(kBadArgument, "quantize_blockwise: a stack whose order the blocksize does not divide (or with unaligned buffers) "
                                 "takes at most 65535 matrices per launch");
         return;
     }
+    // Small inputs are bound by latency: the general kernel, which takes eight elements a thread and not thirty-two, and in 4 bits
+    // searches instead of setting up a bucket table, is the faster one.  us, flat and general, one matrix: 4 bits fp32 with its
+    // diagonal 256 x 256 8.3 and 4.6, 1024 x 1024 7.6 and 5.0, 2048 x 2048 8.1 and 7.6, 2560 x 2560 10.7 and 9.3, 4096 x 4096 19.4
+    // and 21.3; bf16 2560 x 2560 9.2 and 8.8, 3072 x 3072 10.3 and 11.5; 8 bits bf16 256 x 256 6.8 and 5.5, 1024 x 1024 7.1 and 6.0,
+    // 1280 x 1280 7.2 and 7.0 (fp32 6.7 and 6.7), 2048 x 2048 7.9 and 9.2.
+    if ((uint64_t)order * order * batch < (BITS == 4 ? 7u << 20 : 3u << 19)) flat = false;
     if (flat) {
         switch (blocksize) {
             case 64: launch_flat<T, BITS, 64, DIAG>(A, code, order, (uint32_t)batch, absmax, diag, out, stream); break;

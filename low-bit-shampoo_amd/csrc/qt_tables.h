@@ -19,13 +19,13 @@ namespace qt {
 constexpr int kFlagAscending = 1;  // caller's table was already non-decreasing (perm = identity)
 constexpr int kFlagLut = 2;        // bucket table usable (at most one threshold per bucket, none near 0)
 
-// Bucket table geometry: buckets are (sign, exponent, top 6 mantissa bits) of v, for
-// |v| from 2^-24 up to 1.0; anything smaller shares the innermost bucket of its sign.
-constexpr int kLutShift = 17;
-constexpr int kLutBinades = 24;
-constexpr int kLutPerSign = kLutBinades * 64 + 1;
-constexpr int kLutBias = (127 - kLutBinades) << 6;
-constexpr int kLutEntries = 2 * kLutPerSign;
+// Bucket table geometry: a bucket is what an fp16 number with six mantissa bits is, v rounded towards zero (sign, exponent
+// and six bits of the twelve that are left of v's conversion: one instruction for two values, then a shift and a mask).
+// |v| reaches up to 1; below 2^-14, where fp16 has no exponents left, the buckets are 2^-20 wide.
+constexpr int kLutTop = 0x3c0;             // 1.0; what lies beyond shares its bucket
+constexpr int kLutNegative = 0x800;
+constexpr int kLutEntries = kLutNegative + kLutTop + 1;
+constexpr int kLutPlaces = 2 * (kLutTop + 1);      // buckets that are used, in ascending order of their values: lut_place
 
 #if defined(__HIPCC__)
 
@@ -34,9 +34,9 @@ struct alignas(16) CodeTables {
     float code[NCODE];     // ascending
     float thr[NCODE];      // thr[i], i < NCODE-1; last slot = +inf
     float raw[NCODE];      // caller's order
-    uint16_t bucket[NCODE];
     uint8_t perm[NCODE];   // ascending position -> caller's index
     int flags;
+    uint32_t wave_sum[4];
 };
 
 __device__ __forceinline__ bool takes_upper(float v, float clo, float chi) {
@@ -46,13 +46,15 @@ __device__ __forceinline__ bool takes_upper(float v, float clo, float chi) {
     return fabsf(dlo) > fabsf(dhi);
 }
 
-__device__ __forceinline__ int lut_bucket(float v) {
-    uint32_t b = __float_as_uint(v);
-    int fb = (int)((b & 0x7fffffffu) >> kLutShift) - kLutBias;
-    fb = min(max(fb, 0), kLutPerSign - 1);
-    int s = (int)b >> 31;
-    return kLutPerSign + (fb ^ s);
+// Two values as packed fp16, towards zero.
+__device__ __forceinline__ uint32_t lut_pair(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
 }
+__device__ __forceinline__ int lut_bucket(float v) {
+    const uint32_t p = lut_pair(v, 0.0f) >> 4;
+    return (int)((p & kLutNegative) | min(p & 0x7ffu, (uint32_t)kLutTop));
+}
+__device__ __forceinline__ int lut_place(int p) { return p <= kLutTop ? kLutNegative + kLutTop - p : p - kLutTop - 1; }
 
 // #{i < NCODE-1 : !(v < thr[i])}; thr ascending.  NaN counts everything -> NCODE-1.
 template <int NCODE>
@@ -72,93 +74,121 @@ __device__ __forceinline__ int count_thresholds(float v, const float *thr) {
     }
 }
 
-// All threads of the workgroup call this; ends with a barrier.  lut may be nullptr.
-// Bound by latency: a few chains of dependent LDS reads that every workgroup runs before its first element, so what
-// shortens the chains shows in every launch.  A table that ascends is not sorted (256 comparisons per thread), a threshold
-// is bracketed around the middle of its gap (5 evaluations of the rule instead of up to 32) and the bucket table's
-// searches run four at a time.  Quantizing one 4096 x 4096 bf16 matrix, back to back, with 8-bit / 4-bit codes: 18.4 /
-// 16.6 us; with a sort of every table 24.9 / 16.8, with bisection from the ends of the gaps 20.1 / 18.6, with one bucket
-// at a time 20.1 / 17.2, with none of the three 27.8 / 19.1.
+// The smallest value from which the upper of two neighbouring entries is taken.
+__device__ __forceinline__ float entry_threshold(float clo, float chi) {
+    if (takes_upper(clo, clo, chi)) return clo;      // repeated entry
+    // the flip lies a few values from the middle of the gap: bracket it there, by the predicate itself, so
+    // that three halvings remain of up to thirty-two
+    uint32_t lo = float_to_key(clo), hi = float_to_key(chi);
+    const uint32_t centre = float_to_key(0.5f * clo + 0.5f * chi);
+    if (centre > lo && centre < hi) {
+        const uint32_t below = centre - lo > 4u ? centre - 4u : lo, above = hi - centre > 4u ? centre + 4u : hi;
+        if (takes_upper(key_to_float(below), clo, chi)) hi = below; else lo = below;
+        if (lo < above && above < hi) {
+            if (takes_upper(key_to_float(above), clo, chi)) hi = above; else lo = above;
+        }
+    }
+    for (int it = 0; it < 32; ++it) {
+        if (hi - lo <= 1u) break;
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        if (takes_upper(key_to_float(mid), clo, chi)) hi = mid; else lo = mid;
+    }
+    return key_to_float(hi);
+}
+
+// Sum over the lanes up to and with this one.
+__device__ __forceinline__ uint32_t wave_running_sum(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);       // row_shr:1, 2, 4, 8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);       // row_bcast:15 into rows 1 and 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);       // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// All 256 threads of the workgroup call this; ends with a barrier.  lut may be nullptr.
+// Bound by latency: a chain that every workgroup runs before its first element, so what shortens it shows in every launch.
+// A thread finds the threshold behind its entry from the two entries as they come from memory, as if the table ascended --
+// one that does not is found out on the way and takes the longer way below -- with one barrier behind it; the clearing
+// of the bucket table and the first barrier lie in the shadow of that load.  The bucket table's counts are a running sum over
+// marks, nine buckets a thread.  Against five barriers, the entries through LDS between them, and a binary search per bucket,
+// us: 4 bits, no bucket table, 256 x 256 5.1 -> 4.2; 8 bits 1024 x 1024 9.9 -> 7.1, bf16 4096 x 4096 19.9 -> 15.9.
 template <int NCODE>
 __device__ void build_code_tables(const float *__restrict__ code, CodeTables<NCODE> &t, uint2 *lut) {
-    const int tid = threadIdx.x, nt = blockDim.x;
-    for (int i = tid; i < NCODE; i += nt) t.raw[i] = code[i];
-    if (tid == 0) t.flags = kFlagAscending | kFlagLut;
+    static_assert(NCODE <= 256, "a thread per entry");
+    const int tid = threadIdx.x, i = min(tid, NCODE - 1);
+    const float own = code[i], next = code[min(i + 1, NCODE - 1)];
+    auto clear = [&]() {
+        if (lut != nullptr)
+            for (int b = tid; b < kLutEntries; b += 256) lut[b] = make_uint2(0x7f800000u, 0u);
+    };
+    // threshold i: into the table, and a mark on its bucket
+    auto place = [&](float th) {
+        // The fast quotient is only exact for |v| >= 2^-40; below that the chosen index
+        // must not depend on v, so no threshold may sit that close to zero.
+        if ((__float_as_uint(th) & 0x7fffffffu) < 0x2c800000u) atomicAnd(&t.flags, ~kFlagLut);
+        t.thr[i] = th;
+        if (lut != nullptr) {
+            uint2 *at = lut + lut_bucket(th);
+            at->x = __float_as_uint(th);
+            atomicAdd(&at->y, 1u);
+        }
+    };
+    if (tid == 0) { t.flags = kFlagAscending | kFlagLut; t.thr[NCODE - 1] = __uint_as_float(0x7f800000u); }
+    clear();
     __syncthreads();
-    // a table that already ascends (no NaN in it, then) ranks where it stands; only another one is sorted
-    for (int i = tid; i < NCODE - 1; i += nt)
-        if (!(t.raw[i] <= t.raw[i + 1])) atomicAnd(&t.flags, ~kFlagAscending);
+    if (tid < NCODE) {
+        t.raw[i] = own;
+        t.code[i] = own;
+        t.perm[i] = (uint8_t)i;
+        if (i < NCODE - 1) {
+            if (!(own <= next)) atomicAnd(&t.flags, ~kFlagAscending);          // (a NaN, too)
+            place(entry_threshold(own, next));
+        }
+    }
     __syncthreads();
-    const bool in_order = (t.flags & kFlagAscending) != 0;
-    // rank sort, ties by position
-    for (int i = tid; i < NCODE; i += nt) {
-        const float c = t.raw[i];
-        int rank = i;
-        if (!in_order) {
-            rank = 0;
+    if ((t.flags & kFlagAscending) == 0) {           // (the same for the whole workgroup)
+        // rank sort, ties by position
+        int rank = 0;
+        if (tid < NCODE)
             for (int j = 0; j < NCODE; ++j) {
                 const float d = t.raw[j];
-                rank += (d < c) || (d == c && j < i);
+                rank += (d < own) || (d == own && j < i);
             }
+        __syncthreads();
+        if (tid == 0) t.flags = kFlagLut;
+        if (tid < NCODE) {
+            t.code[rank] = own;
+            t.perm[rank] = (uint8_t)i;
         }
-        t.code[rank] = c;
-        t.perm[rank] = (uint8_t)i;
+        clear();
+        __syncthreads();
+        if (tid < NCODE - 1) place(entry_threshold(t.code[i], t.code[i + 1]));
+        __syncthreads();
     }
-    __syncthreads();
-    for (int i = tid; i < NCODE; i += nt) {
-        float th = __uint_as_float(0x7f800000u);
-        if (i < NCODE - 1) {
-            const float clo = t.code[i], chi = t.code[i + 1];
-            if (takes_upper(clo, clo, chi)) {
-                th = clo;  // repeated entry
-            } else {
-                // the flip lies a few values from the middle of the gap: bracket it there, by the predicate itself, so
-                // that three halvings remain of up to thirty-two
-                uint32_t lo = float_to_key(clo), hi = float_to_key(chi);
-                const uint32_t centre = float_to_key(0.5f * clo + 0.5f * chi);
-                if (centre > lo && centre < hi) {
-                    const uint32_t below = centre - lo > 4u ? centre - 4u : lo, above = hi - centre > 4u ? centre + 4u : hi;
-                    if (takes_upper(key_to_float(below), clo, chi)) hi = below; else lo = below;
-                    if (lo < above && above < hi) {
-                        if (takes_upper(key_to_float(above), clo, chi)) hi = above; else lo = above;
-                    }
-                }
-                for (int it = 0; it < 32; ++it) {
-                    if (hi - lo <= 1u) break;
-                    const uint32_t mid = lo + ((hi - lo) >> 1);
-                    if (takes_upper(key_to_float(mid), clo, chi)) hi = mid; else lo = mid;
-                }
-                th = key_to_float(hi);
-            }
-            // The fast quotient is only exact for |v| >= 2^-40; below that the chosen index
-            // must not depend on v, so no threshold may sit that close to zero.
-            if ((__float_as_uint(th) & 0x7fffffffu) < 0x2c800000u) atomicAnd(&t.flags, ~kFlagLut);
-            t.bucket[i] = (uint16_t)lut_bucket(th);
-        }
-        t.thr[i] = th;
-    }
-    __syncthreads();
     if (lut != nullptr) {
-        // four buckets at a time: their searches are chains of dependent LDS reads that run side by side
-        constexpr int kAtOnce = 4;
-        for (int b0 = tid; b0 < kLutEntries; b0 += kAtOnce * nt) {
-            int base[kAtOnce];   // #{i : bucket[i] < b}
+        constexpr int kEach = 9;                                               // (odd: with eight, lanes 64 bytes apart meet in the banks)
+        static_assert(256 * kEach >= kLutPlaces, "");
+        const int p0 = tid * kEach;
+        uint32_t marks[kEach], sum = 0;
 #pragma unroll
-            for (int u = 0; u < kAtOnce; ++u) base[u] = 0;
+        for (int u = 0; u < kEach; ++u) marks[u] = p0 + u < kLutPlaces ? lut[lut_place(p0 + u)].y : 0u;
 #pragma unroll
-            for (int step = NCODE / 2; step >= 1; step >>= 1)
+        for (int u = 0; u < kEach; ++u) {
+            if (marks[u] > 1u) atomicAnd(&t.flags, ~kFlagLut);                 // two thresholds in a bucket
+            sum += marks[u];
+        }
+        const uint32_t upto = wave_running_sum(sum);
+        if ((tid & 63) == 63) t.wave_sum[tid >> 6] = upto;
+        __syncthreads();
+        uint32_t base = upto - sum;
 #pragma unroll
-                for (int u = 0; u < kAtOnce; ++u)
-                    if ((int)t.bucket[base[u] + step - 1] < b0 + u * nt) base[u] += step;
+        for (int w = 0; w < 3; ++w) base += w < tid >> 6 ? t.wave_sum[w] : 0u;
 #pragma unroll
-            for (int u = 0; u < kAtOnce; ++u) {
-                const int b = b0 + u * nt;
-                if (b >= kLutEntries) break;
-                const bool one = base[u] < NCODE - 1 && (int)t.bucket[base[u]] == b;
-                const bool two = base[u] + 1 < NCODE - 1 && (int)t.bucket[base[u] + 1] == b;
-                if (two) atomicAnd(&t.flags, ~kFlagLut);
-                lut[b] = make_uint2(one ? __float_as_uint(t.thr[base[u]]) : 0x7f800000u, (uint32_t)base[u]);
-            }
+        for (int u = 0; u < kEach; ++u) {
+            if (p0 + u < kLutPlaces) lut[lut_place(p0 + u)].y = base;
+            base += marks[u];
         }
         __syncthreads();
     }
@@ -175,22 +205,23 @@ __device__ __forceinline__ uint32_t exact_index(float x, uint32_t amax_bits, con
     return t.perm[count_thresholds<NCODE>(q, t.thr)];
 }
 
-// Bucket of a quotient known to satisfy |q| <= 1 (no upper clamp needed).
-__device__ __forceinline__ int lut_bucket_unit(float q) {
-    const uint32_t b = __float_as_uint(q);
-    int fb = (int)((b & 0x7fffffffu) >> kLutShift) - kLutBias;
-    fb = max(fb, 0);
-    return kLutPerSign + (fb ^ ((int)b >> 31));
+template <int NCODE>
+__device__ __forceinline__ uint32_t fast_index(float x, float a, float r, const CodeTables<NCODE> &t) {
+    return (uint32_t)count_thresholds<NCODE>(quotient(x, a, r), t.thr);
 }
 
-template <int NCODE, bool USE_LUT>
-__device__ __forceinline__ uint32_t fast_index(float x, float a, float r, const CodeTables<NCODE> &t, const uint2 *lut) {
-    const float q = quotient(x, a, r);
-    if (USE_LUT) {
-        const uint2 e = lut[lut_bucket_unit(q)];
-        return e.y + (uint32_t)!(q < __uint_as_float(e.x));
+// Four of them through the bucket table (quotients of magnitude 1 at most).
+__device__ __forceinline__ void fast_four(const float x[4], float a, float r, const uint2 *lut, uint32_t idx[4]) {
+    float q[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] = quotient(x[e], a, r);
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {
+        const uint32_t p = lut_pair(q[e], q[e + 1]);
+        const uint2 lo = lut[(p >> 4) & 0xfffu], hi = lut[p >> 20];
+        idx[e] = lo.y + (uint32_t)!(q[e] < __uint_as_float(lo.x));
+        idx[e + 1] = hi.y + (uint32_t)!(q[e + 1] < __uint_as_float(hi.x));
     }
-    return (uint32_t)count_thresholds<NCODE>(q, t.thr);
 }
 
 // Four consecutive elements per lane, G lanes per segment: the segment maximum (as bits; a NaN
@@ -210,7 +241,7 @@ __device__ __forceinline__ uint32_t encode_four(const float x[4], const CodeTabl
         const float r = exact_reciprocal(amax);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            idx[e] = fast_index<NCODE, false>(x[e], amax, r, tab, nullptr);
+            idx[e] = fast_index<NCODE>(x[e], amax, r, tab);
             if (!ascending) idx[e] = tab.perm[idx[e]];
         }
     }

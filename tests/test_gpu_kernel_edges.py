@@ -314,6 +314,36 @@ def test_threshold_tables_of_unusual_code_tables(X, bits, order, table):
     assert all(entry_of[b] < entry_of[a] for b, a in zip(below.tolist(), above.tolist()))
 
 
+@pytest.mark.parametrize("bits,order,table", [(b, n, t) for b, lines in ((4, (2688, 2752)), (8, (1216, 1280))) for n in lines
+                                              for t in ("as it ships", "shuffled", "neighbours", "tiny", "lopsided")] +
+                         [(b, n, "as it ships") for b in (4, 8) for n in (1408, 1472, 1728, 1792)])
+def test_whole_segments_on_either_side_of_the_lines_between_the_kernels(X, bits, order, table):
+    """Orders that the blocksize divides take the general kernels when small and the flat ones, with their bucket table, from some
+    size on (quantizer: 7 x 2^20 elements in 4 bits, 3 x 2^19 in 8; dequantizer: 2^21, with a diagonal and for bf16 3 x 2^20):
+    codes, maxima, diagonal and the dequantized matrix are the oracle's, bit for bit, around every threshold of the table."""
+    import numpy as np
+    import qtensor.functional as F
+    from oracle import quant_np as Q
+    code = table_of(table, bits)
+    values, _, _ = around_the_thresholds(code)
+    A = torch.from_numpy(np.resize(values, order * order).copy()).view(order, order)
+    A[:, ::64] = 1.0                                   # segments of 64 with a 1 in each: the quotients are the values themselves
+    A[order // 2] = 0.0
+    for diag, dtype in ((False, torch.float32), (True, torch.bfloat16), (True, torch.float32)):
+        if diag and table != "as it ships":
+            continue
+        given = A.to(dtype)
+        want = Q.quantize_c(given.float().numpy(), code.numpy(), order, 64, bits, diag)
+        quantize, dequantize = ((F.quantize_blockwise_diagreal, F.dequantize_blockwise_diagreal) if diag else
+                                (F.quantize_blockwise, F.dequantize_blockwise))
+        got = quantize(given.cuda(), code.cuda(), order, blocksize=64, bits=bits)
+        back = dequantize(got[0], code.cuda(), order, *got[1:], outdtype=dtype, blocksize=64, bits=bits)
+        assert all(np.array_equal(a.cpu().numpy(), b) for a, b in zip(got, want))
+        full = Q.dequantize_c(want[0], code.numpy(), order, want[1], bits=bits, blocksize=64, diag=want[2] if diag else None,
+                              to_bf16=dtype == torch.bfloat16)
+        assert np.array_equal(back.float().cpu().numpy(), full.reshape(order, order))
+
+
 @pytest.mark.parametrize("trans", ["", "a", "b"])
 @pytest.mark.parametrize("k", [32, 48, 64, 80, 96, 112, 144, 1216])
 @pytest.mark.parametrize("m,n", [(64, 64), (65, 128), (2, 3), (200, 70)])
