@@ -22,6 +22,7 @@ class Preconditioner(PreconditionerBase):
 
     inv_root_mode 0: inverse root from the stored eigenpairs (QTensorSVDFast.computepower);
     inv_root_mode 1: coupled Newton iteration on the dequantized statistic."""
+    statistics_in_stacks = True
 
     def __init__(self, var, name2qmap, stat_decay=0.95, matrix_eps=1e-6, prec_maxorder=1200,
                  prec_bits=32, min_lowbit_size=4096, quan_blocksize=64, rect_t1=1, rect_t2=4, inv_root_mode=0):
@@ -44,6 +45,14 @@ class Preconditioner(PreconditionerBase):
         stat, basis = holder.dequantize()
         decay_and_add_gram(stat, block, axis, w1, w2)
         holder.quantize(stat, basis)
+
+    def _begin(self, holder, block, axis, w1, w2):
+        stat, basis = holder.dequantize()
+        decay_and_add_gram(stat, block, axis, w1, w2)
+        return holder.power_step(stat, basis)
+
+    def _finish(self, holder, stat, Q):
+        holder.adopt_basis(stat, Q)
 
     def _inverse_root(self, holder, exp, eps):
         if self.inv_root_mode == 0:

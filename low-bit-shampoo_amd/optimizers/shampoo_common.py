@@ -141,6 +141,21 @@ class PreconditionerBase:
             for axis in range(rank):
                 self._accumulate(self.statistics[j * rank + axis], block, axis, w1, w2)
 
+    # Whether the update of a statistic is a long chain of launches that the optimizers queue for many of them together
+    # (_ShampooOptimizer._statistics_together), and its two ends, around the orthonormalisation that is done in stacks:
+    # _begin(holder, block, axis, w1, w2) -> (statistic, matrix to orthonormalise) and _finish(holder, statistic, Q).
+    statistics_in_stacks = False
+
+    def statistics_updates(self, grad):
+        """add_statistics as its independent pieces: [arguments of _accumulate], one per statistic."""
+        if not self.statistics:
+            return []
+        w1 = self.stat_decay
+        w2 = 1.0 if w1 == 1.0 else (1.0 - w1)
+        rank = len(self._transformed_shape)
+        blocks = [b.float() for b in self._partitioner.partition(torch.reshape(grad, self._transformed_shape))]
+        return [(self.statistics[j * rank + axis], block, axis, w1, w2) for j, block in enumerate(blocks) for axis in range(rank)]
+
     def compute_preconditioners(self, v0=None):
         """Refresh every preconditioner with the inverse 4th root of its statistic.
         v0 (not in the reference): optional start vectors of the power iteration, one per
@@ -292,6 +307,91 @@ class _ShampooOptimizer(optim.Optimizer):
         kwargs = {k: group[k] for k in _PREC_KEYS + tuple(self.extra_keys)}
         return self.preconditioner_class(p, self.name2qmap, **kwargs)
 
+    LANES = 3                        # streams that the stacks of statistics are dealt out to
+    STACK_BYTES = 256 << 20          # of the matrices that are orthonormalised at a time (the update holds about five times this)
+
+    def _statistics_together(self, group):
+        """This step's statistics of a group's parameters, ahead of everything else the step does; returns the parameters whose
+        statistics are through.
+
+        The update of one statistic is a chain of up to three hundred dependent launches on one matrix, each of a few
+        workgroups: one chain after the other leaves the device idle.  Here the matrices of equal order are orthonormalised
+        as a stack, and the stacks' chains are queued on a few streams, all of them before the host looks at the first
+        one's outcome.  FIGURES
+        No update draws random numbers or looks at another one's result: it is what add_statistics does, up to the rounding of
+        products that are cut otherwise in a stack.  Only where the step would come to them: parameters from the second step
+        on, with a dense fp32 gradient on one GPU, up to the first whose gradient stops the step."""
+        done, updates = [], []
+        for p in group['params']:
+            if p.grad is None:
+                continue
+            if p.grad.is_sparse:
+                break
+            state = self.state.get(p)
+            prec = state.get('preconditioner') if state else None
+            if (prec is None or not prec.statistics_in_stacks or not prec.statistics
+                    or type(prec).add_statistics is not PreconditionerBase.add_statistics
+                    or not p.grad.is_cuda or p.grad.dtype != torch.float32 or (done and p.grad.device != done[0].grad.device)
+                    or any(h.var.device != p.grad.device for h in prec.statistics)
+                    or (state['step'] + 1) % group['stat_compute_steps'] != 0):
+                continue
+            done.append(p)
+            updates += [(prec, one) for one in prec.statistics_updates(p.grad.data)]
+        if len(updates) < 2 or F.lib is None:
+            return ()
+        from optimizers.engine import shared_stream
+        from qtensor import fused as X
+        device = done[0].grad.device
+        by_order = {}
+        for one in updates:
+            by_order.setdefault(one[1][1].shape[one[1][2]], []).append(one)
+        stacks = []
+        for order in sorted(by_order, reverse=True):
+            X.completion_columns(device, -(-order // 64) * 64, order)         # made by one stream, read by all
+            per = max(1, self.STACK_BYTES // (4 * order * order))
+            stacks += [by_order[order][i:i + per] for i in range(0, len(by_order[order]), per)]
+        main = torch.cuda.current_stream(device)
+        lanes = [shared_stream(device, i) for i in range(min(self.LANES, len(stacks)))]
+        for lane in lanes:
+            lane.wait_stream(main)
+        try:
+            while stacks:                                                      # as many at a time as the bound allows
+                running, size, loads = [], 0, [0.0] * len(lanes)
+                while stacks and (not running or size + self._stack_bytes(stacks[0]) <= self.STACK_BYTES):
+                    stack = stacks.pop(0)
+                    size += self._stack_bytes(stack)
+                    i = loads.index(min(loads))
+                    loads[i] += stack[0][1][1].shape[stack[0][1][2]] ** 1.5    # (about what its chain takes)
+                    with torch.cuda.stream(lanes[i]):
+                        begun = [prec._begin(*one) for prec, one in stack]
+                        running.append((lanes[i], stack, [L for L, _ in begun], X.CholeskyQR(torch.stack([Y for _, Y in begun]))))
+                    del begun
+                while running:
+                    # the one whose outcome is there already, else the first
+                    lane, stack, statistics, solver = running.pop(next((i for i, r in enumerate(running) if r[3].landed()), 0))
+                    with torch.cuda.stream(lane):
+                        if solver.swept:
+                            solver.check()
+                        elif not solver.poll():
+                            solver.advance()
+                            if not solver.finished:
+                                solver.check()
+                        if not solver.finished:
+                            running.append((lane, stack, statistics, solver))
+                            continue
+                        Q, _ = solver.result()
+                        for (prec, one), L, V in zip(stack, statistics, Q):
+                            prec._finish(one[0], L, V)
+        finally:
+            for lane in lanes:
+                main.wait_stream(lane)
+        return done
+
+    @staticmethod
+    def _stack_bytes(stack):
+        _, (_, block, axis, _, _) = stack[0]
+        return 4 * len(stack) * block.shape[axis] ** 2
+
     def _shampoo_direction(self, p, grad, group, state, statistics_done=False, roots_done=False):
         """Statistics / inverse-root bookkeeping for this step and the grafted direction
         (statistics_done / roots_done: the caller has already run this step's add_statistics /
@@ -323,6 +423,7 @@ class ShampooSGDBase(_ShampooOptimizer):
     @torch.no_grad()
     def step(self, closure=None):
         for group in self.param_groups:
+            ahead = {id(p) for p in self._statistics_together(group)}
             for p in group['params']:
                 if p.grad is None:
                     continue
@@ -335,7 +436,7 @@ class ShampooSGDBase(_ShampooOptimizer):
                     state['preconditioner'] = self._make_preconditioner(p, group)
                     state['momentum'] = torch.zeros_like(p, memory_format=torch.preserve_format)
                 state['step'] += 1
-                direction = self._shampoo_direction(p, grad, group, state)
+                direction = self._shampoo_direction(p, grad, group, state, statistics_done=id(p) in ahead)
                 if group['weight_decay'] != 0.0:
                     direction.add_(p.data, alpha=group['weight_decay'])
                 buf = state['momentum'].mul_(group['momentum']).add_(direction)
@@ -357,6 +458,7 @@ class ShampooAdamWBase(_ShampooOptimizer):
     @torch.no_grad()
     def step(self, closure=None):
         for group in self.param_groups:
+            ahead = {id(p) for p in self._statistics_together(group)}
             for p in group['params']:
                 if p.grad is None:
                     continue
@@ -371,7 +473,7 @@ class ShampooAdamWBase(_ShampooOptimizer):
                     state['exp_avg_sq'] = torch.zeros_like(p, memory_format=torch.preserve_format)
                 state['step'] += 1
                 p.mul_(1 - group['lr'] * group['weight_decay'])           # decoupled weight decay
-                direction = self._shampoo_direction(p, grad, group, state)
+                direction = self._shampoo_direction(p, grad, group, state, statistics_done=id(p) in ahead)
                 beta1, beta2 = group['betas']
                 correction1 = 1 - beta1 ** state['step']
                 correction2 = 1 - beta2 ** state['step']

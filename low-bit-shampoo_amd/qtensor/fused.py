@@ -904,6 +904,10 @@ class CholeskyQR:
         self.ids, self.near, self.mended = self.ids[keep], self.near[keep], self.mended[keep]
         self.far_before, self.stuck = self.far_before[keep], self.stuck[keep]
 
+    def landed(self):
+        """Whether what the host has to see next, the outcome of the sweep or of the last test, is there."""
+        return (self.info_host if self.swept else self.far_host)[1].query()
+
     def check(self):
         if self.swept:
             self.swept = False

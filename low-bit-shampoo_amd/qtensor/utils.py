@@ -212,19 +212,32 @@ class QTensorSVDFast(_LowBitState):
         L = var.float()
         from qtensor import fused
         if fused.on_matrix_cores(L, Vt) and L.dim() == 2:
-            # the same products on the matrix cores; the Rayleigh quotients diag(V^T (L V)) without the product
-            V = _orthonormal_basis(fused.gemm(L, Vt, trans_b=True))
-            quotients = (V * fused.gemm(L, V.contiguous())).sum(dim=0)
+            L, Y = self.power_step(L, Vt)
+            self.adopt_basis(L, _orthonormal_basis(Y), var.dtype)
         else:
             V = _orthonormal_basis(L @ Vt.T.float())
-            quotients = (V.T @ L @ V).diag()
+            self._adopt(V, (V.T @ L @ V).diag(), var.dtype)
 
+    # the same in two parts, for callers that orthonormalise many of them at a time; fp32 matrices on the GPU
+    @staticmethod
+    def power_step(var, Vt):
+        """(L, L Vt^T), on the matrix cores"""
+        from qtensor import fused
+        L = var.float()
+        return L, fused.gemm(L, Vt, trans_b=True)
+
+    def adopt_basis(self, L, V, dtype=torch.float32):
+        """The rest of `quantize` behind the orthonormalisation: the Rayleigh quotients diag(V^T (L V)) without the product."""
+        from qtensor import fused
+        self._adopt(V, (V * fused.gemm(L, V.contiguous())).sum(dim=0), dtype)
+
+    def _adopt(self, V, quotients, dtype):
         keep = max(1, quotients.numel() // 2)
         ascending, where = torch.sort(quotients)
         self.keep_indices = where[:keep].to(dtype=torch.int64)
-        self.Svalue = ascending[:keep].to(var.dtype)
-        dropped = ascending[keep:].to(var.dtype)
-        self.max_eigenvalue = quotients.max().to(var.dtype)
+        self.Svalue = ascending[:keep].to(dtype)
+        dropped = ascending[keep:].to(dtype)
+        self.max_eigenvalue = quotients.max().to(dtype)
 
         if self.bits >= 16:
             self.var = V.T.contiguous()

@@ -763,3 +763,54 @@ def test_a_dependent_column_next_to_an_ill_conditioned_panel_is_flagged(mods):
         gram = Q[0].double().T @ Q[0].double()
         assert float((gram - torch.eye(n, dtype=torch.float64, device="cuda")).abs().max()) <= 5e-5
     assert flagged >= len(mats) // 2                                        # these matrices are rank deficient: most must be flagged
+
+
+@pytest.mark.parametrize("stack_bytes,lanes", [(256 << 20, 3), (1, 2), (4 * 96 * 96, 1)])
+def test_statistics_taken_together_are_those_taken_one_by_one(monkeypatch, stack_bytes, lanes):
+    """fused=False: the statistics of all parameters in stacks on a few streams, or parameter by parameter: quotients, maxima and
+    parameters over five steps, every second of which takes statistics, with a parameter that has no gradient at times.  (Square
+    gradients with singular values between 1/2 and 2: statistics whose eigenvectors rounding does not choose.)  A stack's products may be cut along k in another way than
+    a single matrix's, which rounds sums of up to 130 fp32 products differently: 130 x 2^-24 = 8e-6 of a quotient, and where
+    a maximum or a code sits on an edge the element moves a level, in few places."""
+    from optimizers import shampoo2, shampoo_common
+    monkeypatch.setattr(shampoo_common._ShampooOptimizer, "STACK_BYTES", stack_bytes)
+    monkeypatch.setattr(shampoo_common._ShampooOptimizer, "LANES", lanes)
+    shapes = [(96, 96), (128, 128), (64, 64), (100, 100), (130, 130), (45, 5, 3, 3), (17,), (96, 96)]
+    gen = torch.Generator().manual_seed(5)
+    start = [0.1 * torch.randn(s, generator=gen) for s in shapes]
+
+    def gradient(shape):
+        n = shape[0]
+        if len(shape) == 1:
+            return torch.randn(n, generator=gen)
+        (u, _), (v, _) = [torch.linalg.qr(torch.randn(n, n, generator=gen)) for _ in range(2)]
+        return ((u * torch.logspace(-1, 1, n, base=2.0)) @ v).reshape(shape)
+
+    grads = [[gradient(s) for s in shapes] for _ in range(5)]
+    made, taken = [], []
+    together = shampoo_common._ShampooOptimizer._statistics_together
+    for alone in (False, True):
+        def spy(self, group):
+            done = () if alone else together(self, group)
+            taken.append(len(done))
+            return done
+        monkeypatch.setattr(shampoo_common._ShampooOptimizer, "_statistics_together", spy)
+        params = [torch.nn.Parameter(t.cuda()) for t in start]
+        opt = shampoo2.ShampooAdamW(params, lr=1e-2, start_prec_step=1, stat_compute_steps=2, prec_compute_steps=4, prec_maxorder=1200,
+                                    prec_bits=4, quan_blocksize=64, min_lowbit_size=4096)
+        for step, gs in enumerate(grads):
+            for i, (p, g) in enumerate(zip(params, gs)):
+                p.grad = None if (i == 2 and step in (1, 2)) or (i == 7 and step == 0) else g.cuda()
+            opt.step()
+        made.append((params, opt))
+    # the first step finds no state; then parameters at an even count: (step, counts of parameters 2 and 7)
+    assert taken[:5] == [0, 5, 1, 6, 1] and taken[5:] == [0] * 5
+    for pa, pb in zip(made[0][0], made[1][0]):
+        a, b = pa.detach(), pb.detach()
+        stats = [opt.state[p]["preconditioner"].statistics for (_, opt), p in zip(made, (pa, pb))]
+        for x, y in zip(*stats):
+            assert float((x.Svalue - y.Svalue).norm() / y.Svalue.norm()) <= 1e-5 * 4
+            assert torch.equal(x.keep_indices, y.keep_indices)
+            if x.bits < 16:
+                assert float((x.absmax - y.absmax).norm() / y.absmax.norm()) <= 1e-3
+        assert float((a - b).abs().max()) <= 1e-4 * 5e-2                       # five steps of 1e-2
