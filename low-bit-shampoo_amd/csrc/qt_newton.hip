@@ -4,7 +4,7 @@
 //
 // Every one of them is a small kernel or one pass over the stack, and what they cost is launches: as torch operations a
 // round took 22 of them beside its four products and a power iteration's step 11, most of 3 to 5 us in a chain.  One
-// launch each here.  Inverse roots over a ViT-B/32's weights (248 matrices, seven parts): 3409 -> 706 launches.
+// launch each here.  Inverse roots over a ViT-B/32's weights (248 matrices, seven parts): 3409 -> 591 launches.
 #include "qt_common.h"
 #include "qt_half.h"
 
