@@ -414,3 +414,40 @@ def test_fused_step_with_parameters_the_bank_does_not_take(setup, monkeypatch):
         assert [opt.state[p]["step"] for p in params] == [sum(row[k] for row in present) for k in range(4)]
     for k, (a, b) in enumerate(zip(*finals)):
         assert rel(a, b) <= (2e-4 if dtypes[k] == torch.float32 else 2e-2), k
+
+
+@pytest.mark.parametrize("sizes", [(1 << 24, 16384 * 70 + 3, 5), (16384 * 3 + 1, 64 * 16384, 3, 16385)])
+@pytest.mark.parametrize("kind", ["adamw", "sgd"])
+def test_fused_update_of_large_tensors_and_odd_ends(sizes, kind):
+    """Tensors of 2^24 elements and more in all stream past the caches; the norms of a tensor are the sums of more chunks than a wave
+    has lanes; ends that are no multiple of four, and rows that are not 16-byte aligned.  One update against float64: a norm is a
+    sum of fp32 squares over 16384 elements (64 per thread) and a few roundings, 1e-5 of the step; a parameter is rounded twice
+    (decay, step), 2^-24 of it each."""
+    from optimizers.tail import TailPlan
+    gen = torch.Generator(device="cuda").manual_seed(3)
+
+    def make(scale, shift=0):
+        return [(scale * torch.randn(n + shift, device="cuda", generator=gen))[shift:] for n in sizes]
+
+    params, dirs, grads, m = make(1.0), make(3.0), make(0.1, 1), make(0.1)
+    v = [t.abs() for t in make(0.01)]
+    graft = [True] * (len(sizes) - 1) + [False]
+    before = [[t.double() for t in ts] for ts in (params, m, v)]
+    plan = TailPlan()
+    if kind == "adamw":
+        plan.adamw(params, dirs, grads, m, v, graft, 1e-2, (0.9, 0.999), 1e-8, 0.05, 3)
+    else:
+        plan.sgd(params, dirs, grads, m, graft, 1e-2, 0.9, 5e-4, False)
+    for i, (p, d, g) in enumerate(zip(params, dirs, grads)):
+        d = d.double()
+        if graft[i]:
+            d = d * (g.double().norm() / (d.norm() + 1e-12))
+        P, M, V = [b[i] for b in before]
+        if kind == "adamw":
+            M, V = 0.9 * M + 0.1 * d, 0.999 * V + 0.001 * d * d
+            want = P * (1 - 1e-2 * 0.05) - 1e-2 / (1 - 0.9 ** 3) * M / (V.sqrt() / (1 - 0.999 ** 3) ** 0.5 + 1e-8)
+        else:
+            M = 0.9 * M + d + 5e-4 * P
+            want = P - 1e-2 * M
+        assert float((m[i].double() - M).norm() / M.norm()) <= 1e-5
+        assert float((p.double() - want).norm()) <= 1e-5 * float((want - P).norm()) + 2.0 ** -23 * float(P.norm())
