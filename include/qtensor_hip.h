@@ -108,6 +108,12 @@ void qtensor_hip_dequantize_batched(const unsigned char *q, const float *code, i
  * Needs blocksize in {64, 128, 256} dividing order, order a multiple of 64, 16-byte aligned A. */
 void qtensor_hip_quantize_transposed_batched(const float *A, const float *code, int bits, int order, int batch,
                                              float *absmax, unsigned char *out, int blocksize, qtensor_stream_t stream);
+/* out[b][i] = row rows[b][i] of matrix b of a stack (batch x count x order), from 4- or 8-bit codes without exact diagonal (bits 4,
+ * 8) or fp32 (bits 32: code and absmax ignored); scaled, if not NULL: the same times weight[b][i].  Replaces dequantize, index and multiply at
+ * qtensor/utils.py:200-203 and 205-215 of the reference.  order a multiple of four, from aligned to four elements, out and scaled to
+ * 16 bytes; a row number outside the matrix makes a row of NaN. */
+void qtensor_hip_rows_batched(const void *from, int bits, const float *code, const float *absmax, int blocksize, int order, int batch,
+                              const long long *rows, int count, const float *weight, float *out, float *scaled, qtensor_stream_t stream);
 
 /* ---- self check and calibration (no counterpart in the reference) ------------------------
  * The flat-path quantizer replaces IEEE division by the segment maximum a with r = rcp(a) refined

@@ -127,12 +127,15 @@ class ShampooBank2(ShampooBank):
 
     # ---- pieces of QTensorSVDFast, for a whole stack ---------------------------------------------
     def _pick(self, order, rows):
-        """(basis, kept row indices, kept quotients, largest quotient) of the whole stack (rows None) or of a copy
-        of the given rows of it."""
+        """(basis, kept row indices, kept quotients, largest quotient) of the whole stack (rows None), of a range (first,
+        count) of it as views, or of a copy of the given rows of it."""
+        parts = self.basis[order], self.keep[order], self.svalue[order], self.max_eig[order]
         if rows is None:
-            return self.basis[order], self.keep[order], self.svalue[order], self.max_eig[order]
-        return (self.basis[order].select(rows), self.keep[order].index_select(0, rows),
-                self.svalue[order].index_select(0, rows), self.max_eig[order].index_select(0, rows))
+            return parts
+        if isinstance(rows, tuple):
+            first, count = rows
+            return (parts[0].rows(first, count),) + tuple(t[first:first + count] for t in parts[1:])
+        return (parts[0].select(rows),) + tuple(t.index_select(0, rows) for t in parts[1:])
 
     def _measured(self, order):
         """Whether the largest elements of this order's matrices are looked up for the pipe that wants to know them: a
@@ -145,8 +148,9 @@ class ShampooBank2(ShampooBank):
         those of vt, None: not looked at) of the result are.  (The deviation from the identity: its elements are of one
         size to the last step, where vt vt^T itself ends as the identity and rounding noise.)"""
         eye = torch.eye(vt.shape[1], device=vt.device).expand(vt.shape[0], -1, -1) if steps > 0 else None
-        for _ in range(steps):
-            square, after = (None, None) if size is None else torch.zeros(2, 2, vt.shape[0], device=vt.device)
+        found = None if size is None else torch.zeros(steps, 2, 2, vt.shape[0], device=vt.device)
+        for step in range(steps):
+            square, after = (None, None) if size is None else found[step]
             gram = X.gemm(vt, vt, trans_b=True, symmetric=True, addend=eye, beta=-1.0, amax=None if size is None else (size, size),
                           amax_out=square)
             vt = X.gemm(gram, vt, addend=vt, alpha=-0.5, amax=None if size is None else (square, size), beta=1.0, amax_out=after)
@@ -162,19 +166,11 @@ class ShampooBank2(ShampooBank):
             vt, size = self._rectify(vt, self.rect_t1, X.measure(basis) if self._measured(order) else None)
         return (vt, size) if with_size else vt
 
-    @staticmethod
-    def _gather_rows(vt, keep):
-        n = vt.shape[2]
-        return torch.gather(vt, 1, keep.unsqueeze(2).expand(-1, -1, n))
-
-    def _kept_rows(self, order, vt, rows=None):
-        return self._gather_rows(vt, self._pick(order, rows)[1])
-
     def _statistic(self, order, vt, out=None, rows=None):
         """Vt[keep]^T diag(S) Vt[keep] (utils.py:200-203)."""
         _, keep, svalue, _ = self._pick(order, rows)
-        kept = self._gather_rows(vt, keep)
-        return X.gemm(kept * svalue.unsqueeze(2), kept, trans_a=True, symmetric=True, out=out)
+        kept, weighted = X.rows_of(vt, keep, svalue)
+        return X.gemm(weighted, kept, trans_a=True, symmetric=True, out=out)
 
     # ---- the operations of the reference's Preconditioner ----------------------------------------
     @torch.no_grad()
@@ -468,12 +464,9 @@ class ShampooBank2(ShampooBank):
             def run():
                 rows = self._rows(order, only)
                 for part in self._newton_parts(order, rows):
-                    # (a part of the whole stack is gathered like a chosen set of rows: one copy of its 4-bit basis)
-                    index = torch.arange(part[0], part[0] + part[1], device=self.device) if rows is None else part
-                    whole = rows is None and part[1] == self.per_order[order]
-                    basis, keep, svalue, max_eig = self._pick(order, None if whole else index)
+                    basis, keep, svalue, max_eig = self._pick(order, part)
                     if self.inv_root_mode == 0:
-                        kept, size = self._gather_rows(X.load_stack(basis), keep), None
+                        kept, size = X.rows_of(basis, keep), None
                         if not isinstance(basis, X.DenseStack):          # (a basis held in fp32 is not rectified: utils.py:205-227)
                             kept, size = self._rectify(kept, self.rect_t2, X.measure(basis) if self._measured(order) else None)
                         ridge = self.matrix_eps * max_eig
@@ -481,15 +474,15 @@ class ShampooBank2(ShampooBank):
                         roots = X.gemm(kept * weights.unsqueeze(2), kept, trans_a=True, symmetric=True,
                                        amax=None if size is None else ((size[0] * weights.amax(dim=1), size[1] / weights.amin(dim=1)), size))
                     else:
-                        L = self._statistic(order, self._rectified_basis(order, None if whole else index), rows=None if whole else index)
-                        start = starts[order] if whole else starts[order].index_select(0, index)
+                        L = self._statistic(order, self._rectified_basis(order, part), rows=part)
+                        start = starts[order][part[0]:part[0] + part[1]] if rows is None else starts[order].index_select(0, part)
                         # L is symmetric up to the rounding inside its diagonal tiles: half products are fine
                         roots = ComputePowerBatched(L, 4, ridge_epsilon=self.matrix_eps, v0=start, symmetric=True,
                                                     stack=self.per_order[order])
                     if rows is None:
                         X.store_stack(roots, self.precs[order].rows(part[0], part[1]))
                     else:
-                        self.precs[order].put(index, X.store_stack(roots, self.precs[order].select(index)))
+                        self.precs[order].put(part, X.store_stack(roots, self.precs[order].select(part)))
             return run
 
         self._fan_out([job(o) for o in orders], inline=not self.NEWTON_SIDE_BY_SIDE)

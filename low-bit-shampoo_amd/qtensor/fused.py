@@ -610,6 +610,37 @@ def load_stack(q) -> Tensor:
     return q.data if isinstance(q, DenseStack) else dequantize_stack(q)
 
 
+if F.lib is not None:
+    F.lib.qtensor_hip_rows_batched.restype = None
+    F.lib.qtensor_hip_rows_batched.argtypes = ([ct.c_void_p, ct.c_int, ct.c_void_p, ct.c_void_p] + [ct.c_int] * 3 +
+                                               [ct.c_void_p, ct.c_int] + [ct.c_void_p] * 4)
+
+
+def rows_of(stack, rows: Tensor, weights: Optional[Tensor] = None):
+    """[batch, count, order]: the rows rows[b] (int64 [batch, count]) of every matrix of a stack -- a `Quantized` without diagonal,
+    a `DenseStack` or an fp32 tensor [batch, order, order] -- and with weights [batch, count] a pair of them and of the
+    rows times their weights."""
+    quantized = isinstance(stack, Quantized)
+    src = stack.codes if quantized else stack.data if isinstance(stack, DenseStack) else stack
+    batch, count = rows.shape
+    n = stack.order if quantized else src.shape[2]
+    if src.shape[0] != batch or rows.dtype != torch.int64 or (quantized and stack.diag is not None) or (
+            weights is not None and (weights.shape != rows.shape or weights.dtype != torch.float32)):
+        raise ValueError("rows_of takes int64 rows and fp32 weights [batch, count] of a stack without exact diagonal")
+    if F.lib is None or n % 4 or batch > 65535 or not src.is_contiguous() or src.data_ptr() % (4 if quantized else 16):
+        # (an order whose rows do not begin with whole, aligned fours)
+        out = torch.gather(load_stack(stack) if quantized else src, 1, rows.unsqueeze(2).expand(-1, -1, n))
+        return out if weights is None else (out, out * weights.unsqueeze(2))
+    out = torch.empty(batch, count, n, device=src.device)
+    scaled, rows = None, rows.contiguous()
+    if weights is not None:
+        scaled, weights = torch.empty_like(out), weights.contiguous()
+    F._call(F.lib.qtensor_hip_rows_batched, src.device, src.data_ptr(), stack.bits if quantized else 32, stack.code.data_ptr() if quantized else None,
+            stack.absmax.data_ptr() if quantized else None, stack.blocksize if quantized else 0, n, batch, rows.data_ptr(), count,
+            None if weights is None else weights.data_ptr(), out.data_ptr(), None if scaled is None else scaled.data_ptr())
+    return out if weights is None else (out, scaled)
+
+
 def store_stack(mats: Tensor, q, transposed: bool = False):
     """Inverse of load_stack: mats (their transposes with transposed=True) into q's buffers."""
     if isinstance(q, DenseStack):

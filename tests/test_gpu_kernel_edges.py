@@ -491,3 +491,32 @@ def test_reencoding_products_with_tiles_of_either_size_equal_update_then_quantiz
     assert torch.equal(one.codes, two.codes)
     assert torch.equal(one.absmax.view(torch.int32), two.absmax.view(torch.int32))
     assert torch.equal(one.diag.nan_to_num(7.0), two.diag.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("order,blocksize,count,batch", [(4, 64, 2, 3), (64, 64, 1, 5), (68, 64, 34, 3), (256, 256, 256, 2), (1200, 64, 600, 2),
+                                                         (1024, 128, 512, 3), (65, 64, 32, 2)])
+@pytest.mark.parametrize("bits", [4, 8, 32])
+def test_chosen_rows_of_a_stack_equal_dequantize_index_and_multiply(order, blocksize, count, batch, bits):
+    """Whole matrices and views of a stack that begin anywhere, an order whose rows do not begin with whole fours (the general
+    way), repeated rows, segments that are zero, infinite or NaN: bit for bit."""
+    import qtensor.functional as F
+    from qtensor import fused
+    g = torch.Generator().manual_seed(order + bits)
+    if bits == 32:
+        stack = fused.DenseStack(torch.randn(batch, order, order, generator=g).cuda())
+    else:
+        code = (F.create_linear_map(True, 4, 2) if bits == 4 else F.create_dynamic_map(True, 8, 1)).cuda()
+        stack = fused.quantize_stack(torch.randn(batch, order, order, generator=g).cuda(),
+                                     fused.empty_quantized(batch, order, blocksize, bits, code, False))
+        stack.absmax[0, 0], stack.absmax[-1, 1], stack.absmax[-1, -1] = 0.0, float("inf"), float("nan")
+    rows = torch.randint(0, order, (batch, count), generator=g).cuda()
+    rows[:, -1] = order - 1
+    weights = torch.randn(batch, count, generator=g).cuda()
+    full = fused.load_stack(stack)
+    for first in (0, 1):
+        part = stack.rows(first, batch - first)
+        want = full[first:].gather(1, rows[first:].unsqueeze(2).expand(-1, -1, order))
+        kept, weighted = fused.rows_of(part, rows[first:], weights[first:])
+        for got, w in ((kept, want), (weighted, want * weights[first:].unsqueeze(2)), (fused.rows_of(part, rows[first:]), want),
+                       (fused.rows_of(full[first:], rows[first:]), want)):
+            assert torch.equal(got.nan_to_num(7.0), w.nan_to_num(7.0)) and torch.equal(got.isnan(), w.isnan())
