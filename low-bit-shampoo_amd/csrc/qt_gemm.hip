@@ -194,23 +194,26 @@ __device__ __forceinline__ float dequant_element(const uint8_t *codes, const flo
     return a == 0.0f ? 0.0f : s_code[id] * a;
 }
 
+// Four elements from the word that holds their codes and the maximum of their segment.
+template <int BITS>
+__device__ __forceinline__ void expand_four(uint32_t w, float a, const float *s_code, float out[4]) {
+    uint32_t id[4];
+    if (BITS == 8) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) id[e] = (w >> (8 * e)) & 255u;
+    } else {
+        id[0] = (w >> 4) & 15u; id[1] = w & 15u; id[2] = (w >> 12) & 15u; id[3] = (w >> 8) & 15u;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = a == 0.0f ? 0.0f : s_code[id[e]] * a;
+}
+
 // Four consecutive off-diagonal elements (r, c0 .. c0+3), c0 a multiple of 4, of the same matrix.
 template <int BITS>
 __device__ __forceinline__ void dequant_four(const uint8_t *codes, const float *absmax, const float *s_code, int order,
                                              int bs_shift, int r, int c0, float out[4]) {
     const long long k = (long long)r * order + c0;
-    uint32_t id[4];
-    if (BITS == 8) {
-        const uint32_t w = gload_u32(codes + k);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) id[e] = (w >> (8 * e)) & 255u;
-    } else {
-        const uint32_t w = gload_u16(codes + (k >> 1));
-        id[0] = (w >> 4) & 15u; id[1] = w & 15u; id[2] = (w >> 12) & 15u; id[3] = (w >> 8) & 15u;
-    }
-    const float a = gload(absmax + (k >> bs_shift));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) out[e] = a == 0.0f ? 0.0f : s_code[id[e]] * a;
+    expand_four<BITS>(BITS == 8 ? gload_u32(codes + k) : gload_u16(codes + (k >> 1)), gload(absmax + (k >> bs_shift)), s_code, out);
 }
 
 // ---- tile loaders: global -> registers -> LDS ([k][row], row stride rows + LDS_PAD) -------------
@@ -1170,6 +1173,22 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         float *o_absmax = const_cast<float *>(e_absmax), *o_diag = const_cast<float *>(e_diag);
         const bool fast_ok = (tab.flags & kFlagLut) != 0, ascending = (tab.flags & kFlagAscending) != 0;
         const int order = args.Eq.order, per_row = order >> 6;
+        // The addend of a wave's rows is asked for in one go, ahead of their staging: the compiler cannot move a load of it
+        // above the stores of the row before, and the latencies of 32 loads one after the other were a tenth of a tile's time.
+        // A step that takes statistics in 3.10 -> 3.04 ms.
+        uint32_t held[ROWS / 4];
+        float held_max[ROWS / 4], held_diag[ROWS / 4];
+        auto fetch_rows = [&](int row_base, int col_base) {
+            if (col_base >= order) return;
+#pragma unroll
+            for (int q = 0; q < ROWS / 4; ++q) {
+                const int row = min(row_base + q * 4 + (lane >> 4), order - 1);
+                const long long k = (long long)row * order + col_base + (lane & 15) * 4;
+                held[q] = EBITS == 8 ? gload_u32(e_codes + k) : gload_u16(e_codes + (k >> 1));
+                held_max[q] = gload(e_absmax + (k >> 6));
+                held_diag[q] = o_diag != nullptr ? gload(o_diag + row) : 0.0f;
+            }
+        };
         auto encode_rows = [&](int row_base, int col_base) {
             if (col_base >= order) return;
 #pragma unroll
@@ -1180,12 +1199,11 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                 const int row = row_base + rl, col = col_base + c4;
                 if (row >= order) continue;                      // the 16 lanes of a segment share the row
                 float e[4], y[4];
-                dequant_four<EBITS>(e_codes, e_absmax, s_code, order, 6, row, col, e);
+                expand_four<EBITS>(held[q], held_max[q], s_code, e);
                 const bool on_diag = o_diag != nullptr && (unsigned)(row - col) < 4u;
                 if (on_diag) {
-                    const float d = gload(o_diag + row);
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) if (row == col + k) e[k] = d;
+                    for (int k = 0; k < 4; ++k) if (row == col + k) e[k] = held_diag[q];
                 }
 #pragma unroll
                 for (int k = 0; k < 4; ++k) y[k] = __builtin_fmaf(args.alpha, a[k], args.beta * e[k]);
@@ -1205,12 +1223,14 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
             }
         };
         if constexpr (SMALL) {
+            fetch_rows(m0 + wave * ROWS, n0);
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 s_mem[(wm + 8 * (r / 4) + 4 * (lane >> 5) + r % 4) * REQUANT_LD + wn + (lane & 31)] = acc[0][0][r];
             __syncthreads();
             encode_rows(m0 + wave * ROWS, n0);
             if (mirror) {                                            // (the same for the whole workgroup)
+                fetch_rows(n0 + wave * ROWS, m0);
                 __syncthreads();
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
@@ -1222,6 +1242,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         }
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
+            fetch_rows(m0 + wm + i * 32, n0 + wn);
 #pragma unroll
             for (int j = 0; j < NI; ++j)
 #pragma unroll
@@ -1234,6 +1255,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         if (mirror) {
 #pragma unroll
             for (int j = 0; j < NI; ++j) {
+                fetch_rows(n0 + wn + j * 32, m0 + wm);
 #pragma unroll
                 for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -1261,7 +1283,16 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
+            // (a dense addend's elements of a block likewise: result and addend may be one buffer, each element read and written
+            // by the same lane.  Newton roots of the ViT-B/32 55.4 -> 54.8 ms, its eigenbasis step 17.15 -> 16.9)
+            float4 held[4];
             if (direct_vec) {
+                if (kDenseAddend) {
+#pragma unroll
+                    for (int p = 0; p < 4; ++p)
+                        held[p] = gload4(E + (long long)min(m0 + wm + i * 32 + p * 8 + (lane >> 3), args.M - 1) * args.lde +
+                                         min(n0 + wn + j * 32 + (lane & 7) * 4, args.N - 4));
+                }
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     stage[(8 * (r / 4) + 4 * (lane >> 5) + r % 4) * STAGE_LD + (lane & 31)] = acc[i][j][r];
@@ -1274,8 +1305,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                     const int row = m0 + wm + i * 32 + ml, col4 = n0 + wn + j * 32 + nl;
                     if (row >= args.M || col4 >= args.N) continue;           // N % 4 == 0: col4 + 3 < N
                     if (kDenseAddend) {
-                        const float4 x = gload4(E + (long long)row * args.lde + col4);
-                        const float e[4] = {x.x, x.y, x.z, x.w};
+                        const float e[4] = {held[p].x, held[p].y, held[p].z, held[p].w};
 #pragma unroll
                         for (int q = 0; q < 4; ++q) y[q] = args.beta * e[q] + args.alpha * y[q];
                     } else if (kQuantAddend) {
@@ -1334,6 +1364,12 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                 }
             }
             if (!mirror) continue;
+            if (kDenseAddend && mirror_vec) {
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+                    held[p] = gload4(E + (long long)min(n0 + wn + j * 32 + p * 8 + (lane >> 3), args.N - 1) * args.lde +
+                                     min(m0 + wm + i * 32 + (lane & 7) * 4, args.M - 4));
+            }
             // The mirror image of the block: staged as [column][row], read back as 16 bytes along the row
             // index, stored as 128-byte runs of the mirrored rows.
 #pragma unroll
@@ -1352,7 +1388,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                 float y[4], e[4] = {0.f, 0.f, 0.f, 0.f};
                 const bool whole = mirror_vec;                  // M % 4 == 0: mcol + 3 < M
                 if (kDenseAddend) {
-                    if (whole) { const float4 x = gload4(E + (long long)mrow * args.lde + mcol); e[0] = x.x; e[1] = x.y; e[2] = x.z; e[3] = x.w; }
+                    if (whole) { e[0] = held[p].x; e[1] = held[p].y; e[2] = held[p].z; e[3] = held[p].w; }
                     else
 #pragma unroll
                         for (int q = 0; q < 4; ++q) if (mcol + q < args.M) e[q] = gload(E + (long long)mrow * args.lde + mcol + q);

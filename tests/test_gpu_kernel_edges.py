@@ -520,3 +520,21 @@ def test_chosen_rows_of_a_stack_equal_dequantize_index_and_multiply(order, block
         for got, w in ((kept, want), (weighted, want * weights[first:].unsqueeze(2)), (fused.rows_of(part, rows[first:]), want),
                        (fused.rows_of(full[first:], rows[first:]), want)):
             assert torch.equal(got.nan_to_num(7.0), w.nan_to_num(7.0)) and torch.equal(got.isnan(), w.isnan())
+
+
+@pytest.mark.parametrize("n,k,batch", [(4, 16, 3), (68, 32, 2), (132, 64, 3), (260, 256, 2), (1028, 288, 1)])
+@pytest.mark.parametrize("symmetric,known", [(True, False), (False, False), (True, True)])
+def test_products_added_to_their_own_result_buffer(X, n, k, batch, symmetric, known):
+    """The addend's elements are read ahead of the stores of the same block, at the mirrored places too: an addend that is not symmetric
+    and is the result as well, rows and columns that end inside a block.  fp32 sums of k terms: k 2^-24 |G| |G|^T bounds the
+    products' error, two roundings the rest."""
+    g = torch.Generator().manual_seed(n + k)
+    G = torch.randn(batch, n, k, generator=g).cuda()
+    E = torch.randn(batch, n, n, generator=g).cuda()
+    G64, E64 = G.double(), E.double()
+    want = 0.75 * E64 + 0.5 * (G64 @ G64.transpose(1, 2))
+    size = X.measure(G) if known else None
+    out = X.gemm(G, G, trans_b=True, addend=E, out=E, alpha=0.5, beta=0.75, symmetric=symmetric, amax=(size, size) if known else None)
+    assert out.data_ptr() == E.data_ptr()
+    bound = 2 ** -24 * (0.5 * k * (G64.abs() @ G64.abs().transpose(1, 2)) + 2 * want.abs() + 2 * E64.abs())
+    assert float(((E.double() - want).abs() - bound).max()) <= 0.0
