@@ -973,8 +973,13 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
         using LB = SplitLayout<BN>;
         // products in the order of their size, smallest first: (h, l), (l, h), (m, m), (h, m), (m, h), (h, h)
         constexpr int pa_of[6] = {0, 2, 1, 0, 1, 0}, pb_of[6] = {2, 0, 1, 1, 0, 0};
-        for (int t = 0; t < n_tiles; ++t) {
-            const int cur = t & 1;
+        // `more`: a tile follows.  The last tile is a copy of the body without commits and loads, and the loads past the end that are
+        // left repeat the last tile: behind a branch around a commit or a load the next wait is one for all loads in flight,
+        // those of the other operand that are half a tile old too.  us, 99 x 1024^3 1064 -> 1044, with the left operand stored
+        // transposed 1057 -> 1006; 99 x 512 x 128 over 1024 (a sweep's coefficients) 97 -> 87.
+        auto multiply_tile = [&](int t, auto more) {
+            constexpr bool MORE = decltype(more)::value;
+            const int cur = t & 1, ahead = k_begin + min(t + 2, n_tiles - 1) * BK;
             const unsigned char *sa = reinterpret_cast<const unsigned char *>(s_mem) + cur * SPLIT_STAGE + half * LA::kHalf + (wm + frag_row) * 16;
             const unsigned char *sb = reinterpret_cast<const unsigned char *>(s_mem) + cur * SPLIT_STAGE + SPLIT_A + half * LB::kHalf + (wn + frag_row) * 16;
             qt_bf16x8 fa[3][MI], fb[3][NI];
@@ -989,7 +994,7 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
             for (int q = 0; q < 6; ++q) {
                 if constexpr (KB >= kQuant4) {        // the turned commit of the right factor, spread over the products
                     unsigned char *next_b = reinterpret_cast<unsigned char *>(s_mem) + (cur ^ 1) * SPLIT_STAGE + SPLIT_A;
-                    if (t + 1 < n_tiles) {
+                    if constexpr (MORE) {
                         if (q == 1) lb.stage(next_b, s_code);
                         if (q == 2) lb.turn(next_b);
                         if (q == 4) lb.finish(next_b);
@@ -999,17 +1004,17 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                     // dense operands: the split of the next tile in two halves between the product groups (A, then B),
                     // each followed by its loads of the tile after
                     unsigned char *next = reinterpret_cast<unsigned char *>(s_mem) + (cur ^ 1) * SPLIT_STAGE;
-                    if (q == 2 && t + 1 < n_tiles) {
+                    if (MORE && q == 2) {
                         la.commit_split(next);
-                        if (t + 2 < n_tiles) la.fetch_fast(A + (KA == kDense ? (long long)(k_begin + (t + 2) * BK) : (long long)(k_begin + (t + 2) * BK) * args.lda));
+                        la.fetch_fast(A + (KA == kDense ? (long long)ahead : (long long)ahead * args.lda));
                     }
-                    if (q == 4 && t + 1 < n_tiles) {
+                    if (MORE && q == 4) {
                         lb.commit_split(next + SPLIT_A);
-                        if (t + 2 < n_tiles) lb.fetch_fast(B + (KB == kDenseT ? (long long)(k_begin + (t + 2) * BK) : (long long)(k_begin + (t + 2) * BK) * args.ldb));
+                        lb.fetch_fast(B + (KB == kDenseT ? (long long)ahead : (long long)ahead * args.ldb));
                     }
-                } else if (q == 3 && t + 1 < n_tiles) {
+                } else if (MORE && q == 3) {
                     commit(cur ^ 1, true);
-                    if (t + 2 < n_tiles) fetch(k_begin + (t + 2) * BK);
+                    fetch(ahead);
                 }
 #pragma unroll
                 for (int i = 0; i < MI; ++i)
@@ -1018,7 +1023,9 @@ __global__ __launch_bounds__(256, (kWavesPerSimd<BM, BN, KA, KB, EPI, PREC>)) vo
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa_of[q]][i], fb[pb_of[q]][j], acc[i][j], 0, 0, 0);
             }
             __syncthreads();
-        }
+        };
+        for (int t = 0; t + 1 < n_tiles; ++t) multiply_tile(t, std::true_type{});
+        multiply_tile(n_tiles - 1, std::false_type{});
     } else
     for (int t = 0; t < n_tiles; ++t) {
         const int cur = t & 1;
