@@ -563,7 +563,7 @@ def main():
         "pct_of_hbm_peak": round(100 * value / HBM_PEAK_GBS, 2),
         "roofline": {
             "bound": "hbm",
-            "kernel": "quantize_flat_kernel<float,4,64,false,true,true>",
+            "kernel": "quantize_flat_kernel<float,4,64,false,true>",
             "achieved": round(q_gbs, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
@@ -574,7 +574,7 @@ def main():
             "algorithmic_bytes_per_launch": int(algo),
         },
         "dequantize": {
-            "kernel": "dequantize_flat_kernel<float,4,false,true>",
+            "kernel": "dequantize_flat_kernel<float,4,0,true,128>",
             "traffic": MEASURED_TRAFFIC["dequantize"],
             "achieved": round(d_gbs, 1),
             "frac": round(d_gbs / HBM_PEAK_GBS, 4),
