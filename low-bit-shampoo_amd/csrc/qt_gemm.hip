@@ -634,10 +634,14 @@ struct LoadQuant {
     }
 };
 
-// (the 256-entry tables of the 8-bit re-encoding leave LDS for two; the half pipe's two accumulators take 128 registers)
+// (the 256-entry tables of the 8-bit re-encoding leave LDS for two; the half pipe's two accumulators take 128 registers, and its
+// 128 x 64 and 64 x 128 tiles with a quantized right factor reloaded twenty a k tile from scratch at three, each reload a wait for all
+// loads in flight: 4 and 8 bits, us, 14 x 1088 x 576 by 576 96 and 124 -> 73 and 71, 10 x 1088 x 1088 164 and 217 -> 134 and
+// 136, 3072 x 3072 313 and 480 -> 286 and 289)
 template <int BM, int BN, int KA, int KB, int EPI, int PREC>
 constexpr int kWavesPerSimd = (PREC >= kPipeSplit && BM == 128 && BN == 128 &&
-                               (KA >= kQuant4 || KB >= kQuant4 || EPI == kRequant8 || PREC == kPipeHalf)) ? 2 : 3;
+                               (KA >= kQuant4 || KB >= kQuant4 || EPI == kRequant8 || PREC == kPipeHalf)) ||
+                              (PREC == kPipeHalf && BM * BN == 128 * 64 && KB >= kQuant4) ? 2 : 3;
 template <int PREC> using KernelArgs = typename std::conditional<PREC == kPipeHalf, RangedArgs, GemmArgs>::type;
 
 template <int BM, int BN, int KA, int KB, int EPI, int PREC = kPipeF32, bool DEEP = false>
