@@ -7,13 +7,14 @@
 // 17.9 -> 12.1 us (the kernels are what is left), 1200 x 1200 17.7 -> 11.1.
 //
 // It takes plainly good calls only.  Anything else -- an argument that is not what it should be, a device that is not the current one, a
-// tensor subclass or wrapper, a torch function mode -- returns None, nothing done, and the caller's own checks say what
-// is wrong or do it the long way: there is one place that words errors.
+// tensor subclass or wrapper, a function or dispatch mode, a transformation (torch.func) or trace around the call -- returns None,
+// nothing launched, and the caller's own checks say what is wrong or do it the long way: there is one place that words errors.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
@@ -28,23 +29,37 @@ void *entry[2][2][2][2];
 int (*last_error)();
 const char *(*last_error_string)();
 
-// A tensor that is itself, in plain memory of the current GPU: no subclass, no wrapper that a transformation or mode has put
-// around it.
+using K = c10::DispatchKey;
+
+// Memory of the GPU `device` and nothing around it: no wrapper that a transformation or mode has made.
+bool in_plain_memory(const at::Tensor &t, int device) {
+    static const c10::DispatchKeySet wrapped({K::Python, K::PythonTLSSnapshot, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Functionalize,
+                                              K::Batched, K::Conjugate, K::Negative, K::ZeroTensor});
+    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(wrapped) && t.has_storage() &&
+           t.get_device() == device && t.is_contiguous();
+}
+
+// A tensor that is itself (no subclass), in plain memory of the current GPU.
 const at::Tensor *plain(PyObject *obj, int device) {
     if (!THPVariable_CheckExact(obj)) return nullptr;
     const at::Tensor &t = THPVariable_Unpack(obj);
-    using K = c10::DispatchKey;
-    static const c10::DispatchKeySet wrapped({K::Python, K::PythonTLSSnapshot, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Functionalize,
-                                              K::Batched, K::Conjugate, K::Negative, K::ZeroTensor});
-    if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.key_set().has_any(wrapped) || !t.has_storage()) return nullptr;
-    return t.get_device() == device && t.is_contiguous() ? &t : nullptr;
+    return in_plain_memory(t, device) ? &t : nullptr;
 }
 
-// A buffer of `numel` elements: nullptr where what is given does not fit; made if nothing is given.
+// Whether something is set up around the call that would see, or wrap, the tensors it makes: with plain inputs, too, what
+// at::empty returns inside a level of torch.func is a wrapper without memory of its own.
+bool watched() {
+    static const c10::DispatchKeySet levels({K::Python, K::PythonTLSSnapshot, K::PythonDispatcher, K::PreDispatch, K::Functionalize, K::Tracer,
+                                             K::FuncTorchVmapMode, K::VmapMode, K::FuncTorchDynamicLayerFrontMode,
+                                             K::FuncTorchDynamicLayerBackMode});
+    return c10::impl::tls_local_dispatch_key_set().included_.has_any(levels) || at::impl::torch_function_mode_enabled();
+}
+
+// A buffer of `numel` elements: false where what is given does not fit; made if nothing is given.
 bool buffer(PyObject *given, int device, long long numel, at::ScalarType type, const at::TensorOptions &like, at::Tensor &out) {
     if (given == Py_None) {
         out = at::empty({numel}, like.dtype(type));
-        return true;
+        return in_plain_memory(out, device);
     }
     const at::Tensor *t = plain(given, device);
     if (t == nullptr || t->scalar_type() != type || t->numel() != numel) return false;
@@ -60,11 +75,13 @@ bool whole(PyObject *obj, long long &value) {
 }
 
 struct Format { long long order, blocksize, bits, codes, maxima; int device; };
-bool format(PyObject *order, PyObject *blocksize, PyObject *bits, Format &f) {
+bool format(PyObject *data, PyObject *order, PyObject *blocksize, PyObject *bits, Format &f) {
+    // (before the device is asked for: that would start the GPU's runtime for a tensor that is not there)
+    if (!THPVariable_CheckExact(data) || !THPVariable_Unpack(data).is_cuda()) return false;
     if (!whole(order, f.order) || !whole(blocksize, f.blocksize) || !whole(bits, f.bits)) return false;
     if (f.bits != 4 && f.bits != 8) return false;
     if (f.blocksize < 64 || f.blocksize > 2048 || (f.blocksize & (f.blocksize - 1)) != 0) return false;
-    if (f.order < 1 || f.order > 46340 || at::impl::torch_function_mode_enabled()) return false;
+    if (f.order < 1 || f.order > 46340 || watched()) return false;
     f.codes = (f.order * f.order * f.bits + 7) / 8;
     f.maxima = f.order * ((f.order + f.blocksize - 1) / f.blocksize);
     f.device = c10::hip::current_device();
@@ -78,17 +95,20 @@ const at::Tensor *code_table(PyObject *obj, const Format &f) {
 
 int slot_of(at::ScalarType type) { return type == at::kFloat ? 0 : type == at::kBFloat16 ? 1 : -1; }
 
-// The launch itself, without the interpreter's lock (a full queue blocks); false with a Python error set.
+// The launch itself, without the interpreter's lock (a full queue blocks); false with a Python error set.  Addresses first:
+// asking for one may throw (a lazy copy that has to be made, memory that is not there), and nothing may between letting go
+// of the lock and taking it again.
 bool launch(void *fn, const at::Tensor &a, const at::Tensor &code, const Format &f, const at::Tensor &absmax, const at::Tensor *diag,
             const at::Tensor &out) {
     void *stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(f.device)).stream();
+    const void *from = a.data_ptr(), *table = code.data_ptr();
+    void *maxima = absmax.data_ptr(), *diagonal = diag != nullptr ? diag->data_ptr() : nullptr, *to = out.data_ptr();
+    const int order = (int)f.order, blocksize = (int)f.blocksize;
+    const bool with_diag = diag != nullptr;
     int error = 0;
     Py_BEGIN_ALLOW_THREADS
-    if (diag != nullptr)
-        reinterpret_cast<WithDiagonal>(fn)(a.data_ptr(), code.data_ptr(), (int)f.order, absmax.data_ptr(), diag->data_ptr(), out.data_ptr(),
-                                           (int)f.blocksize, stream);
-    else
-        reinterpret_cast<Plain>(fn)(a.data_ptr(), code.data_ptr(), (int)f.order, absmax.data_ptr(), out.data_ptr(), (int)f.blocksize, stream);
+    if (with_diag) reinterpret_cast<WithDiagonal>(fn)(from, table, order, maxima, diagonal, to, blocksize, stream);
+    else reinterpret_cast<Plain>(fn)(from, table, order, maxima, to, blocksize, stream);
     error = last_error();
     Py_END_ALLOW_THREADS
     if (error == 0) return true;
@@ -99,7 +119,7 @@ bool launch(void *fn, const at::Tensor &a, const at::Tensor &code, const Format 
 // quantize(A, code, order, absmax, diag, out, blocksize, bits, with_diag) -> (out, absmax[, diag]) or None
 PyObject *quantize_checked(PyObject *const *args) {
     Format f;
-    if (!format(args[2], args[6], args[7], f)) Py_RETURN_NONE;
+    if (!format(args[0], args[2], args[6], args[7], f)) Py_RETURN_NONE;
     const bool with_diag = args[8] == Py_True;
     const at::Tensor *a = plain(args[0], f.device), *code = code_table(args[1], f);
     if (a == nullptr || code == nullptr || a->numel() != f.order * f.order) Py_RETURN_NONE;
@@ -126,7 +146,7 @@ PyObject *quantize_checked(PyObject *const *args) {
 // dequantize(A, code, order, absmax, diag, outdtype, out, blocksize, bits, with_diag) -> out or None
 PyObject *dequantize_checked(PyObject *const *args) {
     Format f;
-    if (!format(args[2], args[7], args[8], f)) Py_RETURN_NONE;
+    if (!format(args[0], args[2], args[7], args[8], f)) Py_RETURN_NONE;
     const bool with_diag = args[9] == Py_True;
     const at::Tensor *a = plain(args[0], f.device), *code = code_table(args[1], f), *absmax = plain(args[3], f.device);
     if (a == nullptr || code == nullptr || absmax == nullptr) Py_RETURN_NONE;
@@ -139,6 +159,7 @@ PyObject *dequantize_checked(PyObject *const *args) {
         const at::ScalarType type = reinterpret_cast<THPDtype *>(args[5])->scalar_type;
         if (slot_of(type) < 0) Py_RETURN_NONE;
         out = at::empty({f.order, f.order}, at::TensorOptions().device(a->device()).dtype(type));
+        if (!in_plain_memory(out, f.device)) Py_RETURN_NONE;
     } else {
         const at::Tensor *t = plain(args[6], f.device);
         if (t == nullptr || t->numel() != f.order * f.order) Py_RETURN_NONE;
@@ -154,8 +175,8 @@ PyObject *dequantize_checked(PyObject *const *args) {
     return THPVariable_Wrap(std::move(out));
 }
 
-// C++ exceptions (out of memory, a failed look-up) end here: the caller's long way meets the same one and raises it in
-// torch's words.
+// C++ exceptions (out of memory, a failed look-up) end here, with the interpreter's lock held: the caller's long way meets
+// the same one and raises it in torch's words.
 template <PyObject *(*body)(PyObject *const *), Py_ssize_t COUNT>
 PyObject *guarded(PyObject *, PyObject *const *args, Py_ssize_t count) {
     if (count != COUNT || last_error == nullptr) Py_RETURN_NONE;

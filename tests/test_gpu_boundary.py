@@ -164,3 +164,54 @@ def test_native_host_side_takes_the_good_calls_and_no_others(bits, blocksize, or
         with pytest.raises(error):
             call()
     assert len(taken) == 10 and all(t is None for t in taken)
+
+
+def _inside(what, call):
+    """What `call` returns, or the error it raises, with a transformation or a dispatch mode around it."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    seen = []
+
+    def body(x):
+        try:
+            seen.append(call())
+        except RuntimeError as error:
+            seen.append(error)
+        return (x * x).sum() if what == "grad" else x * x
+
+    x = torch.ones(3, device="cuda")
+    if what == "mode":
+        class Mode(TorchDispatchMode):
+            def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+                return func(*args, **(kwargs or {}))
+        with Mode():
+            body(x)
+    elif what == "jvp":
+        torch.func.jvp(body, (x,), (x,))
+    elif what in ("vmap", "functionalize", "grad"):
+        getattr(torch.func, what)(body)(x)
+    else:
+        torch.func.vjp(body, x)
+    return seen[0]
+
+
+@pytest.mark.parametrize("what", ["grad", "vjp", "jvp", "vmap", "functionalize", "mode"])
+def test_calls_inside_a_transformation_or_mode_go_from_python(what, monkeypatch):
+    """Plain tensors in, buffers to be made: what is made there may be a wrapper without memory.  The call ends as the one
+    from Python does: the same error, the same tensors."""
+    native, code = F._direct, F.create_linear_map(True, 4, 2).cuda()
+    A = torch.randn(64, 64, device="cuda")
+    codes, absmax = F.quantize_blockwise(A, code, 64, blocksize=64, bits=4)
+    calls = (lambda: F.quantize_blockwise(A, code, 64, blocksize=64, bits=4),
+             lambda: (F.dequantize_blockwise(codes, code, 64, absmax, blocksize=64, bits=4),))
+    assert _inside(what, lambda: native.quantize(A, code, 64, None, None, None, 64, 4, False)) is None
+    assert _inside(what, lambda: native.dequantize(codes, code, 64, absmax, None, torch.float32, None, 64, 4, False)) is None
+    for call in calls:
+        got = _inside(what, call)
+        monkeypatch.setattr(F, "_direct", None)
+        want = _inside(what, call)
+        monkeypatch.setattr(F, "_direct", native)
+        if isinstance(want, RuntimeError):
+            assert isinstance(got, RuntimeError) and str(got) == str(want)
+        else:
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert what not in ("grad", "vjp", "jvp") or isinstance(want, RuntimeError)
