@@ -411,7 +411,7 @@ void qtensor_hip_power_step_batched(const float *product, float *u, float *value
  * Start: mats [batch, n, n] += ridge * top[b] on the diagonal, in place; z = (1 + p) / (2 |mats|_F), c = z^(1/p);
  * M = z mats, E = M - I, R = c (I - E / p) (the root after the first round, should that be accepted), first_root = c,
  * err (zeroed by the caller) = max |E|; fine (optional, zeroed by the caller; n a multiple of 4): raised to the fineness of
- * E and M (qtensor_gemm_fineness).  partial: scratch of batch * ceil(n / 8) doubles. */
+ * E and M (qtensor_gemm_fineness), to infinity where M, E and R are not all 16-byte aligned.  partial: scratch of batch * ceil(n / 8) doubles. */
 void qtensor_hip_newton_first_batched(float *mats, const float *top, float ridge, int p, int n, int batch, double *partial, float *M,
                                       float *E, float *R, float *first_root, float *err, float *fine, qtensor_stream_t stream);
 /* Stopping rules: new_err NULL before the first round, else max |E| after a round.  A round is accepted unless new_err > 1.2 err;

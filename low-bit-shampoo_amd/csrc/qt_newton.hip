@@ -46,6 +46,11 @@ __global__ __launch_bounds__(256) void power_step_kernel(const float *product, f
     for (int i = threadIdx.x; i < n; i += 256) at[i] = v[i] / norm;
 }
 
+// Four elements of a stack that need not begin on a 16-byte boundary (wide: it does).
+__device__ __forceinline__ float4 load_four(const float *p, bool wide) {
+    return wide ? load_f32x4<false>(p) : make_float4(p[0], p[1], p[2], p[3]);
+}
+
 // The ridge onto the diagonal, and the sum of squares of every band of rows.
 __global__ __launch_bounds__(256) void newton_norm_kernel(float *mats, const float *top, float ridge, int n, int bands, double *partial) {
     __shared__ double s_wave[4];
@@ -56,9 +61,10 @@ __global__ __launch_bounds__(256) void newton_norm_kernel(float *mats, const flo
     if ((int)threadIdx.x < rows) base[(long long)threadIdx.x * n + r0 + threadIdx.x] += add;
     __syncthreads();
     double sum = 0.0;
-    if ((n & 3) == 0 && is_aligned16(mats)) {
+    if ((n & 3) == 0) {
+        const bool wide = is_aligned16(mats);
         for (int i = threadIdx.x; i < rows * (n >> 2); i += 256) {
-            const float4 x = load_f32x4<false>(base + 4ll * i);
+            const float4 x = load_four(base + 4ll * i, wide);
             sum += ((double)x.x * x.x + (double)x.y * x.y) + ((double)x.z * x.z + (double)x.w * x.w);
         }
     } else {
@@ -70,7 +76,8 @@ __global__ __launch_bounds__(256) void newton_norm_kernel(float *mats, const flo
 
 // First iterates: M = z A with z = (1 + p) / (2 |A|), E = M - I, the candidate root of the first round c (I + w E) with
 // c = z^(1/p), w = -1/p; err = max |E|; fine (optional): raised to the fineness of E and M.  A thread takes squares of 8 rows by
-// 4 columns, so that the pieces lie inside one thread.
+// 4 columns, so that the pieces lie inside one thread.  Where M, E or R do not lie on 16-byte boundaries, nobody looks at the pieces
+// and the fineness is that of pieces of any size, infinity, as behind a product whose output does not.
 __global__ __launch_bounds__(256) void newton_first_kernel(const float *mats, const double *partial, int p, int n, int bands, float *M, float *E,
                                                            float *R, float *first_root, float *err, float *fine) {
     __shared__ double s_wave[4];
@@ -84,13 +91,14 @@ __global__ __launch_bounds__(256) void newton_first_kernel(const float *mats, co
     const long long base = (b * n + r0) * n;
     uint32_t top = 0;
     Pieces seen;
-    if ((n & 3) == 0 && is_aligned16(mats) && is_aligned16(M) && is_aligned16(E) && is_aligned16(R)) {
+    if ((n & 3) == 0 && is_aligned16(M) && is_aligned16(E) && is_aligned16(R)) {
+        const bool wide = is_aligned16(mats);
         for (int q = threadIdx.x; q < n >> 2; q += 256) {
             const int c0 = q * 4;
             Pieces seen_m;                                             // (a run of rows of each)
             float4 x[kBand];
 #pragma unroll
-            for (int r = 0; r < kBand; ++r) x[r] = load_f32x4<false>(mats + base + (long long)min(r, rows - 1) * n + c0);
+            for (int r = 0; r < kBand; ++r) x[r] = load_four(mats + base + (long long)min(r, rows - 1) * n + c0, wide);
 #pragma unroll
             for (int r = 0; r < kBand; ++r) {
                 if (r >= rows) break;
@@ -116,7 +124,8 @@ __global__ __launch_bounds__(256) void newton_first_kernel(const float *mats, co
             seen.end();
             seen.low = min(seen.low, seen_m.low);
         }
-    } else {                                                           // (no fineness: the half pipe takes orders in multiples of 32)
+    } else {
+        seen.low = 0;
         for (int i = threadIdx.x; i < rows * n; i += 256) {
             const bool diagonal = i % n == r0 + i / n;
             const float m = mats[base + i] * z, e = diagonal ? m - 1.0f : m;
