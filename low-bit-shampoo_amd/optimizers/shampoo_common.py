@@ -318,8 +318,8 @@ class _ShampooOptimizer(optim.Optimizer):
         workgroups: one chain after the other leaves the device idle.  Here the matrices of equal order are orthonormalised
         as a stack, and the stacks' chains are queued on a few streams, all of them before the host looks at the first
         one's outcome.  FIGURES
-        No update draws random numbers or looks at another one's result: it is what add_statistics does, up to the rounding of
-        products that are cut otherwise in a stack.  Only where the step would come to them: parameters from the second step
+        No update draws random numbers or looks at another one's result: it is what add_statistics does, to the bit, whichever
+        parameters have a gradient in this step (CholeskyQR(apart=True)).  Only where the step would come to them: parameters from the second step
         on, with a dense fp32 gradient on one GPU, up to the first whose gradient stops the step."""
         done, updates = [], []
         for p in group['params']:
@@ -364,7 +364,7 @@ class _ShampooOptimizer(optim.Optimizer):
                     loads[i] += stack[0][1][1].shape[stack[0][1][2]] ** 1.5    # (about what its chain takes)
                     with torch.cuda.stream(lanes[i]):
                         begun = [prec._begin(*one) for prec, one in stack]
-                        running.append((lanes[i], stack, [L for L, _ in begun], X.CholeskyQR(torch.stack([Y for _, Y in begun]))))
+                        running.append((lanes[i], stack, [L for L, _ in begun], X.CholeskyQR(torch.stack([Y for _, Y in begun]), apart=True)))
                     del begun
                 while running:
                     # the one whose outcome is there already, else the first

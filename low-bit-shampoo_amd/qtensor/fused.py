@@ -826,8 +826,11 @@ class CholeskyQR:
     library).  All calls for one object must be made with the same current stream."""
 
     def __init__(self, Y, max_rounds=12, pivot_floor=PIVOT_FLOOR, tolerance=2e-5, sweep=True, replace_first=False,
-                 remake=None, leave=()):
-        """leave: matrices of the stack (their numbers) that the caller orthonormalises some other way: whatever the
+                 remake=None, leave=(), apart=False):
+        """apart: the matrices have nothing to do with each other, and each is to come out as if it were alone in its stack: column
+        lengths summed matrix by matrix, no decision that looks at other matrices (every fourth one far, a repair that
+        leaves all of them three rounds), the library's routine on one at a time.
+        leave: matrices of the stack (their numbers) that the caller orthonormalises some other way: whatever the
         sweep makes of them is final here, they are neither tested nor polished.
         remake: optional callable, int64 GPU vector of matrix numbers -> those matrices of Y again.  With it Y is
         given up: its columns are scaled in place and it becomes the working set (one stack less held through the
@@ -837,11 +840,11 @@ class CholeskyQR:
         B, self.true_n, _ = Y.shape
         n = -(-self.true_n // 64) * 64
         self.batch, self.n, self.device, self.remake = B, n, Y.device, remake
-        self.leave = np.asarray(sorted(leave), dtype=np.int64)
+        self.leave, self.apart = np.asarray(sorted(leave), dtype=np.int64), apart
         if n != self.true_n:
             Y = self._padded(Y)
-        self.pivot_floor, self.tolerance, self.rounds_left = pivot_floor, tolerance, max_rounds
-        scale = torch.linalg.vector_norm(Y, dim=1, keepdim=True).clamp_min(1e-30)
+        self.pivot_floor, self.tolerance = pivot_floor, tolerance
+        scale = self._lengths(Y)
         if remake is not None and Y.is_contiguous():
             self.Y, self.Q = None, Y.div_(scale)
         else:
@@ -862,6 +865,8 @@ class CholeskyQR:
         self.last = None                              # (pivot flags, near, ids) of the round not yet looked at
         self.far_before = np.full(B, np.inf)          # per working-set entry: ||G - I||_F^2 at the test before this one if it was far
         self.stuck = np.zeros(B, dtype=np.int64)      # per working-set entry: rounds in a row that did not halve that distance
+        self.rounds_left = np.full(B, max_rounds)     # per working-set entry
+        self.tested = np.ones(B, dtype=bool)          # per working-set entry: the next test is of something new
         self.mended = np.zeros(B, dtype=bool)         # per working-set entry: has been through the replacing sweep
         self.stale = False                            # the Gram matrices are those of before a repair: no round on them
         self.swept = sweep
@@ -875,6 +880,11 @@ class CholeskyQR:
             if replace_first:
                 self.mended[:] = True
             self.info_host = self._to_host(self.info)
+
+    def _lengths(self, Y):
+        """[B, 1, n]: lengths of the columns.  (The order in which torch adds up depends on the number of matrices.)"""
+        parts = Y.split(1) if self.apart else (Y,)
+        return torch.cat([torch.linalg.vector_norm(part, dim=1, keepdim=True) for part in parts]).clamp_min(1e-30)
 
     def _to_host(self, t):
         """A copy of a small device tensor on its way into pinned host memory, queued on the current stream right
@@ -934,6 +944,7 @@ class CholeskyQR:
             self.gram = self.gram.index_select(0, index)
         self.ids, self.near, self.mended = self.ids[keep], self.near[keep], self.mended[keep]
         self.far_before, self.stuck = self.far_before[keep], self.stuck[keep]
+        self.rounds_left, self.tested = self.rounds_left[keep], self.tested[keep]
 
     def landed(self):
         """Whether what the host has to see next, the outcome of the sweep or of the last test, is there."""
@@ -962,8 +973,7 @@ class CholeskyQR:
         are swept again from their original columns, three passes, with every column that a pass finds dependent
         replaced by a stand-in column (block_gram_schmidt(replace_dependent=True))."""
         original = self._original(self._index(self.ids[where]))
-        scale = torch.linalg.vector_norm(original, dim=1, keepdim=True).clamp_min(1e-30)
-        again = (original / scale).contiguous()
+        again = (original / self._lengths(original)).contiguous()
         info = torch.zeros(again.shape[0], dtype=torch.int32, device=again.device)
         block_gram_schmidt(again, info, self.pivot_floor, replace_dependent=True, true_n=self.true_n)
         self.Q.index_copy_(0, self._index(where), again)
@@ -988,8 +998,7 @@ class CholeskyQR:
         with np.errstate(invalid="ignore"):
             done = far[:, 0] < self.tolerance                                   # False for NaN as well
             self.near = far[:, 1] < 0.25
-        if self.rounds_left == 0:
-            failed |= ~done
+        failed |= ~done & (self.rounds_left == 0)
         done &= ~failed
         self.redo += self.ids[failed].tolist()
         self._finish(np.nonzero(done)[0], self.Q)
@@ -1002,16 +1011,20 @@ class CholeskyQR:
             # in a row did not bring nearer than half of before -- or a stack where every fourth matrix is far (eight
             # at least) -- is of low numerical rank: rounds diverge there, the replacing sweep does not.
             away = ~self.near
-            many = away.sum() >= 8 and away.sum() * 4 > self.batch
+            many = not self.apart and away.sum() >= 8 and away.sum() * 4 > self.batch
             with np.errstate(invalid="ignore"):
                 no_nearer = away & np.isfinite(self.far_before) & ~(distance < 0.5 * self.far_before)      # (NaN and inf count)
-            self.stuck = np.where(no_nearer, self.stuck + 1, 0)
+            self.stuck = np.where(no_nearer, self.stuck + self.tested, 0)
             again = away & ~self.mended & ((self.stuck >= 2) | many)
+            self.tested = np.ones(self.ids.size, dtype=bool)
             if again.any():
                 self._repair(np.nonzero(again)[0])
                 self.mended |= again
                 self.stale = True
-                self.rounds_left = min(self.rounds_left, 3)   # what is far after the repair and three rounds goes to the library
+                if self.apart:
+                    self.tested = again                       # (the others wait: their next test finds what this one did)
+                # what is far after the repair and three rounds goes to the library
+                self.rounds_left = np.where(again if self.apart else True, np.minimum(self.rounds_left, 3), self.rounds_left)
             self.far_before = np.where(away, distance, np.inf)
         return self.finished
 
@@ -1048,7 +1061,8 @@ class CholeskyQR:
         if self.redo:
             redo = torch.tensor(sorted(set(self.redo)), device=self.device)
             torch.cuda.synchronize()              # the library routine is not trusted to be stream-ordered here
-            self.final[redo] = _householder_qr(self._original(redo))[0]
+            for some in redo.split(1 if self.apart else len(redo)):
+                self.final[some] = _householder_qr(self._original(some))[0]
             torch.cuda.synchronize()
         Q = self.final
         if Q.shape[1] != self.true_n:

@@ -814,3 +814,34 @@ def test_statistics_taken_together_are_those_taken_one_by_one(monkeypatch, stack
             if x.bits < 16:
                 assert float((x.absmax - y.absmax).norm() / y.absmax.norm()) <= 1e-3
         assert float((a - b).abs().max()) <= 1e-4 * 5e-2                       # five steps of 1e-2
+
+
+@pytest.mark.parametrize("stack_bytes", [256 << 20, 4 * 4 * 130 * 130])
+def test_statistics_of_a_parameter_do_not_depend_on_its_neighbours(monkeypatch, stack_bytes):
+    """fused=False: ten statistics of order 130 and three of order 288 and of low rank, for which the orthonormalisation has to decide (stand-in
+    columns, another sweep), beside others of full rank: in stacks, whole or cut small, the bits of the state and of the
+    parameters are those of the parameters taken one by one, also where neighbours have no gradient."""
+    from optimizers import shampoo2, shampoo_common
+    monkeypatch.setattr(shampoo_common._ShampooOptimizer, "STACK_BYTES", stack_bytes)
+    shapes = [(130, 30)] * 10 + [(288, 72)] * 3 + [(130, 130), (64, 288), (200, 64)]
+    gen = torch.Generator().manual_seed(7)
+    start = [0.1 * torch.randn(s, generator=gen) for s in shapes]
+    grads = [[torch.randn(s, generator=gen) for s in shapes] for _ in range(5)]
+    together = shampoo_common._ShampooOptimizer._statistics_together
+    made = []
+    for alone in (False, True):
+        monkeypatch.setattr(shampoo_common._ShampooOptimizer, "_statistics_together", (lambda self, group: ()) if alone else together)
+        torch.manual_seed(3)                                                  # the roots' start vectors
+        params = [torch.nn.Parameter(t.cuda()) for t in start]
+        opt = shampoo2.ShampooAdamW(params, lr=1e-2, start_prec_step=1, stat_compute_steps=1, prec_compute_steps=2, prec_maxorder=1200,
+                                    prec_bits=4, quan_blocksize=64, min_lowbit_size=4096)
+        for step, gs in enumerate(grads):
+            for i, (p, g) in enumerate(zip(params, gs)):
+                p.grad = None if i in (0, 3, 4, 11)[:step] else g.cuda()
+            opt.step()
+        made.append((params, opt))
+    for pa, pb in zip(made[0][0], made[1][0]):
+        assert torch.equal(pa, pb)
+        for x, y in zip(*[opt.state[p]["preconditioner"].statistics for (_, opt), p in zip(made, (pa, pb))]):
+            for name in ("Svalue", "keep_indices", "max_eigenvalue", "var") + (("absmax",) if x.bits < 16 else ()):
+                assert torch.equal(getattr(x, name), getattr(y, name)), (tuple(pa.shape), name)
