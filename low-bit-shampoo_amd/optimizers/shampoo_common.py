@@ -382,6 +382,9 @@ class _ShampooOptimizer(optim.Optimizer):
                         Q, _ = solver.result()
                         for (prec, one), L, V in zip(stack, statistics, Q):
                             prec._finish(one[0], L, V)
+                            for t in vars(one[0]).values():                    # made on the lane, read and let go on this stream
+                                if isinstance(t, torch.Tensor):
+                                    t.record_stream(main)
         finally:
             for lane in lanes:
                 main.wait_stream(lane)

@@ -845,3 +845,47 @@ def test_statistics_of_a_parameter_do_not_depend_on_its_neighbours(monkeypatch, 
         for x, y in zip(*[opt.state[p]["preconditioner"].statistics for (_, opt), p in zip(made, (pa, pb))]):
             for name in ("Svalue", "keep_indices", "max_eigenvalue", "var") + (("absmax",) if x.bits < 16 else ()):
                 assert torch.equal(getattr(x, name), getattr(y, name)), (tuple(pa.shape), name)
+
+
+def test_state_made_on_a_side_stream_outlives_what_the_callers_stream_reads():
+    """fused=False: an optimizer that is let go while its stream still has work to do.  Its statistics were made on the shared
+    side streams, and another optimizer's step must not be handed their memory there before that work is through."""
+    import bisect
+    import gc
+    from optimizers import shampoo2
+    from optimizers.engine import shared_stream
+    device = torch.device("cuda", torch.cuda.current_device())
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    params = [torch.nn.Parameter(torch.randn(96, 96, device="cuda", generator=gen)) for _ in range(6)]
+    opt = shampoo2.ShampooSGD(params, lr=1e-3, start_prec_step=1, stat_compute_steps=1, prec_compute_steps=10 ** 6, prec_bits=4,
+                              quan_blocksize=64, min_lowbit_size=4096)
+    for _ in range(3):
+        for p in params:
+            p.grad = torch.randn(96, 96, device="cuda", generator=gen)
+        opt.step()
+    held = []
+    for p in params:
+        for holder in opt.state[p]["preconditioner"].statistics:
+            held += [(t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()) for t in
+                     (holder.var, holder.absmax, holder.Svalue, holder.keep_indices, holder.max_eigenvalue)]
+    del holder
+    a = torch.randn(8192, 8192, device="cuda", generator=gen)
+    b, done = torch.empty_like(a), torch.cuda.Event()
+    torch.cuda.synchronize()
+    for _ in range(100):
+        torch.mm(a, a, out=b)
+    done.record()
+    del opt, params, p
+    gc.collect()                                         # (an optimizer is in a cycle with its hooks)
+    reused, made = 0, []
+    for lane in range(3):
+        with torch.cuda.stream(shared_stream(device, lane)):
+            reserved = torch.cuda.memory_reserved()
+            while torch.cuda.memory_reserved() == reserved:          # everything that the lane's pool has to give
+                made += [torch.empty(512, dtype=torch.uint8, device="cuda") for _ in range(1000)]
+    still_busy = not done.query()
+    at = sorted(t.data_ptr() for t in made)
+    for low, high in held:
+        i = bisect.bisect_left(at, low - 511)
+        reused += i < len(at) and at[i] < high
+    assert still_busy and reused == 0
