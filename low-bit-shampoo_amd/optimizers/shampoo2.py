@@ -22,7 +22,6 @@ class Preconditioner(PreconditionerBase):
 
     inv_root_mode 0: inverse root from the stored eigenpairs (QTensorSVDFast.computepower);
     inv_root_mode 1: coupled Newton iteration on the dequantized statistic."""
-    statistics_in_stacks = True
 
     def __init__(self, var, name2qmap, stat_decay=0.95, matrix_eps=1e-6, prec_maxorder=1200,
                  prec_bits=32, min_lowbit_size=4096, quan_blocksize=64, rect_t1=1, rect_t2=4, inv_root_mode=0):
@@ -45,6 +44,18 @@ class Preconditioner(PreconditionerBase):
         stat, basis = holder.dequantize()
         decay_and_add_gram(stat, block, axis, w1, w2)
         holder.quantize(stat, basis)
+
+    def statistics_in_stacks(self):
+        # (not where a subclass, a holder of another kind or a wrapped method has its own way of doing a part of it)
+        def own(method, function):
+            return getattr(method, "__func__", None) is function
+
+        def plain(holder):
+            return (type(holder) is QTensorSVDFast and own(holder.quantize, QTensorSVDFast.quantize)
+                    and (holder.var.dtype if holder.bits >= 16 else holder.var_dtype) == torch.float32)
+
+        return (own(self.add_statistics, PreconditionerBase.add_statistics) and own(self._accumulate, Preconditioner._accumulate)
+                and all(plain(h) for h in self.statistics))
 
     def _begin(self, holder, block, axis, w1, w2):
         stat, basis = holder.dequantize()

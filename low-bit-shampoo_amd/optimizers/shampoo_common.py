@@ -141,10 +141,12 @@ class PreconditionerBase:
             for axis in range(rank):
                 self._accumulate(self.statistics[j * rank + axis], block, axis, w1, w2)
 
-    # Whether the update of a statistic is a long chain of launches that the optimizers queue for many of them together
-    # (_ShampooOptimizer._statistics_together), and its two ends, around the orthonormalisation that is done in stacks:
-    # _begin(holder, block, axis, w1, w2) -> (statistic, matrix to orthonormalise) and _finish(holder, statistic, Q).
-    statistics_in_stacks = False
+    def statistics_in_stacks(self):
+        """Whether the update of a statistic is a long chain of launches that the optimizers may queue for many of them together
+        (_ShampooOptimizer._statistics_together) instead of calling add_statistics.  Its two ends then are, around the orthonormalisation
+        that is done in stacks, _begin(holder, block, axis, w1, w2) -> (statistic, matrix to orthonormalise) and
+        _finish(holder, statistic, Q)."""
+        return False
 
     def statistics_updates(self, grad):
         """add_statistics as its independent pieces: [arguments of _accumulate], one per statistic."""
@@ -329,11 +331,10 @@ class _ShampooOptimizer(optim.Optimizer):
                 break
             state = self.state.get(p)
             prec = state.get('preconditioner') if state else None
-            if (prec is None or not prec.statistics_in_stacks or not prec.statistics
-                    or type(prec).add_statistics is not PreconditionerBase.add_statistics
+            if (not isinstance(prec, PreconditionerBase) or not prec.statistics
+                    or (state['step'] + 1) % group['stat_compute_steps'] != 0 or not prec.statistics_in_stacks()
                     or not p.grad.is_cuda or p.grad.dtype != torch.float32 or (done and p.grad.device != done[0].grad.device)
-                    or any(h.var.device != p.grad.device for h in prec.statistics)
-                    or (state['step'] + 1) % group['stat_compute_steps'] != 0):
+                    or any(h.var.device != p.grad.device for h in prec.statistics)):
                 continue
             done.append(p)
             updates += [(prec, one) for one in prec.statistics_updates(p.grad.data)]

@@ -889,3 +889,50 @@ def test_state_made_on_a_side_stream_outlives_what_the_callers_stream_reads():
         i = bisect.bisect_left(at, low - 511)
         reused += i < len(at) and at[i] < high
     assert still_busy and reused == 0
+
+
+@pytest.mark.parametrize("what", ["accumulate", "add_statistics", "holder", "wrapped", "none"])
+def test_an_own_way_of_taking_statistics_is_taken(what, monkeypatch):
+    """fused=False: a preconditioner class with its own _accumulate or add_statistics, one with holders of its own, an object whose
+    method has been wrapped: each is called for every statistic (two parameters of two sides, three steps); "none": the stacks are."""
+    from optimizers import shampoo2
+    from qtensor.utils import QTensorSVDFast
+    calls = []
+
+    class Holder(QTensorSVDFast):
+        def quantize(self, var, Vt=None):
+            calls.append("holder")
+            super().quantize(var, Vt)
+
+    class Prec(shampoo2.Preconditioner):
+        if what == "accumulate":
+            def _accumulate(self, *args):
+                calls.append(what)
+                super()._accumulate(*args)
+        if what == "add_statistics":
+            def add_statistics(self, grad):
+                calls.extend([what] * 2)
+                super().add_statistics(grad)
+        if what == "holder":
+            def _new_statistic(self, order, device, index, rank, quant_args, extra):
+                return Holder(self.matrix_eps * torch.eye(order, device=device), rect_t1=extra["rect_t1"], rect_t2=extra["rect_t2"], **quant_args)
+
+    class Optimizer(shampoo2.ShampooSGD):
+        preconditioner_class = Prec
+
+    params = [torch.nn.Parameter(torch.randn(96, 96, device="cuda")) for _ in range(2)]
+    opt = Optimizer(params, lr=1e-3, start_prec_step=1, stat_compute_steps=1, prec_compute_steps=10 ** 6, prec_bits=4, quan_blocksize=64,
+                    min_lowbit_size=4096)
+    for step in range(3):
+        for p in params:
+            p.grad = torch.randn(96, 96, device="cuda")
+        opt.step()
+        if what == "wrapped" and step == 0:
+            calls.extend([what] * 4)
+            for p in params:
+                prec = opt.state[p]["preconditioner"]
+                plain = prec._accumulate
+                prec._accumulate = lambda *args, plain=plain: (calls.append(what), plain(*args))
+    assert calls == ([] if what == "none" else [what] * 12)
+    taken = [s for p in params for s in [opt.state[p]["preconditioner"].statistics_in_stacks()]]
+    assert taken == [what == "none"] * 2
