@@ -114,6 +114,8 @@ def PowerIterBatched(mats, error_tolerance=1e-6, num_iters=10, v0=None):
         v = torch.rand(B, n, device=mats.device) * 2 - 1
     else:
         v = v0.to(mats.device).expand(B, n).clone()
+        if v.dtype in (torch.bfloat16, torch.float16):
+            v = v.float()
     if X.on_matrix_cores(mats) and mats.is_contiguous():            # the library's kernels: two launches a round
         return X.power_iteration(mats, v.contiguous(), error_tolerance, num_iters)
     value = torch.zeros(B, device=mats.device)

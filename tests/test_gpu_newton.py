@@ -233,3 +233,17 @@ def test_a_stack_that_is_not_aligned_is_measured_like_one_that_is(n, monkeypatch
     pieces += [m.abs().view(2, n // 8, 8, n).amax(dim=2) for m in plain[:2]]
     low = torch.stack([torch.where(p > 0, p, torch.inf).amin(dim=(1, 2)) for p in pieces]).amin(dim=0)
     assert torch.equal(plain[5], 1.0 / low) and bool(torch.isinf(odd[5]).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float64])
+def test_start_vectors_of_other_types(dtype):
+    """16-bit start vectors, one for all matrices or one each, are taken as the fp32 ones they are; others are not."""
+    mats, v0 = psd_stack(3, 128, 1.0, seed=1)
+    mats = mats.cuda()
+    for v in (v0.to(dtype), v0[0].to(dtype)):
+        if dtype == torch.float64:
+            with pytest.raises(ValueError):
+                PowerIterBatched(mats, v0=v)
+            continue
+        assert torch.equal(PowerIterBatched(mats, v0=v), PowerIterBatched(mats, v0=v.float()))
+        assert torch.equal(ComputePowerBatched(mats.clone(), 4, v0=v), ComputePowerBatched(mats.clone(), 4, v0=v.float()))
