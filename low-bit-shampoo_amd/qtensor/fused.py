@@ -627,6 +627,9 @@ def rows_of(stack, rows: Tensor, weights: Optional[Tensor] = None):
     if src.shape[0] != batch or rows.dtype != torch.int64 or (quantized and stack.diag is not None) or (
             weights is not None and (weights.shape != rows.shape or weights.dtype != torch.float32)):
         raise ValueError("rows_of takes int64 rows and fp32 weights [batch, count] of a stack without exact diagonal")
+    if (not quantized and (src.dtype != torch.float32 or src.shape != (batch, n, n))) or any(
+            t is not None and not (t.is_cuda and t.device == src.device) for t in (rows, weights, src)):
+        raise ValueError("rows_of takes a stack of square fp32 matrices, its rows and weights on one GPU")
     if F.lib is None or n % 4 or batch > 65535 or not src.is_contiguous() or src.data_ptr() % (4 if quantized else 16):
         # (an order whose rows do not begin with whole, aligned fours)
         out = torch.gather(load_stack(stack) if quantized else src, 1, rows.unsqueeze(2).expand(-1, -1, n))

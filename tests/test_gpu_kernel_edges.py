@@ -538,3 +538,16 @@ def test_products_added_to_their_own_result_buffer(X, n, k, batch, symmetric, kn
     assert out.data_ptr() == E.data_ptr()
     bound = 2 ** -24 * (0.5 * k * (G64.abs() @ G64.abs().transpose(1, 2)) + 2 * want.abs() + 2 * E64.abs())
     assert float(((E.double() - want).abs() - bound).max()) <= 0.0
+
+
+def test_rows_of_a_stack_that_is_not_one_of_fp32_matrices_are_refused():
+    """Before anything is launched: the kernel reads four bytes an element and takes every address for one of the GPU."""
+    from qtensor import fused
+    stack, rows = torch.randn(2, 64, 64, device="cuda"), torch.zeros(2, 3, dtype=torch.int64, device="cuda")
+    weights = torch.ones(2, 3, device="cuda")
+    assert torch.equal(fused.rows_of(stack, rows), stack[:, :1].expand(-1, 3, -1))
+    for bad, r, w in ((stack.bfloat16(), rows, None), (stack.double(), rows, None), (stack[:, :32].contiguous(), rows, None),
+                      (stack.cpu(), rows, None), (stack, rows.cpu(), None), (stack, rows.int(), None), (stack, rows, weights.cpu()),
+                      (stack, rows, weights.double()), (stack, rows[:1], None)):
+        with pytest.raises(ValueError):
+            fused.rows_of(bad, r, w)
