@@ -472,9 +472,12 @@ void launch_flat(const T *A, const float *code, uint32_t order, uint32_t batch, 
     const uint32_t blocks_needed = (n_steps + kWaves - 1) / kWaves;
     // Inputs far beyond the 256 MB last-level cache are read with the streaming hint, by the fewest workgroups that keep the
     // loads coming.  Below that 4-bit codes do better with five: us with three, four, five, fp32 with its diagonal 3072 x
-    // 3072 14.1 13.2 13.2, 4096 x 4096 19.4 19.4 18.6, bf16 4096 x 4096 14.2 14.1 13.0; 8 bits, bf16 4096 x 4096 15.9 16.3 17.7.
-    const bool streams = total >= (1u << 25);
-    const int grid = grid_for(blocks_needed, BITS == 4 && !streams ? 5 : kFlatBlocksPerCU);
+    // 3072 13.7 12.8 12.8, 4096 x 4096 19.2 19.4 18.4, bf16 4096 x 4096 15.3 14.6 13.5; 8 bits, bf16 4096 x 4096 15.9 16.3 17.7.  Not
+    // where a segment is several vectors of a wave, whose registers leave room for four, and a fifth comes after them: fp32 in
+    // segments of 512 3072 x 3072 12.3 12.2 14.8, 4096 x 4096 17.9 17.8 19.0, of 2048 4096 x 4096 16.6 16.7 18.1; bf16 4096 x 4096 in
+    // segments of 1024 12.0 12.1 11.3, of 2048 11.7 11.8 14.3.
+    const bool streams = total >= (1u << 25), five_fit = BS <= (sizeof(T) == 4 ? 256 : 1024);
+    const int grid = grid_for(blocks_needed, BITS == 4 && !streams && five_fit ? 5 : kFlatBlocksPerCU);
     if (streams)
         hipLaunchKernelGGL((quantize_flat_kernel<T, BITS, BS, DIAG, true>), dim3(grid), dim3(kFlatThreads), 0, stream,
                            A, code, n_steps, rd, od, absmax, diag, out);
@@ -535,10 +538,14 @@ void quantize_dispatch(const T *A, const float *code, int order_i, float *absmax
     }
     // Small inputs are bound by latency: the general kernel, which takes eight elements a thread and not thirty-two, and in 4 bits
     // searches instead of setting up a bucket table, is the faster one.  us, flat and general, one matrix: 4 bits fp32 with its
-    // diagonal 256 x 256 8.3 and 4.6, 1024 x 1024 7.6 and 5.0, 2048 x 2048 8.1 and 7.6, 2560 x 2560 10.7 and 9.3, 4096 x 4096 19.4
-    // and 21.3; bf16 2560 x 2560 9.2 and 8.8, 3072 x 3072 10.3 and 11.5; 8 bits bf16 256 x 256 6.8 and 5.5, 1024 x 1024 7.1 and 6.0,
-    // 1280 x 1280 7.2 and 7.0 (fp32 6.7 and 6.7), 2048 x 2048 7.9 and 9.2.
-    if ((uint64_t)order * order * batch < (BITS == 4 ? 7u << 20 : 3u << 19)) flat = false;
+    // diagonal 256 x 256 8.3 and 4.6, 1024 x 1024 7.6 and 5.0, 2048 x 2048 8.1 and 7.6, 2560 x 2560 9.3 and 8.8, 4096 x 4096 18.4
+    // and 20.4; bf16 2560 x 2560 9.2 and 8.8, 3072 x 3072 10.3 and 11.5; 8 bits bf16 256 x 256 6.8 and 5.5, 1024 x 1024 7.1 and 6.0,
+    // 1280 x 1280 7.2 and 7.0 (fp32 6.7 and 6.7), 2048 x 2048 7.9 and 9.2.  Segments of more than 512 it takes in rounds one
+    // after the other, and reads twice: 4 bits 1024 x 1024 in segments of 1024 5.8 and 5.3, 2048 x 2048 6.9 and 7.1 (with its diagonal
+    // 7.2 and 7.4, bf16 6.9 and 7.2), in segments of 2048 6.5 and 8.8; 8 bits 1024 x 1024 in segments of 1024 5.6 and 6.5.
+    const bool long_segments = bs > 512;
+    const uint32_t flat_from = BITS == 4 ? (long_segments ? 2u << 20 : 7u << 20) : long_segments ? 0u : 3u << 19;
+    if ((uint64_t)order * order * batch < flat_from) flat = false;
     if (flat) {
         switch (blocksize) {
             case 64: launch_flat<T, BITS, 64, DIAG>(A, code, order, (uint32_t)batch, absmax, diag, out, stream); break;
