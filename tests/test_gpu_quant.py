@@ -148,13 +148,52 @@ def test_general_path_ragged_and_odd_orders(F, code_maps, order, bits, bs):
 
 
 def test_large_flat_path_uses_bucket_table(F, code_maps):
-    """>= 2^20 elements switches the quantizer to its bucket-table kernel."""
+    """Segments of 64 and 256, 4 bits on the general kernel still, 8 bits on the flat one with its bucket table."""
     for bits, bs, name in ((4, 64, "linear-2"), (8, 256, "dynamic"), (8, 64, "linear-2"), (4, 256, "dynamic")):
         order = 1536
         A = special_matrix(order, seed=bits + bs)
         for diag in (False, True):
             run_case(F, A, code_maps[(name, bits)], order, bs, bits, diag, "fp32")
     run_case(F, special_matrix(2048, 5), code_maps[("linear-2", 4)], 2048, 64, 4, True, "bf16")
+
+
+# the smallest orders that go to the flat quantizer
+FLAT_ORDERS = {(4, 64): 2752, (4, 128): 2816, (4, 256): 2816, (4, 512): 3072, (4, 1024): 2048, (4, 2048): 2048,
+               (8, 64): 1280, (8, 128): 1280, (8, 256): 1280, (8, 512): 1536, (8, 1024): 1024, (8, 2048): 2048}
+
+
+@pytest.mark.parametrize("bits,bs", CELLS)
+@pytest.mark.parametrize("diag", [False, True])
+def test_flat_quantizer_where_it_is_the_one_that_runs(F, code_maps, bits, bs, diag):
+    """Every segment length at the first order that is the flat kernel's, and one order below it that is the general one's where
+    there is one: segments whose maximum is zero, tiny, denormal, huge, infinite or NaN beside ordinary ones of the same wave, in
+    whole rows and in the one segment of a row alone."""
+    order = FLAT_ORDERS[bits, bs]
+    A = special_matrix(order, seed=bits + bs)
+    for i, value in enumerate((0.0, 1e-41, 1e-30, 1e30, np.inf, np.nan, -np.inf)):
+        A[20 + i, -bs:] = F32(value)                       # a whole segment of it (-bs: the row's last)
+        A[30 + i, -bs // 2] = F32(value)                   # and one element
+    run_case(F, A, code_maps[("linear-2", bits)], order, bs, bits, diag, "fp32")
+    run_case(F, A, code_maps[("dynamic", bits)], order, bs, bits, diag, "bf16")
+    if order - bs >= bs:
+        run_case(F, A[:order - bs, bs:].copy(), code_maps[("linear-2", bits)], order - bs, bs, bits, diag, "bf16")
+
+
+@pytest.mark.parametrize("bits,bs,diag,dtype", [(4, 512, False, "fp32"), (4, 2048, True, "bf16"), (8, 1024, True, "fp32"), (4, 128, False, "bf16")])
+def test_flat_quantizer_past_the_caches(F, code_maps, bits, bs, diag, dtype):
+    """From 2^25 elements on the loads stream."""
+    run_case(F, special_matrix(6144, seed=bs), code_maps[("linear-2", bits)], 6144, bs, bits, diag, dtype)
+
+
+@pytest.mark.parametrize("bits,order", [(4, 2752), (8, 1280)])
+def test_flat_quantizer_with_unusual_tables(F, code_maps, bits, order):
+    """Not ascending, and with thresholds crowded next to zero, where every element takes the exact route."""
+    rng = np.random.default_rng(12)
+    crowded = np.sort(np.concatenate([F32(10.0) ** -np.arange(2, 2 + 2 ** bits // 2, dtype=F32).clip(max=36), np.linspace(-1, 1, 2 ** bits // 2, dtype=F32)]))
+    A = special_matrix(order, seed=order)
+    A[10, :64] = np.array([1e-13, -1e-13, 3e-14, 1.0] * 16, F32)
+    for table in (code_maps[("dynamic", bits)][rng.permutation(2 ** bits)], crowded.astype(F32)):
+        run_case(F, A, table, order, 64, bits, bits == 8, "fp32")
 
 
 def test_unsorted_and_unusual_tables(F, code_maps):
