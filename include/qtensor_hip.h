@@ -445,7 +445,8 @@ void qtensor_hip_newton_result_batched(const float *r0, const float *r1, const i
  * that owns chunk c; a tensor of n elements owns ceil(n / qtensor_hip_tail_chunk()) consecutive
  * chunks starting at first_chunk.  partial: device scratch of 2 * n_chunks floats (only used when
  * graft != 0).  Rows with flags bit 0 set get dir rescaled to the norm of grad (dir itself is not
- * written); the others use dir as it is.  All tensors fp32. */
+ * written); the others use dir as it is.  Bit 1 (of all rows or none): the buffers are read and written past the caches, for
+ * tables of more than they hold.  All tensors fp32. */
 typedef struct {
     float *param;
     const float *dir;           /* preconditioned gradient, or the gradient itself            */
@@ -454,7 +455,7 @@ typedef struct {
     float *v;                   /* AdamW: exp_avg_sq; SGD: unused                             */
     long long n;
     long long first_chunk;
-    long long flags;            /* bit 0: graft                                               */
+    long long flags;            /* bit 0: graft, bit 1: stream                                */
 } qtensor_tail_tensor;
 int qtensor_hip_tail_chunk(void);
 void qtensor_hip_adamw_tail(const qtensor_tail_tensor *table, const int *chunk_tensor, int n_chunks, float *partial, int graft,

@@ -20,7 +20,7 @@ struct TailTensor {            // one row of the device table: 8 x 64 bit
     float *v;                  // AdamW: exp_avg_sq, SGD: unused
     long long n;               // elements
     long long first_chunk;     // index of this tensor's first chunk
-    long long flags;           // bit 0: rescale dir to the norm of grad
+    long long flags;           // bit 0: rescale dir to the norm of grad; bit 1: stream past the caches
 };
 
 namespace {
@@ -57,12 +57,7 @@ __device__ __forceinline__ float block_sum(float x, float *s_part) {
 
 // partial[2c] = sum grad^2, partial[2c+1] = sum dir^2 over chunk c (rows without graft: untouched)
 template <bool STREAM>
-__global__ __launch_bounds__(kThreads) void tail_norms_kernel(const TailTensor *table, const int *chunk_tensor,
-                                                              float *partial) {
-    __shared__ float s_part[4];
-    const int c = blockIdx.x;
-    const TailTensor t = table[chunk_tensor[c]];
-    if (!(t.flags & 1)) return;
+__device__ __forceinline__ void norms_of_chunk(const TailTensor &t, int c, float *partial, float *s_part) {
     const long long start = ((long long)c - t.first_chunk) * kChunk;
     const long long left = t.n - start;
     const int len = left < kChunk ? (int)left : kChunk;
@@ -85,6 +80,15 @@ __global__ __launch_bounds__(kThreads) void tail_norms_kernel(const TailTensor *
     sg = block_sum(sg, s_part);
     sd = block_sum(sd, s_part);
     if (threadIdx.x == 0) { s1(partial + 2 * c, sg); s1(partial + 2 * c + 1, sd); }
+}
+
+__global__ __launch_bounds__(kThreads) void tail_norms_kernel(const TailTensor *table, const int *chunk_tensor,
+                                                              float *partial) {
+    __shared__ float s_part[4];
+    const TailTensor t = table[chunk_tensor[blockIdx.x]];
+    if (!(t.flags & 1)) return;
+    if (t.flags & 2) norms_of_chunk<true>(t, blockIdx.x, partial, s_part);
+    else norms_of_chunk<false>(t, blockIdx.x, partial, s_part);
 }
 
 // |grad| / (|dir| + 1e-12) of the tensor that owns this chunk, summed in an order of its own number of chunks alone (the same
@@ -140,16 +144,12 @@ struct Sgd {
 };
 
 // A thread's first elements are on their way while the scale is summed up, the next ones while it works on the ones before.
-// STREAM: every buffer is touched once a step and all of them are more than the last-level cache holds.  Bound by memory: AdamW
-// over the 87.4 M elements of a ViT-B/32 460 -> 422 us, 5.8 TB/s.
+// STREAM: every buffer is touched once a step, and the buffers of a step are more than the last-level cache holds.  Whether they are
+// is in the table (bit 1 of a row's flags, the same in all), whose writer knows how many elements there are: from 2^24 on, of
+// which they (20 to 28 bytes each) no longer fit its 256 MB.  The number of chunks does not say: a thousand small tensors have as
+// many.  Bound by memory: AdamW over the 87.4 M elements of a ViT-B/32 460 -> 422 us, 5.8 TB/s.
 template <typename RULE, bool HAS_V, bool STREAM>
-__global__ __launch_bounds__(kThreads) void tail_update_kernel(const TailTensor *table, const int *chunk_tensor,
-                                                               const float *partial, const RULE launch_rule) {
-    __shared__ float s_scale;
-    const int c = blockIdx.x;
-    const TailTensor t = table[chunk_tensor[c]];
-    RULE rule = launch_rule;
-    rule.bind(chunk_tensor[c]);
+__device__ __forceinline__ void update_chunk(const TailTensor &t, int c, const float *partial, const RULE &rule, float *s_scale) {
     const bool graft = (t.flags & 1) != 0;
     const long long start = ((long long)c - t.first_chunk) * kChunk;
     const long long left = t.n - start;
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(kThreads) void tail_update_kernel(const TailTensor 
         int i = threadIdx.x * 4;
         Four x = {}, y = {};
         if (i < whole) x = load(i);
-        const float scale = graft_scale(t, partial, &s_scale);
+        const float scale = graft_scale(t, partial, s_scale);
         for (; i < whole; i += kThreads * 4) {
             if (i + kThreads * 4 < whole) y = load(i + kThreads * 4);
             if (graft) { x.d.x *= scale; x.d.y *= scale; x.d.z *= scale; x.d.w *= scale; }
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kThreads) void tail_update_kernel(const TailTensor 
             if (HAS_V) s1(v + e, V);
         }
     } else {
-        const float scale = graft_scale(t, partial, &s_scale);
+        const float scale = graft_scale(t, partial, s_scale);
         for (int e = threadIdx.x; e < len; e += kThreads) {
             float P = g1(p + e), M = g1(m + e), V = HAS_V ? g1(v + e) : 0.f, D = g1(d + e);
             if (graft) D *= scale;
@@ -204,19 +204,15 @@ __global__ __launch_bounds__(kThreads) void tail_update_kernel(const TailTensor 
     }
 }
 
-// Streaming hints from 2^24 elements on, of which the buffers of a step (20 to 28 bytes each) no longer fit the 256 MB
-// last-level cache.
-constexpr int kStreamChunks = (1 << 24) / kChunk;
-void launch_norms(const TailTensor *table, const int *chunk_tensor, int n_chunks, float *partial, hipStream_t stream) {
-    if (n_chunks >= kStreamChunks) hipLaunchKernelGGL(tail_norms_kernel<true>, dim3(n_chunks), dim3(kThreads), 0, stream, table, chunk_tensor, partial);
-    else hipLaunchKernelGGL(tail_norms_kernel<false>, dim3(n_chunks), dim3(kThreads), 0, stream, table, chunk_tensor, partial);
-}
 template <typename RULE, bool HAS_V>
-void launch_update(const TailTensor *table, const int *chunk_tensor, int n_chunks, const float *partial, const RULE &rule, hipStream_t stream) {
-    if (n_chunks >= kStreamChunks)
-        hipLaunchKernelGGL((tail_update_kernel<RULE, HAS_V, true>), dim3(n_chunks), dim3(kThreads), 0, stream, table, chunk_tensor, partial, rule);
-    else
-        hipLaunchKernelGGL((tail_update_kernel<RULE, HAS_V, false>), dim3(n_chunks), dim3(kThreads), 0, stream, table, chunk_tensor, partial, rule);
+__global__ __launch_bounds__(kThreads) void tail_update_kernel(const TailTensor *table, const int *chunk_tensor,
+                                                               const float *partial, const RULE launch_rule) {
+    __shared__ float s_scale;
+    const TailTensor t = table[chunk_tensor[blockIdx.x]];
+    RULE rule = launch_rule;
+    rule.bind(chunk_tensor[blockIdx.x]);
+    if (t.flags & 2) update_chunk<RULE, HAS_V, true>(t, blockIdx.x, partial, rule, &s_scale);
+    else update_chunk<RULE, HAS_V, false>(t, blockIdx.x, partial, rule, &s_scale);
 }
 
 bool tail_args_ok(const void *table, const void *chunk_tensor, int n_chunks, const void *partial, int graft, const char *what) {
@@ -240,7 +236,7 @@ void adamw_tail(const void *table, const int *chunk_tensor, int n_chunks, float 
     if (n_chunks == 0) return;
     const TailTensor *tab = static_cast<const TailTensor *>(table);
     if (graft) {
-        launch_norms(tab, chunk_tensor, n_chunks, partial, (hipStream_t)stream);
+        hipLaunchKernelGGL(tail_norms_kernel, dim3(n_chunks), dim3(kThreads), 0, (hipStream_t)stream, tab, chunk_tensor, partial);
         if (!launch_ok("adamw_tail (norms)")) return;
     }
     AdamW rule;
@@ -253,7 +249,8 @@ void adamw_tail(const void *table, const int *chunk_tensor, int n_chunks, float 
     rule.eps = (float)eps;
     rule.neg_step = row_corrections != nullptr ? 0.0f : (float)(-lr / (1.0 - pow(beta1, (double)step)));
     rule.row_corrections = row_corrections;
-    launch_update<AdamW, true>(tab, chunk_tensor, n_chunks, partial, rule, (hipStream_t)stream);
+    hipLaunchKernelGGL((tail_update_kernel<AdamW, true>), dim3(n_chunks), dim3(kThreads), 0, (hipStream_t)stream, tab,
+                       chunk_tensor, partial, rule);
     launch_ok("adamw_tail");
 }
 }  // namespace
@@ -284,7 +281,7 @@ extern "C" void qtensor_hip_sgd_tail(const void *table, const int *chunk_tensor,
     if (n_chunks == 0) return;
     const TailTensor *tab = static_cast<const TailTensor *>(table);
     if (graft) {
-        launch_norms(tab, chunk_tensor, n_chunks, partial, (hipStream_t)stream);
+        hipLaunchKernelGGL(tail_norms_kernel, dim3(n_chunks), dim3(kThreads), 0, (hipStream_t)stream, tab, chunk_tensor, partial);
         if (!launch_ok("sgd_tail (norms)")) return;
     }
     Sgd rule;
@@ -292,6 +289,7 @@ extern "C" void qtensor_hip_sgd_tail(const void *table, const int *chunk_tensor,
     rule.weight_decay = (float)weight_decay;
     rule.neg_lr = (float)(-lr);
     rule.nesterov = nesterov != 0;
-    launch_update<Sgd, false>(tab, chunk_tensor, n_chunks, partial, rule, (hipStream_t)stream);
+    hipLaunchKernelGGL((tail_update_kernel<Sgd, false>), dim3(n_chunks), dim3(kThreads), 0, (hipStream_t)stream, tab,
+                       chunk_tensor, partial, rule);
     launch_ok("sgd_tail");
 }

@@ -29,6 +29,8 @@ class TailPlan:
     """Device-side table of (param, direction, grad, moment buffers) rows and the chunk map the
     kernels walk.  Rebuilt only when a buffer has moved."""
 
+    STREAM_FROM = 1 << 24            # elements in all whose buffers (20 to 28 bytes each) no longer fit the 256 MB last-level cache
+
     def __init__(self):
         if F.lib is None:
             raise RuntimeError("libqtensor_hip.so is not available")
@@ -44,6 +46,7 @@ class TailPlan:
         if key == self.key:
             return
         rows, owner, first = [], [], 0
+        streams = 2 if sum(p.numel() for p in params) >= self.STREAM_FROM else 0
         for i, (p, d, g, a, b, f) in enumerate(zip(params, dirs, grads, m, v, graft)):
             tensors = [p, d, a] + ([g] if f else []) + ([] if b is None else [b])
             for t in tensors:
@@ -51,7 +54,7 @@ class TailPlan:
                     raise ValueError("the fused update takes contiguous fp32 GPU tensors of equal size per parameter")
             chunks = -(-p.numel() // self.chunk)
             rows.append([p.data_ptr(), d.data_ptr(), g.data_ptr() if f else 0, a.data_ptr(), 0 if b is None else b.data_ptr(),
-                         p.numel(), first, 1 if f else 0])
+                         p.numel(), first, (1 if f else 0) | streams])
             owner += [i] * chunks
             first += chunks
         dev = params[0].device

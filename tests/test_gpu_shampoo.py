@@ -451,3 +451,23 @@ def test_fused_update_of_large_tensors_and_odd_ends(sizes, kind):
             want = P - 1e-2 * M
         assert float((m[i].double() - M).norm() / M.norm()) <= 1e-5
         assert float((p.double() - want).norm()) <= 1e-5 * float((want - P).norm()) + 2.0 ** -23 * float(P.norm())
+
+
+@pytest.mark.parametrize("sizes", [[301] * 1100, [(1 << 24) - 5, 7], [(1 << 24) - 8, 7]])
+def test_fused_update_streams_by_the_number_of_elements(sizes):
+    """A thousand small tensors stay in the caches; the first size that does not, and the last one that does.  Bits do not depend
+    on it: each tensor's update is the one that it gets alone."""
+    from optimizers.tail import TailPlan
+    gen = torch.Generator(device="cuda").manual_seed(5)
+
+    def make(scale):
+        return [scale * torch.randn(n, device="cuda", generator=gen) for n in sizes]
+
+    params, dirs, grads, m, v = make(1.0), make(3.0), make(0.1), make(0.1), [t.abs() for t in make(0.01)]
+    alone = [[t.clone() for t in ts[-2:]] for ts in (params, m, v)]
+    plan = TailPlan()
+    plan.adamw(params, dirs, grads, m, v, [True] * len(sizes), 1e-2, (0.9, 0.999), 1e-8, 0.05, 3)
+    assert plan.table[:, 7].tolist() == [3 if sum(sizes) >= 1 << 24 else 1] * len(sizes)
+    for i in range(2):
+        TailPlan().adamw([alone[0][i]], [dirs[-2 + i]], [grads[-2 + i]], [alone[1][i]], [alone[2][i]], [True], 1e-2, (0.9, 0.999), 1e-8, 0.05, 3)
+        assert all(torch.equal(a[i], ts[-2 + i]) for a, ts in zip(alone, (params, m, v)))
