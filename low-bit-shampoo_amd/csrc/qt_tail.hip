@@ -104,8 +104,9 @@ __device__ __forceinline__ float graft_scale(const TailTensor &t, const float *p
             sg += (double)g1(at);
             sd += (double)g1(at + 1);
         }
+        if (chunks > 1)                                          // (a small tensor's are on lane 0)
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) { sg += __shfl_xor(sg, off, 64); sd += __shfl_xor(sd, off, 64); }
+            for (int off = 32; off > 0; off >>= 1) { sg += __shfl_xor(sg, off, 64); sd += __shfl_xor(sd, off, 64); }
         if (threadIdx.x == 0) {
             const float gn = (float)sqrt(sg), dn = (float)sqrt(sd);
             *s_scale = gn / (dn + 1e-12f);
