@@ -21,14 +21,27 @@ for src in "${here}"/qt_*.hip; do
   "${HIPCC}" "${FLAGS[@]}" "$@" -c "${src}" -o "${o}" &
   pids+=($!)
 done
-# (beside the library that it is bound to: none for a library built somewhere else)
+# Beside the library that it is bound to (none for a library built somewhere else), and from scratch: what is there may be of
+# another torch.  The library does without it, so it is no reason not to link the library.
+build_direct() {
+  local to="${here}/../qtensor/_direct.so" where
+  rm -f "${to}"
+  where="$("${PYTHON:-python3}" -c 'import os, sysconfig, torch; print(os.path.dirname(torch.__file__), sysconfig.get_paths()["include"], torch.__version__, sep="\n")')" || return 1
+  mapfile -t where <<< "${where}"
+  "${CXX:-g++}" -O2 -std=c++17 -shared -fPIC -Wall -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -DQT_TORCH_VERSION="\"${where[2]}\"" \
+    -I"${where[0]}/include" -I"${where[0]}/include/torch/csrc/api/include" -I"${HIP_PATH:-/opt/rocm}/include" -I"${where[1]}" \
+    "${here}/direct_call.cpp" -o "${obj}/_direct.so" \
+    -L"${where[0]}/lib" -lc10 -lc10_hip -ltorch_cpu -ltorch_hip -ltorch -ltorch_python -Wl,-rpath,"${where[0]}/lib" || return 1
+  mv "${obj}/_direct.so" "${to}"
+}
+direct=""
 if [[ -z "${QT_OUT:-}" ]]; then
-  mapfile -t where < <(python3 -c 'import os, sysconfig, torch; print(os.path.dirname(torch.__file__)); print(sysconfig.get_paths()["include"])')
-  g++ -O2 -std=c++17 -shared -fPIC -Wall -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -I"${where[0]}/include" -I"${where[0]}/include/torch/csrc/api/include" \
-    -I"${HIP_PATH:-/opt/rocm}/include" -I"${where[1]}" "${here}/direct_call.cpp" -o "${here}/../qtensor/_direct.so" \
-    -L"${where[0]}/lib" -lc10 -lc10_hip -ltorch_cpu -ltorch_hip -ltorch -ltorch_python -Wl,-rpath,"${where[0]}/lib" &
-  pids+=($!)
+  build_direct &
+  direct=$!
 fi
 for p in "${pids[@]}"; do wait "${p}"; done
 "${HIPCC}" --offload-arch=gfx950 -shared -fPIC "${objs[@]}" -o "${out}"
 echo "built ${out}"
+if [[ -n "${direct}" ]] && ! wait "${direct}"; then
+  echo "warning: qtensor/_direct.so was not built; quantize and dequantize calls have their host side in Python" >&2
+fi

@@ -223,4 +223,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_direct", "one quantize or dequant
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__direct() { return PyModule_Create(&module); }
+// torch_version: what this was compiled against.  It reads torch's objects as they lie in memory, which no other torch promises.
+PyMODINIT_FUNC PyInit__direct() {
+    PyObject *made = PyModule_Create(&module);
+    if (made != nullptr && PyModule_AddStringConstant(made, "torch_version", QT_TORCH_VERSION) != 0) {
+        Py_DECREF(made);
+        return nullptr;
+    }
+    return made;
+}

@@ -71,10 +71,15 @@ if lib is not None:
     _STREAM_FN = _bind_stream_variants()
 
     # the same calls with their host side in native code (csrc/direct_call.cpp): what it does not take goes the way below
+    def _of_this_torch(module):
+        """The module, or None (the same launches from Python) if it was compiled against another torch than this one."""
+        return module if getattr(module, "torch_version", None) == str(torch.__version__) else None
+
     try:
         from qtensor import _direct
     except ImportError:
-        _direct = None                              # not built: the same launches from Python
+        _direct = None                              # not built
+    _direct = _of_this_torch(_direct)
     if _direct is not None:
         _direct.bind([ct.cast(fn, ct.c_void_p).value for fn in
                       [_STREAM_FN[(kind, bits, slot, diag)] for kind in ("quantize", "dequantize") for bits in (4, 8)

@@ -180,3 +180,49 @@ def test_offsets_into_the_largest_quantized_matrices(tmp_path, bits):
         for row, col in ((0, 0), (1, 0), (order // 2, 16), (order - 1, 0), (order - 1, order - 8)):
             out = subprocess.run([str(program)] + [str(x) for x in (row, col, order, shift)], capture_output=True, text=True, check=True).stdout
             assert [int(x) for x in out.split()] == [(row * order + col) * bits // 8, 4 * row * (order >> shift)], (order, row, col)
+
+
+def test_native_host_side_is_of_this_torch(built_library):
+    """The module reads torch's objects as they lie in memory: one compiled against another torch is not used."""
+    import types
+    import qtensor.functional as F
+    assert F._direct is not None and F._direct.torch_version == str(torch.__version__)
+    assert F._of_this_torch(F._direct) is F._direct
+    assert F._of_this_torch(types.SimpleNamespace(torch_version="2.9.0+rocm7.0")) is None
+    assert F._of_this_torch(types.SimpleNamespace()) is None and F._of_this_torch(None) is None
+
+
+@pytest.mark.parametrize("missing", ["torch", "compiler", "hipcc"])
+def test_build_does_without_the_native_host_side(tmp_path, missing):
+    """build.sh on a copy of the sources with stand-ins for the compilers: without torch for its python or with a host compiler that
+    fails the library is linked all the same, and what an earlier build left of the module is gone; a device
+    compiler that fails ends the build."""
+    import os
+    import shutil
+    csrc, qtensor = tmp_path / "pkg" / "csrc", tmp_path / "pkg" / "qtensor"
+    csrc.mkdir(parents=True), qtensor.mkdir()
+    shutil.copy(ROOT / "low-bit-shampoo_amd" / "csrc" / "build.sh", csrc)
+    for name in ("qt_one.hip", "qt_two.hip", "direct_call.cpp"):
+        (csrc / name).touch()
+    (qtensor / "_direct.so").write_text("an earlier build's")
+
+    def stand_in(name, body):
+        path = tmp_path / name
+        path.write_text("#!/usr/bin/env bash\n" + body)
+        path.chmod(0o755)
+        return str(path)
+
+    make_output = 'while [[ $# -gt 0 ]]; do if [[ $1 == -o ]]; then echo made > "$2"; fi; shift; done\n'
+    env = dict(os.environ, HIPCC=stand_in("hipcc", "exit 1\n" if missing == "hipcc" else make_output),
+               CXX=stand_in("cxx", "exit 1\n" if missing == "compiler" else make_output),
+               PYTHON=stand_in("python", "exit 1\n" if missing == "torch" else "printf '/torch\\n/include\\n1.0\\n'\n"))
+    env.pop("QT_OUT", None), env.pop("QT_OBJ", None)
+    done = subprocess.run(["bash", str(csrc / "build.sh")], env=env, capture_output=True, text=True, timeout=60)
+    if missing == "hipcc":
+        assert done.returncode != 0 and not (qtensor / "libqtensor_hip.so").exists()
+        return
+    assert done.returncode == 0 and (qtensor / "libqtensor_hip.so").read_text() == "made\n"
+    assert not (qtensor / "_direct.so").exists() and "_direct.so was not built" in done.stderr
+    env["CXX"], env["PYTHON"] = stand_in("cxx2", make_output), stand_in("python2", "printf '/torch\\n/include\\n1.0\\n'\n")
+    assert subprocess.run(["bash", str(csrc / "build.sh")], env=env, timeout=60).returncode == 0
+    assert (qtensor / "_direct.so").read_text() == "made\n"
