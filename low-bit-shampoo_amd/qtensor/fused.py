@@ -886,8 +886,12 @@ class CholeskyQR:
 
     def _lengths(self, Y):
         """[B, 1, n]: lengths of the columns.  (The order in which torch adds up depends on the number of matrices.)"""
-        parts = Y.split(1) if self.apart else (Y,)
-        return torch.cat([torch.linalg.vector_norm(part, dim=1, keepdim=True) for part in parts]).clamp_min(1e-30)
+        if not self.apart or Y.shape[0] == 1:
+            return torch.linalg.vector_norm(Y, dim=1, keepdim=True).clamp_min(1e-30)
+        out = torch.empty(Y.shape[0], 1, Y.shape[2], device=Y.device)
+        for one, length in zip(Y.split(1), out.split(1)):
+            torch.linalg.vector_norm(one, dim=1, keepdim=True, out=length)
+        return out.clamp_min_(1e-30)
 
     def _to_host(self, t):
         """A copy of a small device tensor on its way into pinned host memory, queued on the current stream right
