@@ -62,8 +62,8 @@ class Preconditioner(PreconditionerBase):
         decay_and_add_gram(stat, block, axis, w1, w2)
         return holder.power_step(stat, basis)
 
-    def _finish(self, holder, stat, Q):
-        holder.adopt_basis(stat, Q)
+    def _finish(self, holder, stat, Q, into):
+        holder.adopt_basis(stat, Q, into=into)
 
     def _inverse_root(self, holder, exp, eps):
         if self.inv_root_mode == 0:

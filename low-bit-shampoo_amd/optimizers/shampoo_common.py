@@ -145,7 +145,7 @@ class PreconditionerBase:
         """Whether the update of a statistic is a long chain of launches that the optimizers may queue for many of them together
         (_ShampooOptimizer._statistics_together) instead of calling add_statistics.  Its two ends then are, around the orthonormalisation
         that is done in stacks, _begin(holder, block, axis, w1, w2) -> (statistic, matrix to orthonormalise) and
-        _finish(holder, statistic, Q)."""
+        _finish(holder, statistic, Q, what holder.room() returned on the caller's stream)."""
         return False
 
     def statistics_updates(self, grad):
@@ -363,13 +363,16 @@ class _ShampooOptimizer(optim.Optimizer):
                     size += self._stack_bytes(stack)
                     i = loads.index(min(loads))
                     loads[i] += stack[0][1][1].shape[stack[0][1][2]] ** 1.5    # (about what its chain takes)
+                    # (memory of this stream, which reads what the holders keep and lets go of it: the lane waits for all that
+                    # this stream has been given so far, and this stream for the lane)
+                    room = [one[0].room() for _, one in stack]
                     with torch.cuda.stream(lanes[i]):
                         begun = [prec._begin(*one) for prec, one in stack]
-                        running.append((lanes[i], stack, [L for L, _ in begun], X.CholeskyQR(torch.stack([Y for _, Y in begun]), apart=True)))
+                        running.append((lanes[i], stack, room, [L for L, _ in begun], X.CholeskyQR(torch.stack([Y for _, Y in begun]), apart=True)))
                     del begun
                 while running:
                     # the one whose outcome is there already, else the first
-                    lane, stack, statistics, solver = running.pop(next((i for i, r in enumerate(running) if r[3].landed()), 0))
+                    lane, stack, room, statistics, solver = running.pop(next((i for i, r in enumerate(running) if r[-1].landed()), 0))
                     with torch.cuda.stream(lane):
                         if solver.swept:
                             solver.check()
@@ -378,14 +381,11 @@ class _ShampooOptimizer(optim.Optimizer):
                             if not solver.finished:
                                 solver.check()
                         if not solver.finished:
-                            running.append((lane, stack, statistics, solver))
+                            running.append((lane, stack, room, statistics, solver))
                             continue
                         Q, _ = solver.result()
-                        for (prec, one), L, V in zip(stack, statistics, Q):
-                            prec._finish(one[0], L, V)
-                            for t in vars(one[0]).values():                    # made on the lane, read and let go on this stream
-                                if isinstance(t, torch.Tensor):
-                                    t.record_stream(main)
+                        for (prec, one), into, L, V in zip(stack, room, statistics, Q):
+                            prec._finish(one[0], L, V, into)
         finally:
             for lane in lanes:
                 main.wait_stream(lane)

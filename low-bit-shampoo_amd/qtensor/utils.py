@@ -226,21 +226,30 @@ class QTensorSVDFast(_LowBitState):
         L = var.float()
         return L, fused.gemm(L, Vt, trans_b=True)
 
-    def adopt_basis(self, L, V, dtype=torch.float32):
-        """The rest of `quantize` behind the orthonormalisation: the Rayleigh quotients diag(V^T (L V)) without the product."""
-        from qtensor import fused
-        self._adopt(V, (V * fused.gemm(L, V.contiguous())).sum(dim=0), dtype)
+    def room(self):
+        """What `adopt_basis` makes anew: a caller who runs it on another stream than the one that uses the holder has the current
+        one own the memory."""
+        n, device = self.var_order if self.bits < 16 else self.var.shape[0], self.var.device
+        return (torch.empty(n, device=device), torch.empty(n, device=device, dtype=torch.int64), torch.empty((), device=device),
+                torch.empty_like(self.var) if self.bits >= 16 else None)
 
-    def _adopt(self, V, quotients, dtype):
+    def adopt_basis(self, L, V, dtype=torch.float32, into=None):
+        """The rest of `quantize` behind the orthonormalisation: the Rayleigh quotients diag(V^T (L V)) without the product.
+        into: what `room` returned, for fp32 statistics."""
+        from qtensor import fused
+        self._adopt(V, (V * fused.gemm(L, V.contiguous())).sum(dim=0), dtype, into)
+
+    def _adopt(self, V, quotients, dtype, into=None):
         keep = max(1, quotients.numel() // 2)
-        ascending, where = torch.sort(quotients)
+        values, places, top, basis = (None,) * 4 if into is None else into
+        ascending, where = torch.sort(quotients) if into is None else torch.sort(quotients, out=(values, places))
         self.keep_indices = where[:keep].to(dtype=torch.int64)
         self.Svalue = ascending[:keep].to(dtype)
         dropped = ascending[keep:].to(dtype)
-        self.max_eigenvalue = quotients.max().to(dtype)
+        self.max_eigenvalue = (quotients.max() if into is None else torch.max(quotients, out=top)).to(dtype)
 
         if self.bits >= 16:
-            self.var = V.T.contiguous()
+            self.var = V.T.contiguous() if into is None else basis.copy_(V.T)
         elif V.is_cuda and V.dtype == torch.float32 and V.is_contiguous() and self.var_order % self.blocksize == 0:
             # the quantizer reads V as it lies and writes the codes of V.T (no transposed copy)
             from qtensor import fused
