@@ -310,7 +310,8 @@ class _ShampooOptimizer(optim.Optimizer):
         return self.preconditioner_class(p, self.name2qmap, **kwargs)
 
     LANES = 3                        # streams that the stacks of statistics are dealt out to
-    STACK_BYTES = 256 << 20          # of the matrices that are orthonormalised at a time (the update holds about five times this)
+    STACK_BYTES = 256 << 20          # of the matrices that are orthonormalised at a time (the update holds about five times this);
+                                     # less on an optimizer that has little room, 1 for a matrix at a time
 
     def _statistics_together(self, group):
         """This step's statistics of a group's parameters, ahead of everything else the step does; returns the parameters whose
@@ -319,7 +320,7 @@ class _ShampooOptimizer(optim.Optimizer):
         The update of one statistic is a chain of up to three hundred dependent launches on one matrix, each of a few
         workgroups: one chain after the other leaves the device idle.  Here the matrices of equal order are orthonormalised
         as a stack, and the stacks' chains are queued on a few streams, all of them before the host looks at the first
-        one's outcome.  Ten convolution and head weights (width 32, blocks of 1200): 31.3 -> 14.8 ms a step.
+        one's outcome.  Ten convolution and head weights (width 32, blocks of 1200): 31.2 -> 15.0 ms a step.
         No update draws random numbers or looks at another one's result: it is what add_statistics does, to the bit, whichever
         parameters have a gradient in this step (CholeskyQR(apart=True)).  Only where the step would come to them: parameters from the second step
         on, with a dense fp32 gradient on one GPU, up to the first whose gradient stops the step."""
