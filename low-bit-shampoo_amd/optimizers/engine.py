@@ -525,6 +525,10 @@ class ShampooBank:
     def state_dict(self):
         return {"active": torch.tensor(self.active), **self._tensors()}
 
+    @staticmethod
+    def check_saved(sd):
+        """ValueError for what no bank can have written, before anything of it is taken."""
+
     def load_state_dict(self, sd):
         active = sd["active"]
         if torch.is_tensor(active) and active.dim() == 1:

@@ -509,7 +509,17 @@ class ShampooBank2(ShampooBank):
                              for row, state in sorted(table.items())], dtype=torch.int64).reshape(-1, 4)
         return {**super().state_dict(), "low_rank": low_rank, "low_rank_rows": rows}
 
+    @staticmethod
+    def check_saved(sd):
+        """ValueError for kept rows that their basis does not have: the kernel that reads rows makes NaN of those."""
+        for name, keep in sd.items():
+            if name.startswith("basis.") and name.endswith(".keep"):
+                order = int(name.split(".")[1])
+                if bool(((keep < 0) | (keep >= order)).any()):
+                    raise ValueError(f"checkpoint holds row numbers that a basis of order {order} does not have")
+
     def load_state_dict(self, sd):
+        self.check_saved(sd)
         super().load_state_dict(sd)
         if "low_rank" in sd:
             self.low_rank = {int(o): [bool(flag), int(count)] for o, flag, count in sd["low_rank"].tolist()}

@@ -82,6 +82,9 @@ class _FusedStep:
         if banks is not None and any(b for b in banks) and not self._fused:
             raise ValueError("this checkpoint was written by an optimizer with fused=True (it carries 'shampoo_bank'); "
                              "load it into an optimizer constructed with fused=True")
+        for saved in banks or []:
+            if saved:
+                self.bank_class().check_saved(saved)
         super().load_state_dict(state_dict)
         if banks is not None:
             self.__dict__.pop('_fused_cache', None)          # rebuilt, then filled, by the next step

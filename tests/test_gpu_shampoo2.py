@@ -936,3 +936,23 @@ def test_an_own_way_of_taking_statistics_is_taken(what, monkeypatch):
     assert calls == ([] if what == "none" else [what] * 12)
     taken = [s for p in params for s in [opt.state[p]["preconditioner"].statistics_in_stacks()]]
     assert taken == [what == "none"] * 2
+
+
+@pytest.mark.parametrize("row", [-1, 96])
+def test_a_checkpoint_with_rows_that_no_basis_has_is_refused(row):
+    """Kept rows outside their basis: refused when the checkpoint is loaded, and nothing of it is taken."""
+    from optimizers import shampoo2
+    params = [torch.nn.Parameter(torch.randn(96, 64, device="cuda")) for _ in range(2)]
+    opt = shampoo2.ShampooSGD(params, lr=1e-3, start_prec_step=1, stat_compute_steps=1, prec_compute_steps=1, prec_bits=4, quan_blocksize=64,
+                              min_lowbit_size=4096, fused=True)
+    for p in params:
+        p.grad = torch.randn(96, 64, device="cuda")
+    opt.step()
+    saved = opt.state_dict()
+    bank = {k: v.clone() if torch.is_tensor(v) else v for k, v in saved["shampoo_bank"][0].items()}
+    held = {k: v.clone() for k, v in opt.state_dict()["shampoo_bank"][0].items() if torch.is_tensor(v)}
+    bank["basis.96.keep"][1, 5] = row
+    bank["basis.96.absmax"] += 1.0
+    with pytest.raises(ValueError):
+        opt.load_state_dict({**saved, "shampoo_bank": [bank]})
+    assert all(torch.equal(v, held[k]) for k, v in opt.state_dict()["shampoo_bank"][0].items() if torch.is_tensor(v))
