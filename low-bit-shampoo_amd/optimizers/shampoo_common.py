@@ -322,8 +322,9 @@ class _ShampooOptimizer(optim.Optimizer):
         as a stack, and the stacks' chains are queued on a few streams, all of them before the host looks at the first
         one's outcome.  Ten convolution and head weights (width 32, blocks of 1200): 31.2 -> 15.0 ms a step.
         No update draws random numbers or looks at another one's result: it is what add_statistics does, to the bit, whichever
-        parameters have a gradient in this step (CholeskyQR(apart=True)).  Only where the step would come to them: parameters from the second step
-        on, with a dense fp32 gradient on one GPU, up to the first whose gradient stops the step."""
+        parameters have a gradient in this step (CholeskyQR(apart=True)).  Only where the step would come to them:
+        parameters from the second step on, with a dense fp32 gradient on one GPU, up to the first whose gradient
+        stops the step."""
         done, updates = [], []
         for p in group['params']:
             if p.grad is None:
@@ -369,7 +370,8 @@ class _ShampooOptimizer(optim.Optimizer):
                     room = [one[0].room() for _, one in stack]
                     with torch.cuda.stream(lanes[i]):
                         begun = [prec._begin(*one) for prec, one in stack]
-                        running.append((lanes[i], stack, room, [L for L, _ in begun], X.CholeskyQR(torch.stack([Y for _, Y in begun]), apart=True)))
+                        solver = X.CholeskyQR(torch.stack([Y for _, Y in begun]), apart=True)
+                    running.append((lanes[i], stack, room, [L for L, _ in begun], solver))
                     del begun
                 while running:
                     # the one whose outcome is there already, else the first
