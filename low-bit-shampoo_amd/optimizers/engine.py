@@ -529,7 +529,10 @@ class ShampooBank:
     def check_saved(sd):
         """ValueError for what no bank can have written, before anything of it is taken."""
 
-    def load_state_dict(self, sd):
+    def load_state_dict(self, sd, checked=False):
+        """checked: the caller has been through check_saved."""
+        if not checked:
+            self.check_saved(sd)
         active = sd["active"]
         if torch.is_tensor(active) and active.dim() == 1:
             self.active = [bool(a) for a in active.tolist()]

@@ -511,16 +511,15 @@ class ShampooBank2(ShampooBank):
 
     @staticmethod
     def check_saved(sd):
-        """ValueError for kept rows that their basis does not have: the kernel that reads rows makes NaN of those."""
-        for name, keep in sd.items():
-            if name.startswith("basis.") and name.endswith(".keep"):
-                order = int(name.split(".")[1])
-                if bool(((keep < 0) | (keep >= order)).any()):
-                    raise ValueError(f"checkpoint holds row numbers that a basis of order {order} does not have")
+        """ValueError for kept rows that their basis does not have: the kernel that reads rows makes NaN of those.  (One read by
+        the host for all orders.)"""
+        keeps = {int(name.split(".")[1]): t for name, t in sd.items() if name.startswith("basis.") and name.endswith(".keep")}
+        outside = [torch.div(t, order, rounding_mode="floor").any() for order, t in keeps.items()]
+        if outside and bool(torch.stack(outside).any()):
+            raise ValueError("checkpoint holds row numbers that a basis of its order does not have")
 
-    def load_state_dict(self, sd):
-        self.check_saved(sd)
-        super().load_state_dict(sd)
+    def load_state_dict(self, sd, checked=False):
+        super().load_state_dict(sd, checked)
         if "low_rank" in sd:
             self.low_rank = {int(o): [bool(flag), int(count)] for o, flag, count in sd["low_rank"].tolist()}
         if "low_rank_rows" in sd:

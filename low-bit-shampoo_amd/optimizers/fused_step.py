@@ -110,7 +110,7 @@ def _entry_for(opt, group, group_index):
             table = torch.tensor(bank.block_table(), dtype=torch.int64)
             if 'block_table' not in saved or not torch.equal(saved['block_table'].cpu(), table):
                 raise ValueError("checkpoint was written for other parameter shapes or block sizes")
-            bank.load_state_dict(saved)
+            bank.load_state_dict(saved, checked=True)
         pending[group_index] = None
     return entry
 
