@@ -531,8 +531,6 @@ class ShampooBank:
 
     def load_state_dict(self, sd, checked=False):
         """checked: the caller has been through check_saved."""
-        if not checked:
-            self.check_saved(sd)
         active = sd["active"]
         if torch.is_tensor(active) and active.dim() == 1:
             self.active = [bool(a) for a in active.tolist()]

@@ -519,7 +519,9 @@ class ShampooBank2(ShampooBank):
             raise ValueError("checkpoint holds row numbers that a basis of its order does not have")
 
     def load_state_dict(self, sd, checked=False):
-        super().load_state_dict(sd, checked)
+        if not checked:
+            self.check_saved(sd)
+        super().load_state_dict(sd)
         if "low_rank" in sd:
             self.low_rank = {int(o): [bool(flag), int(count)] for o, flag, count in sd["low_rank"].tolist()}
         if "low_rank_rows" in sd:
